@@ -65,6 +65,8 @@ SIGNATURES = {
     "fmoe_seg_off_from_host_counts": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
     "fmoe_topk_softmax_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
                                       c_int, c_void_p]),
+    "fmoe_naive_gate_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
+                                    c_void_p, c_int, c_void_p]),
     "fmoe_topk_softmax_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                       c_int32, c_int, c_void_p]),
     "fmoe_scatter_tokens": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64,

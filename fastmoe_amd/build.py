@@ -113,11 +113,12 @@ EXT_HASH_MARKER = "fmoe-ext:"
 
 
 def ext_source_hash() -> str:
-    """Digest of what the extension is compiled from: its source and the C ABI header."""
+    """Digest of what the extension is compiled from: its sources and the C ABI header."""
     import hashlib
 
     h = hashlib.sha256()
-    for path in (EXT_SRC, os.path.join(PKG_DIR, "..", "include", "fmoe_hip.h")):
+    for path in (EXT_SRC, os.path.join(CSRC, "moe_layer.h"),
+                 os.path.join(PKG_DIR, "..", "include", "fmoe_hip.h")):
         with open(path, "rb") as f:
             h.update(f.read() + b"\0")
     return h.hexdigest()[:12]

@@ -531,6 +531,12 @@ Tensor gelu_bwd(Tensor dy, Tensor x, OptTensor n_rows_dev) {
   return dx;
 }
 
+}  // namespace
+
+#include "moe_layer.h"   // the whole layer as one native autograd node
+
+namespace {
+
 void set_gemm_path(int64_t path) { check(fmoe_set_gemm_path((int)path), "set_gemm_path"); }
 
 }  // namespace
@@ -576,6 +582,10 @@ PYBIND11_MODULE(fmoe_cuda, m) {
   m.def("topk_softmax_bwd", &topk_softmax_bwd);
   m.def("gelu_fwd", &gelu_fwd, py::arg("x"), py::arg("n_rows_dev") = py::none());
   m.def("gelu_bwd", &gelu_bwd, py::arg("dy"), py::arg("x"), py::arg("n_rows_dev") = py::none());
+  m.def("expert_layer", &expert_layer, py::arg("x"), py::arg("gate_idx"), py::arg("score"),
+        py::arg("w1"), py::arg("b1"), py::arg("w2"), py::arg("b2"));
+  m.def("gated_layer", &gated_layer, py::arg("x"), py::arg("gate_weight"), py::arg("gate_bias"),
+        py::arg("w1"), py::arg("b1"), py::arg("w2"), py::arg("b2"), py::arg("top_k"));
   m.def("set_gemm_path", &set_gemm_path);
   m.def("_seg_off_from_counts",
         [](Tensor expert_count, py::object device) {

@@ -11,6 +11,8 @@
 // lanes keeps the k best of its share as a sorted list and the rounds pop the
 // overall winners.  The arrays are a few hundred KiB at most: the kernels are
 // bound by launch latency and instruction count, not by memory.
+#include <algorithm>
+
 #include "common.h"
 
 namespace fmoe {
@@ -33,8 +35,9 @@ __device__ __forceinline__ bool better(A v, int e, A w, int f) {
 template <typename T, int KMAX, int LANES>
 __global__ __launch_bounds__(kGateThreads) void topk_softmax_fwd_kernel(
     const T* __restrict__ logits, int64_t n_tokens, int n_expert, int top_k,
-    int64_t* __restrict__ idx, T* __restrict__ score) {
+    int64_t* __restrict__ idx, T* __restrict__ score, float* __restrict__ zero_loss) {
   using acc_t = typename Elem<T>::acc_t;
+  if (zero_loss && blockIdx.x == 0 && threadIdx.x == 0) *zero_loss = 0.f;
   const int g = threadIdx.x % LANES;
   const int64_t t = (int64_t)blockIdx.x * (kGateThreads / LANES) + threadIdx.x / LANES;
   const bool live = t < n_tokens;
@@ -138,8 +141,9 @@ __global__ __launch_bounds__(kGateThreads) void topk_softmax_fwd_kernel(
 template <typename T, int LANES, int C>
 __global__ __launch_bounds__(kGateThreads) void topk_softmax_fwd_flat_kernel(
     const T* __restrict__ logits, int64_t n_tokens, int n_expert, int top_k,
-    int64_t* __restrict__ idx, T* __restrict__ score) {
+    int64_t* __restrict__ idx, T* __restrict__ score, float* __restrict__ zero_loss) {
   using acc_t = typename Elem<T>::acc_t;
+  if (zero_loss && blockIdx.x == 0 && threadIdx.x == 0) *zero_loss = 0.f;
   constexpr int KMAX = FMOE_MAX_GATE_TOP_K;
   static_assert(C <= 32, "one bit per register in the alive mask");
   const int g = threadIdx.x % LANES;
@@ -244,13 +248,13 @@ __global__ __launch_bounds__(kGateThreads) void topk_softmax_bwd_kernel(
 
 template <typename T, int KMAX>
 static int launch_fwd(const void* logits, int64_t n_tokens, int n_expert, int top_k,
-                      int64_t* idx, void* score, hipStream_t s) {
+                      int64_t* idx, void* score, float* zero_loss, hipStream_t s) {
   const T* in = (const T*)logits;
   T* out = (T*)score;
 #define FMOE_GATE_FLAT(LANES, C)                                                              \
   hipLaunchKernelGGL((topk_softmax_fwd_flat_kernel<T, LANES, C>),                             \
-                     dim3(ceil_div(n_tokens, kGateThreads / LANES)), dim3(kGateThreads), 0, s, \
-                     in, n_tokens, n_expert, top_k, idx, out)
+                     dim3(std::max(1, ceil_div(n_tokens, kGateThreads / LANES))), dim3(kGateThreads), 0, s, \
+                     in, n_tokens, n_expert, top_k, idx, out, zero_loss)
   // measured at 128 experts, k = 8, 8192 tokens: 32 lanes x 4 registers 15 us,
   // 8 lanes x 16 registers 19 us (one wave per SIMD, nothing to overlap with),
   // the sorted lists 20 us
@@ -262,8 +266,8 @@ static int launch_fwd(const void* logits, int64_t n_tokens, int n_expert, int to
   else if (n_expert <= 512) FMOE_GATE_FLAT(32, 16);
   else
     hipLaunchKernelGGL((topk_softmax_fwd_kernel<T, KMAX, 32>),
-                       dim3(ceil_div(n_tokens, kGateThreads / 32)), dim3(kGateThreads), 0, s, in,
-                       n_tokens, n_expert, top_k, idx, out);
+                       dim3(std::max(1, ceil_div(n_tokens, kGateThreads / 32))), dim3(kGateThreads), 0, s, in,
+                       n_tokens, n_expert, top_k, idx, out, zero_loss);
 #undef FMOE_GATE_FLAT
   FMOE_LAUNCH_CHECK("topk_softmax_fwd");
   return FMOE_OK;
@@ -312,20 +316,35 @@ using namespace fmoe;
               : top_k <= 4 ? FN<T, 4>(__VA_ARGS__)             \
                            : top_k <= 8 ? FN<T, 8>(__VA_ARGS__) : FN<T, 16>(__VA_ARGS__))
 
+static int gate_fwd(const char* who, const void* logits, int64_t n_tokens, int32_t n_expert,
+                    int32_t top_k, int64_t* idx, void* score, float* zero_loss, int dtype,
+                    void* stream) {
+  int rc = check_gate(who, n_tokens, n_expert, top_k, dtype);
+  if (rc) return rc;
+  if (n_tokens == 0 && zero_loss == nullptr) return FMOE_OK;
+  FMOE_REQUIRE(n_tokens == 0 || (logits && idx && score), FMOE_ERR_INVALID, "%s: null pointer", who);
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case FMOE_F32: return FMOE_GATE_DISPATCH(launch_fwd, float, logits, n_tokens, n_expert, top_k, idx, score, zero_loss, s);
+    case FMOE_F64: return FMOE_GATE_DISPATCH(launch_fwd, double, logits, n_tokens, n_expert, top_k, idx, score, zero_loss, s);
+    case FMOE_F16: return FMOE_GATE_DISPATCH(launch_fwd, __half, logits, n_tokens, n_expert, top_k, idx, score, zero_loss, s);
+    default: return FMOE_GATE_DISPATCH(launch_fwd, __hip_bfloat16, logits, n_tokens, n_expert, top_k, idx, score, zero_loss, s);
+  }
+}
+
 extern "C" int fmoe_topk_softmax_fwd(const void* logits, int64_t n_tokens, int32_t n_expert,
                                      int32_t top_k, int64_t* idx, void* score, int dtype,
                                      void* stream) {
-  int rc = check_gate("topk_softmax_fwd", n_tokens, n_expert, top_k, dtype);
-  if (rc) return rc;
-  if (n_tokens == 0) return FMOE_OK;
-  FMOE_REQUIRE(logits && idx && score, FMOE_ERR_INVALID, "topk_softmax_fwd: null pointer");
-  hipStream_t s = (hipStream_t)stream;
-  switch (dtype) {
-    case FMOE_F32: return FMOE_GATE_DISPATCH(launch_fwd, float, logits, n_tokens, n_expert, top_k, idx, score, s);
-    case FMOE_F64: return FMOE_GATE_DISPATCH(launch_fwd, double, logits, n_tokens, n_expert, top_k, idx, score, s);
-    case FMOE_F16: return FMOE_GATE_DISPATCH(launch_fwd, __half, logits, n_tokens, n_expert, top_k, idx, score, s);
-    default: return FMOE_GATE_DISPATCH(launch_fwd, __hip_bfloat16, logits, n_tokens, n_expert, top_k, idx, score, s);
-  }
+  return gate_fwd("topk_softmax_fwd", logits, n_tokens, n_expert, top_k, idx, score, nullptr, dtype,
+                  stream);
+}
+
+extern "C" int fmoe_naive_gate_fwd(const void* logits, int64_t n_tokens, int32_t n_expert,
+                                   int32_t top_k, int64_t* idx, void* score, float* zero_loss,
+                                   int dtype, void* stream) {
+  FMOE_REQUIRE(zero_loss != nullptr, FMOE_ERR_INVALID, "naive_gate_fwd: zero_loss is null");
+  return gate_fwd("naive_gate_fwd", logits, n_tokens, n_expert, top_k, idx, score, zero_loss, dtype,
+                  stream);
 }
 
 extern "C" int fmoe_topk_softmax_bwd(const void* dscore, const void* score, const int64_t* idx,

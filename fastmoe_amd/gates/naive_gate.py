@@ -1,7 +1,9 @@
 r"""Top-k of a linear layer (fmoe/gates/naive_gate.py)."""
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
+from .. import fmoe_cuda
 from ..functions import topk_softmax
 from .base_gate import BaseGate
 
@@ -15,6 +17,22 @@ class NaiveGate(BaseGate):
         super().__init__(num_expert, world_size)
         self.gate = nn.Linear(d_model, self.tot_expert, bias=gate_bias)
         self.top_k = top_k
+
+    def is_plain(self, x) -> bool:
+        r"""Whether running this module on the 2-d tensor `x` is exactly Linear -> top-k ->
+        softmax in one dtype, with nobody watching: a layer may then fold the gate into its
+        own autograd node."""
+        lin = self.gate
+        return (type(self) is NaiveGate and type(lin) is nn.Linear
+                and lin.weight.dtype == x.dtype and lin.weight.is_cuda
+                and self.top_k <= fmoe_cuda.MAX_GATE_TOP_K
+                and torch.get_default_dtype() == torch.float32
+                and not torch.is_autocast_enabled()
+                and not _has_any_global_hook()
+                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
+                         or self._backward_pre_hooks or lin._forward_hooks
+                         or lin._forward_pre_hooks or lin._backward_hooks
+                         or lin._backward_pre_hooks))
 
     def forward(self, inp, return_all_scores=False):
         logits = self.gate(inp)

@@ -146,6 +146,12 @@ class FMoE(nn.Module):
     def forward(self, moe_inp):
         r"""Gate, dispatch, experts, and the score-weighted sum of each token's
         top-k expert outputs (fmoe/layers.py:205-312)."""
+        whole = getattr(self.experts, "can_run_layer", None) if self.experts_fused else None
+        if (whole is not None and type(self.gate) is NaiveGate and self.gate_hook is None
+                and self.mask is None and whole(moe_inp, self.top_k)):
+            out = self.experts.run_gated_layer(self.gate, moe_inp)
+            if out is not None:
+                return out
         sizes = tree.flatten(tree.map_structure(lambda t: t.shape[0], moe_inp))
         assert all(s == sizes[0] for s in sizes), \
             "MoE inputs must have the same batch size"
@@ -165,7 +171,6 @@ class FMoE(nn.Module):
                 mask = self.mask.view(-1).to(gate_top_k_idx.device)
                 gate_top_k_idx = torch.where((mask == 0).view(-1, 1),
                                              gate_top_k_idx.view(-1, self.top_k), -1)
-            whole = getattr(self.experts, "can_run_layer", None) if self.experts_fused else None
             if whole is not None and whole(moe_inp, self.top_k):
                 # dispatch, experts and combine as one autograd node (least host time)
                 out = self.experts.run_layer(moe_inp, gate_top_k_idx, score)

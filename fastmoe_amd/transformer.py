@@ -140,9 +140,27 @@ class _Expert(nn.Module):
 
     def run_layer(self, inp, gate_idx, score):
         r"""`sum_j score[t, j] * expert_{gate_idx[t, j]}(inp[t])` over the live slots,
-        as one autograd node (FusedExpertLayer)."""
+        as one autograd node: the extension's own, or FusedExpertLayer where a Python node
+        is wanted (ctypes binding, per-op profiling)."""
+        native = fmoe_cuda.native_layers()
+        if native is not None:
+            return native[0](inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
+                             self.h4toh.weight, self.h4toh.bias)
         return FusedExpertLayer.apply(inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
                                       self.h4toh.weight, self.h4toh.bias)
+
+    def run_gated_layer(self, gate, inp):
+        r"""The layer with the plain top-k gate `gate` (NaiveGate) in front of it as one
+        native autograd node, the gate's zero loss included; None where the gate has to run
+        as the module it is.  Only called after can_run_layer()."""
+        native = fmoe_cuda.native_layers()
+        if native is None or not gate.is_plain(inp):
+            return None
+        lin = gate.gate
+        out, loss = native[1](inp, lin.weight, lin.bias, self.htoh4.weight, self.htoh4.bias,
+                              self.h4toh.weight, self.h4toh.bias, gate.top_k)
+        gate.set_loss(loss)
+        return out
 
     def __len__(self):
         return self.htoh4.num_expert

@@ -360,6 +360,14 @@ int fmoe_topk_softmax_fwd(const void* logits, int64_t n_tokens, int32_t n_expert
                           void* stream);
 
 /*
+ * fmoe_topk_softmax_fwd that also writes *zero_loss = 0: the balance loss of the plain
+ * top-k gate (fmoe/gates/naive_gate.py:31-38 with fmoe/gates/base_gate.py:15-22), which
+ * would otherwise be a launch of its own.  No counterpart in the reference's extension.
+ */
+int fmoe_naive_gate_fwd(const void* logits, int64_t n_tokens, int32_t n_expert, int32_t top_k,
+                        int64_t* idx, void* score, float* zero_loss, int dtype, void* stream);
+
+/*
  * Backward of fmoe_topk_softmax_fwd with respect to the logits:
  *   dlogits[t][idx[t][j]] = score_j * (dscore_j - sum_i dscore_i * score_i)
  * and zero for every other expert (all n_tokens * n_expert entries are written).
