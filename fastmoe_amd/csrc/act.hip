@@ -10,11 +10,9 @@
 // multiplication.  That leaves both passes HBM-bound, where evaluating erf
 // per element (some 25 VALU instructions) does not.  f32 / f64 evaluate
 // 0.5 x (1 + erf(x / sqrt 2)) directly.
-#include <math.h>
-
 #include <mutex>
 
-#include "common.h"
+#include "act_math.h"
 
 namespace fmoe {
 namespace {
@@ -35,13 +33,6 @@ __device__ __forceinline__ double bits_to_double(int which, uint16_t b) {
 __device__ __forceinline__ uint16_t float_to_bits(int which, float v) {
   if (which == 0) return __bfloat16_as_ushort(__float2bfloat16(v));
   return __half_as_ushort(__float2half(v));
-}
-
-// gelu(x) = x Phi(x), gelu'(x) = Phi(x) + x phi(x); Phi through erfc so that the
-// negative tail keeps its relative accuracy.
-__device__ __forceinline__ double gelu_f64(double x) { return 0.5 * x * erfc(-x * M_SQRT1_2); }
-__device__ __forceinline__ double gelu_grad_f64(double x) {
-  return 0.5 * erfc(-x * M_SQRT1_2) + x * exp(-0.5 * x * x) * 0.3989422804014327;
 }
 
 __global__ void gelu_table_kernel() {
@@ -156,16 +147,6 @@ __global__ void gelu_bwd_tab_kernel(const T* __restrict__ dy, const uint16_t* __
 }
 
 // ---- f32 / f64: direct evaluation ---------------------------------------------
-__device__ __forceinline__ float gelu_direct(float x) {
-  return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
-}
-__device__ __forceinline__ double gelu_direct(double x) { return gelu_f64(x); }
-__device__ __forceinline__ float gelu_grad_direct(float x) {
-  return 0.5f * (1.f + erff(x * 0.70710678118654752f)) +
-         x * expf(-0.5f * x * x) * 0.3989422804014327f;
-}
-__device__ __forceinline__ double gelu_grad_direct(double x) { return gelu_grad_f64(x); }
-
 template <typename T>
 __global__ void gelu_fwd_direct_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t n,
                                        const int32_t* __restrict__ n_rows_dev,

@@ -119,6 +119,13 @@ static int check_linear(const char* who, int64_t n_rows, int64_t in_feat,
 static int run_gemm(int mode, const GemmArgs& g, int dtype, hipStream_t s) {
   if (g_gemm_path == 0 && gemm_mfma_supported(mode, g, dtype))
     return launch_gemm_mfma(mode, g, dtype, s);
+  if (g_gemm_path == 0 && gemm_plain_supported(g, dtype)) {
+    if (mode == GEMM_FWD) return launch_gemm_plain_fwd(g, dtype, s);
+    GemmArgs none = g;
+    none.c = nullptr;
+    return mode == GEMM_DGRAD ? launch_gemm_plain_bwd(g, none, dtype, s)
+                              : launch_gemm_plain_bwd(none, g, dtype, s);
+  }
   if (g_gemm_path == 0 && gemm_mfma_wide_supported(mode, g, dtype))
     return launch_gemm_mfma_wide(mode, g, dtype, s);
   return launch_gemm_simt(mode, g, dtype, s);
@@ -224,6 +231,13 @@ static int linear_fwd(const char* who, const void* x, const void* w, const void*
     g.act_out = y_act;
     return launch_gemm_mfma(GEMM_FWD, g, dtype, s);
   }
+  // f32: always inside the tiles (the activation costs what evaluating erf costs either
+  // way, and the pass over memory is saved)
+  if (dtype == FMOE_F32 && g_gemm_path == 0 && g_fuse_fwd_act) {
+    g.act_out = y_act;
+    if (gemm_plain_supported(g, dtype)) return launch_gemm_plain_fwd(g, dtype, s);
+    g.act_out = nullptr;
+  }
   rc = run_gemm(GEMM_FWD, g, dtype, s);
   if (rc) return rc;
   return fmoe_gelu_fwd(y, y_act, n_rows * out_feat, seg_off + n_expert, out_feat, dtype, stream);
@@ -293,24 +307,31 @@ static int linear_bwd(const void* dy, const void* x, const void* w, const void* 
   FMOE_REQUIRE(n_rows == 0 || dy != nullptr, FMOE_ERR_INVALID,
                "grouped_linear_bwd: dy is null");
   hipStream_t s = (hipStream_t)stream;
-  // The bf16/f16 matrix-core kernel sums the columns of dY inside its dW tiles;
-  // every other kernel leaves the bias gradient to the reduction kernel below.
+  // The matrix-core kernels for 16-bit types and f32 sum the columns of dY inside their dW
+  // tiles; f64 and the scalar kernel leave the bias gradient to the reduction kernel below.
   GemmArgs gw{dy, x, dw, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
-  const bool mfma_w = dw && g_gemm_path == 0 && (n_rows == 0 || x != nullptr) &&
-                      gemm_mfma_supported(GEMM_WGRAD, gw, dtype);
-  if (mfma_w && dbias) {
+  const bool have_w = dw && g_gemm_path == 0 && (n_rows == 0 || x != nullptr);
+  const bool mfma_w = have_w && gemm_mfma_supported(GEMM_WGRAD, gw, dtype);
+  const bool plain_w = have_w && !mfma_w && gemm_plain_supported(gw, dtype);
+  if ((mfma_w || plain_w) && dbias) {
     gw.bias = dbias;
     dbias = nullptr;  // comes out of the dW launch
   }
   GemmArgs gd{dy, w, dx, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   gd.w_table = w_table;
   void* const dx_out = dx;
-  const bool act_fused = act_pre && dx && n_rows > 0 && dtype == FMOE_BF16 && g_gemm_path == 0 &&
-                         (uintptr_t)act_pre % 16 == 0 && gemm_mfma_supported(GEMM_DGRAD, gd, dtype);
-  if (act_fused) {
+  const bool act_here = act_pre && dx && n_rows > 0 && g_gemm_path == 0;
+  bool act_fused = false;
+  if (act_here && dtype == FMOE_BF16 && (uintptr_t)act_pre % 16 == 0 &&
+      gemm_mfma_supported(GEMM_DGRAD, gd, dtype)) {
     rc = gelu_bwd_table(dtype, s, &gd.act_table);
     if (rc) return rc;
     gd.act_pre = act_pre;
+    act_fused = true;
+  } else if (act_here && dtype == FMOE_F32) {
+    gd.act_pre = act_pre;
+    act_fused = gemm_plain_supported(gd, dtype);
+    if (!act_fused) gd.act_pre = nullptr;
   }
   if (dx && dw && n_rows > 0 && g_gemm_path == 0) {
     FMOE_REQUIRE((w != nullptr || w_table != nullptr) && x != nullptr, FMOE_ERR_INVALID,
@@ -319,6 +340,11 @@ static int linear_bwd(const void* dy, const void* x, const void* w, const void* 
       rc = launch_gemm_mfma_bwd(gd, gw, dtype, s);
       if (rc) return rc;
       dx = nullptr;  // both products are under way
+      dw = nullptr;
+    } else if (plain_w && gemm_plain_supported(gd, dtype)) {
+      rc = launch_gemm_plain_bwd(gd, gw, dtype, s);
+      if (rc) return rc;
+      dx = nullptr;
       dw = nullptr;
     }
   }

@@ -31,14 +31,14 @@ struct GemmArgs {
   int out_feat;
   int n_expert;
   int tile;             // 0 = choose the tile shape automatically, 1..4 = force one
-  // DGRAD on the bf16 matrix-core kernel only: if not null, dx = (dy W) * gelu'(act_pre)
+  // DGRAD on the bf16 matrix-core and f32 kernels only: if not null, dx = (dy W) * gelu'(act_pre)
   // with act_pre [n_rows, in_feat] the pre-activations behind the layer's input,
-  // and act_table the device table of gelu'(-|x|) (gelu_bwd_table()).
+  // and act_table (bf16) the device table of gelu'(-|x|) (gelu_bwd_table()).
   const void* act_pre = nullptr;
   const float* act_table = nullptr;
-  // FWD on the bf16 matrix-core kernel only: if not null, act_out [n_rows, out_feat]
-  // receives gelu(y) next to y, through act_fwd_table, the device table of gelu(x)
-  // by 16-bit pattern of x (gelu_fwd_table()).
+  // FWD on the bf16 matrix-core and f32 kernels only: if not null, act_out
+  // [n_rows, out_feat] receives gelu(y) next to y; bf16 through act_fwd_table, the device
+  // table of gelu(x) by 16-bit pattern of x (gelu_fwd_table()).
   void* act_out = nullptr;
   const uint16_t* act_fwd_table = nullptr;
   // Experts whose parameters are separate allocations (the reference keeps one module
@@ -108,7 +108,15 @@ int launch_gemm_mfma(int mode, const GemmArgs& g, int dtype, hipStream_t s);
 // grouped linear, in one launch where the tile shapes allow it.
 int launch_gemm_mfma_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s);
 
-// f32 / f64 grouped GEMM on the matrix cores, for 4-element-aligned shapes.
+// f32 grouped GEMM of any shape and bf16 / f16 of even feature sizes on the matrix cores.
+// f32 applies the activation inside its tiles: act_out (forward) and act_pre (dX) without
+// a table.
+bool gemm_plain_supported(const GemmArgs& g, int dtype);
+int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s);
+// dX (gd) and dW (gw) in one launch; a null gd.c or gw.c leaves that product out.
+int launch_gemm_plain_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s);
+
+// f64 grouped GEMM on the matrix cores, for 4-element-aligned shapes.
 bool gemm_mfma_wide_supported(int mode, const GemmArgs& g, int dtype);
 int launch_gemm_mfma_wide(int mode, const GemmArgs& g, int dtype, hipStream_t s);
 

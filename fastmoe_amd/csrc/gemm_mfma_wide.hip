@@ -1,16 +1,13 @@
-// f32 / f64 grouped GEMM on the matrix cores (v_mfma_f32_32x32x2_f32,
-// v_mfma_f64_16x16x4_f64): the full-precision half of the reference's dtype
-// dispatch (cuda/parallel_linear.cu:33,76 -> cublasSgemm / cublasDgemm,
+// f64 grouped GEMM on the matrix cores (v_mfma_f64_16x16x4_f64): the double-precision part
+// of the reference's dtype dispatch (cuda/parallel_linear.cu:33,76 -> cublasDgemm,
 // cuda/utils/cublas_wrapper.h:51-90).
 //
-// These MFMAs run at 1/16 (f32) and 1/32 (f64) of the bf16 rate, so one K slice
-// of a 128x128 tile keeps the matrix cores busy for microseconds and a plain
-// design is enough: global -> registers -> LDS with two LDS stages of 16 values
-// of K, one barrier per slice, and several blocks per CU (four for f32: their
-// stages fill the 160 KB of LDS exactly; two for f64) so that one block's barrier and LDS writes hide behind the
-// others' MFMAs.  Operand roles and the ragged rows are those of the
-// bf16 kernel (gemm.h); the row tiles of an expert are found as in the scalar
-// kernel (virtual_row_tiles).
+// This MFMA runs at 1/32 of the bf16 rate, so one K slice of a 128x128 tile keeps the
+// matrix cores busy for microseconds and a plain design is enough: global -> registers ->
+// LDS with two LDS stages of 16 values of K, one barrier per slice, and two blocks per CU
+// so that one block's barrier and LDS writes hide behind the other's MFMAs.  Operand roles
+// and the ragged rows are those of the bf16 kernel (gemm.h); the row tiles of an expert
+// are found as in the scalar kernel (virtual_row_tiles).
 //
 // Both operand layouts are copied into LDS as they come, pack by pack: operands
 // whose rows are contiguous in memory (W in DGRAD, both in WGRAD) as [k][row],
@@ -23,33 +20,18 @@
 namespace fmoe {
 namespace {
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWideTile = 128;     // output tile is kWideTile x kWideTile
 constexpr int kWideThreads = 256;  // 2 x 2 waves of 64 x 64
 
 template <typename F> struct WideMma;
-template <> struct WideMma<float> {
-  static constexpr int kBlk = 32;   // rows / columns of one MFMA block
-  static constexpr int kAcc = 16;   // accumulators per lane and block
-  static constexpr int kBK = 16;    // values of K per LDS slice
-  static constexpr int kPad = 4;    // row padding of the LDS image, in elements
-  static constexpr int kWaves = 4;      // waves per SIMD the registers are budgeted for
-  static constexpr bool kSwap = true;   // feed (B, A): a lane then owns runs of 4 columns
-  using acc_t = f32x16_t;
-  typedef float vec_t __attribute__((ext_vector_type(4)));             // 16-byte pack
-  static __device__ __forceinline__ acc_t run(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
 template <> struct WideMma<double> {
   static constexpr int kBlk = 16;
   static constexpr int kAcc = 4;
   static constexpr int kBK = 16;
   static constexpr int kPad = 2;
   static constexpr int kWaves = 2;
-  static constexpr bool kSwap = false;  // a lane owns one column, 16 lanes a row segment
   using acc_t = f64x4_t;
   typedef double vec_t __attribute__((ext_vector_type(4), aligned(16)));  // two 16-byte packs
   static __device__ __forceinline__ acc_t run(double a, double b, acc_t c) {
@@ -175,9 +157,6 @@ __global__ __launch_bounds__(kWideThreads, (WideMma<F>::kWaves)) void gemm_wide_
   using a_kc = std::integral_constant<bool, A_KC>;
   using b_kc = std::integral_constant<bool, B_KC>;
 
-  // f32: acc[i][j] holds the TRANSPOSE of block (i, j) of C (the MFMA is fed
-  // (B value, A value)): a lane owns row lane % 32 and runs of 4 consecutive
-  // columns, which leave as one 16-byte store each.  f64: block (i, j) itself.
   typename Mma::acc_t acc[TB][TB];
 #pragma unroll
   for (int i = 0; i < TB; ++i)
@@ -234,8 +213,7 @@ __global__ __launch_bounds__(kWideThreads, (WideMma<F>::kWaves)) void gemm_wide_
         for (int i = 0; i < TB; ++i)
 #pragma unroll
           for (int j = 0; j < TB; ++j)
-            acc[i][j] = Mma::kSwap ? Mma::run(b[j][c], a[i][c], acc[i][j])
-                                   : Mma::run(a[i][c], b[j][c], acc[i][j]);
+            acc[i][j] = Mma::run(a[i][c], b[j][c], acc[i][j]);
     }
     if (more) {
       // the other stage was last read in iteration kt - 1, which every wave
@@ -248,40 +226,18 @@ __global__ __launch_bounds__(kWideThreads, (WideMma<F>::kWaves)) void gemm_wide_
   }
 
   const F* bias = MODE == GEMM_FWD ? expert_operand<F>(g.bias, g.bias_table, e, out_f) : nullptr;
-  if constexpr (Mma::kSwap) {
-    // 32x32 block, operands swapped: accumulator r of a lane is row lane % 32,
-    // column 8 * (r / 4) + 4 * (lane / 32) + r % 4
+  // 16x16 block: accumulator r of a lane is row 4 * r + lane / 16, column
+  // lane % 16; 16 lanes store 128 contiguous bytes of a row
+#pragma unroll
+  for (int j = 0; j < TB; ++j) {
+    const int n = n0 + wave_n * 64 + j * BLK + lr;
+    const F bv = bias && n < N ? load_global<F>(bias + n) : (F)0;
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
-      const int m = m0 + wave_m * 64 + i * BLK + lr;
 #pragma unroll
-      for (int j = 0; j < TB; ++j) {
-#pragma unroll
-        for (int q = 0; q < Mma::kAcc / 4; ++q) {
-          const int n = n0 + wave_n * 64 + j * BLK + 8 * q + 4 * lk;
-          if (m < M && n < N) {  // N is a multiple of 4
-            Vec4 o;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) o[c] = acc[i][j][4 * q + c] + (bias ? load_global<F>(bias + n + c) : (F)0);
-            *reinterpret_cast<Vec4*>(C + (int64_t)m * ldc + n) = o;
-          }
-        }
-      }
-    }
-  } else {
-    // 16x16 block: accumulator r of a lane is row 4 * r + lane / 16, column
-    // lane % 16; 16 lanes store 128 contiguous bytes of a row
-#pragma unroll
-    for (int j = 0; j < TB; ++j) {
-      const int n = n0 + wave_n * 64 + j * BLK + lr;
-      const F bv = bias && n < N ? load_global<F>(bias + n) : (F)0;
-#pragma unroll
-      for (int i = 0; i < TB; ++i) {
-#pragma unroll
-        for (int r = 0; r < Mma::kAcc; ++r) {
-          const int m = m0 + wave_m * 64 + i * BLK + 4 * r + lk;
-          if (m < M && n < N) C[(int64_t)m * ldc + n] = acc[i][j][r] + bv;
-        }
+      for (int r = 0; r < Mma::kAcc; ++r) {
+        const int m = m0 + wave_m * 64 + i * BLK + 4 * r + lk;
+        if (m < M && n < N) C[(int64_t)m * ldc + n] = acc[i][j][r] + bv;
       }
     }
   }
@@ -324,7 +280,7 @@ int launch_wide_t(int mode, const GemmArgs& g, hipStream_t s) {
 // from 16 tiles up, so size does not enter the choice.
 bool gemm_mfma_wide_supported(int mode, const GemmArgs& g, int dtype) {
   (void)mode;
-  if (dtype != FMOE_F32 && dtype != FMOE_F64) return false;
+  if (dtype != FMOE_F64) return false;
   if (g.in_feat % 4 != 0 || g.out_feat % 4 != 0) return false;
   if (((uintptr_t)g.a | (uintptr_t)g.b | (uintptr_t)g.c) % 16 != 0) return false;
   return true;
@@ -333,7 +289,6 @@ bool gemm_mfma_wide_supported(int mode, const GemmArgs& g, int dtype) {
 int launch_gemm_mfma_wide(int mode, const GemmArgs& g, int dtype, hipStream_t s) {
   if (!gemm_mfma_wide_supported(mode, g, dtype))
     return set_error(FMOE_ERR_UNSUPPORTED, "grouped GEMM: shape not MFMA-aligned");
-  if (dtype == FMOE_F32) return launch_wide_t<float>(mode, g, s);
   return launch_wide_t<double>(mode, g, s);
 }
 

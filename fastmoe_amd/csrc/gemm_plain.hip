@@ -1,0 +1,683 @@
+// Grouped GEMM on the matrix cores for what the 256-row bf16/f16 kernels
+// (gemm_mfma_impl.h) do not take: f32 of any shape, and bf16/f16 whose feature sizes
+// are even but no multiples of 8 (rows then start on 4-byte boundaries).
+//
+// One pipeline for all of them.  A workgroup of 4 waves (2 x 2) computes a BM x BN tile;
+// a K slice is 128 BYTES of every operand row (32 values of f32, 64 of bf16/f16), two LDS
+// stages of it alternate, copied by `buffer_load ... lds` (16 or 4 bytes per lane,
+// no staging registers), with one wait and one barrier per slice.  There is no
+// interleaving plan as in the 256-row kernels: f32 MFMAs are 16 times slower, so one
+// slice of a 64 x 128 tile is 2048 cycles of them per SIMD, and three or four workgroups per
+// CU cover each other's barriers; with 4-byte copies (dword-aligned rows) the CU's address
+// unit bounds the kernel (a quarter of a KiB per 20 cycles).
+//
+// Both operand layouts are kept in LDS as they come:
+//   K-contiguous rows  [row][128 bytes], 16-byte packs XORed by row bits;
+//   K-strided          [k][rows], plain for f32, 32-byte segments XORed by k bits for
+//                      bf16/f16 (ds_read_b64_tr_b16 transposes on the way to registers).
+// f32 fragments: the 32x32x2 MFMA takes one value of K per lane, and WHICH value of a
+// slice that is, and which row of the wave's patch, only has to agree with the other
+// operand and the epilogue.  With 16-byte copies lane group g = l / 32 takes
+// k = 8 s + 4 g + c in round c of group s, so a K-contiguous operand is one 16-byte read
+// per four rounds; with 4-byte copies (feature sizes off the 16-byte grid) it takes
+// k = 8 s + 2 c + g, i.e. the sums run over K in ascending order.  Both orders are those
+// of the kernels that ran before, so results are the same bits (a ReLU behind the layer
+// turns any difference of a sum around zero into a whole gradient).  Block i of lane l is
+// row (l % 32) * blocks + i: a K-strided operand is then one read per round for all
+// blocks, and a lane's blocks are adjacent columns of the output, so that 32 lanes store
+// up to 256 contiguous bytes straight from the accumulators.
+//
+// Tile shape: the cost model and the measurements at the end.
+#include <algorithm>
+
+#include "act_math.h"
+#include "dma_desc.h"
+#include "gemm_tiles.h"
+
+namespace fmoe {
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+constexpr int kThreads = 256, kWaves = 4;
+constexpr int kSliceBytes = 128;               // of one operand row per K slice
+constexpr int kRsrcFlags = 0x00020000;         // raw buffer, 32-bit data format
+
+template <typename T> struct Half;             // the 16-bit types' instructions
+template <> struct Half<__hip_bfloat16> {
+  static __device__ __forceinline__ f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ float add(uint32_t pair, float s) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pair),
+                                           __builtin_bit_cast(bf16x2_t, 0x3f803f80u), s, false);
+  }
+};
+template <> struct Half<__half> {
+  static __device__ __forceinline__ f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ float add(uint32_t pair, float s) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, pair),
+                                  __builtin_bit_cast(f16x2_t, 0x3c003c00u), s, false);
+  }
+};
+
+// One operand tile: R rows of the M or N index by one K slice.  ES bytes per element, BLOCKS
+// 16-row blocks per wave, DMA bytes per lane and copy.
+template <int R, int ES, int BLOCKS, bool KC, int DMA>
+struct SliceTile {
+  static constexpr int kBytes = R * kSliceBytes;
+  static constexpr int kBK = kSliceBytes / ES;                 // values of K per slice
+  static constexpr int kLoads = kBytes / (64 * DMA) / kWaves;  // copies per wave and slice
+  static constexpr int kRowBytes = R * ES;                     // of a [k] row (not KC)
+  static_assert(kBytes % (64 * DMA * kWaves) == 0 && kLoads >= 1, "tile must split evenly");
+
+  // which of the 8 packs of a [row][128 bytes] row holds pack p: rows that the lanes of
+  // one read touch together differ in the bits used here
+  static __device__ __forceinline__ int row_swizzle(int row) {
+    return (row / (ES == 4 ? BLOCKS : 2)) & 7;
+  }
+  // XOR of the 32-byte segment index of a [k] row (16-bit types)
+  static __device__ __forceinline__ int k_swizzle(int k) {
+    return ES == 2 ? (((k & 3) << 1) ^ ((k >> 3) & 1)) & (kRowBytes / 32 - 1) : 0;
+  }
+
+  uint32_t voff[kLoads];   // per lane: source offset of every copy
+  i32x4_t rsrc;            // descriptor of the current slice; num_records ends the valid data
+  int64_t remaining;       // bytes from the slice origin to the end of the valid data
+  int step, k_left;
+
+  // K value (inside the slice) of the bytes this lane copies in copy i (KC only)
+  static __device__ __forceinline__ int copy_k(int i, int wave, int lane) {
+    const int off = (wave * kLoads + i) * 64 * DMA + lane * DMA;
+    const int row = off / kSliceBytes, in = off % kSliceBytes;
+    return (((in / 16) ^ row_swizzle(row)) * 16 + in % 16) / ES;
+  }
+
+  __device__ __forceinline__ void init(const char* origin, int wave, int lane, int ld, int r_valid,
+                                       int r_span, int k_total) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int off = (wave * kLoads + i) * 64 * DMA + lane * DMA;
+      if (KC) {
+        voff[i] = (uint32_t)(off / kSliceBytes * ld + copy_k(i, wave, lane)) * ES;
+      } else {
+        const int k = off / kRowBytes, in = off % kRowBytes;
+        const int r = (((in / 32) ^ k_swizzle(k)) * 32 + in % 32) / ES;
+        voff[i] = r < r_valid ? (uint32_t)(k * ld + r) * ES : kDmaOutOfRange;
+      }
+    }
+    int64_t bytes = 0;
+    if (k_total > 0)
+      bytes = KC ? ((int64_t)(r_valid - 1) * ld + k_total) * ES
+                 : ((int64_t)(k_total - 1) * ld + r_span) * ES;
+    remaining = ((int64_t)__builtin_amdgcn_readfirstlane((int)(bytes >> 32)) << 32) |
+                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
+    step = __builtin_amdgcn_readfirstlane(KC ? kSliceBytes : kBK * ld * ES);
+    k_left = k_total;
+    const uint64_t p = (uint64_t)origin;
+    rsrc[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
+    rsrc[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(p >> 32) & 0xffff);
+    rsrc[2] = dma_num_records(remaining);
+    rsrc[3] = kRsrcFlags;
+    mask_k_tail(wave, lane);
+  }
+
+  // the one slice that holds the end of K: what lies past it is pointed out of range for
+  // good (the slices behind it are empty)
+  __device__ __forceinline__ void mask_k_tail(int wave, int lane) {
+    if (KC && k_left < kBK) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        if (copy_k(i, wave, lane) >= k_left) voff[i] = kDmaOutOfRange;
+    }
+  }
+
+  __device__ __forceinline__ void advance(int wave, int lane) {
+    const uint64_t p = (((uint64_t)(uint32_t)rsrc[1] << 32) | (uint32_t)rsrc[0]) + (uint32_t)step;
+    rsrc[0] = (int)(uint32_t)p;
+    rsrc[1] = (int)(uint32_t)(p >> 32);
+    remaining -= step;
+    rsrc[2] = dma_num_records(remaining);
+    k_left -= kBK;
+    mask_k_tail(wave, lane);
+  }
+
+  // All copies of this wave for the current slice.  Inline assembly, so that the compiler
+  // neither counts them nor waits for them at every LDS read: the kernel waits itself.
+  __device__ __forceinline__ void issue(uint32_t tile_lds, int wave) const {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const uint32_t dst = tile_lds + (uint32_t)(wave * kLoads + i) * (64 * DMA);
+      if (DMA == 16)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :: "s"(dst), "v"(voff[i]), "s"(rsrc) : "memory", "m0");
+      else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                     :: "s"(dst), "v"(voff[i]), "s"(rsrc) : "memory", "m0");
+    }
+  }
+
+  // f32, K group s (8 values): f[c][i] = the value of K that round c multiplies, of row
+  // row0 + (lane % 32) * BLOCKS + i
+  static __device__ __forceinline__ void frags32(const char* lds, int row0, int s, int lane,
+                                                 float (&f)[4][BLOCKS]) {
+    const int a = lane & 31, g = lane >> 5;
+    if (KC) {
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) {
+        const int row = row0 + a * BLOCKS + i;
+        const char* p = lds + row * kSliceBytes;
+        if (DMA == 16) {
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + (((s * 2 + g) ^ row_swizzle(row)) * 16));
+#pragma unroll
+          for (int c = 0; c < 4; ++c) f[c][i] = v[c];
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            f[c][i] = *reinterpret_cast<const float*>(
+                p + (((s * 2 + c / 2) ^ row_swizzle(row)) * 16) + ((c & 1) * 2 + g) * 4);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int k = s * 8 + (DMA == 16 ? 4 * g + c : 2 * c + g);
+        const char* p = lds + k * kRowBytes + (row0 + a * BLOCKS) * 4;
+        if (BLOCKS == 2) {
+          const f32x2_t v = *reinterpret_cast<const f32x2_t*>(p);
+#pragma unroll
+          for (int i = 0; i < BLOCKS; ++i) f[c][i] = v[i];
+        } else {
+          f[c][0] = *reinterpret_cast<const float*>(p);
+        }
+      }
+    }
+  }
+
+  // bf16 / f16, K group s (32 values): lane l holds row row16 + l % 16, values
+  // 8 (l / 16) .. + 7 of the group
+  static __device__ __forceinline__ uint4 frag16(const char* lds, int row16, int s, int lane) {
+    if (KC) {
+      const int row = row16 + (lane & 15);
+      return *reinterpret_cast<const uint4*>(
+          lds + row * kSliceBytes + (((s * 4 + (lane >> 4)) ^ row_swizzle(row)) * 16));
+    }
+    const int k = s * 32 + 8 * (lane >> 4) + ((lane & 15) >> 2);
+    const int m = row16 + 4 * (lane & 3);
+    const char* p = lds + k * kRowBytes + ((m >> 4) ^ k_swizzle(k)) * 32 + (m & 15) * 2;
+    const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4_t*)(p));
+    const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4_t*)(p + 4 * kRowBytes));
+    const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+    return make_uint4(l2.x, l2.y, h2.x, h2.y);
+  }
+};
+
+// The activation behind the forward product / in front of the backward one, f32 only.
+__device__ __forceinline__ float act_fwd(float v) { return gelu_direct(v); }
+__device__ __forceinline__ float act_bwd(float g, float pre) { return g * gelu_grad_direct(pre); }
+
+template <typename T, int BM, int BN, int MODE, int DMA>
+__device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRows where,
+                                           int n_origin) {
+  constexpr bool kF32 = std::is_same<T, float>::value;
+  constexpr int ES = sizeof(T);
+  // blocks of a wave: 32x32 for f32, 16x16 for the 16-bit types
+  constexpr int TM = BM / 2 / (kF32 ? 32 : 16), TN = BN / 2 / (kF32 ? 32 : 16);
+  using Acc = typename std::conditional<kF32, f32x16_t, f32x4_t>::type;
+  constexpr bool A_KC = MODE != GEMM_WGRAD, B_KC = MODE == GEMM_FWD;
+  using ATile = SliceTile<BM, ES, TM, A_KC, DMA>;
+  using BTile = SliceTile<BN, ES, TN, B_KC, DMA>;
+  constexpr int kStage = ATile::kBytes + BTile::kBytes;
+  static_assert(!kF32 || (TM <= 2 && TN <= 2), "fragment reads cover 1 or 2 blocks");
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_m = wave >> 1, wave_n = wave & 1;
+  const int in_f = g.in_feat, out_f = g.out_feat;
+  const int e = __builtin_amdgcn_readfirstlane(where.e);
+  const int row0 = __builtin_amdgcn_readfirstlane(where.row0);
+  const int cnt = __builtin_amdgcn_readfirstlane(where.cnt);
+
+  int M, N, K, lda, ldb, ldc;
+  const T *A, *B;
+  T* C;
+  if (MODE == GEMM_FWD) {
+    M = cnt; N = out_f; K = in_f;
+    A = (const T*)g.a + (int64_t)row0 * in_f;                      lda = in_f;
+    B = expert_operand<T>(g.b, g.w_table, e, (int64_t)out_f * in_f); ldb = in_f;
+    C = (T*)g.c + (int64_t)row0 * out_f;                           ldc = out_f;
+  } else if (MODE == GEMM_DGRAD) {
+    M = cnt; N = in_f; K = out_f;
+    A = (const T*)g.a + (int64_t)row0 * out_f;                     lda = out_f;
+    B = expert_operand<T>(g.b, g.w_table, e, (int64_t)out_f * in_f); ldb = in_f;
+    C = (T*)g.c + (int64_t)row0 * in_f;                            ldc = in_f;
+  } else {
+    M = out_f; N = in_f; K = cnt;
+    A = (const T*)g.a + (int64_t)row0 * out_f;                     lda = out_f;
+    B = (const T*)g.b + (int64_t)row0 * in_f;                      ldb = in_f;
+    C = (T*)g.c + (int64_t)e * out_f * in_f;                       ldc = in_f;
+  }
+  const int m0 = __builtin_amdgcn_readfirstlane(where.m0);
+  const int n0 = __builtin_amdgcn_readfirstlane(n_origin);
+  if (m0 >= M || n0 >= N) return;   // the same for the whole block
+  const int m_valid = min(BM, M - m0), n_valid = min(BN, N - n0);
+
+  const uint32_t lds_base = (uint32_t)(size_t)(lds_ptr_t)smem;
+  ATile ta;
+  BTile tb;
+  ta.init((const char*)(A_KC ? A + (int64_t)m0 * lda : A + m0), wave, lane, lda, m_valid, M - m0, K);
+  tb.init((const char*)(B_KC ? B + (int64_t)n0 * ldb : B + n0), wave, lane, ldb, n_valid, N - n0, K);
+
+  Acc acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = (Acc)(0.f);
+
+  // dW tiles of the first column also sum the columns of dY: the bias gradient
+  const bool colsum = MODE == GEMM_WGRAD && g.bias != nullptr && n0 == 0;
+  float cs[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) cs[i] = 0.f;
+
+  const int k_tiles = (K + ATile::kBK - 1) / ATile::kBK;
+  ta.issue(lds_base, wave);
+  tb.issue(lds_base + ATile::kBytes, wave);
+  ta.advance(wave, lane);
+  tb.advance(wave, lane);
+  for (int kt = 0; kt < k_tiles; ++kt) {
+    // slice kt has landed here (my share) and, behind the barrier, everywhere; behind it
+    // nobody reads the stage of slice kt - 1 any more, which slice kt + 1 takes
+    const int stage = kt & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ta.issue(lds_base + (stage ^ 1) * kStage, wave);
+    tb.issue(lds_base + (stage ^ 1) * kStage + ATile::kBytes, wave);
+    ta.advance(wave, lane);
+    tb.advance(wave, lane);
+    const char* la = smem + stage * kStage;
+    const char* lb = la + ATile::kBytes;
+    if constexpr (kF32) {
+#pragma unroll
+      for (int s = 0; s < kSliceBytes / 32; ++s) {
+        float fa[4][TM], fb[4][TN];
+        ATile::frags32(la, wave_m * (BM / 2), s, lane, fa);
+        BTile::frags32(lb, wave_n * (BN / 2), s, lane, fb);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[c][i], fb[c][j], acc[i][j], 0, 0, 0);
+        }
+        if (MODE == GEMM_WGRAD && colsum) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i) cs[i] += (fa[0][i] + fa[1][i]) + (fa[2][i] + fa[3][i]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint4 fa[TM], fb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[i] = ATile::frag16(la, wave_m * (BM / 2) + i * 16, s, lane);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fb[j] = BTile::frag16(lb, wave_n * (BN / 2) + j * 16, s, lane);
+        // operands swapped: a lane then owns 4 adjacent columns of a row of C
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = Half<T>::mma(fb[j], fa[i], acc[i][j]);
+        if (MODE == GEMM_WGRAD && colsum) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            cs[i] = Half<T>::add(fa[i].x, cs[i]);
+            cs[i] = Half<T>::add(fa[i].y, cs[i]);
+            cs[i] = Half<T>::add(fa[i].z, cs[i]);
+            cs[i] = Half<T>::add(fa[i].w, cs[i]);
+          }
+        }
+      }
+    }
+  }
+  // the zero-filled slices past the end of K are still landing
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  const int a = lane & (kF32 ? 31 : 15), gr = lane / (kF32 ? 32 : 16);
+  if (MODE == GEMM_WGRAD && colsum) {
+    T* db = (T*)const_cast<void*>(g.bias) + (int64_t)e * out_f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      float total = cs[i] + __shfl_xor(cs[i], 32, 64);
+      if (!kF32) total += __shfl_xor(total, 16, 64);
+      const int m = m0 + wave_m * (BM / 2) + (kF32 ? a * TM + i : i * 16 + a);
+      if (wave_n == 0 && gr == 0 && m < M) db[m] = Elem<T>::from_acc(total);
+    }
+  }
+
+  const T* bias = MODE == GEMM_FWD ? expert_operand<T>(g.bias, g.bias_table, e, out_f) : nullptr;
+  if constexpr (kF32) {
+    // accumulator r of block (i, j): row (8 (r / 4) + 4 gr + r % 4) TM + i, column a TN + j
+    struct alignas(DMA == 16 ? 4 * TN : 4) Vec { float v[TN]; };
+    const int col = n0 + wave_n * (BN / 2) + a * TN;
+    float bv[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      bv[j] = bias && col + j < N ? load_global<float>(bias + col + j) : 0.f;
+    const float* pre = MODE == GEMM_DGRAD ? (const float*)g.act_pre : nullptr;
+    float* act_out = MODE == GEMM_FWD ? (float*)g.act_out : nullptr;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = wave_m * (BM / 2) + (8 * (r / 4) + 4 * gr + r % 4) * TM + i;
+        if (m >= m_valid || col >= N) continue;
+        Vec o;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) o.v[j] = acc[i][j][r] + bv[j];
+        const int64_t at = (int64_t)(m0 + m) * ldc + col;
+        const bool whole = DMA == 16 || col + TN <= N;   // 16-byte rows: N is a multiple of 4
+        if (MODE == GEMM_DGRAD && pre) {
+          const float* p = pre + (int64_t)row0 * ldc + at;
+          Vec x;
+          if (whole) {
+            x = *reinterpret_cast<const Vec*>(p);
+          } else {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) x.v[j] = col + j < N ? p[j] : 0.f;
+          }
+#pragma unroll
+          for (int j = 0; j < TN; ++j) o.v[j] = act_bwd(o.v[j], x.v[j]);
+        }
+        if (whole) {
+          *reinterpret_cast<Vec*>(C + at) = o;
+        } else {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            if (col + j < N) C[at + j] = o.v[j];
+        }
+        if (MODE == GEMM_FWD && act_out) {
+          float* q = act_out + (int64_t)row0 * ldc + at;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) o.v[j] = act_fwd(o.v[j]);
+          if (whole) {
+            *reinterpret_cast<Vec*>(q) = o;
+          } else {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              if (col + j < N) q[j] = o.v[j];
+          }
+        }
+      }
+  } else {
+    // accumulator r of block (i, j): row 16 i + a, column 16 j + 4 gr + r of the patch; rows
+    // start on 4-byte boundaries and N is even, so a pair is all in or all out
+    struct alignas(4) Pair { T v[2]; };
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + wave_n * (BN / 2) + j * 16 + 4 * gr;
+      float bv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        bv[r] = bias && col + r < N ? Elem<T>::to_acc(load_global<T>(bias + col + r)) : 0.f;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = wave_m * (BM / 2) + i * 16 + a;
+        if (m >= m_valid) continue;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (col + 2 * h >= N) continue;
+          Pair o;
+          o.v[0] = Elem<T>::from_acc(acc[i][j][2 * h] + bv[2 * h]);
+          o.v[1] = Elem<T>::from_acc(acc[i][j][2 * h + 1] + bv[2 * h + 1]);
+          *reinterpret_cast<Pair*>(C + (int64_t)(m0 + m) * ldc + col + 2 * h) = o;
+        }
+      }
+    }
+  }
+}
+
+template <int BM, int BN>
+constexpr size_t plain_lds() { return (size_t)2 * (BM + BN) * kSliceBytes; }
+// workgroups per CU the LDS allows, at most 4 (the registers are budgeted for them)
+template <int BM, int BN>
+constexpr int plain_blocks() {
+  constexpr int fit = 160 * 1024 / (int)(plain_lds<BM, BN>() + 128);
+  return fit < 4 ? fit : 4;
+}
+
+template <typename T, int BM, int BN, int DMA>
+__global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_fwd_kernel(GemmArgs g, int tiles_n) {
+  extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
+  __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
+  RowTiles<BM, false, kWaves> rows;
+  rows.scan(g.seg_off, g.n_expert, s_wave_sum);
+  const int live = rows.rows_f * tiles_n;
+  if (live == 0) return;
+  const int t = tile_number(blockIdx.x, live);
+  if (t >= live) return;
+  int v, n_tile;
+  tile_order(t, rows.rows_f, tiles_n, v, n_tile);
+  const TileRows where = rows.find(g.seg_off, v, false, s_owner);
+  plain_tile<T, BM, BN, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * BN);
+}
+
+// dX and dW (with the bias gradient) in one launch, dX tiles first; either may be absent
+// (no tiles).
+template <typename T, int BM, int BN, int DMA>
+__global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_bwd_kernel(GemmArgs gd, GemmArgs gw,
+                                                                int tiles_n_d, int tiles_n_w,
+                                                                int tiles_m_w) {
+  extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
+  __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
+  RowTiles<BM, false, kWaves> rows;
+  rows.scan(gd.seg_off, gd.n_expert, s_wave_sum);
+  const int live_d = rows.rows_f * tiles_n_d;
+  const int per_expert_w = tiles_n_w * tiles_m_w;
+  const int live = live_d + per_expert_w * gw.n_expert;
+  if (live == 0) return;
+  const int t = tile_number(blockIdx.x, live);
+  if (t >= live) return;
+  if (t >= live_d) {
+    const int tw = t - live_d, e = tw / per_expert_w;
+    int m_tile, n_tile;
+    tile_order(tw % per_expert_w, tiles_m_w, tiles_n_w, m_tile, n_tile);
+    const int row0 = gw.seg_off[e];
+    plain_tile<T, BM, BN, GEMM_WGRAD, DMA>(
+        gw, plain_smem, {e, m_tile * BM, row0, gw.seg_off[e + 1] - row0}, n_tile * BN);
+    return;
+  }
+  int v, n_tile;
+  tile_order(t, rows.rows_f, tiles_n_d, v, n_tile);
+  const TileRows where = rows.find(gd.seg_off, v, false, s_owner);
+  plain_tile<T, BM, BN, GEMM_DGRAD, DMA>(gd, plain_smem, where, n_tile * BN);
+}
+
+// ------------------------------------------------------------------ host side
+
+int round_up_blocks(int64_t tiles, unsigned* blocks) {
+  const int64_t b = ceil_div(tiles, 8 * kXcdRun) * (int64_t)(8 * kXcdRun);
+  FMOE_REQUIRE(b < ((int64_t)1 << 31), FMOE_ERR_UNSUPPORTED, "grouped GEMM: too many tiles");
+  *blocks = (unsigned)b;
+  return FMOE_OK;
+}
+
+template <typename T, int BM, int BN, int DMA>
+int launch_fwd(const GemmArgs& g, hipStream_t s) {
+  constexpr size_t lds = plain_lds<BM, BN>();
+  auto kern = plain_fwd_kernel<T, BM, BN, DMA>;
+  FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds);
+  const int tiles_n = ceil_div(g.out_feat, BN);
+  unsigned blocks = 0;
+  const int rc = round_up_blocks(tiles_n * (g.n_rows / BM + (int64_t)g.n_expert), &blocks);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds, s, g, tiles_n);
+  FMOE_LAUNCH_CHECK("gemm_plain");
+  return FMOE_OK;
+}
+
+template <typename T, int BM, int BN, int DMA>
+int launch_bwd(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
+  constexpr size_t lds = plain_lds<BM, BN>();
+  auto kern = plain_bwd_kernel<T, BM, BN, DMA>;
+  FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds);
+  const int tiles_n_d = gd.c ? ceil_div(gd.in_feat, BN) : 0;
+  const int tiles_n_w = gw.c ? ceil_div(gw.in_feat, BN) : 0;
+  const int tiles_m_w = ceil_div(gw.out_feat, BM);
+  unsigned blocks = 0;
+  const int rc = round_up_blocks(tiles_n_d * (gd.n_rows / BM + (int64_t)gd.n_expert) +
+                                     (int64_t)tiles_n_w * tiles_m_w * gw.n_expert, &blocks);
+  if (rc || blocks == 0) return rc;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds, s, gd, gw, tiles_n_d, tiles_n_w,
+                     tiles_m_w);
+  FMOE_LAUNCH_CHECK("gemm_plain_bwd");
+  return FMOE_OK;
+}
+
+// Tile shape: the matrix cores of a CU take `us` per K slice of a tile, whatever the
+// number of workgroups that share them, and at least one whole tile is walked.  The tiles
+// of a launch are dealt over 256 CUs, half-way between evenly and in whole rounds.  The
+// shape with the least estimated time wins: the bigger one where there are enough tiles of
+// it, the smaller one where the chip would idle.
+struct Shape { int bm, bn; double us; };
+double rounds(double tiles) { return std::max(1.0, 0.5 * (tiles / 256 + ceil(tiles / 256))); }
+
+// every expert's last row tile is half empty on average
+double row_tiles(const GemmArgs& g, int bm) {
+  return (double)g.n_rows / bm + 0.5 * g.n_expert;
+}
+
+// Two stages and as many workgroups per CU as fit: they cover each other's waits better
+// than more stages do.  Measured in f32, forward / dX + dW, us (4 stages of the 64 x 64
+// tile, 2 of 128 x 128, 64 x 128, 64 x 64, against the register-staged 128 x 128 kernel
+// before):
+//   4 experts, 1024 rows, 128 -> 256       8.0/10.0  15.5/25.4  9.7/14.7  7.6/10.0  (26/50)
+//   8 experts, 4000 rows, 512 -> 2048      106/169   118/208    90/163    88/151    (110/250)
+//   8 experts, 4000 rows, 2048 -> 512      126/175   138/171    128/158   109/156   (160/255)
+//   32 experts, 15567 rows, 512 -> 2176    393/642   336/619    300/560   320/588
+//   64 experts, 32000 rows, 1024 -> 4096   2741/4897 2245/4288  2110/4261 2296/4460 (127 TFLOP/s)
+constexpr Shape kShapesF32[2] = {{64, 128, 1.06}, {64, 64, 0.56}};
+// bound by the address unit: 4-byte copies
+constexpr Shape kShapes16[2] = {{128, 128, 1.36}, {64, 64, 0.42}};
+
+int fwd_shape(const GemmArgs& g, const Shape (&shapes)[2], int es) {
+  if (g.tile) return (g.tile - 1) % 2;   // forced (tests)
+  const double slices = ceil_div((int64_t)g.in_feat * es, kSliceBytes);
+  double cost[2];
+  for (int i = 0; i < 2; ++i)
+    cost[i] = rounds(row_tiles(g, shapes[i].bm) * ceil_div(g.out_feat, shapes[i].bn)) * slices *
+              shapes[i].us;
+  return cost[0] <= cost[1] ? 0 : 1;
+}
+
+template <typename T, int DMA>
+int fwd_typed(const GemmArgs& g, hipStream_t s) {
+  if constexpr (std::is_same<T, float>::value) {
+    switch (fwd_shape(g, kShapesF32, 4)) {
+      case 0: return launch_fwd<T, 64, 128, DMA>(g, s);
+      default: return launch_fwd<T, 64, 64, DMA>(g, s);
+    }
+  } else {
+    switch (fwd_shape(g, kShapes16, 2)) {
+      case 0: return launch_fwd<T, 128, 128, DMA>(g, s);
+      default: return launch_fwd<T, 64, 64, DMA>(g, s);
+    }
+  }
+}
+
+// Both gradients share one shape: the estimate counts the tiles of both, each with its own
+// number of slices.
+int bwd_shape(const GemmArgs& gd, const GemmArgs& gw, const Shape (&shapes)[2], int es) {
+  const int forced = gd.tile ? gd.tile : gw.tile;
+  if (forced) return (forced - 1) % 2;
+  const double ks_d = gd.c ? ceil_div((int64_t)gd.out_feat * es, kSliceBytes) : 0;
+  const double ks_w = gw.c ? (double)gw.n_rows / gw.n_expert * es / kSliceBytes + 0.5 : 0;
+  double cost[2];
+  for (int i = 0; i < 2; ++i) {
+    const double td = row_tiles(gd, shapes[i].bm) * ceil_div(gd.in_feat, shapes[i].bn);
+    const double tw = (double)gw.n_expert * ceil_div(gw.out_feat, shapes[i].bm) *
+                      ceil_div(gw.in_feat, shapes[i].bn);
+    // (the last tiles to finish run alone for a while: a fifth of the longest)
+    const double longest = std::max(ks_d, ks_w);
+    cost[i] = std::max(longest, (td * ks_d + tw * ks_w) / 256 + 0.2 * longest) * shapes[i].us;
+  }
+  return cost[0] <= cost[1] ? 0 : 1;
+}
+
+template <typename T, int DMA>
+int bwd_typed(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
+  if constexpr (std::is_same<T, float>::value) {
+    switch (bwd_shape(gd, gw, kShapesF32, 4)) {
+      case 0: return launch_bwd<T, 64, 128, DMA>(gd, gw, s);
+      default: return launch_bwd<T, 64, 64, DMA>(gd, gw, s);
+    }
+  } else {
+    switch (bwd_shape(gd, gw, kShapes16, 2)) {
+      case 0: return launch_bwd<T, 128, 128, DMA>(gd, gw, s);
+      default: return launch_bwd<T, 64, 64, DMA>(gd, gw, s);
+    }
+  }
+}
+
+// bytes per lane of the copies: 16 where every row of every operand starts on a 16-byte
+// boundary, 4 where it starts on a 4-byte one, 0 = not this kernel's
+int copy_width(const GemmArgs& g, int dtype) {
+  const int es = (int)dtype_size(dtype);
+  const uintptr_t bases = (uintptr_t)g.a | (uintptr_t)g.b | (uintptr_t)g.c |
+                          (uintptr_t)g.act_pre | (uintptr_t)g.act_out;
+  const int64_t rows = ((int64_t)g.in_feat | g.out_feat) * es;
+  if (rows % 16 == 0 && bases % 16 == 0) return 16;
+  return rows % 4 == 0 && bases % 4 == 0 ? 4 : 0;
+}
+
+}  // namespace
+
+bool gemm_plain_supported(const GemmArgs& g, int dtype) {
+  if (dtype != FMOE_F32 && dtype != FMOE_BF16 && dtype != FMOE_F16) return false;
+  // tile-relative byte offsets are 32-bit: 128 rows of f32 are the bytes of 256 of bf16
+  if (!dma_ld_supported(g.in_feat) || !dma_ld_supported(g.out_feat)) return false;
+  if (dtype != FMOE_F32 && (g.act_pre || g.act_out)) return false;
+  return copy_width(g, dtype) != 0;
+}
+
+int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s) {
+  if (!gemm_plain_supported(g, dtype))
+    return set_error(FMOE_ERR_UNSUPPORTED, "grouped GEMM: rows not on 4-byte boundaries");
+  switch (dtype) {
+    case FMOE_F32:
+      return copy_width(g, dtype) == 16 ? fwd_typed<float, 16>(g, s) : fwd_typed<float, 4>(g, s);
+    case FMOE_F16: return fwd_typed<__half, 4>(g, s);
+    default: return fwd_typed<__hip_bfloat16, 4>(g, s);
+  }
+}
+
+int launch_gemm_plain_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s) {
+  if (!gemm_plain_supported(gd, dtype) || !gemm_plain_supported(gw, dtype))
+    return set_error(FMOE_ERR_UNSUPPORTED, "grouped GEMM: rows not on 4-byte boundaries");
+  switch (dtype) {
+    case FMOE_F32:
+      return copy_width(gd, dtype) == 16 && copy_width(gw, dtype) == 16
+                 ? bwd_typed<float, 16>(gd, gw, s)
+                 : bwd_typed<float, 4>(gd, gw, s);
+    case FMOE_F16: return bwd_typed<__half, 4>(gd, gw, s);
+    default: return bwd_typed<__hip_bfloat16, 4>(gd, gw, s);
+  }
+}
+
+}  // namespace fmoe

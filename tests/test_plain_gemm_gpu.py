@@ -1,0 +1,60 @@
+"""The plain-pipeline matrix-core GEMMs (f32 of any shape; bf16 / f16 whose feature sizes
+are even but no multiples of 8): every tile shape forced at sizes on and around the edges
+of its tiles and K slices, against float64; the f32 activation inside the tiles against
+the activation kernel, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import DTYPES, TOL, max_rel_err, randn
+from test_linear_gpu import _run
+
+pytestmark = pytest.mark.gpu
+
+# counts per expert, in_feat, out_feat
+EDGES = [
+    ([1], 2, 2),
+    ([64, 65, 0, 127, 129], 62, 66),
+    ([63, 128, 1, 0, 200], 130, 126),
+    ([33, 31, 0, 2], 258, 34),
+    ([70, 300], 36, 300),
+]
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("counts,in_f,out_f", EDGES)
+def test_every_tile_shape_at_its_edges(dt, tile, counts, in_f, out_f):
+    _run(counts, in_f, out_f, DTYPES[dt], True, tile + 1 if tile else 0, extra_rows=3)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("counts,in_f,out_f", [([64, 65, 0, 127], 64, 68), ([130, 5], 132, 128)])
+def test_f32_sixteen_byte_rows(tile, counts, in_f, out_f):
+    _run(counts, in_f, out_f, torch.float32, True, tile + 1 if tile else 0, extra_rows=1)
+
+
+@pytest.mark.parametrize("in_f,out_f", [(64, 132), (38, 66)])
+def test_f32_activation_inside_the_tiles(in_f, out_f):
+    from fastmoe_amd import fmoe_cuda
+
+    counts = [70, 0, 129, 3]
+    seg = torch.from_numpy(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)).cuda()
+    n, e = sum(counts), len(counts)
+    x, w, b = (randn(s, torch.float32, i, 0.5).cuda()
+               for i, s in enumerate([(n, in_f), (e, out_f, in_f), (e, out_f)]))
+    y, a = fmoe_cuda.grouped_linear_fwd(x, seg, w, b, with_gelu=True)
+    assert torch.equal(y, fmoe_cuda.grouped_linear_fwd(x, seg, w, b))
+    assert torch.equal(a, fmoe_cuda.gelu_fwd(y))
+    dy = randn((n, out_f), torch.float32, 7).cuda()
+    pre = randn((n, in_f), torch.float32, 8).cuda()
+    dx, dw, db = fmoe_cuda.grouped_linear_bwd(dy, x, seg, w, act_pre=pre)
+    dh, dw0, db0 = fmoe_cuda.grouped_linear_bwd(dy, x, seg, w)
+    assert torch.equal(dw, dw0) and torch.equal(db, db0)
+    assert torch.equal(dx, fmoe_cuda.gelu_bwd(dh, pre))
+    # each product alone runs the same tiles
+    for kw, want in (({"need_dw": False, "need_bias": False}, (dh, None, None)),
+                     ({"need_dx": False}, (None, dw, db))):
+        for got, ref in zip(fmoe_cuda.grouped_linear_bwd(dy, x, seg, w, **kw), want):
+            assert (got is None) == (ref is None)
+            assert got is None or max_rel_err(got, ref) <= TOL[torch.float32]
