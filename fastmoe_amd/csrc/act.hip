@@ -25,6 +25,10 @@ constexpr int kTabBwd = 32768;           // entries: every pattern without its s
 // One copy per GPU; [0] = bf16, [1] = f16.
 __device__ uint16_t g_gelu_fwd_tab[2][kTabFwd];
 __device__ float g_gelu_bwd_tab[2][kTabBwd];
+// The same for ReLU; the backward one (for both types) by pattern of the activation, which is
+// never negative: 1 for zero, 0 for everything else, NaNs included.
+__device__ uint16_t g_relu_fwd_tab[2][kTabFwd];
+__device__ float g_relu_bwd_tab[kTabBwd];
 
 __device__ __forceinline__ double bits_to_double(int which, uint16_t b) {
   if (which == 0) return (double)__uint_as_float((uint32_t)b << 16);
@@ -44,6 +48,10 @@ __global__ void gelu_table_kernel() {
     g_gelu_fwd_tab[which][i] = float_to_bits(which, (float)gelu_f64(x));
     if (i < kTabBwd) g_gelu_bwd_tab[which][i] = (float)gelu_grad_f64(-x);
   }
+  // negative numbers to zero, negative NaNs as they are
+  g_relu_fwd_tab[0][i] = i >= 0x8000 && i <= 0xff80 ? 0 : (uint16_t)i;
+  g_relu_fwd_tab[1][i] = i >= 0x8000 && i <= 0xfc00 ? 0 : (uint16_t)i;
+  if (i < kTabBwd) g_relu_bwd_tab[i] = i == 0 ? 1.f : 0.f;
 }
 
 // Elements that need work: all n, or the first *n_rows_dev rows of row_len when
@@ -167,6 +175,31 @@ __global__ void gelu_bwd_direct_kernel(const T* __restrict__ dy, const T* __rest
     dx[i] = dy[i] * gelu_grad_direct(x[i]);
 }
 
+// ---- ReLU: 16-byte packs of any type, and a tail ------------------------------
+template <typename T>
+__device__ __forceinline__ bool positive_or_nan(T v) { return !(Elem<T>::to_acc(v) <= 0); }
+
+template <typename T, bool BWD>
+__global__ void relu_kernel(const T* __restrict__ dy, const T* __restrict__ x, T* __restrict__ out,
+                            int64_t n, const int32_t* __restrict__ n_rows_dev, int64_t row_len,
+                            bool packed) {
+  n = live_elems(n, n_rows_dev, row_len);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int kN = Pack16<T>::kN;
+  const int64_t n_packs = packed ? n / kN : 0;
+  for (int64_t i = t; i < n_packs; i += stride) {
+    const Pack16<T> a = reinterpret_cast<const Pack16<T>*>(x)[i];
+    const Pack16<T> b = BWD ? reinterpret_cast<const Pack16<T>*>(dy)[i] : a;
+    Pack16<T> o;
+#pragma unroll
+    for (int c = 0; c < kN; ++c) o.v[c] = positive_or_nan(a.v[c]) ? b.v[c] : Elem<T>::from_acc(0);
+    reinterpret_cast<Pack16<T>*>(out)[i] = o;
+  }
+  for (int64_t i = n_packs * kN + t; i < n; i += stride)
+    out[i] = positive_or_nan(x[i]) ? (BWD ? dy[i] : x[i]) : Elem<T>::from_acc(0);
+}
+
 // ---- host side ------------------------------------------------------------
 constexpr int kMaxDevices = 64;
 std::mutex g_setup_mutex;          // guards everything below
@@ -247,6 +280,52 @@ int gelu_fwd_table(int dtype, hipStream_t s, const uint16_t** table) {
   FMOE_HIP_CHECK(hipGetSymbolAddress((void**)&base, HIP_SYMBOL(g_gelu_fwd_tab)));
   *table = base + (dtype == FMOE_BF16 ? 0 : kTabFwd);
   return FMOE_OK;
+}
+
+int relu_fwd_table(int dtype, hipStream_t s, const uint16_t** table) {
+  int cus = 0;
+  const int rc = ensure_tables(s, &cus);
+  if (rc) return rc;
+  uint16_t* base = nullptr;
+  FMOE_HIP_CHECK(hipGetSymbolAddress((void**)&base, HIP_SYMBOL(g_relu_fwd_tab)));
+  *table = base + (dtype == FMOE_BF16 ? 0 : kTabFwd);
+  return FMOE_OK;
+}
+int relu_bwd_table(hipStream_t s, const float** table) {
+  int cus = 0;
+  const int rc = ensure_tables(s, &cus);
+  if (rc) return rc;
+  FMOE_HIP_CHECK(hipGetSymbolAddress((void**)table, HIP_SYMBOL(g_relu_bwd_tab)));
+  return FMOE_OK;
+}
+
+template <typename T, bool BWD>
+static int launch_relu(const void* dy, const void* x, void* out, int64_t n,
+                       const int32_t* n_rows_dev, int64_t row_len, hipStream_t s) {
+  const bool packed = aligned16(x) && aligned16(out) && (!BWD || aligned16(dy));
+  const int64_t work = packed ? n / Pack16<T>::kN + Pack16<T>::kN : n;
+  hipLaunchKernelGGL((relu_kernel<T, BWD>), dim3(direct_blocks(work)), dim3(256), 0, s, (const T*)dy,
+                     (const T*)x, (T*)out, n, n_rows_dev, row_len, packed);
+  FMOE_LAUNCH_CHECK("relu");
+  return FMOE_OK;
+}
+int relu_fwd(const void* x, void* y, int64_t n, const int32_t* n_rows_dev, int64_t row_len,
+             int dtype, hipStream_t s) {
+  switch (dtype) {
+    case FMOE_F32: return launch_relu<float, false>(nullptr, x, y, n, n_rows_dev, row_len, s);
+    case FMOE_F64: return launch_relu<double, false>(nullptr, x, y, n, n_rows_dev, row_len, s);
+    case FMOE_F16: return launch_relu<__half, false>(nullptr, x, y, n, n_rows_dev, row_len, s);
+    default: return launch_relu<__hip_bfloat16, false>(nullptr, x, y, n, n_rows_dev, row_len, s);
+  }
+}
+int relu_bwd(const void* dy, const void* x, void* dx, int64_t n, const int32_t* n_rows_dev,
+             int64_t row_len, int dtype, hipStream_t s) {
+  switch (dtype) {
+    case FMOE_F32: return launch_relu<float, true>(dy, x, dx, n, n_rows_dev, row_len, s);
+    case FMOE_F64: return launch_relu<double, true>(dy, x, dx, n, n_rows_dev, row_len, s);
+    case FMOE_F16: return launch_relu<__half, true>(dy, x, dx, n, n_rows_dev, row_len, s);
+    default: return launch_relu<__hip_bfloat16, true>(dy, x, dx, n, n_rows_dev, row_len, s);
+  }
 }
 
 }  // namespace fmoe

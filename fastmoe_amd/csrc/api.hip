@@ -116,19 +116,65 @@ static int check_linear(const char* who, int64_t n_rows, int64_t in_feat,
   return FMOE_OK;
 }
 
-static int run_gemm(int mode, const GemmArgs& g, int dtype, hipStream_t s) {
-  if (g_gemm_path == 0 && gemm_mfma_supported(mode, g, dtype))
-    return launch_gemm_mfma(mode, g, dtype, s);
-  if (g_gemm_path == 0 && gemm_plain_supported(g, dtype)) {
-    if (mode == GEMM_FWD) return launch_gemm_plain_fwd(g, dtype, s);
-    GemmArgs none = g;
-    none.c = nullptr;
-    return mode == GEMM_DGRAD ? launch_gemm_plain_bwd(g, none, dtype, s)
-                              : launch_gemm_plain_bwd(none, g, dtype, s);
+// Which family of kernels runs a product (fmoe_set_gemm_path may force one).
+enum Family { kScalar, kWide, kPlain, kBig };
+
+static Family fwd_family(const GemmArgs& g, int dtype) {
+  if (g_gemm_path != 0) return kScalar;
+  const bool plain = gemm_plain_supported(g, dtype);
+  if (gemm_mfma_supported(GEMM_FWD, g, dtype))
+    return plain && gemm_plain_fwd_preferred(g, dtype) ? kPlain : kBig;
+  if (plain) return kPlain;
+  return gemm_mfma_wide_supported(GEMM_FWD, g, dtype) ? kWide : kScalar;
+}
+
+// dX (gd) and dW (gw), either of which may be absent (c null).
+static Family bwd_family(const GemmArgs& gd, const GemmArgs& gw, int dtype) {
+  if (g_gemm_path != 0) return kScalar;
+  const bool plain = gemm_plain_supported(gd, dtype) && gemm_plain_supported(gw, dtype);
+  if ((!gd.c || gemm_mfma_supported(GEMM_DGRAD, gd, dtype)) &&
+      (!gw.c || gemm_mfma_supported(GEMM_WGRAD, gw, dtype)))
+    return plain && gemm_plain_bwd_preferred(gd, gw, dtype) ? kPlain : kBig;
+  if (plain) return kPlain;
+  return gemm_mfma_wide_supported(GEMM_DGRAD, gd, dtype) &&
+                 gemm_mfma_wide_supported(GEMM_WGRAD, gw, dtype) ? kWide : kScalar;
+}
+
+static int run_fwd(Family family, const GemmArgs& g, int dtype, hipStream_t s) {
+  switch (family) {
+    case kBig: return launch_gemm_mfma(GEMM_FWD, g, dtype, s);
+    case kPlain: return launch_gemm_plain_fwd(g, dtype, s);
+    case kWide: return launch_gemm_mfma_wide(GEMM_FWD, g, dtype, s);
+    default: return launch_gemm_simt(GEMM_FWD, g, dtype, s);
   }
-  if (g_gemm_path == 0 && gemm_mfma_wide_supported(mode, g, dtype))
-    return launch_gemm_mfma_wide(mode, g, dtype, s);
-  return launch_gemm_simt(mode, g, dtype, s);
+}
+
+static int run_bwd(Family family, const GemmArgs& gd, const GemmArgs& gw, int dtype,
+                   hipStream_t s) {
+  if (family == kPlain) return launch_gemm_plain_bwd(gd, gw, dtype, s);
+  if (family == kBig && gd.c && gw.c) return launch_gemm_mfma_bwd(gd, gw, dtype, s);
+  for (int mode : {GEMM_DGRAD, GEMM_WGRAD}) {
+    const GemmArgs& g = mode == GEMM_DGRAD ? gd : gw;
+    if (!g.c) continue;
+    const int rc = family == kBig ? launch_gemm_mfma(mode, g, dtype, s)
+                   : family == kWide ? launch_gemm_mfma_wide(mode, g, dtype, s)
+                                     : launch_gemm_simt(mode, g, dtype, s);
+    if (rc) return rc;
+  }
+  return FMOE_OK;
+}
+
+// Up to this many values the small 16-bit tiles look the activation up in its table in
+// memory while they store; a bigger product leaves it to the activation kernel, which
+// keeps the table in LDS.
+constexpr int64_t kTableInMemoryMax = 4 << 20;
+
+// The tables of a 16-bit activation.
+static int act_tables(int act, int dtype, hipStream_t s, GemmArgs* g, bool fwd) {
+  if (dtype != FMOE_BF16 && dtype != FMOE_F16) return FMOE_OK;
+  if (act == FMOE_ACT_RELU)
+    return fwd ? relu_fwd_table(dtype, s, &g->act_fwd_table) : relu_bwd_table(s, &g->act_table);
+  return fwd ? gelu_fwd_table(dtype, s, &g->act_fwd_table) : gelu_bwd_table(dtype, s, &g->act_table);
 }
 
 }  // namespace fmoe
@@ -160,7 +206,8 @@ extern "C" int fmoe_init(void* stream) {
 
 extern "C" int fmoe_set_gemm_path(int path) {
   FMOE_REQUIRE(path >= 0 && path <= 6, FMOE_ERR_INVALID, "gemm path must be 0..6");
-  // 2..5: matrix-core kernel with tile configuration 1..4 forced; 6: automatic, but
+  // 2..5: tile configuration 1..4 forced (16-bit types: 256 rows, 128, 64, 256 with K slices of
+  // 64 in two stages; f32 and odd feature sizes: their larger, smaller shape); 6: automatic, but
   // the forward activation runs as a kernel of its own behind the GEMM
   g_gemm_path = path == 1 ? 1 : 0;
   g_tile = path >= 2 && path <= 5 ? path - 1 : 0;
@@ -201,46 +248,58 @@ extern "C" int fmoe_seg_off_from_host_counts(const int64_t* expert_count_host,
 }
 
 // Forward of the grouped linear layer, with the weights (and the bias) as one
-// [E, ...] array or as tables of per-expert pointers, and optionally the activation
-// behind it: y_act = gelu(y) from the same tiles where the bf16 matrix-core kernel
-// runs, by the activation kernel over y otherwise.
+// [E, ...] array or as tables of per-expert pointers, and optionally an activation
+// behind it: y_act = act(y) from the same tiles where the kernel can, by the activation
+// kernel over y otherwise.  With an activation y may be null (not kept).
 static int linear_fwd(const char* who, const void* x, const void* w, const void* const* w_table,
                       const void* bias, const void* const* bias_table, const int32_t* seg_off,
-                      void* y, void* y_act, bool want_act, int64_t n_rows, int64_t in_feat,
+                      void* y, void* y_act, int act, int64_t n_rows, int64_t in_feat,
                       int64_t out_feat, int64_t n_expert, int dtype, void* stream) {
   int rc = check_linear(who, n_rows, in_feat, out_feat, n_expert, dtype);
   if (rc) return rc;
+  FMOE_REQUIRE(act >= FMOE_ACT_NONE && act <= FMOE_ACT_RELU, FMOE_ERR_INVALID,
+               "%s: unknown activation %d", who, act);
   if (n_rows == 0) return FMOE_OK;
-  FMOE_REQUIRE(x && (w || w_table) && seg_off && y && (y_act || !want_act), FMOE_ERR_INVALID,
+  FMOE_REQUIRE(x && (w || w_table) && seg_off && (act ? y_act : y), FMOE_ERR_INVALID,
                "%s: null pointer", who);
   hipStream_t s = (hipStream_t)stream;
-  GemmArgs g{x, w, y, bias, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
+  GemmArgs g{x, w, y ? y : y_act, bias, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   g.w_table = w_table;
   g.bias_table = bias_table;
-  if (!want_act) return run_gemm(GEMM_FWD, g, dtype, s);
-  // Worth it from about 768 rows per expert on (measured: 12 % of GEMM + activation
-  // kernel at 1024 rows per expert, 5 % at 4096, level at 512, where half of the tiles
-  // are remainder tiles that pay the table and the second store for few rows); a
-  // forced tile shape (tests, tuning) takes the fused tiles at any size.
-  const bool fused = dtype == FMOE_BF16 && g_gemm_path == 0 && (uintptr_t)y_act % 16 == 0 &&
-                     g_fuse_fwd_act && (g_tile != 0 || n_rows >= 768 * n_expert) &&
-                     gemm_mfma_supported(GEMM_FWD, g, dtype);
+  Family family = fwd_family(g, dtype);
+  if (!act) return run_fwd(family, g, dtype, s);
+  // 256-row tiles: worth it from about 768 rows per expert on (measured: 12 % of GEMM +
+  // activation kernel at 1024 rows per expert, 5 % at 4096, level at 512, where half of the
+  // tiles are remainder tiles that pay the table and the second store for few rows).  Small
+  // tiles: f32 always (the activation costs what evaluating it costs either way, and the
+  // pass over memory is saved).  A forced tile shape (tests, tuning) fuses at any size.
+  bool fused = g_fuse_fwd_act && (uintptr_t)y_act % 16 == 0;
+  if (family == kBig)
+    fused = fused && dtype == FMOE_BF16 && (g_tile != 0 || n_rows >= 768 * n_expert);
+  else if (family == kPlain)
+    fused = fused && (dtype == FMOE_F32 || g_tile != 0 || n_rows * out_feat <= kTableInMemoryMax);
+  else
+    fused = false;
+  // A pre-activation whose sign is decided in its last bit switches a whole gradient on or
+  // off behind a ReLU: feature sizes off the 8-element grid keep the sums in ascending order.
+  if (act == FMOE_ACT_RELU && dtype != FMOE_F32 && family == kPlain &&
+      !gemm_mfma_supported(GEMM_FWD, g, dtype)) {
+    family = kScalar;
+    fused = false;
+  }
   if (fused) {
-    rc = gelu_fwd_table(dtype, s, &g.act_fwd_table);
+    g.act = act;
+    g.act_out = y_act;
+    g.c = y;
+    rc = act_tables(act, dtype, s, &g, true);
     if (rc) return rc;
-    g.act_out = y_act;
-    return launch_gemm_mfma(GEMM_FWD, g, dtype, s);
+    return run_fwd(family, g, dtype, s);
   }
-  // f32: always inside the tiles (the activation costs what evaluating erf costs either
-  // way, and the pass over memory is saved)
-  if (dtype == FMOE_F32 && g_gemm_path == 0 && g_fuse_fwd_act) {
-    g.act_out = y_act;
-    if (gemm_plain_supported(g, dtype)) return launch_gemm_plain_fwd(g, dtype, s);
-    g.act_out = nullptr;
-  }
-  rc = run_gemm(GEMM_FWD, g, dtype, s);
+  rc = run_fwd(family, g, dtype, s);
   if (rc) return rc;
-  return fmoe_gelu_fwd(y, y_act, n_rows * out_feat, seg_off + n_expert, out_feat, dtype, stream);
+  if (act == FMOE_ACT_RELU)
+    return relu_fwd(g.c, y_act, n_rows * out_feat, seg_off + n_expert, out_feat, dtype, s);
+  return fmoe_gelu_fwd(g.c, y_act, n_rows * out_feat, seg_off + n_expert, out_feat, dtype, stream);
 }
 
 extern "C" int fmoe_grouped_linear_fwd(const void* x, const void* w,
@@ -249,15 +308,16 @@ extern "C" int fmoe_grouped_linear_fwd(const void* x, const void* w,
                                        int64_t out_feat, int64_t n_expert,
                                        int dtype, void* stream) {
   return linear_fwd("grouped_linear_fwd", x, w, nullptr, bias, nullptr, seg_off, y, nullptr,
-                    false, n_rows, in_feat, out_feat, n_expert, dtype, stream);
+                    FMOE_ACT_NONE, n_rows, in_feat, out_feat, n_expert, dtype, stream);
 }
 
 extern "C" int fmoe_grouped_linear_fwd_act(const void* x, const void* w, const void* bias,
                                            const int32_t* seg_off, void* y, void* y_act,
                                            int64_t n_rows, int64_t in_feat, int64_t out_feat,
                                            int64_t n_expert, int dtype, void* stream) {
+  FMOE_REQUIRE(n_rows == 0 || y != nullptr, FMOE_ERR_INVALID, "grouped_linear_fwd_act: y is null");
   return linear_fwd("grouped_linear_fwd_act", x, w, nullptr, bias, nullptr, seg_off, y, y_act,
-                    true, n_rows, in_feat, out_feat, n_expert, dtype, stream);
+                    FMOE_ACT_GELU, n_rows, in_feat, out_feat, n_expert, dtype, stream);
 }
 
 extern "C" int fmoe_grouped_linear_fwd_ptrs(const void* x, const void* const* w_ptrs,
@@ -265,8 +325,19 @@ extern "C" int fmoe_grouped_linear_fwd_ptrs(const void* x, const void* const* w_
                                             const int32_t* seg_off, void* y, void* y_act,
                                             int64_t n_rows, int64_t in_feat, int64_t out_feat,
                                             int64_t n_expert, int dtype, void* stream) {
+  FMOE_REQUIRE(n_rows == 0 || y != nullptr, FMOE_ERR_INVALID,
+               "grouped_linear_fwd_ptrs: y is null");
   return linear_fwd("grouped_linear_fwd_ptrs", x, nullptr, w_ptrs, nullptr, bias_ptrs, seg_off, y,
-                    y_act, y_act != nullptr, n_rows, in_feat, out_feat, n_expert, dtype, stream);
+                    y_act, y_act ? FMOE_ACT_GELU : FMOE_ACT_NONE, n_rows, in_feat, out_feat, n_expert, dtype, stream);
+}
+
+extern "C" int fmoe_expert_linear_fwd(const void* x, const void* w, const void* const* w_ptrs,
+                                      const void* bias, const void* const* bias_ptrs,
+                                      const int32_t* seg_off, void* y, void* y_act, int act,
+                                      int64_t n_rows, int64_t in_feat, int64_t out_feat,
+                                      int64_t n_expert, int dtype, void* stream) {
+  return linear_fwd("expert_linear_fwd", x, w, w_ptrs, bias, bias_ptrs, seg_off, y, y_act, act,
+                    n_rows, in_feat, out_feat, n_expert, dtype, stream);
 }
 
 // A device array of pointers from a host array, written by a small kernel that
@@ -293,72 +364,50 @@ extern "C" int fmoe_pointer_table(const void* const* host_ptrs, int64_t n, const
 }
 
 // Backward of the grouped linear layer; with act_pre, dx is further multiplied
-// by gelu'(act_pre): inside the DGRAD tiles' epilogue where the bf16 matrix-core
-// kernel runs, by the activation kernel over dx otherwise.
+// by act'(act_pre): inside the dX tiles where the kernel can, by the activation kernel over
+// dx otherwise.  ReLU: act_pre may be the activation itself.
 static int linear_bwd(const void* dy, const void* x, const void* w, const void* const* w_table,
-                      const int32_t* seg_off,
-                      const void* act_pre, void* dx, void* dw, void* dbias, int64_t n_rows,
-                      int64_t in_feat, int64_t out_feat, int64_t n_expert, int dtype,
-                      void* stream) {
+                      const int32_t* seg_off, const void* act_pre, int act, void* dx, void* dw,
+                      void* dbias, int64_t n_rows, int64_t in_feat, int64_t out_feat,
+                      int64_t n_expert, int dtype, void* stream) {
   int rc = check_linear("grouped_linear_bwd", n_rows, in_feat, out_feat, n_expert, dtype);
   if (rc) return rc;
   FMOE_REQUIRE(seg_off != nullptr, FMOE_ERR_INVALID,
                "grouped_linear_bwd: seg_off is null");
   FMOE_REQUIRE(n_rows == 0 || dy != nullptr, FMOE_ERR_INVALID,
                "grouped_linear_bwd: dy is null");
+  FMOE_REQUIRE(n_rows == 0 || !dx || w || w_table, FMOE_ERR_INVALID,
+               "grouped_linear_bwd: w is null");
+  FMOE_REQUIRE(n_rows == 0 || !dw || x, FMOE_ERR_INVALID, "grouped_linear_bwd: x is null");
   hipStream_t s = (hipStream_t)stream;
-  // The matrix-core kernels for 16-bit types and f32 sum the columns of dY inside their dW
-  // tiles; f64 and the scalar kernel leave the bias gradient to the reduction kernel below.
+  if (n_rows == 0) dx = nullptr;   // (dw runs all the same: experts without rows get zeros)
   GemmArgs gw{dy, x, dw, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
-  const bool have_w = dw && g_gemm_path == 0 && (n_rows == 0 || x != nullptr);
-  const bool mfma_w = have_w && gemm_mfma_supported(GEMM_WGRAD, gw, dtype);
-  const bool plain_w = have_w && !mfma_w && gemm_plain_supported(gw, dtype);
-  if ((mfma_w || plain_w) && dbias) {
-    gw.bias = dbias;
-    dbias = nullptr;  // comes out of the dW launch
-  }
   GemmArgs gd{dy, w, dx, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   gd.w_table = w_table;
-  void* const dx_out = dx;
-  const bool act_here = act_pre && dx && n_rows > 0 && g_gemm_path == 0;
-  bool act_fused = false;
-  if (act_here && dtype == FMOE_BF16 && (uintptr_t)act_pre % 16 == 0 &&
-      gemm_mfma_supported(GEMM_DGRAD, gd, dtype)) {
-    rc = gelu_bwd_table(dtype, s, &gd.act_table);
-    if (rc) return rc;
-    gd.act_pre = act_pre;
-    act_fused = true;
-  } else if (act_here && dtype == FMOE_F32) {
-    gd.act_pre = act_pre;
-    act_fused = gemm_plain_supported(gd, dtype);
-    if (!act_fused) gd.act_pre = nullptr;
+  const Family family = bwd_family(gd, gw, dtype);
+  // The matrix-core kernels for 16-bit types and f32 sum the columns of dY inside their dW
+  // tiles; f64 and the scalar kernel leave the bias gradient to the reduction kernel below.
+  if (dw && dbias && (family == kBig || family == kPlain)) {
+    gw.bias = dbias;
+    dbias = nullptr;
   }
-  if (dx && dw && n_rows > 0 && g_gemm_path == 0) {
-    FMOE_REQUIRE((w != nullptr || w_table != nullptr) && x != nullptr, FMOE_ERR_INVALID,
-                 "grouped_linear_bwd: w or x is null");
-    if (gemm_mfma_supported(GEMM_DGRAD, gd, dtype) && mfma_w) {
-      rc = launch_gemm_mfma_bwd(gd, gw, dtype, s);
-      if (rc) return rc;
-      dx = nullptr;  // both products are under way
-      dw = nullptr;
-    } else if (plain_w && gemm_plain_supported(gd, dtype)) {
-      rc = launch_gemm_plain_bwd(gd, gw, dtype, s);
-      if (rc) return rc;
-      dx = nullptr;
-      dw = nullptr;
-    }
-  }
-  if (dx && n_rows > 0) {
-    FMOE_REQUIRE(w != nullptr || w_table != nullptr, FMOE_ERR_INVALID,
-                 "grouped_linear_bwd: w is null");
-    rc = run_gemm(GEMM_DGRAD, gd, dtype, s);
+  bool act_fused = act_pre && dx && (uintptr_t)act_pre % 16 == 0;
+  if (family == kBig)
+    act_fused = act_fused && dtype == FMOE_BF16;
+  else if (family == kPlain)
+    // (f16 GELU: the activation kernel rounds its product once, not through f32 first)
+    act_fused = act_fused && (dtype != FMOE_F16 || act == FMOE_ACT_RELU) &&
+                (dtype == FMOE_F32 || g_tile != 0 || n_rows * in_feat <= kTableInMemoryMax);
+  else
+    act_fused = false;
+  if (act_fused) {
+    gd.act = act;
+    gd.act_pre = act_pre;
+    rc = act_tables(act, dtype, s, &gd, false);
     if (rc) return rc;
   }
-  if (dw) {
-    // runs also for n_rows == 0: experts without rows get zero gradients
-    FMOE_REQUIRE(n_rows == 0 || x != nullptr, FMOE_ERR_INVALID,
-                 "grouped_linear_bwd: x is null");
-    rc = run_gemm(GEMM_WGRAD, gw, dtype, s);
+  if (dx || dw) {
+    rc = run_bwd(family, gd, gw, dtype, s);
     if (rc) return rc;
   }
   if (dbias) {
@@ -370,10 +419,13 @@ static int linear_bwd(const void* dy, const void* x, const void* w, const void* 
     }
     if (rc) return rc;
   }
-  if (act_pre && !act_fused && dx_out && n_rows > 0)
+  if (act_pre && !act_fused && dx) {
     // rows of experts only: the device-side row total is the table's last entry
-    return fmoe_gelu_bwd(dx_out, act_pre, dx_out, n_rows * in_feat, seg_off + n_expert, in_feat,
-                         dtype, stream);
+    if (act == FMOE_ACT_RELU)
+      return relu_bwd(dx, act_pre, dx, n_rows * in_feat, seg_off + n_expert, in_feat, dtype, s);
+    return fmoe_gelu_bwd(dx, act_pre, dx, n_rows * in_feat, seg_off + n_expert, in_feat, dtype,
+                         stream);
+  }
   return FMOE_OK;
 }
 
@@ -383,7 +435,7 @@ extern "C" int fmoe_grouped_linear_bwd(const void* dy, const void* x,
                                        int64_t n_rows, int64_t in_feat,
                                        int64_t out_feat, int64_t n_expert,
                                        int dtype, void* stream) {
-  return linear_bwd(dy, x, w, nullptr, seg_off, nullptr, dx, dw, dbias, n_rows, in_feat,
+  return linear_bwd(dy, x, w, nullptr, seg_off, nullptr, FMOE_ACT_NONE, dx, dw, dbias, n_rows, in_feat,
                     out_feat, n_expert, dtype, stream);
 }
 
@@ -395,7 +447,7 @@ extern "C" int fmoe_grouped_linear_bwd_act(const void* dy, const void* x,
                                            int dtype, void* stream) {
   FMOE_REQUIRE(act_pre != nullptr || n_rows == 0 || dx == nullptr, FMOE_ERR_INVALID,
                "grouped_linear_bwd_act: act_pre is null");
-  return linear_bwd(dy, x, w, nullptr, seg_off, act_pre, dx, dw, dbias, n_rows, in_feat,
+  return linear_bwd(dy, x, w, nullptr, seg_off, act_pre, FMOE_ACT_GELU, dx, dw, dbias, n_rows, in_feat,
                     out_feat, n_expert, dtype, stream);
 }
 
@@ -407,6 +459,20 @@ extern "C" int fmoe_grouped_linear_bwd_ptrs(const void* dy, const void* x,
                                             int dtype, void* stream) {
   FMOE_REQUIRE(w_ptrs != nullptr || dx == nullptr || n_rows == 0, FMOE_ERR_INVALID,
                "grouped_linear_bwd_ptrs: w_ptrs is null");
-  return linear_bwd(dy, x, nullptr, w_ptrs, seg_off, act_pre, dx, dw, dbias, n_rows, in_feat,
+  return linear_bwd(dy, x, nullptr, w_ptrs, seg_off, act_pre, FMOE_ACT_GELU, dx, dw, dbias, n_rows, in_feat,
                     out_feat, n_expert, dtype, stream);
+}
+
+extern "C" int fmoe_expert_linear_bwd(const void* dy, const void* x, const void* w,
+                                      const void* const* w_ptrs, const int32_t* seg_off,
+                                      const void* act_pre, int act, void* dx, void* dw,
+                                      void* dbias, int64_t n_rows, int64_t in_feat,
+                                      int64_t out_feat, int64_t n_expert, int dtype,
+                                      void* stream) {
+  FMOE_REQUIRE(act >= FMOE_ACT_NONE && act <= FMOE_ACT_RELU, FMOE_ERR_INVALID,
+               "expert_linear_bwd: unknown activation %d", act);
+  FMOE_REQUIRE(act == FMOE_ACT_NONE || act_pre != nullptr || n_rows == 0 || dx == nullptr,
+               FMOE_ERR_INVALID, "expert_linear_bwd: act_pre is null");
+  return linear_bwd(dy, x, w, w_ptrs, seg_off, act == FMOE_ACT_NONE ? nullptr : act_pre, act, dx,
+                    dw, dbias, n_rows, in_feat, out_feat, n_expert, dtype, stream);
 }

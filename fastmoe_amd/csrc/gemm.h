@@ -39,6 +39,8 @@ struct GemmArgs {
   // FWD on the bf16 matrix-core and f32 kernels only: if not null, act_out
   // [n_rows, out_feat] receives gelu(y) next to y; bf16 through act_fwd_table, the device
   // table of gelu(x) by 16-bit pattern of x (gelu_fwd_table()).
+  // With act_out the forward product's c may be null: only the activation is wanted.
+  int act = FMOE_ACT_GELU;      // fmoe_activation behind act_pre / act_out
   void* act_out = nullptr;
   const uint16_t* act_fwd_table = nullptr;
   // Experts whose parameters are separate allocations (the reference keeps one module
@@ -88,6 +90,16 @@ constexpr int kActTabLdsOffset = 256 * (256 + 8) * 2;   // bytes from the start 
 int gelu_bwd_table(int dtype, hipStream_t s, const float** table);
 // Device table of gelu(x) by the 16-bit pattern of x (65536 results of the dtype).
 int gelu_fwd_table(int dtype, hipStream_t s, const uint16_t** table);
+// The same two for ReLU: a forward table of max(x, 0) by pattern, and (for either dtype)
+// 1 - relu'(a) by pattern of the ACTIVATION a = relu(x) (never negative), so that the
+// kernels' rule "a positive argument takes 1 - the entry" holds for both activations.
+int relu_fwd_table(int dtype, hipStream_t s, const uint16_t** table);
+int relu_bwd_table(hipStream_t s, const float** table);
+// y = max(x, 0) and dx = x > 0 ? dy : 0 (NaN passes), over the first *n_rows_dev rows
+int relu_fwd(const void* x, void* y, int64_t n, const int32_t* n_rows_dev, int64_t row_len,
+             int dtype, hipStream_t s);
+int relu_bwd(const void* dy, const void* x, void* dx, int64_t n, const int32_t* n_rows_dev,
+             int64_t row_len, int dtype, hipStream_t s);
 
 // Virtual row-tile index space of the scalar kernel: expert e owns the tiles
 // from seg_off[e] / BM + e on (the starts are strictly increasing, so tiles
@@ -108,10 +120,14 @@ int launch_gemm_mfma(int mode, const GemmArgs& g, int dtype, hipStream_t s);
 // grouped linear, in one launch where the tile shapes allow it.
 int launch_gemm_mfma_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s);
 
-// f32 grouped GEMM of any shape and bf16 / f16 of even feature sizes on the matrix cores.
-// f32 applies the activation inside its tiles: act_out (forward) and act_pre (dX) without
-// a table.
+// f32 grouped GEMM of any shape and bf16 / f16 of even feature sizes on the matrix cores,
+// the activation inside the tiles: act_out (forward) and act_pre (dX), for the 16-bit types
+// through act_fwd_table / act_table.
 bool gemm_plain_supported(const GemmArgs& g, int dtype);
+// Whether these kernels are expected to beat the 256-row ones (16-bit types that both take;
+// always for f32, which only these take).
+bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype);
+bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype);
 int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s);
 // dX (gd) and dW (gw) in one launch; a null gd.c or gw.c leaves that product out.
 int launch_gemm_plain_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s);

@@ -706,7 +706,9 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
   // per-row condition; a pack past the last column (N is a multiple of 8: a pack
   // is all in or all out) gets an offset no descriptor reaches.
   const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(C + (int64_t)m0 * ldc + n0), (short)0, ((m_valid - 1) * ldc + n_valid) * 2,
+      (void*)(C + (int64_t)m0 * ldc + n0), (short)0,
+      // (FWD_ACT without a place for the pre-activations: an empty descriptor drops the stores)
+      MODE == GEMM_FWD_ACT && g.c == nullptr ? 0 : ((m_valid - 1) * ldc + n_valid) * 2,
       kRsrcFlags);
   const int c_off = n0 + pk * 8 < N ? (r0 * ldc + pk * 8) * 2 : (int)kOutOfRange;
   // FWD with the activation fused in (g.act_out): the tile is written twice, as it
@@ -1631,45 +1633,15 @@ static int launch_cfg(const GemmArgs& g, hipStream_t s) {
   return FMOE_OK;
 }
 
-// Tile shape by a small cost model: blocks run in rounds over the CUs that
-// take a block at a time (256 CUs; live tiles come first in launch order, so a
-// round is really 256 wide), a tile costs a fixed prologue/epilogue
-// plus a per-K-slice time that depends on its shape (measured microseconds).
-// The shape with the least estimated time wins; `g.tile` overrides the choice
-// for tuning (1..3 = the three shapes, 4 = 256x256 with two stages of 64).
-// Ragged experts add at most one partial tile each, which the estimate ignores.
-template <int MODE>
-static int pick_tile(const GemmArgs& g) {
-  if (g.tile >= 1 && g.tile <= 4) return g.tile;
-  const int64_t N = is_fwd(MODE) ? g.out_feat : g.in_feat;
-  const int64_t K = MODE == GEMM_WGRAD ? g.n_rows / g.n_expert
-                                       : (is_fwd(MODE) ? g.in_feat : g.out_feat);
-  auto cost = [&](int bm, int bn, double us_per_slice, int blocks_per_cu) -> double {
-    const int64_t tiles = MODE == GEMM_WGRAD
-        ? (int64_t)g.n_expert * ceil_div(g.out_feat, bm) * ceil_div(g.in_feat, bn)
-        : (int64_t)ceil_div(g.n_rows, bm) * ceil_div(N, bn);
-    const int64_t slots = 256 * blocks_per_cu;
-    const double rounds = (double)((tiles + slots - 1) / slots);
-    return rounds * (8.0 + (double)ceil_div(K, 32) * us_per_slice * blocks_per_cu);
-  };
-  const double c1 = cost(256, 256, 0.78, 1), c2 = cost(128, 256, 0.45, 1),
-               c3 = cost(128, 128, 0.27, 2);
-  return c1 <= c2 && c1 <= c3 ? 1 : (c2 <= c3 ? 2 : 3);
-}
-
+// Every product runs 256x256 tiles; what they do not suit (few rows, few tiles) goes to the
+// smaller tiles of gemm_plain.hip, by the estimate there.
 template <typename T, int MODE>
 static int launch_mode(const GemmArgs& g, hipStream_t s) {
-  switch (pick_tile<MODE>(g)) {
-    case 1:
-      // A [row][k] operand (both in FWD, dY in DGRAD) moves whole 128-byte
-      // lines with K slices of 64: measured 7-8% faster for FWD, 2% for DGRAD;
-      // WGRAD, with two [k][row] operands, is level with four stages of 32.
-      if constexpr (MODE != GEMM_WGRAD) return launch_cfg<T, 256, 256, 64, 2, 2, 2, MODE>(g, s);
-      else return launch_cfg<T, 256, 256, 32, 2, 2, 4, MODE>(g, s);
-    case 2: return launch_cfg<T, 128, 256, 32, 2, 2, 4, MODE>(g, s);
-    case 4: return launch_cfg<T, 256, 256, 64, 2, 2, 2, MODE>(g, s);
-    default: return launch_cfg<T, 128, 128, 32, 2, 2, 4, MODE>(g, s);
-  }
+  // A [row][k] operand (both in FWD, dY in DGRAD) moves whole 128-byte lines with K slices
+  // of 64: measured 7-8% faster for FWD, 2% for DGRAD; WGRAD, with two [k][row] operands,
+  // is level with four stages of 32.
+  if constexpr (MODE != GEMM_WGRAD) return launch_cfg<T, 256, 256, 64, 2, 2, 2, MODE>(g, s);
+  else return launch_cfg<T, 256, 256, 32, 2, 2, 4, MODE>(g, s);
 }
 
 template <typename T>
@@ -1732,19 +1704,12 @@ static int launch_bwd_fused(const GemmArgs& gd, const GemmArgs& gw, hipStream_t 
   return FMOE_OK;
 }
 
-// dX and dW in one launch when both products would use the 256x256 tiles
-// anyway; otherwise one launch each.
+// dX and dW in one launch.
 template <typename T>
 static int launch_bwd_t(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
-  const int pd = pick_tile<GEMM_DGRAD>(gd), pw = pick_tile<GEMM_WGRAD>(gw);
-  if (pd == 4 && pw == 4) return launch_bwd_fused<T, 64, 2>(gd, gw, s);  // forced
-  if (pd != 1 || pw != 1) {
-    const int rc = launch_t<T>(GEMM_DGRAD, gd, s);
-    return rc ? rc : launch_mode<T, GEMM_WGRAD>(gw, s);
-  }
   // K slices of 64 in two stages measured 2-3% faster than four stages of 32
   // when dW's K (the rows of an expert) is long, 2% slower at ~500 rows
-  if (gd.tile != 1 && gd.n_rows / gd.n_expert >= 1024)
+  if (gd.tile == 4 || (gd.tile != 1 && gd.n_rows / gd.n_expert >= 1024))
     return launch_bwd_fused<T, 64, 2>(gd, gw, s);
   return launch_bwd_fused<T, 32, 4>(gd, gw, s);
 }

@@ -76,10 +76,10 @@ template <> struct Half<__half> {
 
 // One operand tile: R rows of the M or N index by one K slice.  ES bytes per element, BLOCKS
 // 16-row blocks per wave, DMA bytes per lane and copy.
-template <int R, int ES, int BLOCKS, bool KC, int DMA>
+template <int R, int ES, int BLOCKS, bool KC, int DMA, int SB>
 struct SliceTile {
-  static constexpr int kBytes = R * kSliceBytes;
-  static constexpr int kBK = kSliceBytes / ES;                 // values of K per slice
+  static constexpr int kBytes = R * SB;
+  static constexpr int kBK = SB / ES;                 // values of K per slice
   static constexpr int kLoads = kBytes / (64 * DMA) / kWaves;  // copies per wave and slice
   static constexpr int kRowBytes = R * ES;                     // of a [k] row (not KC)
   static_assert(kBytes % (64 * DMA * kWaves) == 0 && kLoads >= 1, "tile must split evenly");
@@ -87,6 +87,7 @@ struct SliceTile {
   // which of the 8 packs of a [row][128 bytes] row holds pack p: rows that the lanes of
   // one read touch together differ in the bits used here
   static __device__ __forceinline__ int row_swizzle(int row) {
+    if (SB == 64) return ((row >> 4) & 1) | (((row >> 2) & 1) << 1);
     return (row / (ES == 4 ? BLOCKS : 2)) & 7;
   }
   // XOR of the 32-byte segment index of a [k] row (16-bit types)
@@ -102,7 +103,7 @@ struct SliceTile {
   // K value (inside the slice) of the bytes this lane copies in copy i (KC only)
   static __device__ __forceinline__ int copy_k(int i, int wave, int lane) {
     const int off = (wave * kLoads + i) * 64 * DMA + lane * DMA;
-    const int row = off / kSliceBytes, in = off % kSliceBytes;
+    const int row = off / SB, in = off % SB;
     return (((in / 16) ^ row_swizzle(row)) * 16 + in % 16) / ES;
   }
 
@@ -112,7 +113,7 @@ struct SliceTile {
     for (int i = 0; i < kLoads; ++i) {
       const int off = (wave * kLoads + i) * 64 * DMA + lane * DMA;
       if (KC) {
-        voff[i] = (uint32_t)(off / kSliceBytes * ld + copy_k(i, wave, lane)) * ES;
+        voff[i] = (uint32_t)(off / SB * ld + copy_k(i, wave, lane)) * ES;
       } else {
         const int k = off / kRowBytes, in = off % kRowBytes;
         const int r = (((in / 32) ^ k_swizzle(k)) * 32 + in % 32) / ES;
@@ -125,7 +126,7 @@ struct SliceTile {
                  : ((int64_t)(k_total - 1) * ld + r_span) * ES;
     remaining = ((int64_t)__builtin_amdgcn_readfirstlane((int)(bytes >> 32)) << 32) |
                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
-    step = __builtin_amdgcn_readfirstlane(KC ? kSliceBytes : kBK * ld * ES);
+    step = __builtin_amdgcn_readfirstlane(KC ? SB : kBK * ld * ES);
     k_left = k_total;
     const uint64_t p = (uint64_t)origin;
     rsrc[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
@@ -179,7 +180,7 @@ struct SliceTile {
 #pragma unroll
       for (int i = 0; i < BLOCKS; ++i) {
         const int row = row0 + a * BLOCKS + i;
-        const char* p = lds + row * kSliceBytes;
+        const char* p = lds + row * SB;
         if (DMA == 16) {
           const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + (((s * 2 + g) ^ row_swizzle(row)) * 16));
 #pragma unroll
@@ -213,7 +214,7 @@ struct SliceTile {
     if (KC) {
       const int row = row16 + (lane & 15);
       return *reinterpret_cast<const uint4*>(
-          lds + row * kSliceBytes + (((s * 4 + (lane >> 4)) ^ row_swizzle(row)) * 16));
+          lds + row * SB + (((s * 4 + (lane >> 4)) ^ row_swizzle(row)) * 16));
     }
     const int k = s * 32 + 8 * (lane >> 4) + ((lane & 15) >> 2);
     const int m = row16 + 4 * (lane & 3);
@@ -227,22 +228,53 @@ struct SliceTile {
   }
 };
 
-// The activation behind the forward product / in front of the backward one, f32 only.
-__device__ __forceinline__ float act_fwd(float v) { return gelu_direct(v); }
-__device__ __forceinline__ float act_bwd(float g, float pre) { return g * gelu_grad_direct(pre); }
+// A tile's shape and pipeline: BM x BN outputs, NS stages of SB bytes per operand row.
+template <int BM_, int BN_, int NS_, int SB_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, NS = NS_, SB = SB_;
+  // pipeline stages; the 16-bit epilogue stages an output tile in the same place
+  static constexpr size_t kLds = std::max((size_t)NS * (BM + BN) * SB, (size_t)BM * (BN + 8) * 2);
+};
+// workgroups per CU that LDS allows, at most 4 (the registers are budgeted for them)
+constexpr int workgroups_per_cu(size_t lds) {
+  return std::min<int>(4, (int)(160 * 1024 / (lds + 128)));
+}
 
-template <typename T, int BM, int BN, int MODE, int DMA>
+// The activation behind the forward product and in front of the backward one.  GELU of the
+// 16-bit types comes from the activation kernels' tables in memory (they stay in L2; these
+// are small products), ReLU takes the activation itself as `pre`: its sign is all it needs.
+// A NaN stays one in both directions, as in torch.
+__device__ __forceinline__ float act_fwd(const GemmArgs& g, float v) {
+  return g.act == FMOE_ACT_RELU ? (v < 0.f ? 0.f : v) : gelu_direct(v);
+}
+__device__ __forceinline__ float act_bwd(const GemmArgs& g, float d, float pre) {
+  return g.act == FMOE_ACT_RELU ? (pre <= 0.f ? 0.f : d) : d * gelu_grad_direct(pre);
+}
+__device__ __forceinline__ uint16_t act_fwd16(const GemmArgs& g, uint16_t v) {
+  return load_global<uint16_t>(g.act_fwd_table + v);
+}
+template <typename T>
+__device__ __forceinline__ uint16_t act_bwd16(const GemmArgs& g, uint16_t d, uint16_t pre) {
+  const float n = load_global<float>(g.act_table + (pre & 0x7fffu));
+  return __builtin_bit_cast(uint16_t, Elem<T>::from_acc(
+      Elem<T>::to_acc(__builtin_bit_cast(T, d)) * ((pre & 0x8000u) ? n : 1.f - n)));
+}
+
+template <typename T, typename S, int MODE, int DMA>
 __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRows where,
                                            int n_origin) {
+  constexpr int BM = S::BM, BN = S::BN, NS = S::NS, SB = S::SB;
   constexpr bool kF32 = std::is_same<T, float>::value;
   constexpr int ES = sizeof(T);
   // blocks of a wave: 32x32 for f32, 16x16 for the 16-bit types
   constexpr int TM = BM / 2 / (kF32 ? 32 : 16), TN = BN / 2 / (kF32 ? 32 : 16);
   using Acc = typename std::conditional<kF32, f32x16_t, f32x4_t>::type;
   constexpr bool A_KC = MODE != GEMM_WGRAD, B_KC = MODE == GEMM_FWD;
-  using ATile = SliceTile<BM, ES, TM, A_KC, DMA>;
-  using BTile = SliceTile<BN, ES, TN, B_KC, DMA>;
+  using ATile = SliceTile<BM, ES, TM, A_KC, DMA, SB>;
+  using BTile = SliceTile<BN, ES, TN, B_KC, DMA, SB>;
   constexpr int kStage = ATile::kBytes + BTile::kBytes;
+  constexpr int kLoads = ATile::kLoads + BTile::kLoads;
+  static_assert((NS - 2) * kLoads < 64, "vmcnt is a 6-bit counter");
   static_assert(!kF32 || (TM <= 2 && TN <= 2), "fragment reads cover 1 or 2 blocks");
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -296,25 +328,29 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
   for (int i = 0; i < TM; ++i) cs[i] = 0.f;
 
   const int k_tiles = (K + ATile::kBK - 1) / ATile::kBK;
-  ta.issue(lds_base, wave);
-  tb.issue(lds_base + ATile::kBytes, wave);
-  ta.advance(wave, lane);
-  tb.advance(wave, lane);
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) {
+    ta.issue(lds_base + s * kStage, wave);
+    tb.issue(lds_base + s * kStage + ATile::kBytes, wave);
+    ta.advance(wave, lane);
+    tb.advance(wave, lane);
+  }
+  int stage = 0;
   for (int kt = 0; kt < k_tiles; ++kt) {
     // slice kt has landed here (my share) and, behind the barrier, everywhere; behind it
-    // nobody reads the stage of slice kt - 1 any more, which slice kt + 1 takes
-    const int stage = kt & 1;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // nobody reads the stage of slice kt - 1 any more, which slice kt + NS - 1 takes
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * kLoads) : "memory");
     __syncthreads();
-    ta.issue(lds_base + (stage ^ 1) * kStage, wave);
-    tb.issue(lds_base + (stage ^ 1) * kStage + ATile::kBytes, wave);
+    const int free_stage = stage == 0 ? NS - 1 : stage - 1;
+    ta.issue(lds_base + free_stage * kStage, wave);
+    tb.issue(lds_base + free_stage * kStage + ATile::kBytes, wave);
     ta.advance(wave, lane);
     tb.advance(wave, lane);
     const char* la = smem + stage * kStage;
     const char* lb = la + ATile::kBytes;
     if constexpr (kF32) {
 #pragma unroll
-      for (int s = 0; s < kSliceBytes / 32; ++s) {
+      for (int s = 0; s < SB / 32; ++s) {
         float fa[4][TM], fb[4][TN];
         ATile::frags32(la, wave_m * (BM / 2), s, lane, fa);
         BTile::frags32(lb, wave_n * (BN / 2), s, lane, fb);
@@ -333,7 +369,7 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
       }
     } else {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
+      for (int s = 0; s < SB / 64; ++s) {
         uint4 fa[TM], fb[TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i) fa[i] = ATile::frag16(la, wave_m * (BM / 2) + i * 16, s, lane);
@@ -355,8 +391,10 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
         }
       }
     }
+    stage = stage + 1 == NS ? 0 : stage + 1;
   }
-  // the zero-filled slices past the end of K are still landing
+  // the zero-filled slices past the end of K are still landing; behind the barrier the LDS
+  // is free to stage an output tile
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   const int a = lane & (kF32 ? 31 : 15), gr = lane / (kF32 ? 32 : 16);
@@ -403,9 +441,10 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
             for (int j = 0; j < TN; ++j) x.v[j] = col + j < N ? p[j] : 0.f;
           }
 #pragma unroll
-          for (int j = 0; j < TN; ++j) o.v[j] = act_bwd(o.v[j], x.v[j]);
+          for (int j = 0; j < TN; ++j) o.v[j] = act_bwd(g, o.v[j], x.v[j]);
         }
-        if (whole) {
+        if (MODE == GEMM_FWD && g.c == nullptr) {   // only the activation is wanted
+        } else if (whole) {
           *reinterpret_cast<Vec*>(C + at) = o;
         } else {
 #pragma unroll
@@ -415,7 +454,7 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
         if (MODE == GEMM_FWD && act_out) {
           float* q = act_out + (int64_t)row0 * ldc + at;
 #pragma unroll
-          for (int j = 0; j < TN; ++j) o.v[j] = act_fwd(o.v[j]);
+          for (int j = 0; j < TN; ++j) o.v[j] = act_fwd(g, o.v[j]);
           if (whole) {
             *reinterpret_cast<Vec*>(q) = o;
           } else {
@@ -426,47 +465,74 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
         }
       }
   } else {
-    // accumulator r of block (i, j): row 16 i + a, column 16 j + 4 gr + r of the patch; rows
-    // start on 4-byte boundaries and N is even, so a pair is all in or all out
-    struct alignas(4) Pair { T v[2]; };
+    // Accumulator r of block (i, j) is row 16 i + a, column 16 j + 4 gr + r of the patch: the
+    // tile goes through LDS (rows padded by 16 bytes) and leaves in units of 16 bytes (4
+    // where rows start on 4-byte boundaries), 128 to 256 contiguous bytes per row.
+    constexpr int kLdc = BN + 8, kUnit = DMA / 2;             // elements
+    constexpr int kRowUnits = BN / kUnit, kUnits = BM * kRowUnits / kThreads;
+  
+    using Unit = typename std::conditional<DMA == 16, uint4, uint32_t>::type;
+    uint16_t* staged = reinterpret_cast<uint16_t*>(smem);
+    // pre-activations (ReLU: activations) in front of the dX product: under way while the
+    // tile is staged
+    constexpr bool kDgrad = MODE == GEMM_DGRAD, kFwd = MODE == GEMM_FWD;
+    const uint16_t* pre = kDgrad ? (const uint16_t*)g.act_pre : nullptr;
+    Unit pv[kDgrad ? kUnits : 1];
+    if (kDgrad && pre) {
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u) {
+        const int m = (tid + u * kThreads) / kRowUnits, c = (tid + u * kThreads) % kRowUnits * kUnit;
+        pv[u] = Unit{};
+        if (m < m_valid && c < n_valid)
+          pv[u] = *reinterpret_cast<const Unit*>(pre + (int64_t)(row0 + m0 + m) * ldc + n0 + c);
+      }
+    }
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = n0 + wave_n * (BN / 2) + j * 16 + 4 * gr;
+      const int col = wave_n * (BN / 2) + j * 16 + 4 * gr;
       float bv[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        bv[r] = bias && col + r < N ? Elem<T>::to_acc(load_global<T>(bias + col + r)) : 0.f;
+        bv[r] = bias && n0 + col + r < N ? Elem<T>::to_acc(load_global<T>(bias + n0 + col + r)) : 0.f;
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        const int m = wave_m * (BM / 2) + i * 16 + a;
-        if (m >= m_valid) continue;
+        struct alignas(8) Quad { T v[4]; } o;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (col + 2 * h >= N) continue;
-          Pair o;
-          o.v[0] = Elem<T>::from_acc(acc[i][j][2 * h] + bv[2 * h]);
-          o.v[1] = Elem<T>::from_acc(acc[i][j][2 * h + 1] + bv[2 * h + 1]);
-          *reinterpret_cast<Pair*>(C + (int64_t)(m0 + m) * ldc + col + 2 * h) = o;
-        }
+        for (int r = 0; r < 4; ++r)
+          o.v[r] = Elem<T>::from_acc(kFwd ? acc[i][j][r] + bv[r] : acc[i][j][r]);
+        *reinterpret_cast<Quad*>(staged + (wave_m * (BM / 2) + i * 16 + a) * kLdc + col) = o;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      const int m = (tid + u * kThreads) / kRowUnits, c = (tid + u * kThreads) % kRowUnits * kUnit;
+      if (m >= m_valid || c >= n_valid) continue;   // N is a multiple of the unit
+      const int64_t at = (int64_t)(m0 + m) * ldc + n0 + c;
+      union { Unit u; uint16_t h[kUnit]; } v, p;
+      v.u = *reinterpret_cast<const Unit*>(staged + m * kLdc + c);
+      if (kDgrad && pre) {
+        p.u = pv[u];
+#pragma unroll
+        for (int q = 0; q < kUnit; ++q) v.h[q] = act_bwd16<T>(g, v.h[q], p.h[q]);
+      }
+      if (!kFwd || g.c) *reinterpret_cast<Unit*>(C + at) = v.u;
+      if (kFwd && g.act_out) {
+#pragma unroll
+        for (int q = 0; q < kUnit; ++q) v.h[q] = act_fwd16(g, v.h[q]);
+        *reinterpret_cast<Unit*>((uint16_t*)g.act_out + (int64_t)row0 * ldc + at) = v.u;
       }
     }
   }
 }
 
-template <int BM, int BN>
-constexpr size_t plain_lds() { return (size_t)2 * (BM + BN) * kSliceBytes; }
-// workgroups per CU the LDS allows, at most 4 (the registers are budgeted for them)
-template <int BM, int BN>
-constexpr int plain_blocks() {
-  constexpr int fit = 160 * 1024 / (int)(plain_lds<BM, BN>() + 128);
-  return fit < 4 ? fit : 4;
-}
-
-template <typename T, int BM, int BN, int DMA>
-__global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_fwd_kernel(GemmArgs g, int tiles_n) {
+template <typename T, typename S, int DMA>
+__global__ __launch_bounds__(kThreads, (workgroups_per_cu(S::kLds))) void plain_fwd_kernel(
+    GemmArgs g, int tiles_n) {
   extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
   __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
-  RowTiles<BM, false, kWaves> rows;
+  RowTiles<S::BM, false, kWaves> rows;
   rows.scan(g.seg_off, g.n_expert, s_wave_sum);
   const int live = rows.rows_f * tiles_n;
   if (live == 0) return;
@@ -475,18 +541,17 @@ __global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_fwd_
   int v, n_tile;
   tile_order(t, rows.rows_f, tiles_n, v, n_tile);
   const TileRows where = rows.find(g.seg_off, v, false, s_owner);
-  plain_tile<T, BM, BN, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * BN);
+  plain_tile<T, S, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * S::BN);
 }
 
-// dX and dW (with the bias gradient) in one launch, dX tiles first; either may be absent
-// (no tiles).
-template <typename T, int BM, int BN, int DMA>
-__global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_bwd_kernel(GemmArgs gd, GemmArgs gw,
-                                                                int tiles_n_d, int tiles_n_w,
-                                                                int tiles_m_w) {
+// dX (tiles D) and dW with the bias gradient (tiles W) in one launch, dX tiles first;
+// either may be absent (no tiles).
+template <typename T, typename D, typename W, int DMA>
+__global__ __launch_bounds__(kThreads, (workgroups_per_cu(std::max(D::kLds, W::kLds)))) void
+plain_bwd_kernel(GemmArgs gd, GemmArgs gw, int tiles_n_d, int tiles_n_w, int tiles_m_w) {
   extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
   __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
-  RowTiles<BM, false, kWaves> rows;
+  RowTiles<D::BM, false, kWaves> rows;
   rows.scan(gd.seg_off, gd.n_expert, s_wave_sum);
   const int live_d = rows.rows_f * tiles_n_d;
   const int per_expert_w = tiles_n_w * tiles_m_w;
@@ -499,18 +564,17 @@ __global__ __launch_bounds__(kThreads, (plain_blocks<BM, BN>())) void plain_bwd_
     int m_tile, n_tile;
     tile_order(tw % per_expert_w, tiles_m_w, tiles_n_w, m_tile, n_tile);
     const int row0 = gw.seg_off[e];
-    plain_tile<T, BM, BN, GEMM_WGRAD, DMA>(
-        gw, plain_smem, {e, m_tile * BM, row0, gw.seg_off[e + 1] - row0}, n_tile * BN);
+    plain_tile<T, W, GEMM_WGRAD, DMA>(
+        gw, plain_smem, {e, m_tile * W::BM, row0, gw.seg_off[e + 1] - row0}, n_tile * W::BN);
     return;
   }
   int v, n_tile;
   tile_order(t, rows.rows_f, tiles_n_d, v, n_tile);
   const TileRows where = rows.find(gd.seg_off, v, false, s_owner);
-  plain_tile<T, BM, BN, GEMM_DGRAD, DMA>(gd, plain_smem, where, n_tile * BN);
+  plain_tile<T, D, GEMM_DGRAD, DMA>(gd, plain_smem, where, n_tile * D::BN);
 }
 
 // ------------------------------------------------------------------ host side
-
 int round_up_blocks(int64_t tiles, unsigned* blocks) {
   const int64_t b = ceil_div(tiles, 8 * kXcdRun) * (int64_t)(8 * kXcdRun);
   FMOE_REQUIRE(b < ((int64_t)1 << 31), FMOE_ERR_UNSUPPORTED, "grouped GEMM: too many tiles");
@@ -518,30 +582,29 @@ int round_up_blocks(int64_t tiles, unsigned* blocks) {
   return FMOE_OK;
 }
 
-template <typename T, int BM, int BN, int DMA>
+template <typename T, typename S, int DMA>
 int launch_fwd(const GemmArgs& g, hipStream_t s) {
-  constexpr size_t lds = plain_lds<BM, BN>();
-  auto kern = plain_fwd_kernel<T, BM, BN, DMA>;
-  FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds);
-  const int tiles_n = ceil_div(g.out_feat, BN);
+  auto kern = plain_fwd_kernel<T, S, DMA>;
+  FMOE_SET_DYNAMIC_LDS_ONCE(kern, S::kLds);
+  const int tiles_n = ceil_div(g.out_feat, S::BN);
   unsigned blocks = 0;
-  const int rc = round_up_blocks(tiles_n * (g.n_rows / BM + (int64_t)g.n_expert), &blocks);
+  const int rc = round_up_blocks(tiles_n * (g.n_rows / S::BM + (int64_t)g.n_expert), &blocks);
   if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds, s, g, tiles_n);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), S::kLds, s, g, tiles_n);
   FMOE_LAUNCH_CHECK("gemm_plain");
   return FMOE_OK;
 }
 
-template <typename T, int BM, int BN, int DMA>
+template <typename T, typename D, typename W, int DMA>
 int launch_bwd(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
-  constexpr size_t lds = plain_lds<BM, BN>();
-  auto kern = plain_bwd_kernel<T, BM, BN, DMA>;
+  constexpr size_t lds = std::max(D::kLds, W::kLds);
+  auto kern = plain_bwd_kernel<T, D, W, DMA>;
   FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds);
-  const int tiles_n_d = gd.c ? ceil_div(gd.in_feat, BN) : 0;
-  const int tiles_n_w = gw.c ? ceil_div(gw.in_feat, BN) : 0;
-  const int tiles_m_w = ceil_div(gw.out_feat, BM);
+  const int tiles_n_d = gd.c ? ceil_div(gd.in_feat, D::BN) : 0;
+  const int tiles_n_w = gw.c ? ceil_div(gw.in_feat, W::BN) : 0;
+  const int tiles_m_w = ceil_div(gw.out_feat, W::BM);
   unsigned blocks = 0;
-  const int rc = round_up_blocks(tiles_n_d * (gd.n_rows / BM + (int64_t)gd.n_expert) +
+  const int rc = round_up_blocks(tiles_n_d * (gd.n_rows / D::BM + (int64_t)gd.n_expert) +
                                      (int64_t)tiles_n_w * tiles_m_w * gw.n_expert, &blocks);
   if (rc || blocks == 0) return rc;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds, s, gd, gw, tiles_n_d, tiles_n_w,
@@ -586,21 +649,6 @@ int fwd_shape(const GemmArgs& g, const Shape (&shapes)[2], int es) {
   return cost[0] <= cost[1] ? 0 : 1;
 }
 
-template <typename T, int DMA>
-int fwd_typed(const GemmArgs& g, hipStream_t s) {
-  if constexpr (std::is_same<T, float>::value) {
-    switch (fwd_shape(g, kShapesF32, 4)) {
-      case 0: return launch_fwd<T, 64, 128, DMA>(g, s);
-      default: return launch_fwd<T, 64, 64, DMA>(g, s);
-    }
-  } else {
-    switch (fwd_shape(g, kShapes16, 2)) {
-      case 0: return launch_fwd<T, 128, 128, DMA>(g, s);
-      default: return launch_fwd<T, 64, 64, DMA>(g, s);
-    }
-  }
-}
-
 // Both gradients share one shape: the estimate counts the tiles of both, each with its own
 // number of slices.
 int bwd_shape(const GemmArgs& gd, const GemmArgs& gw, const Shape (&shapes)[2], int es) {
@@ -620,18 +668,154 @@ int bwd_shape(const GemmArgs& gd, const GemmArgs& gw, const Shape (&shapes)[2], 
   return cost[0] <= cost[1] ? 0 : 1;
 }
 
+// ---- bf16 / f16 on 16-byte rows: this file's tiles or the 256-row kernels?
+//
+// Estimated microseconds of a launch from the experts' average number of rows (and what
+// random routing spreads around it).  Per tile: a fixed cost and a cost per K slice, alone
+// on its CU or sharing it; per launch: what HBM needs for the operands and results.  The
+// constants are fits to measured launches (us: 256-row kernels, 128 x 128, 64 x 64 tiles):
+//   forward  16 experts,   64 rows, 1024 -> 4096     25   24   25
+//            16,   64, 4096 -> 1024                  24   55   23
+//             8,  128, 14336 -> 4096                179  221  162
+//            32, 4096, 3072 -> 768                   81   41   49
+//            16, 6002, 768 -> 3072                   52   53   75
+//             8, 2000, 256 -> 1024                   13  8.4  7.2
+//           128, 16376, 2048 -> 1408                190  235  270
+//            32, 16000, 1024 -> 2048                 88  108  154
+//   dX + dW (and 64 x 64 dX tiles with 128 x 128 dW tiles of half slices)
+//            16,   64, 1024 -> 4096                  80   78   83  (61)
+//             8,  128, 14336 -> 4096                470  521  632  (382)
+//            32, 4096, 768 -> 3072                  143   92  140  (105)
+//             4, 1000, 256 -> 512                    16  9.6  7.1  (8.2)
+//             8, 8000, 512 -> 2048                   56   49   69  (71)
+//            32, 16000, 1024 -> 2048                167  196  275
+enum Kind { k256, k128, k64, kMixed };
+
+struct Spread {   // rows of an expert: three equally spaced points and their weights
+  double rows[3];
+  explicit Spread(const GemmArgs& g) {
+    const double r = (double)g.n_rows / g.n_expert, dev = std::max(sqrt(r), 0.03 * r);
+    rows[0] = std::max(0.0, r - dev);
+    rows[1] = r;
+    rows[2] = r + dev;
+  }
+  template <typename F> double mean(F f) const {
+    return 0.25 * f(rows[0]) + 0.5 * f(rows[1]) + 0.25 * f(rows[2]);
+  }
+};
+
+// Work of one product over the experts' rows (forward or dX): CU microseconds over all
+// tiles and the longest tile.  N columns, K values per sum.
+struct Work { double total, longest, tiles; };
+Work row_product(Kind kind, const GemmArgs& g, double N, double K, bool narrow_quarter) {
+  const Spread sp(g);
+  const double slices = ceil(K / 64);
+  if (kind == k256) {
+    const double cols = ceil(N / 128) / 2, tile = 8 + slices * 1.56;
+    double full = 0, half = 0, quarter = 0;
+    full = sp.mean([&](double r) { const double q = floor(r / 256); return q + (r - 256 * q > 128); });
+    half = sp.mean([&](double r) { const double m = r - 256 * floor(r / 256); return m > 64 && m <= 128; });
+    quarter = sp.mean([&](double r) { const double m = r - 256 * floor(r / 256); return m > 0 && m <= 64; });
+    full *= g.n_expert * cols;
+    half *= g.n_expert * cols;
+    quarter *= g.n_expert * cols;
+    Work w{full * tile + (half * 0.6 + quarter * 0.45) * tile, full > 0 ? tile : 0.6 * tile,
+           full + half + quarter};
+    if (K >= 2048 && half + quarter <= 128) {   // narrow remainder tiles
+      const double f = narrow_quarter ? 4 : 2, narrow = 4 + slices * (narrow_quarter ? 0.31 : 0.4);
+      w.total = full * tile + (half * 1.5 + quarter) * f * narrow;
+      w.longest = full > 0 ? tile : narrow;
+      w.tiles = full + (half + quarter) * f;
+    }
+    return w;
+  }
+  const double side = kind == k128 ? 128 : 64;
+  const double tiles = g.n_expert * sp.mean([&](double r) { return ceil(r / side); }) * ceil(N / side);
+  return kind == k128 ? Work{tiles * (slices * 0.65 + 0.8), slices * 0.8, tiles}
+                      : Work{tiles * (slices * 0.256 + 1.0), slices * 0.31, tiles};
+}
+
+// HBM time of one pass over the weights and `passes` over the rows of both sides; weights
+// are read again for every further row tile of an expert as far as caches do not hold them
+double memory_us(const GemmArgs& g, double weight_passes, double row_passes, double side) {
+  const double tiles = ceil((double)g.n_rows / g.n_expert / side);
+  const double again = std::min(2.0, 1 + 0.5 * std::max(0.0, tiles - 1));
+  return 2.0 * ((double)g.n_expert * g.in_feat * g.out_feat * (weight_passes - 1 + again) +
+                row_passes * g.n_rows * ((double)g.in_feat + g.out_feat)) / 5.3e6 + 3;
+}
+
+double launch_us(const Work& w, double tail) {
+  return w.tiles <= 256 ? w.longest : std::max(w.longest, w.total / 256 + tail * w.longest);
+}
+
+double fwd_us(Kind kind, const GemmArgs& g) {
+  const Work w = row_product(kind, g, g.out_feat, g.in_feat, true);
+  const double side = kind == k256 ? 256 : kind == k128 ? 128 : 64;
+  const double tiles = kind == k256 ? launch_us(w, 0.6) : 4 + launch_us(w, 0.15);
+  return std::max(tiles, memory_us(g, 1, 1, side));
+}
+
+double bwd_us(Kind kind, const GemmArgs& gd, const GemmArgs& gw) {
+  const double r = (double)gw.n_rows / gw.n_expert, E = gw.n_expert;
+  Work w{0, 0, 0};
+  if (gd.c) w = row_product(kind == kMixed ? k64 : kind, gd, gd.in_feat, gd.out_feat, false);
+  if (gw.c) {
+    const double side = kind == k256 ? 256 : kind == k64 ? 64 : 128;
+    const double n = E * ceil(gw.out_feat / side) * ceil(gw.in_feat / side);
+    const double tile = kind == k256 ? 8.7 + ceil(r / 32) * 0.7
+                        : kind == k128 ? 2.2 + ceil(r / 64) * 0.42
+                        : kind == kMixed ? 1.45 + ceil(r / 32) * 0.23 : 0.9 + ceil(r / 64) * 0.15;
+    w.total += n * tile;
+    w.longest = std::max(w.longest, tile * (kind == k256 ? 1 : 2));
+    w.tiles += n;
+  }
+  const double side = kind == k256 ? 256 : kind == k128 ? 128 : 64;
+  const double tiles = kind == k256 ? launch_us(w, 0.5) : 4 + launch_us(w, 0.3);
+  return std::max(tiles, memory_us(gw, (gd.c ? 1 : 0) + (gw.c ? 1 : 0), 1.5, side));
+}
+
+int bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
+  const double a = bwd_us(k128, gd, gw), b = bwd_us(kMixed, gd, gw), c = bwd_us(k64, gd, gw);
+  return a <= b && a <= c ? k128 : b <= c ? kMixed : k64;
+}
+
+template <typename T, int DMA>
+int fwd_typed(const GemmArgs& g, hipStream_t s) {
+  if constexpr (std::is_same<T, float>::value) {
+    return fwd_shape(g, kShapesF32, 4) == 0 ? launch_fwd<T, Tile<64, 128, 2, 128>, DMA>(g, s)
+                                            : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
+  } else if constexpr (DMA == 16) {
+    const bool big = g.tile ? g.tile != 3 : fwd_us(k128, g) <= fwd_us(k64, g);
+    return big ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
+               : launch_fwd<T, Tile<64, 64, 4, 128>, DMA>(g, s);
+  } else {
+    return fwd_shape(g, kShapes16, 2) == 0 ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
+                                           : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
+  }
+}
+
 template <typename T, int DMA>
 int bwd_typed(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
   if constexpr (std::is_same<T, float>::value) {
-    switch (bwd_shape(gd, gw, kShapesF32, 4)) {
-      case 0: return launch_bwd<T, 64, 128, DMA>(gd, gw, s);
-      default: return launch_bwd<T, 64, 64, DMA>(gd, gw, s);
-    }
+    using Wide = Tile<64, 128, 2, 128>;
+    using Small = Tile<64, 64, 2, 128>;
+    return bwd_shape(gd, gw, kShapesF32, 4) == 0 ? launch_bwd<T, Wide, Wide, DMA>(gd, gw, s)
+                                                 : launch_bwd<T, Small, Small, DMA>(gd, gw, s);
+  } else if constexpr (DMA == 16) {
+    const int forced = gd.tile ? gd.tile : gw.tile;
+    const int kind = forced ? (forced == 3 ? kMixed : k128) : bwd_choice(gd, gw);
+    using Big = Tile<128, 128, 2, 128>;
+    if (kind == k128) return launch_bwd<T, Big, Big, DMA>(gd, gw, s);
+    // short dW sums: half as deep slices, so that four workgroups fit a CU and their output
+    // stores (which bound such products) overlap
+    if (kind == kMixed)
+      return launch_bwd<T, Tile<64, 64, 2, 128>, Tile<128, 128, 2, 64>, DMA>(gd, gw, s);
+    return launch_bwd<T, Tile<64, 64, 3, 128>, Tile<64, 64, 3, 128>, DMA>(gd, gw, s);
   } else {
-    switch (bwd_shape(gd, gw, kShapes16, 2)) {
-      case 0: return launch_bwd<T, 128, 128, DMA>(gd, gw, s);
-      default: return launch_bwd<T, 64, 64, DMA>(gd, gw, s);
-    }
+    using Big = Tile<128, 128, 2, 128>;
+    using Small = Tile<64, 64, 2, 128>;
+    return bwd_shape(gd, gw, kShapes16, 2) == 0 ? launch_bwd<T, Big, Big, DMA>(gd, gw, s)
+                                                : launch_bwd<T, Small, Small, DMA>(gd, gw, s);
   }
 }
 
@@ -652,8 +836,20 @@ bool gemm_plain_supported(const GemmArgs& g, int dtype) {
   if (dtype != FMOE_F32 && dtype != FMOE_BF16 && dtype != FMOE_F16) return false;
   // tile-relative byte offsets are 32-bit: 128 rows of f32 are the bytes of 256 of bf16
   if (!dma_ld_supported(g.in_feat) || !dma_ld_supported(g.out_feat)) return false;
-  if (dtype != FMOE_F32 && (g.act_pre || g.act_out)) return false;
   return copy_width(g, dtype) != 0;
+}
+
+bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype) {
+  if (dtype == FMOE_F32 || !gemm_plain_supported(g, dtype)) return dtype == FMOE_F32;
+  if (g.tile) return g.tile == 2 || g.tile == 3;   // forced (tests)
+  return std::min(fwd_us(k128, g), fwd_us(k64, g)) < fwd_us(k256, g);
+}
+
+bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype) {
+  if (dtype == FMOE_F32 || !gemm_plain_supported(gd, dtype) || !gemm_plain_supported(gw, dtype))
+    return dtype == FMOE_F32;
+  if (gd.tile) return gd.tile == 2 || gd.tile == 3;
+  return bwd_us((Kind)bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw);
 }
 
 int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s) {
@@ -662,8 +858,11 @@ int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s) {
   switch (dtype) {
     case FMOE_F32:
       return copy_width(g, dtype) == 16 ? fwd_typed<float, 16>(g, s) : fwd_typed<float, 4>(g, s);
-    case FMOE_F16: return fwd_typed<__half, 4>(g, s);
-    default: return fwd_typed<__hip_bfloat16, 4>(g, s);
+    case FMOE_F16:
+      return copy_width(g, dtype) == 16 ? fwd_typed<__half, 16>(g, s) : fwd_typed<__half, 4>(g, s);
+    default:
+      return copy_width(g, dtype) == 16 ? fwd_typed<__hip_bfloat16, 16>(g, s)
+                                        : fwd_typed<__hip_bfloat16, 4>(g, s);
   }
 }
 
@@ -675,8 +874,14 @@ int launch_gemm_plain_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hip
       return copy_width(gd, dtype) == 16 && copy_width(gw, dtype) == 16
                  ? bwd_typed<float, 16>(gd, gw, s)
                  : bwd_typed<float, 4>(gd, gw, s);
-    case FMOE_F16: return bwd_typed<__half, 4>(gd, gw, s);
-    default: return bwd_typed<__hip_bfloat16, 4>(gd, gw, s);
+    case FMOE_F16:
+      return copy_width(gd, dtype) == 16 && copy_width(gw, dtype) == 16
+                 ? bwd_typed<__half, 16>(gd, gw, s)
+                 : bwd_typed<__half, 4>(gd, gw, s);
+    default:
+      return copy_width(gd, dtype) == 16 && copy_width(gw, dtype) == 16
+                 ? bwd_typed<__hip_bfloat16, 16>(gd, gw, s)
+                 : bwd_typed<__hip_bfloat16, 4>(gd, gw, s);
   }
 }
 

@@ -49,6 +49,13 @@ typedef enum fmoe_dtype {
   FMOE_BF16 = 3
 } fmoe_dtype;
 
+/* The activation between the two linear layers of an expert. */
+typedef enum fmoe_activation {
+  FMOE_ACT_NONE = 0,
+  FMOE_ACT_GELU = 1, /* the exact, erf-based one */
+  FMOE_ACT_RELU = 2
+} fmoe_activation;
+
 /* Largest number of experts the routing kernels keep in LDS. */
 #define FMOE_MAX_EXPERTS 4096
 /* Largest top_k of the fused gate kernels. */
@@ -323,6 +330,28 @@ int fmoe_grouped_linear_bwd_ptrs(const void* dy, const void* x, const void* cons
                                  void* dw, void* dbias, int64_t n_rows, int64_t in_feat,
                                  int64_t out_feat, int64_t n_expert, int dtype,
                                  void* stream);
+
+/*
+ * The two linear layers of an expert with any activation between them (fmoe/transformer.py:
+ * 25-33; the reference's activation is an arbitrary module between two calls of
+ * fmoe_cuda.linear_forward).  Parameters as one [E, ...] array (w, bias) or as pointer tables
+ * (w_ptrs, bias_ptrs); whichever is not used is NULL.
+ *   _fwd  y = x W^T + b and, with act != FMOE_ACT_NONE, y_act = act(y); y may then be NULL
+ *         (the pre-activations are not kept).
+ *   _bwd  as fmoe_grouped_linear_bwd; with act != FMOE_ACT_NONE, dx is multiplied by
+ *         act'(act_pre).  For ReLU act_pre is the activation (y_act of the forward call), for
+ *         GELU the pre-activations.
+ */
+int fmoe_expert_linear_fwd(const void* x, const void* w, const void* const* w_ptrs,
+                           const void* bias, const void* const* bias_ptrs,
+                           const int32_t* seg_off, void* y, void* y_act, int act, int64_t n_rows,
+                           int64_t in_feat, int64_t out_feat, int64_t n_expert, int dtype,
+                           void* stream);
+int fmoe_expert_linear_bwd(const void* dy, const void* x, const void* w,
+                           const void* const* w_ptrs, const int32_t* seg_off,
+                           const void* act_pre, int act, void* dx, void* dw, void* dbias,
+                           int64_t n_rows, int64_t in_feat, int64_t out_feat, int64_t n_expert,
+                           int dtype, void* stream);
 
 /*
  * table[i] = host_ptrs[i] for i < n: fills a DEVICE array of pointers (the w_ptrs /
