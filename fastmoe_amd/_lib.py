@@ -71,6 +71,14 @@ SIGNATURES = {
     "fmoe_seg_off_from_host_counts": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
     "fmoe_topk_softmax_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
                                       c_int, c_void_p]),
+    "fmoe_limit_gate": (c_int, [c_void_p, c_int64, c_int32, c_int64, c_void_p, c_void_p, c_void_p,
+                                c_int64, c_void_p]),
+    "fmoe_balance_gate_workspace_bytes": (c_int64, [c_int32]),
+    "fmoe_balance_gate_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int, c_int64, c_void_p,
+                                      c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
+                                      c_void_p]),
+    "fmoe_balance_gate_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                      c_void_p, c_int64, c_int32, c_int, c_int, c_void_p]),
     "fmoe_naive_gate_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
                                     c_void_p, c_int, c_void_p]),
     "fmoe_topk_softmax_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32,

@@ -62,13 +62,12 @@ void* stream_of(const Tensor& t) {
 
 void* ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
-// Routing workspace for a call on torch's current stream of `like`'s device.  One
-// buffer per (device, stream) is kept and reused: launches on one stream run in
-// order, and nothing in the workspace outlives a call.  A stream under graph capture
-// gets a fresh tensor instead, which then belongs to the graph's own memory pool.
-Tensor workspace(int64_t numel, int64_t n_expert, const Tensor& like) {
-  int64_t bytes = fmoe_route_workspace_bytes(numel, (int32_t)n_expert);
-  need(bytes >= 0, "route workspace: bad sizes");
+// Scratch memory for a call on torch's current stream of `like`'s device.  One buffer per
+// (device, stream) is kept and reused: launches on one stream run in order, and nothing in
+// it outlives a call.  A stream under graph capture gets a fresh tensor instead, which then
+// belongs to the graph's own memory pool.
+Tensor workspace_of(int64_t bytes, const Tensor& like) {
+  need(bytes >= 0, "workspace: bad sizes");
   if (bytes < 1) bytes = 1;
   auto opts = like.options().dtype(at::kByte);
   void* stream = stream_of(like);
@@ -86,6 +85,9 @@ Tensor workspace(int64_t numel, int64_t n_expert, const Tensor& like) {
   Tensor& ws = (*cache)[{(int)like.device().index(), stream}];
   if (!ws.defined() || ws.numel() < bytes) ws = torch::empty({std::max<int64_t>(bytes, 1 << 16)}, opts);
   return ws;
+}
+Tensor workspace(int64_t numel, int64_t n_expert, const Tensor& like) {
+  return workspace_of(fmoe_route_workspace_bytes(numel, (int32_t)n_expert), like);
 }
 
 // ---------------------------------------------------------------- reference surface
@@ -582,10 +584,19 @@ PYBIND11_MODULE(fmoe_cuda, m) {
   m.def("topk_softmax_bwd", &topk_softmax_bwd);
   m.def("gelu_fwd", &gelu_fwd, py::arg("x"), py::arg("n_rows_dev") = py::none());
   m.def("gelu_bwd", &gelu_bwd, py::arg("dy"), py::arg("x"), py::arg("n_rows_dev") = py::none());
+  py::class_<ParamTables>(m, "ParamTables").def(py::init<>());
   m.def("expert_layer", &expert_layer, py::arg("x"), py::arg("gate_idx"), py::arg("score"),
-        py::arg("w1"), py::arg("b1"), py::arg("w2"), py::arg("b2"));
+        py::arg("params"), py::arg("n_expert"), py::arg("has_b1"), py::arg("has_b2"),
+        py::arg("act"), py::arg("tables") = py::none());
   m.def("gated_layer", &gated_layer, py::arg("x"), py::arg("gate_weight"), py::arg("gate_bias"),
-        py::arg("w1"), py::arg("b1"), py::arg("w2"), py::arg("b2"), py::arg("top_k"));
+        py::arg("params"), py::arg("n_expert"), py::arg("has_b1"), py::arg("has_b2"),
+        py::arg("act"), py::arg("top_k"), py::arg("tables") = py::none());
+  m.def("limit_gate", &limit_gate, py::arg("gate"), py::arg("n_expert"), py::arg("capacity"));
+  m.def("balance_gate", &balance_gate, py::arg("logits"), py::arg("kind"), py::arg("capacity"));
+  m.attr("GATE_GSHARD") = (int)FMOE_GATE_GSHARD;
+  m.attr("GATE_SWITCH") = (int)FMOE_GATE_SWITCH;
+  m.attr("ACT_GELU") = (int)FMOE_ACT_GELU;
+  m.attr("ACT_RELU") = (int)FMOE_ACT_RELU;
   m.def("set_gemm_path", &set_gemm_path);
   m.def("_seg_off_from_counts",
         [](Tensor expert_count, py::object device) {

@@ -1,20 +1,27 @@
-// The whole MoE layer of GELU expert MLPs as ONE native autograd node: route ->
-// scatter -> linear + GELU -> linear -> gather fused with the top-k combine
+// The whole MoE layer of two-layer expert MLPs as ONE native autograd node: route ->
+// scatter -> linear + activation -> linear -> gather fused with the top-k combine
 // (fmoe/layers.py:26-78,281-295 around fmoe/transformer.py:25-33 of the reference),
 // optionally with the top-k gate in front of it (fmoe/gates/naive_gate.py:31-38), and
 // the mirror image backwards.  Part of the extension (fmoe_cuda_ext.cpp).
 //
 // Why native: a small layer costs what the host needs to enqueue it (512 tokens,
-// 128 -> 256, 4 experts: 377 us per step, of which the GPU works for about 170).  As a
+// 128 -> 256, 4 experts: 377 us per step, of which the GPU worked for about 170).  As a
 // torch::autograd::Function neither direction enters Python between two launches, the
 // backward needs no interpreter lock, the routing results share one allocation, and a
-// forward without gradients saves nothing.
+// forward without gradients saves nothing and keeps no pre-activations.
+//
+// Expert parameters come as four [E, ...] arrays or as lists of E single-expert tensors
+// (the reference's module per expert, fmoe/transformer.py:51-55), whose addresses the
+// kernels read from device tables; the gradients of a list are views of one array.
 #pragma once
 #include <torch/extension.h>
 
 #include <ATen/core/grad_mode.h>
 
 namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
 
 // Byte offsets of the routing results inside their one allocation.
 struct RouteLayout {
@@ -23,41 +30,120 @@ struct RouteLayout {
       : inv(slots * 8), seg(inv + slots * 4), bytes(seg + (n_expert + 1) * 4) {}
 };
 
+// Device pointer tables of per-expert parameter lists (w1, b1, w2, b2), rebuilt only when a
+// parameter's storage has moved (optimizers update in place, so normally never).
+struct ParamTables {
+  std::vector<const void*> key;
+  Tensor table;   // int64 [4, E]; rows of absent biases stay zero
+
+  const Tensor& get(const std::vector<Tensor>& params, int64_t n_expert, bool has_b1, bool has_b2) {
+    std::vector<const void*> now(4 * n_expert, nullptr);
+    const bool present[4] = {true, has_b1, true, has_b2};
+    size_t at = 0;
+    for (int row = 0; row < 4; ++row)
+      if (present[row])
+        for (int64_t e = 0; e < n_expert; ++e) now[row * n_expert + e] = params[at++].data_ptr();
+    if (!table.defined() || table.device() != params[0].device() || now != key) {
+      for (const Tensor& t : params) {
+        dev(t, "expert parameter", params[0].scalar_type());
+        need(t.device() == params[0].device(), "expert parameters must share their device");
+        need((uintptr_t)t.data_ptr() % 16 == 0, "expert parameters must be 16-byte aligned");
+      }
+      // (a new tensor: kernels of an earlier call may still be reading the old one)
+      table = torch::empty({4, n_expert}, params[0].options().dtype(at::kLong));
+      check(fmoe_pointer_table(now.data(), (int64_t)now.size(), (const void**)table.data_ptr(),
+                               stream_of(params[0])),
+            "pointer_table");
+      key = std::move(now);
+    }
+    return table;
+  }
+};
+
+struct LayerConfig {
+  int64_t top_k = 0, act = FMOE_ACT_GELU, n_expert = 0;
+  bool gated = false, has_bg = false, has_b1 = false, has_b2 = false, list = false;
+  Tensor table;       // list: pointers of w1, b1, w2, b2
+  Tensor zero_loss;   // gated: the plain gate's balance loss, written by its kernel
+
+  std::vector<int64_t> ints() const {
+    return {top_k, act, n_expert, gated, has_bg, has_b1, has_b2, list};
+  }
+  static LayerConfig from(const std::vector<int64_t>& v) {
+    LayerConfig c;
+    c.top_k = v[0]; c.act = v[1]; c.n_expert = v[2];
+    c.gated = v[3]; c.has_bg = v[4]; c.has_b1 = v[5]; c.has_b2 = v[6]; c.list = v[7];
+    return c;
+  }
+  int64_t per_kind() const { return list ? n_expert : 1; }   // tensors per parameter kind
+};
+
+// One linear layer's parameters as the C ABI takes them.
+struct LinearParams {
+  const void* w = nullptr;
+  const void* const* w_ptrs = nullptr;
+  const void* b = nullptr;
+  const void* const* b_ptrs = nullptr;
+};
+struct ExpertParams {
+  LinearParams first, second;
+};
+
 struct LayerSizes {
   int64_t t, d, h, e, k, n;   // tokens, features, hidden features, experts, top-k, slots
   int dtype;
 };
 
-LayerSizes layer_sizes(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2,
-                       const Tensor& b2, int64_t top_k) {
-  dev(w1, "w1", x.scalar_type());
-  dev(w2, "w2", x.scalar_type());
-  need(x.dim() == 2 && w1.dim() == 3 && w2.dim() == 3, "x must be 2-d and the weights 3-d");
-  LayerSizes s{x.size(0), x.size(1), w1.size(1), w1.size(0), top_k, x.size(0) * top_k, dt(x, "x")};
-  need(w1.size(2) == s.d && w2.size(0) == s.e && w2.size(1) == s.d && w2.size(2) == s.h,
-       "the expert weights must be [E, hidden, in] and [E, in, hidden]");
-  if (b1.defined()) {
-    dev(b1, "b1", x.scalar_type());
-    need(b1.numel() == s.e * s.h, "b1 must be [E, hidden]");
-  }
-  if (b2.defined()) {
-    dev(b2, "b2", x.scalar_type());
-    need(b2.numel() == s.e * s.d, "b2 must be [E, in]");
-  }
+// `params`: w1, b1 (if any), w2, b2 (if any), each one tensor or n_expert of them.
+LayerSizes layer_sizes(const LayerConfig& c, const Tensor& x, at::TensorList params) {
+  const int64_t per = c.per_kind();
+  need(x.dim() == 2, "x must be 2-d");
+  need((int64_t)params.size() == per * (2 + c.has_b1 + c.has_b2), "wrong number of expert parameters");
+  const Tensor& w1 = params[0];
+  const Tensor& w2 = params[per * (1 + c.has_b1)];
+  need(w1.dim() == 3 && w2.dim() == 3, "the expert weights must be 3-d");
+  LayerSizes s{x.size(0), x.size(1), w1.size(1), c.n_expert, c.top_k, x.size(0) * c.top_k, dt(x, "x")};
+  const int64_t lead = c.list ? 1 : s.e;
+  size_t at = 0;
+  auto kind = [&](const char* name, std::initializer_list<int64_t> shape) {
+    for (int64_t i = 0; i < per; ++i) {
+      const Tensor& t = params[at++];
+      dev(t, name, x.scalar_type());
+      need(t.sizes() == at::IntArrayRef(shape), std::string(name) + " has the wrong shape");
+    }
+  };
+  kind("w1", {lead, s.h, s.d});
+  if (c.has_b1) kind("b1", {lead, s.h});
+  kind("w2", {lead, s.d, s.h});
+  if (c.has_b2) kind("b2", {lead, s.d});
   return s;
 }
 
-Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
-const void* raw(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+ExpertParams expert_params(const LayerConfig& c, at::TensorList params) {
+  ExpertParams p;
+  if (c.list) {
+    const void* const* base = (const void* const*)c.table.data_ptr();
+    p.first.w_ptrs = base;
+    if (c.has_b1) p.first.b_ptrs = base + c.n_expert;
+    p.second.w_ptrs = base + 2 * c.n_expert;
+    if (c.has_b2) p.second.b_ptrs = base + 3 * c.n_expert;
+    return p;
+  }
+  size_t at = 0;
+  p.first.w = params[at++].data_ptr();
+  if (c.has_b1) p.first.b = params[at++].data_ptr();
+  p.second.w = params[at++].data_ptr();
+  if (c.has_b2) p.second.b = params[at++].data_ptr();
+  return p;
+}
 
 // What the backward needs of a forward pass, and the output.
 struct LayerPass {
   Tensor y, buf, pre, act, out, score, route;
 };
 
-LayerPass experts_forward(const LayerSizes& s, const Tensor& x, const Tensor& idx,
-                          const Tensor& score, const Tensor& w1, const Tensor& b1,
-                          const Tensor& w2, const Tensor& b2) {
+LayerPass experts_forward(const LayerConfig& c, const LayerSizes& s, const ExpertParams& w,
+                          const Tensor& x, const Tensor& idx, const Tensor& score, bool train) {
   const auto opts = x.options();
   void* stream = stream_of(x);
   const RouteLayout at_(s.n, s.e);
@@ -80,15 +166,19 @@ LayerPass experts_forward(const LayerSizes& s, const Tensor& x, const Tensor& id
     check(fmoe_local_scatter(x.data_ptr(), pos, p.buf.data_ptr(), s.n, s.d, s.k, seg + s.e, s.dtype,
                              stream),
           "local_scatter");
-  p.pre = at::empty({s.n, s.h}, opts);
+  // GELU's backward needs the pre-activations, ReLU's the activations, inference neither
+  const bool keep_pre = train && c.act == FMOE_ACT_GELU;
+  if (keep_pre) p.pre = at::empty({s.n, s.h}, opts);
   p.act = at::empty({s.n, s.h}, opts);
-  check(fmoe_grouped_linear_fwd_act(p.buf.data_ptr(), w1.data_ptr(), raw(b1), seg, p.pre.data_ptr(),
-                                    p.act.data_ptr(), s.n, s.d, s.h, s.e, s.dtype, stream),
-        "grouped_linear_fwd_act");
+  check(fmoe_expert_linear_fwd(p.buf.data_ptr(), w.first.w, w.first.w_ptrs, w.first.b,
+                               w.first.b_ptrs, seg, keep_pre ? p.pre.data_ptr() : nullptr,
+                               p.act.data_ptr(), (int)c.act, s.n, s.d, s.h, s.e, s.dtype, stream),
+        "expert_linear_fwd");
   p.out = at::empty({s.n, s.d}, opts);
-  check(fmoe_grouped_linear_fwd(p.act.data_ptr(), w2.data_ptr(), raw(b2), seg, p.out.data_ptr(), s.n,
-                                s.h, s.d, s.e, s.dtype, stream),
-        "grouped_linear_fwd");
+  check(fmoe_expert_linear_fwd(p.act.data_ptr(), w.second.w, w.second.w_ptrs, w.second.b,
+                               w.second.b_ptrs, seg, p.out.data_ptr(), nullptr, FMOE_ACT_NONE, s.n,
+                               s.h, s.d, s.e, s.dtype, stream),
+        "expert_linear_fwd");
   p.y = at::empty({s.t, s.d}, opts);
   check(fmoe_gather_combine_fwd(p.out.data_ptr(), inv, score.data_ptr(), p.y.data_ptr(), s.t, s.k,
                                 s.d, s.dtype, stream),
@@ -103,8 +193,10 @@ struct LayerNeeds {
   bool dx, w1, b1, w2, b2;
 };
 
-LayerGrads experts_backward(const LayerSizes& s, const LayerPass& p, const Tensor& dy,
-                            const Tensor& w1, const Tensor& w2, const LayerNeeds& want) {
+void* out_ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const ExpertParams& w,
+                            const LayerPass& p, const Tensor& dy, const LayerNeeds& want) {
   const auto opts = dy.options();
   void* stream = stream_of(dy);
   const RouteLayout at_(s.n, s.e);
@@ -120,30 +212,23 @@ LayerGrads experts_backward(const LayerSizes& s, const LayerPass& p, const Tenso
   const bool first = want.dx || want.w1 || want.b1;   // whether the first layer has a backward
   Tensor dpre;
   if (first) dpre = at::empty({s.n, s.h}, opts);
-  if (want.w2) g.dw2 = at::empty_like(w2);
+  if (want.w2) g.dw2 = at::empty({s.e, s.d, s.h}, opts);
   if (want.b2) g.db2 = at::empty({s.e, s.d}, opts);
-  void* dw2 = g.dw2.defined() ? g.dw2.data_ptr() : nullptr;
-  void* db2 = g.db2.defined() ? g.db2.data_ptr() : nullptr;
-  if (first)
-    check(fmoe_grouped_linear_bwd_act(d_out.data_ptr(), p.act.data_ptr(), w2.data_ptr(), seg,
-                                      p.pre.data_ptr(), dpre.data_ptr(), dw2, db2, s.n, s.h, s.d, s.e,
-                                      s.dtype, stream),
-          "grouped_linear_bwd_act");
-  else if (dw2 || db2)
-    check(fmoe_grouped_linear_bwd(d_out.data_ptr(), p.act.data_ptr(), w2.data_ptr(), seg, nullptr,
-                                  dw2, db2, s.n, s.h, s.d, s.e, s.dtype, stream),
-          "grouped_linear_bwd");
+  if (first || want.w2 || want.b2)
+    check(fmoe_expert_linear_bwd(d_out.data_ptr(), p.act.data_ptr(), w.second.w, w.second.w_ptrs, seg,
+                                 p.pre.defined() ? p.pre.data_ptr() : p.act.data_ptr(),
+                                 first ? (int)c.act : FMOE_ACT_NONE, out_ptr(dpre), out_ptr(g.dw2),
+                                 out_ptr(g.db2), s.n, s.h, s.d, s.e, s.dtype, stream),
+          "expert_linear_bwd");
   if (!first) return g;
   Tensor dbuf;
   if (want.dx) dbuf = at::empty({s.n, s.d}, opts);
-  if (want.w1) g.dw1 = at::empty_like(w1);
+  if (want.w1) g.dw1 = at::empty({s.e, s.h, s.d}, opts);
   if (want.b1) g.db1 = at::empty({s.e, s.h}, opts);
-  check(fmoe_grouped_linear_bwd(dpre.data_ptr(), p.buf.data_ptr(), w1.data_ptr(), seg,
-                                dbuf.defined() ? dbuf.data_ptr() : nullptr,
-                                g.dw1.defined() ? g.dw1.data_ptr() : nullptr,
-                                g.db1.defined() ? g.db1.data_ptr() : nullptr, s.n, s.d, s.h, s.e,
-                                s.dtype, stream),
-        "grouped_linear_bwd");
+  check(fmoe_expert_linear_bwd(dpre.data_ptr(), p.buf.data_ptr(), w.first.w, w.first.w_ptrs, seg,
+                               nullptr, FMOE_ACT_NONE, out_ptr(dbuf), out_ptr(g.dw1),
+                               out_ptr(g.db1), s.n, s.d, s.h, s.e, s.dtype, stream),
+        "expert_linear_bwd");
   if (want.dx) {
     g.dx = at::empty({s.t, s.d}, opts);
     check(fmoe_scatter_reduce(dbuf.data_ptr(), inv, g.dx.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
@@ -155,7 +240,8 @@ LayerGrads experts_backward(const LayerSizes& s, const LayerPass& p, const Tenso
 // The gate's top-k and softmax.  `zero_loss` (float[1]) is the gate's balance loss, which is
 // zero for the plain top-k gate: the kernel writes it, so that it costs no launch of its own.
 void gate_topk(const LayerSizes& s, const Tensor& logits, Tensor& idx, Tensor& score,
-               Tensor& zero_loss) {
+               const Tensor& zero_loss) {
+  need(logits.size(1) == s.e, "the gate must have one output per expert");
   idx = at::empty({s.t, s.k}, logits.options().dtype(at::kLong));
   score = at::empty({s.t, s.k}, logits.options());
   check(fmoe_naive_gate_fwd(logits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k,
@@ -164,164 +250,274 @@ void gate_topk(const LayerSizes& s, const Tensor& logits, Tensor& idx, Tensor& s
         "naive_gate_fwd");
 }
 
-// Which of a node's gradients the current backward wants: edges count the node's tensor
-// arguments in order, an optional one only where it is given.
-struct Edges {
-  torch::autograd::AutogradContext* ctx;
-  size_t next = 0;
-  bool operator()(bool defined) { return defined && ctx->needs_input_grad(next++); }
-};
-
-using torch::autograd::AutogradContext;
-using torch::autograd::variable_list;
-
-// The layer behind any gate: (x, idx, score, w1, b1, w2, b2) -> y
-struct ExpertLayerNode : public torch::autograd::Function<ExpertLayerNode> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& inp, const Tensor& idx,
-                        const Tensor& score_in, const Tensor& w1, const OptTensor& b1_,
-                        const Tensor& w2, const OptTensor& b2_, int64_t top_k) {
-    const Tensor b1 = or_undefined(b1_), b2 = or_undefined(b2_);
-    at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor x = inp.contiguous();
-    c10::DeviceGuard guard(x.device());
-    const LayerSizes s = layer_sizes(x, w1, b1, w2, b2, top_k);
-    const Tensor score = score_in.reshape({s.t, s.k}).contiguous().to(x.scalar_type());
-    LayerPass p = experts_forward(s, x, idx, score, w1, b1, w2, b2);
-    ctx->saved_data["k"] = top_k;
-    ctx->saved_data["shape"] = score_in.sizes();
-    ctx->saved_data["dtype"] = (int64_t)score_in.scalar_type();
-    ctx->saved_data["b1"] = b1.defined();
-    ctx->saved_data["b2"] = b2.defined();
-    ctx->save_for_backward({p.buf, p.pre, p.act, p.out, p.score, p.route, w1, w2});
-    return p.y;
+// Forward of the layer.  vars: x, then (wg, bg if any) of a gate to be run here, or (idx,
+// score) of a gate that has been run; then the expert parameters.  The gate's linear map
+// stays the library call it is in torch.nn.Linear, in both directions, so the logits (and
+// with them the routing) and every gradient have the bits of the gate module.
+LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, LayerSizes* sizes,
+                        Tensor* x_out, Tensor* idx_out) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor x = vars[0].contiguous();
+  c10::DeviceGuard guard(x.device());
+  const at::TensorList params = vars.slice(c.gated ? 2 + c.has_bg : 3);
+  const LayerSizes s = layer_sizes(c, x, params);
+  Tensor idx, score;
+  if (c.gated) {
+    gate_topk(s, at::linear(x, vars[1], c.has_bg ? OptTensor(vars[2]) : OptTensor()), idx, score,
+              c.zero_loss);
+  } else {
+    idx = vars[1];
+    score = vars[2].reshape({s.t, s.k}).contiguous().to(x.scalar_type());
   }
+  LayerPass p = experts_forward(c, s, expert_params(c, params), x, idx, score, train);
+  if (sizes) *sizes = s;
+  if (x_out) *x_out = x;
+  if (idx_out) *idx_out = idx;
+  return p;
+}
 
-  static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const variable_list v = ctx->get_saved_variables();
-    const Tensor &w1 = v[6], &w2 = v[7];
-    Edges edge{ctx};
-    const bool dx = edge(true);
-    edge(true);   // idx
-    const bool ds = edge(true), nw1 = edge(true), nb1 = edge(ctx->saved_data["b1"].toBool()),
-               nw2 = edge(true), nb2 = edge(ctx->saved_data["b2"].toBool());
-    const Tensor dy = grads[0].contiguous();
-    c10::DeviceGuard guard(dy.device());
-    LayerPass p{Tensor(), v[0], v[1], v[2], v[3], v[4], v[5]};
-    const int64_t k = ctx->saved_data["k"].toInt();
-    const LayerSizes s{dy.size(0), dy.size(1), w1.size(1), w1.size(0), k, dy.size(0) * k, dt(dy, "dy")};
-    LayerGrads g = experts_backward(s, p, dy, w1, w2, {dx, nw1, nb1, nw2, nb2});
-    Tensor dscore;
-    if (ds)
-      dscore = g.dscore.reshape(ctx->saved_data["shape"].toIntVector())
-                   .to((at::ScalarType)ctx->saved_data["dtype"].toInt());
-    return {g.dx, Tensor(), dscore, g.dw1, g.db1, g.dw2, g.db2, Tensor()};
-  }
-};
-
-// The layer with the top-k gate in front: (x, wg, bg, w1, b1, w2, b2) -> y.  The gate's
-// linear map stays the library call it is in torch.nn.Linear, in both directions, so the
-// logits (and with them the routing) and every gradient have the bits of the gate module.
-struct GatedLayerNode : public torch::autograd::Function<GatedLayerNode> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& inp, const Tensor& wg,
-                        const OptTensor& bg_, const Tensor& w1, const OptTensor& b1_,
-                        const Tensor& w2, const OptTensor& b2_, int64_t top_k, Tensor zero_loss) {
-    const Tensor bg = or_undefined(bg_), b1 = or_undefined(b1_), b2 = or_undefined(b2_);
-    at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor x = inp.contiguous();
-    c10::DeviceGuard guard(x.device());
-    const LayerSizes s = layer_sizes(x, w1, b1, w2, b2, top_k);
-    const Tensor logits = at::linear(x, wg, bg);
-    need(logits.size(1) == s.e, "the gate must have one output per expert");
-    Tensor idx, score;
-    gate_topk(s, logits, idx, score, zero_loss);
-    LayerPass p = experts_forward(s, x, idx, score, w1, b1, w2, b2);
-    ctx->saved_data["bg"] = bg.defined();
-    ctx->saved_data["b1"] = b1.defined();
-    ctx->saved_data["b2"] = b2.defined();
-    ctx->save_for_backward({p.buf, p.pre, p.act, p.out, p.score, p.route, w1, w2, x, wg, idx});
-    return p.y;
-  }
-
-  static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const variable_list v = ctx->get_saved_variables();
-    const Tensor &w1 = v[6], &w2 = v[7], &x = v[8], &wg = v[9], &idx = v[10];
-    Edges edge{ctx};
-    const bool dx = edge(true), nwg = edge(true), nbg = edge(ctx->saved_data["bg"].toBool()),
-               nw1 = edge(true), nb1 = edge(ctx->saved_data["b1"].toBool()), nw2 = edge(true),
-               nb2 = edge(ctx->saved_data["b2"].toBool());
-    at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor dy = grads[0].contiguous();
-    c10::DeviceGuard guard(dy.device());
-    LayerPass p{Tensor(), v[0], v[1], v[2], v[3], v[4], v[5]};
-    const int64_t k = idx.size(1);
-    const LayerSizes s{dy.size(0), dy.size(1), w1.size(1), w1.size(0), k, dy.size(0) * k, dt(dy, "dy")};
-    LayerGrads g = experts_backward(s, p, dy, w1, w2, {dx, nw1, nb1, nw2, nb2});
-    Tensor dwg, dbg;
-    if (dx || nwg || nbg) {
-      Tensor dlogits = at::empty({s.t, s.e}, dy.options());
-      check(fmoe_topk_softmax_bwd(g.dscore.data_ptr(), p.score.data_ptr(), idx.data_ptr<int64_t>(),
-                                  dlogits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k, s.dtype,
-                                  stream_of(dy)),
-            "topk_softmax_bwd");
-      if (nwg) dwg = at::mm(dlogits.t(), x);
-      if (nbg) dbg = dlogits.sum(0);
-      if (dx) g.dx.add_(at::mm(dlogits, wg));
+struct LayerNode : public torch::autograd::Function<LayerNode> {
+  static Tensor forward(AutogradContext* ctx, at::TensorList vars, const LayerConfig& c) {
+    Tensor x, idx;
+    LayerSizes s;
+    LayerPass p = layer_forward(c, vars, true, &s, &x, &idx);
+    variable_list saved{p.buf, p.pre, p.act, p.out, p.score, p.route};
+    if (c.gated) {
+      saved.push_back(x);
+      saved.push_back(vars[1]);
+      saved.push_back(idx);
+    } else {
+      ctx->saved_data["shape"] = vars[2].sizes();
+      ctx->saved_data["dtype"] = (int64_t)vars[2].scalar_type();
     }
-    return {g.dx, dwg, dbg, g.dw1, g.db1, g.dw2, g.db2, Tensor(), Tensor()};
+    if (c.list) saved.push_back(c.table);
+    // the weights (not the biases) are operands of the backward
+    const int64_t first = c.gated ? 2 + c.has_bg : 3, per = c.per_kind();
+    for (int64_t i = 0; i < per; ++i) saved.push_back(vars[first + i]);
+    for (int64_t i = 0; i < per; ++i) saved.push_back(vars[first + per * (1 + c.has_b1) + i]);
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["c"] = c.ints();
+    return p.y;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    LayerConfig c = LayerConfig::from(ctx->saved_data["c"].toIntVector());
+    const variable_list v = ctx->get_saved_variables();
+    const int64_t per = c.per_kind();
+    size_t at = 6 + (c.gated ? 3 : 0);
+    if (c.list) c.table = v[at++];
+    const at::TensorList weights = at::TensorList(v).slice(at);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor dy = grads[0].contiguous();
+    c10::DeviceGuard guard(dy.device());
+    const LayerPass p{Tensor(), v[0], v[1], v[2], v[3], v[4], v[5]};
+    const LayerSizes s{dy.size(0), dy.size(1), weights[0].size(1), c.n_expert, c.top_k,
+                       dy.size(0) * c.top_k, dt(dy, "dy")};
+    ExpertParams w;
+    if (c.list) {
+      w = expert_params(c, {});
+    } else {
+      w.first.w = weights[0].data_ptr();
+      w.second.w = weights[1].data_ptr();
+    }
+    // which gradients are wanted: edges in the order of the forward's tensors
+    size_t edge = 0;
+    auto any = [&](bool present, int64_t count) {
+      bool r = false;
+      if (present)
+        for (int64_t i = 0; i < count; ++i) r = ctx->needs_input_grad(edge++) || r;
+      return r;
+    };
+    const bool dx = any(true, 1);
+    bool nwg = false, nbg = false, ds = false;
+    if (c.gated) {
+      nwg = any(true, 1);
+      nbg = any(c.has_bg, 1);
+    } else {
+      any(true, 1);   // idx
+      ds = any(true, 1);
+    }
+    const size_t first_param = edge;
+    LayerNeeds want{dx, false, false, false, false};
+    want.w1 = any(true, per);
+    want.b1 = any(c.has_b1, per);
+    want.w2 = any(true, per);
+    want.b2 = any(c.has_b2, per);
+    LayerGrads g = experts_backward(c, s, w, p, dy, want);
+    variable_list out;
+    if (c.gated) {
+      const Tensor &x = v[6], &wg = v[7], &idx = v[8];
+      Tensor dwg, dbg;
+      if (dx || nwg || nbg) {
+        Tensor dlogits = at::empty({s.t, s.e}, dy.options());
+        check(fmoe_topk_softmax_bwd(g.dscore.data_ptr(), p.score.data_ptr(), idx.data_ptr<int64_t>(),
+                                    dlogits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k, s.dtype,
+                                    stream_of(dy)),
+              "topk_softmax_bwd");
+        if (nwg) dwg = at::mm(dlogits.t(), x);
+        if (nbg) dbg = dlogits.sum(0);
+        if (dx) g.dx.add_(at::mm(dlogits, wg));
+      }
+      out = {g.dx, dwg};
+      if (c.has_bg) out.push_back(dbg);
+    } else {
+      Tensor dscore;
+      if (ds)
+        dscore = g.dscore.reshape(ctx->saved_data["shape"].toIntVector())
+                     .to((at::ScalarType)ctx->saved_data["dtype"].toInt());
+      out = {g.dx, Tensor(), dscore};
+    }
+    auto give = [&](bool present, const Tensor& t) {
+      if (!present) return;
+      for (int64_t i = 0; i < per; ++i) {
+        const bool need_it = t.defined() && ctx->needs_input_grad(out.size());
+        out.push_back(!need_it ? Tensor() : c.list ? t.narrow(0, i, 1) : t);
+      }
+    };
+    need(out.size() == first_param, "layer node: gradients out of order");
+    give(true, g.dw1);
+    give(c.has_b1, g.db1);
+    give(true, g.dw2);
+    give(c.has_b2, g.db2);
+    out.push_back(Tensor());   // the configuration
+    return out;
   }
 };
 
-bool wants_grad(std::initializer_list<const Tensor*> ts) {
+bool wants_grad(at::TensorList ts) {
   if (!at::GradMode::is_enabled()) return false;
-  for (const Tensor* t : ts)
-    if (t->defined() && t->requires_grad()) return true;
+  for (const Tensor& t : ts)
+    if (t.requires_grad()) return true;
   return false;
 }
 
-Tensor expert_layer(const Tensor& inp, const Tensor& gate_idx, const Tensor& score, const Tensor& w1,
-                    const OptTensor& b1_, const Tensor& w2, const OptTensor& b2_) {
+Tensor run_layer(const LayerConfig& c, at::TensorList vars) {
+  if (wants_grad(vars)) return LayerNode::apply(vars, c);
+  return layer_forward(c, vars, false, nullptr, nullptr, nullptr).y;
+}
+
+// The expert parameters' share of a call: `params` holds w1, b1, w2, b2 in that order, the
+// absent biases left out; one tensor each, or n_expert with `tables`.
+void set_experts(LayerConfig& c, const std::vector<Tensor>& params, int64_t n_expert, bool has_b1,
+                 bool has_b2, ParamTables* tables) {
+  c.n_expert = n_expert;
+  c.has_b1 = has_b1;
+  c.has_b2 = has_b2;
+  c.list = tables != nullptr;
+  need((int64_t)params.size() == c.per_kind() * (2 + has_b1 + has_b2),
+       "wrong number of expert parameters");
+  if (c.list) {
+    c10::DeviceGuard guard(params[0].device());
+    c.table = tables->get(params, n_expert, has_b1, has_b2);
+  }
+}
+
+Tensor expert_layer(const Tensor& inp, const Tensor& gate_idx, const Tensor& score,
+                    std::vector<Tensor> params, int64_t n_expert, bool has_b1, bool has_b2,
+                    int64_t act, ParamTables* tables) {
   need(inp.is_cuda() && gate_idx.is_cuda(), "x and gate_idx must be CUDA tensors");
   need(gate_idx.scalar_type() == at::kLong, "gate_idx has the wrong dtype");
-  const Tensor b1 = or_undefined(b1_), b2 = or_undefined(b2_);
-  const int64_t k = gate_idx.dim() >= 2 ? gate_idx.size(-1) : 1;
-  need(k >= 1 && k <= 64 && gate_idx.numel() == inp.size(0) * k && score.numel() == gate_idx.numel(),
+  LayerConfig c;
+  c.top_k = gate_idx.dim() >= 2 ? gate_idx.size(-1) : 1;
+  c.act = act;
+  need(c.top_k >= 1 && c.top_k <= 64 && gate_idx.numel() == inp.size(0) * c.top_k &&
+           score.numel() == gate_idx.numel(),
        "gate_idx and score must have tokens * top_k entries");
-  const Tensor idx = gate_idx.contiguous();
-  if (wants_grad({&inp, &score, &w1, &b1, &w2, &b2}))
-    return ExpertLayerNode::apply(inp, idx, score, w1, b1_, w2, b2_, k);
-  at::AutoDispatchBelowADInplaceOrView below;
-  const Tensor x = inp.contiguous();
-  c10::DeviceGuard guard(x.device());
-  const LayerSizes s = layer_sizes(x, w1, b1, w2, b2, k);
-  return experts_forward(s, x, idx, score.reshape({s.t, s.k}).contiguous().to(x.scalar_type()), w1, b1,
-                         w2, b2)
-      .y;
+  set_experts(c, params, n_expert, has_b1, has_b2, tables);
+  variable_list vars{inp, gate_idx.contiguous(), score};
+  vars.insert(vars.end(), params.begin(), params.end());
+  return run_layer(c, vars);
 }
 
 // (y, balance loss): the loss is the zero of the plain top-k gate, a leaf that wants a
 // gradient as the gate module makes it
-std::tuple<Tensor, Tensor> gated_layer(const Tensor& inp, const Tensor& wg, const OptTensor& bg_,
-                                       const Tensor& w1, const OptTensor& b1_, const Tensor& w2,
-                                       const OptTensor& b2_, int64_t top_k) {
+std::tuple<Tensor, Tensor> gated_layer(const Tensor& inp, const Tensor& wg, const OptTensor& bg,
+                                       std::vector<Tensor> params, int64_t n_expert, bool has_b1,
+                                       bool has_b2, int64_t act, int64_t top_k,
+                                       ParamTables* tables) {
   need(inp.is_cuda() && inp.dim() == 2, "x must be a 2-d CUDA tensor");
-  const Tensor bg = or_undefined(bg_), b1 = or_undefined(b1_), b2 = or_undefined(b2_);
   c10::DeviceGuard guard(inp.device());
-  Tensor loss = at::empty({1}, inp.options().dtype(at::kFloat));
-  Tensor y;
-  if (wants_grad({&inp, &wg, &bg, &w1, &b1, &w2, &b2})) {
-    y = GatedLayerNode::apply(inp, wg, bg_, w1, b1_, w2, b2_, top_k, loss);
-  } else {
+  LayerConfig c;
+  c.top_k = top_k;
+  c.act = act;
+  c.gated = true;
+  c.has_bg = bg.has_value() && bg->defined();
+  c.zero_loss = at::empty({1}, inp.options().dtype(at::kFloat));
+  set_experts(c, params, n_expert, has_b1, has_b2, tables);
+  variable_list vars{inp, wg};
+  if (c.has_bg) vars.push_back(*bg);
+  vars.insert(vars.end(), params.begin(), params.end());
+  Tensor y = run_layer(c, vars);
+  c.zero_loss.set_requires_grad(true);
+  return {y, c.zero_loss};
+}
+
+// ---------------------------------------------------------------- gates
+// fmoe/gates/utils.py:9-26 at one worker in one call: (slots per expert that survive, gate with
+// -1 where dropped)
+std::tuple<Tensor, Tensor> limit_gate(const Tensor& gate_in, int64_t n_expert, int64_t capacity) {
+  const Tensor gate = gate_in.contiguous();
+  dev(gate, "gate", at::kLong);
+  c10::DeviceGuard guard(gate.device());
+  Tensor count = at::empty({n_expert}, gate.options()), out = at::empty_like(gate);
+  Tensor ws = workspace(gate.numel(), n_expert, gate);
+  check(fmoe_limit_gate(gate.data_ptr<int64_t>(), gate.numel(), (int32_t)n_expert, capacity,
+                        out.data_ptr<int64_t>(), count.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(),
+                        stream_of(gate)),
+        "limit_gate");
+  return {count, out};
+}
+
+// A gate with a balance loss behind its linear map: logits -> (idx limited to the capacity,
+// score, loss)
+struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, int64_t kind,
+                               int64_t capacity) {
     at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor x = inp.contiguous();
-    const LayerSizes s = layer_sizes(x, w1, b1, w2, b2, top_k);
-    const Tensor logits = at::linear(x, wg, bg);
-    need(logits.size(1) == s.e, "the gate must have one output per expert");
-    Tensor idx, score;
-    gate_topk(s, logits, idx, score, loss);
-    y = experts_forward(s, x, idx, score, w1, b1, w2, b2).y;
+    const Tensor logits = logits_in.contiguous();
+    const int64_t t = logits.size(0), e = logits.size(1), k = kind == FMOE_GATE_GSHARD ? 2 : 1;
+    Tensor idx = at::empty({t, k}, logits.options().dtype(at::kLong));
+    Tensor score = at::empty({t, k}, logits.options());
+    const auto f32 = logits.options().dtype(at::kFloat);
+    Tensor loss = at::empty({}, f32), coef = at::empty({e}, f32);
+    Tensor ws = workspace_of(fmoe_balance_gate_workspace_bytes((int32_t)e), logits);
+    check(fmoe_balance_gate_fwd(logits.data_ptr(), t, (int32_t)e, (int)kind, capacity,
+                                idx.data_ptr<int64_t>(), score.data_ptr(), loss.data_ptr<float>(),
+                                coef.data_ptr<float>(), ws.data_ptr(), ws.numel(),
+                                dt(logits, "logits"), stream_of(logits)),
+          "balance_gate_fwd");
+    Tensor kept = std::get<1>(limit_gate(idx, e, capacity));
+    ctx->save_for_backward({logits, coef, score, idx});
+    ctx->saved_data["kind"] = kind;
+    ctx->mark_non_differentiable({kept});
+    ctx->set_materialize_grads(false);
+    return {kept, score, loss};
   }
-  loss.set_requires_grad(true);
-  return {y, loss};
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const Tensor &logits = v[0], &coef = v[1], &score = v[2], &idx = v[3];
+    const Tensor dscore = grads[1].defined() ? grads[1].contiguous() : Tensor();
+    const Tensor dloss = grads[2];
+    if (!dscore.defined() && !dloss.defined()) return {Tensor(), Tensor(), Tensor()};
+    c10::DeviceGuard guard(logits.device());
+    Tensor dlogits = at::empty_like(logits);
+    check(fmoe_balance_gate_bwd(logits.data_ptr(), coef.data_ptr<float>(),
+                                dloss.defined() ? dloss.data_ptr<float>() : nullptr,
+                                dscore.defined() ? dscore.data_ptr() : nullptr, score.data_ptr(),
+                                idx.data_ptr<int64_t>(), dlogits.data_ptr(), logits.size(0),
+                                (int32_t)logits.size(1), (int)ctx->saved_data["kind"].toInt(),
+                                dt(logits, "logits"), stream_of(logits)),
+          "balance_gate_bwd");
+    return {dlogits, Tensor(), Tensor()};
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor> balance_gate(const Tensor& logits, int64_t kind,
+                                                int64_t capacity) {
+  need(logits.is_cuda() && logits.dim() == 2, "logits must be a 2-d CUDA tensor");
+  c10::DeviceGuard guard(logits.device());
+  variable_list r = BalanceGateNode::apply(logits, kind, capacity);
+  return {r[0], r[1], r[2]};
 }
 
 }  // namespace

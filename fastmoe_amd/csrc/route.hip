@@ -15,6 +15,8 @@
 //
 // Semantics follow cuda/local_exchange.cuh:5-16,36-69 and
 // cuda/balancing.cuh:5-21,32-45 of the reference.
+#include <algorithm>
+
 #include "common.h"
 
 namespace fmoe {
@@ -25,7 +27,8 @@ constexpr int kRowsPerWave = 8;                               // 64-slot rows
 constexpr int kRouteChunk = kRouteThreads * kRowsPerWave;     // slots per block
 constexpr int kScanThreads = 1024;
 
-enum { MODE_ROUTE = 0, MODE_ASSIGN = 1, MODE_PRUNE = 2 };
+enum { MODE_ROUTE = 0, MODE_ASSIGN = 1, MODE_PRUNE = 2,
+       MODE_LIMIT = 3 };   // PRUNE with one capacity for all experts; counts what survives
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
@@ -70,7 +73,7 @@ template <int MODE>
 __global__ __launch_bounds__(kScanThreads) void route_scan_kernel(
     int32_t* __restrict__ block_hist, int n_blocks, int n_expert,
     int64_t* __restrict__ count64, int32_t* __restrict__ seg_off,
-    int32_t* __restrict__ cum_or_cap, int32_t* __restrict__ cap_copy) {
+    int32_t* __restrict__ cum_or_cap, int32_t* __restrict__ cap_copy, int32_t limit) {
   extern __shared__ int32_t lds_scan[];
   int32_t* cnt = lds_scan;                  // [E]
   int32_t* off = lds_scan + n_expert;       // [E+1]
@@ -122,6 +125,8 @@ __global__ __launch_bounds__(kScanThreads) void route_scan_kernel(
     } else if (MODE == MODE_ASSIGN) {
       // inclusive cumulative count in, exclusive one out
       cum_or_cap[e] = cum_or_cap[e] - c;
+    } else if (MODE == MODE_LIMIT) {
+      count64[e] = min(c, limit);
     } else {
       const int32_t cap = cum_or_cap[e];
       cap_copy[e] = cap;
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
     const int64_t* __restrict__ gate, int64_t n, int n_expert,
     const int32_t* __restrict__ block_hist, const int32_t* __restrict__ base_off,
     int64_t* __restrict__ pos, int32_t* __restrict__ inv,
-    int64_t* __restrict__ new_gate, const int32_t* __restrict__ cap) {
+    int64_t* __restrict__ new_gate, const int32_t* __restrict__ cap, int32_t limit) {
   extern __shared__ int32_t wave_cnt[];  // [kRouteWaves][E]
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
   // per-expert start of every wave: block base (+ segment start) + earlier waves
   for (int e = threadIdx.x; e < n_expert; e += kRouteThreads) {
     int32_t run = block_hist[(int64_t)blockIdx.x * n_expert + e];
-    if (MODE != MODE_PRUNE) run += base_off[e];
+    if (MODE != MODE_PRUNE && MODE != MODE_LIMIT) run += base_off[e];
 #pragma unroll
     for (int w2 = 0; w2 < kRouteWaves; ++w2) {
       const int32_t t = wave_cnt[w2 * n_expert + e];
@@ -195,9 +200,10 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
     // every lane of the wave has read its counter before the leader of each
     // expert advances it (one wave issues its LDS operations in order)
     if (valid && first) wave_cnt[w * n_expert + key] = p + cnt;
-    if (MODE == MODE_PRUNE) {
-      if (i < n) new_gate[i] = valid ? (p < cap[key] ? (int64_t)key : (int64_t)-1)
-                                     : gate[i];
+    if (MODE == MODE_PRUNE || MODE == MODE_LIMIT) {
+      if (i < n)
+        new_gate[i] = !valid ? gate[i]
+                      : p < (MODE == MODE_LIMIT ? limit : cap[key]) ? (int64_t)key : (int64_t)-1;
     } else {
       if (valid) pos[p] = i;
       if (inv != nullptr && i < n) inv[i] = valid ? p : -1;
@@ -221,10 +227,13 @@ constexpr int kSingleMaxSlots = 4096;
 constexpr int kSingleRows = kSingleMaxSlots / kSingleThreads;   // 64-slot rows per wave
 constexpr int kSingleMaxExperts = 512;
 
-template <int ROWS>
+// LIMIT: instead of routing, new_gate[i] = gate[i] or -1 where the expert already has `limit`
+// earlier slots, and count64 = what survives.
+template <int ROWS, bool LIMIT>
 __global__ __launch_bounds__(kSingleThreads) void route_single_kernel(
     const int64_t* __restrict__ gate, int64_t n, int n_expert, int64_t* __restrict__ count64,
-    int32_t* __restrict__ seg_off, int64_t* __restrict__ pos, int32_t* __restrict__ inv) {
+    int32_t* __restrict__ seg_off, int64_t* __restrict__ pos, int32_t* __restrict__ inv,
+    int64_t* __restrict__ new_gate, int32_t limit) {
   extern __shared__ int32_t lds_single[];
   int32_t* wave_cnt = lds_single;                            // [kSingleWaves][E]
   int32_t* cnt = lds_single + kSingleWaves * n_expert;       // [E]
@@ -262,9 +271,10 @@ __global__ __launch_bounds__(kSingleThreads) void route_single_kernel(
       run += t;
     }
     cnt[e] = run;
+    if (LIMIT) count64[e] = min(run, limit);
   }
   __syncthreads();
-  if (threadIdx.x < kWave) {   // exclusive scan over the experts, 64 per step
+  if (!LIMIT && threadIdx.x < kWave) {   // exclusive scan over the experts, 64 per step
     int32_t carry = 0;
     for (int base = 0; base < n_expert; base += kWave) {
       const int e = base + lane;
@@ -280,16 +290,18 @@ __global__ __launch_bounds__(kSingleThreads) void route_single_kernel(
     }
     if (lane == 0) off[n_expert] = carry;
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < n_expert; e += kSingleThreads) {
-    const int32_t o = off[e];
+  if (!LIMIT) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < n_expert; e += kSingleThreads) {
+      const int32_t o = off[e];
 #pragma unroll
-    for (int w2 = 0; w2 < kSingleWaves; ++w2) wave_cnt[w2 * n_expert + e] += o;
-    if (count64) count64[e] = cnt[e];
-    seg_off[e] = o;
+      for (int w2 = 0; w2 < kSingleWaves; ++w2) wave_cnt[w2 * n_expert + e] += o;
+      if (count64) count64[e] = cnt[e];
+      seg_off[e] = o;
+    }
+    if (threadIdx.x == 0) seg_off[n_expert] = off[n_expert];
+    __syncthreads();
   }
-  if (threadIdx.x == 0) seg_off[n_expert] = off[n_expert];
-  __syncthreads();
 
   const uint64_t lt_mask = ((uint64_t)1 << lane) - 1;
   const int key_bits = 32 - __clz(max(n_expert - 1, 1));
@@ -310,8 +322,12 @@ __global__ __launch_bounds__(kSingleThreads) void route_single_kernel(
     if (valid) p = wave_cnt[w * n_expert + key] + rank;
     // every lane has read its counter before the leader of each expert advances it
     if (valid && first) wave_cnt[w * n_expert + key] = p + __popcll(same);
-    if (valid) pos[p] = i;
-    if (inv != nullptr && i < n) inv[i] = valid ? p : -1;
+    if (LIMIT) {
+      if (i < n) new_gate[i] = !valid ? gate[i] : p < limit ? (int64_t)key : (int64_t)-1;
+    } else {
+      if (valid) pos[p] = i;
+      if (inv != nullptr && i < n) inv[i] = valid ? p : -1;
+    }
   }
 }
 
@@ -455,8 +471,8 @@ static int route_impl(const int64_t* gate, int64_t numel, int32_t n_expert,
   hipStream_t s = (hipStream_t)stream;
   if (single_launch && numel <= kSingleMaxSlots && n_expert <= kSingleMaxExperts) {
     const size_t lds = ((kSingleWaves + 2) * n_expert + 1) * sizeof(int32_t);
-    hipLaunchKernelGGL(route_single_kernel<kSingleRows>, dim3(1), dim3(kSingleThreads), lds, s,
-                       gate, numel, (int)n_expert, count64, seg_off, pos, inv);
+    hipLaunchKernelGGL((route_single_kernel<kSingleRows, false>), dim3(1), dim3(kSingleThreads), lds,
+                       s, gate, numel, (int)n_expert, count64, seg_off, pos, inv, (int64_t*)nullptr, 0);
     FMOE_LAUNCH_CHECK("route_single");
     return FMOE_OK;
   }
@@ -469,14 +485,14 @@ static int route_impl(const int64_t* gate, int64_t numel, int32_t n_expert,
   hipLaunchKernelGGL(route_scan_kernel<MODE_ROUTE>, dim3(1), dim3(kScanThreads),
                      (2 * n_expert + 1) * sizeof(int32_t), s, ws.block_hist,
                      ws.n_blocks, (int)n_expert, count64, seg_off,
-                     (int32_t*)nullptr, (int32_t*)nullptr);
+                     (int32_t*)nullptr, (int32_t*)nullptr, 0);
   FMOE_LAUNCH_CHECK("route_scan");
   if (ws.n_blocks > 0) {
     hipLaunchKernelGGL(route_place_kernel<MODE_ROUTE>, dim3(ws.n_blocks),
                        dim3(kRouteThreads),
                        kRouteWaves * n_expert * sizeof(int32_t), s, gate, numel,
                        (int)n_expert, ws.block_hist, seg_off, pos, inv,
-                       (int64_t*)nullptr, (const int32_t*)nullptr);
+                       (int64_t*)nullptr, (const int32_t*)nullptr, 0);
     FMOE_LAUNCH_CHECK("route_place");
   }
   return FMOE_OK;
@@ -530,14 +546,14 @@ extern "C" int fmoe_assign_pos(int32_t* cum_count, const int64_t* gate,
   hipLaunchKernelGGL(route_scan_kernel<MODE_ASSIGN>, dim3(1), dim3(kScanThreads),
                      (2 * n_expert + 1) * sizeof(int32_t), s, ws.block_hist,
                      ws.n_blocks, (int)n_expert, (int64_t*)nullptr,
-                     (int32_t*)nullptr, cum_count, (int32_t*)nullptr);
+                     (int32_t*)nullptr, cum_count, (int32_t*)nullptr, 0);
   FMOE_LAUNCH_CHECK("route_scan");
   hipLaunchKernelGGL(route_place_kernel<MODE_ASSIGN>, dim3(ws.n_blocks),
                      dim3(kRouteThreads),
                      kRouteWaves * n_expert * sizeof(int32_t), s, gate, numel,
                      (int)n_expert, ws.block_hist, cum_count, pos,
                      (int32_t*)nullptr, (int64_t*)nullptr,
-                     (const int32_t*)nullptr);
+                     (const int32_t*)nullptr, 0);
   FMOE_LAUNCH_CHECK("route_place");
   return FMOE_OK;
 }
@@ -582,13 +598,50 @@ extern "C" int fmoe_prune_gate_by_capacity(const int64_t* gate_idx,
   FMOE_LAUNCH_CHECK("route_hist");
   hipLaunchKernelGGL(route_scan_kernel<MODE_PRUNE>, dim3(1), dim3(kScanThreads),
                      (2 * E + 1) * sizeof(int32_t), s, ws.block_hist, ws.n_blocks,
-                     E, (int64_t*)nullptr, (int32_t*)nullptr, ec, ws.cap_copy);
+                     E, (int64_t*)nullptr, (int32_t*)nullptr, ec, ws.cap_copy, 0);
   FMOE_LAUNCH_CHECK("route_scan");
   hipLaunchKernelGGL(route_place_kernel<MODE_PRUNE>, dim3(ws.n_blocks),
                      dim3(kRouteThreads), kRouteWaves * E * sizeof(int32_t), s,
                      gate_idx, numel, E, ws.block_hist, (const int32_t*)nullptr,
                      (int64_t*)nullptr, (int32_t*)nullptr, new_gate_idx,
-                     ws.cap_copy);
+                     ws.cap_copy, 0);
+  FMOE_LAUNCH_CHECK("route_place");
+  return FMOE_OK;
+}
+
+extern "C" int fmoe_limit_gate(const int64_t* gate, int64_t numel, int32_t n_expert,
+                               int64_t capacity, int64_t* new_gate, int64_t* new_count,
+                               void* workspace, int64_t workspace_bytes, void* stream) {
+  int rc = check_route_args(numel, n_expert);
+  if (rc) return rc;
+  FMOE_REQUIRE(new_count && (numel == 0 || (gate && new_gate)), FMOE_ERR_INVALID,
+               "limit_gate: null pointer");
+  RouteWs ws;
+  rc = carve_ws(workspace, workspace_bytes, numel, n_expert, &ws);
+  if (rc) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  const int32_t limit = (int32_t)std::min<int64_t>(std::max<int64_t>(capacity, 0), 0x7fffffff);
+  if (numel <= kSingleMaxSlots && n_expert <= kSingleMaxExperts) {
+    const size_t lds = ((kSingleWaves + 2) * n_expert + 1) * sizeof(int32_t);
+    hipLaunchKernelGGL((route_single_kernel<kSingleRows, true>), dim3(1), dim3(kSingleThreads), lds,
+                       s, gate, numel, (int)n_expert, new_count, (int32_t*)nullptr,
+                       (int64_t*)nullptr, (int32_t*)nullptr, new_gate, limit);
+    FMOE_LAUNCH_CHECK("limit_gate_single");
+    return FMOE_OK;
+  }
+  hipLaunchKernelGGL(route_hist_kernel, dim3(ws.n_blocks), dim3(kRouteThreads),
+                     n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert, ws.block_hist,
+                     (int32_t*)nullptr);
+  FMOE_LAUNCH_CHECK("route_hist");
+  hipLaunchKernelGGL(route_scan_kernel<MODE_LIMIT>, dim3(1), dim3(kScanThreads),
+                     (2 * n_expert + 1) * sizeof(int32_t), s, ws.block_hist, ws.n_blocks,
+                     (int)n_expert, new_count, (int32_t*)nullptr, (int32_t*)nullptr,
+                     (int32_t*)nullptr, limit);
+  FMOE_LAUNCH_CHECK("route_scan");
+  hipLaunchKernelGGL(route_place_kernel<MODE_LIMIT>, dim3(ws.n_blocks), dim3(kRouteThreads),
+                     kRouteWaves * n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert,
+                     ws.block_hist, (const int32_t*)nullptr, (int64_t*)nullptr, (int32_t*)nullptr,
+                     new_gate, (const int32_t*)nullptr, limit);
   FMOE_LAUNCH_CHECK("route_place");
   return FMOE_OK;
 }

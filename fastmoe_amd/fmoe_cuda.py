@@ -86,19 +86,15 @@ def _hooked(op_name, fn):
     return op
 
 
-# The whole layer as one native autograd node (compiled binding only, else None); see
-# native_layers().
-_expert_layer = _gated_layer = None
+_compiled = None    # the extension, once bound
 
 
-def native_layers():
-    """(expert_layer, gated_layer) of the compiled extension: the layer behind any gate, and
-    the layer with the plain top-k gate in front, each as one autograd node that enters
-    Python nowhere between its launches.  None where they do not apply: on the ctypes
-    binding, and while `profile_hook` watches the single operators."""
-    if _gated_layer is None or profile_hook is not None:
-        return None
-    return _expert_layer, _gated_layer
+def native():
+    """The compiled extension with its whole-layer and gate nodes (expert_layer, gated_layer,
+    balance_gate, limit_gate): one autograd node each that enters Python nowhere between its
+    launches.  None where they do not apply: on the ctypes binding, and while `profile_hook`
+    watches the single operators."""
+    return None if profile_hook is not None else _compiled
 
 
 def _bind(binding: str) -> None:
@@ -109,7 +105,7 @@ def _bind(binding: str) -> None:
         compiled = _ext.load()
         for name in OPERATORS:
             g[name] = _hooked(name, getattr(compiled, name))
-        g["_expert_layer"], g["_gated_layer"] = compiled.expert_layer, compiled.gated_layer
+        g["_compiled"] = compiled
     else:
         for name in OPERATORS:
             g[name] = getattr(ctypes_ops, name)

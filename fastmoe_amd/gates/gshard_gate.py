@@ -5,6 +5,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import fmoe_cuda as fmoe_native
+from ..functions import topk_softmax
 from .naive_gate import NaiveGate
 
 
@@ -31,19 +32,24 @@ class GShardGate(NaiveGate):
         self.random_routing = random_routing
 
     def forward(self, x):
-        topk_idx, topk_val, logits = super().forward(x, return_all_scores=True)
-        n_tok = logits.shape[0]
-        top1 = topk_idx.view(-1, self.top_k)[:, 0]
-        frac = _histogram(top1, self.tot_expert).to(torch.float) / n_tok
-        prob = F.softmax(logits, dim=1).mean(dim=0)
-        self.set_loss(torch.mean(frac * prob) * (self.num_expert ** 2))
-
+        logits = self.gate(x)
         rate = self.capacity[0 if self.training else 1]
         cap = math.ceil(rate * x.shape[0]) * self.top_k // (self.world_size * self.num_expert)
-        budget = torch.full((self.tot_expert,), cap, dtype=torch.int32,
-                            device=topk_idx.device)
-        topk_idx = fmoe_native.prune_gate_by_capacity(
-            topk_idx.contiguous(), budget, self.num_expert, self.world_size)
+        native = self.native_balance(logits)
+        if native is not None:
+            # top-2, both softmaxes, load statistics, loss and capacity limit as one node
+            topk_idx, topk_val, loss = native.balance_gate(logits, native.GATE_GSHARD, cap)
+            self.set_loss(loss)
+        else:
+            topk_idx, topk_val = topk_softmax(logits, self.top_k)
+            top1 = topk_idx.view(-1, self.top_k)[:, 0]
+            frac = _histogram(top1, self.tot_expert).to(torch.float) / logits.shape[0]
+            prob = F.softmax(logits, dim=1).mean(dim=0)
+            self.set_loss(torch.mean(frac * prob) * (self.num_expert ** 2))
+            budget = torch.full((self.tot_expert,), cap, dtype=torch.int32,
+                                device=topk_idx.device)
+            topk_idx = fmoe_native.prune_gate_by_capacity(
+                topk_idx.contiguous(), budget, self.num_expert, self.world_size)
 
         if self.random_routing:
             coin = torch.rand(logits.size(0), device=x.device)

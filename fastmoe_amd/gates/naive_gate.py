@@ -23,7 +23,7 @@ class NaiveGate(BaseGate):
         softmax in one dtype, with nobody watching: a layer may then fold the gate into its
         own autograd node."""
         lin = self.gate
-        return (type(self) is NaiveGate and type(lin) is nn.Linear
+        return (type(self).forward is NaiveGate.forward and type(lin) is nn.Linear
                 and lin.weight.dtype == x.dtype and lin.weight.is_cuda
                 and self.top_k <= fmoe_cuda.MAX_GATE_TOP_K
                 and torch.get_default_dtype() == torch.float32
@@ -33,6 +33,14 @@ class NaiveGate(BaseGate):
                          or self._backward_pre_hooks or lin._forward_hooks
                          or lin._forward_pre_hooks or lin._backward_hooks
                          or lin._backward_pre_hooks))
+
+    def native_balance(self, logits):
+        r"""The extension where its balance-gate node takes these logits, else None."""
+        if (logits.is_cuda and logits.dim() == 2 and logits.shape[0] > 0
+                and 2 <= logits.shape[1] <= 512 and self.world_size == 1
+                and logits.dtype in (torch.float32, torch.float16, torch.bfloat16)):
+            return fmoe_cuda.native()
+        return None
 
     def forward(self, inp, return_all_scores=False):
         logits = self.gate(inp)

@@ -26,12 +26,18 @@ class SwitchGate(NaiveGate):
         if self.training:
             noise = torch.rand_like(score)
             score = score + (noise * 2 * self.switch_eps + 1.0 - self.switch_eps)
+        rate = self.capacity[0 if self.training else 1]
+        cap = math.ceil(rate * inp.shape[0] / self.num_expert)
+        native = self.native_balance(score) if score.dtype == inp.dtype else None
+        if native is not None:
+            # softmax, top-1, capacity limit, load statistics and loss as one node
+            top1_idx, top1_score, loss = native.balance_gate(score, native.GATE_SWITCH, cap)
+            self.set_loss(loss)
+            return top1_idx, top1_score
         score = F.softmax(score.float(), dim=-1)
         top1_score, top1_idx = torch.topk(score, k=1, dim=-1, largest=True)
         top1_score = top1_score.to(dtype=inp.dtype)
 
-        rate = self.capacity[0 if self.training else 1]
-        cap = math.ceil(rate * inp.shape[0] / self.num_expert)
         _lec, _gec, top1_idx = limit_by_capacity(top1_idx, self.num_expert,
                                                  self.world_size, cap)
 

@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from . import _tree as tree
+from . import _tree as tree, fmoe_cuda
 from .functions import (FusedGatherCombine, FusedScatter, MOEGather, MOEScatter,
                         RoutePlan, prepare_forward)
 from .gates import NaiveGate
@@ -142,16 +142,44 @@ class FMoE(nn.Module):
             return self.experts(x, segments)
         return type(self.experts[0]).run_list(self.experts, x, segments)
 
+    def _run_native_list(self, inp):
+        r"""The layer over a list of expert modules as one native autograd node (the gate
+        included where it is the plain one); None where the modules do not allow it."""
+        native = fmoe_cuda.native()
+        get = getattr(type(self.experts[0]), "native_list_args", None) if len(self.experts) else None
+        if (native is None or get is None or not torch.is_tensor(inp) or inp.dim() != 2
+                or not inp.is_cuda or not 1 <= self.top_k <= 64):
+            return None
+        args = get(self.experts, inp)
+        if args is None:
+            return None
+        if self.gate_hook is None and isinstance(self.gate, NaiveGate) and self.gate.is_plain(inp):
+            lin = self.gate.gate
+            out, loss = native.gated_layer(inp, lin.weight, lin.bias, *args[:5],
+                                           self.gate.top_k, args[5])
+            self.gate.set_loss(loss)
+            return out
+        idx, score = self.gate(inp)
+        if self.gate_hook is not None:
+            self.gate_hook(idx, score, None)
+        return native.expert_layer(inp, idx.reshape(-1, self.top_k),
+                                   score.reshape(-1, self.top_k), *args)
+
     # ------------------------------------------------------------- forward
     def forward(self, moe_inp):
         r"""Gate, dispatch, experts, and the score-weighted sum of each token's
         top-k expert outputs (fmoe/layers.py:205-312)."""
         whole = getattr(self.experts, "can_run_layer", None) if self.experts_fused else None
-        if (whole is not None and type(self.gate) is NaiveGate and self.gate_hook is None
-                and self.mask is None and whole(moe_inp, self.top_k)):
-            out = self.experts.run_gated_layer(self.gate, moe_inp)
-            if out is not None:
-                return out
+        if self.mask is None or self.mask_dict is None:
+            if whole is not None and self.gate_hook is None and isinstance(self.gate, NaiveGate) \
+                    and whole(moe_inp, self.top_k):
+                out = self.experts.run_gated_layer(self.gate, moe_inp)
+                if out is not None:
+                    return out
+            elif not self.experts_fused:
+                out = self._run_native_list(moe_inp)
+                if out is not None:
+                    return out
         sizes = tree.flatten(tree.map_structure(lambda t: t.shape[0], moe_inp))
         assert all(s == sizes[0] for s in sizes), \
             "MoE inputs must have the same batch size"

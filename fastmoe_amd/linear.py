@@ -275,6 +275,14 @@ def is_exact_gelu(activation, x: torch.Tensor) -> bool:
             and x.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16))
 
 
+def native_act(activation, x: torch.Tensor) -> int:
+    r"""The library's code of `activation` (FMOE_ACT_*), 0 if it has no kernels for it."""
+    if is_exact_gelu(activation, x):
+        return 1
+    return 2 if type(activation) is torch.nn.ReLU or activation is torch.relu \
+        or activation is torch.nn.functional.relu else 0
+
+
 def act_linear(activation, pre, fwd_expert_count, weight, bias):
     r"""`linear(activation(pre))` over the experts' row segments."""
     if is_exact_gelu(activation, pre) and pre.dtype == weight.dtype:

@@ -9,7 +9,7 @@ from . import fmoe_cuda
 from .functions import SegmentTable
 from .layers import FMoE
 from .linear import (FMoELinear, MOELinear, ParamTables, act_linear, is_exact_gelu,
-                     linear_act_linear, linear_act_linear_list)
+                     linear_act_linear, linear_act_linear_list, native_act)
 
 
 def _watched(*modules) -> bool:
@@ -19,6 +19,13 @@ def _watched(*modules) -> bool:
                (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or
                 getattr(m, "_backward_pre_hooks", None))
                for m in modules)
+
+
+def _hooked(module) -> bool:
+    r"""_watched() of one module, through its dictionary."""
+    d = module.__dict__
+    return bool(d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                or d.get("_backward_pre_hooks"))
 
 
 class FusedExpertLayer(Function):
@@ -130,22 +137,31 @@ class _Expert(nn.Module):
 
     def can_run_layer(self, inp, top_k) -> bool:
         r"""Whether the whole layer (dispatch included) can run as one autograd node:
-        one 2-d GPU tensor in the parameters' dtype, the exact GELU between the two
-        layers, and nobody watching the modules inside."""
+        one 2-d GPU tensor in the parameters' dtype, an activation the library has kernels
+        for (ReLU in the extension only) between the two layers, and nobody watching the
+        modules inside."""
         w1, w2 = self.htoh4.weight, self.h4toh.weight
         return (torch.is_tensor(inp) and inp.dim() == 2 and inp.is_cuda
                 and inp.dtype == w1.dtype == w2.dtype and 1 <= top_k <= 64
-                and is_exact_gelu(self.activation, inp)
+                and (is_exact_gelu(self.activation, inp)
+                     or (native_act(self.activation, inp) != 0
+                         and fmoe_cuda.native() is not None))
                 and not _watched(self, self.htoh4, self.h4toh, self.activation))
+
+    def _native_args(self, inp):
+        r"""The experts' share of a call of the extension's layer nodes."""
+        l1, l2 = self.htoh4, self.h4toh
+        params = [p for p in (l1.weight, l1.bias, l2.weight, l2.bias) if p is not None]
+        return (params, l1.num_expert, l1.bias is not None, l2.bias is not None,
+                native_act(self.activation, inp))
 
     def run_layer(self, inp, gate_idx, score):
         r"""`sum_j score[t, j] * expert_{gate_idx[t, j]}(inp[t])` over the live slots,
         as one autograd node: the extension's own, or FusedExpertLayer where a Python node
         is wanted (ctypes binding, per-op profiling)."""
-        native = fmoe_cuda.native_layers()
+        native = fmoe_cuda.native()
         if native is not None:
-            return native[0](inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
-                             self.h4toh.weight, self.h4toh.bias)
+            return native.expert_layer(inp, gate_idx, score, *self._native_args(inp))
         return FusedExpertLayer.apply(inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
                                       self.h4toh.weight, self.h4toh.bias)
 
@@ -153,12 +169,12 @@ class _Expert(nn.Module):
         r"""The layer with the plain top-k gate `gate` (NaiveGate) in front of it as one
         native autograd node, the gate's zero loss included; None where the gate has to run
         as the module it is.  Only called after can_run_layer()."""
-        native = fmoe_cuda.native_layers()
+        native = fmoe_cuda.native()
         if native is None or not gate.is_plain(inp):
             return None
         lin = gate.gate
-        out, loss = native[1](inp, lin.weight, lin.bias, self.htoh4.weight, self.htoh4.bias,
-                              self.h4toh.weight, self.h4toh.bias, gate.top_k)
+        out, loss = native.gated_layer(inp, lin.weight, lin.bias, *self._native_args(inp),
+                                       gate.top_k)
         gate.set_loss(loss)
         return out
 
@@ -199,6 +215,49 @@ class _Expert(nn.Module):
                     and not _watched(e, e.htoh4, e.h4toh)):
                 return False
         return not _watched(first.activation)
+
+    @staticmethod
+    def native_list_args(experts, inp):
+        r"""The share of a list of single-expert modules in a call of the extension's layer
+        nodes (which read every expert's parameters where they lie), or None where the list
+        has to run some other way.  The conditions of can_run_list(), checked on the
+        modules' own dictionaries: a list is looked through on every call."""
+        first = None
+        kinds = ([], [], [], [])
+        for e in experts:
+            if type(e) is not _Expert or _hooked(e):
+                return None
+            mods = e.__dict__["_modules"]
+            l1, l2 = mods["htoh4"], mods["h4toh"]
+            if (type(l1) is not FMoELinear or type(l2) is not FMoELinear or _hooked(l1)
+                    or _hooked(l2) or l1.num_expert != 1 or l2.num_expert != 1):
+                return None
+            act = mods["activation"] if "activation" in mods else e.activation
+            if first is None:
+                first = act
+            elif act is not first:
+                return None
+            p1, p2 = l1.__dict__["_parameters"], l2.__dict__["_parameters"]
+            for kind, p in zip(kinds, (p1["weight"], p1["bias"], p2["weight"], p2["bias"])):
+                kind.append(p)
+        act = native_act(first, inp)
+        if not act or _watched(first):
+            return None
+        params = []
+        for kind in kinds:
+            present = kind[0] is not None
+            for p in kind:
+                if (p is not None) != present or (present and (
+                        p.dtype != inp.dtype or p.shape != kind[0].shape or not p.is_cuda)):
+                    return None
+            if present:
+                params += kind
+        tables = getattr(experts, "_fmoe_native_tables", None)
+        if tables is None:
+            tables = fmoe_cuda.native().ParamTables()
+            object.__setattr__(experts, "_fmoe_native_tables", tables)
+        return (params, len(kinds[0]), kinds[1][0] is not None, kinds[3][0] is not None, act,
+                tables)
 
     @staticmethod
     def run_list(experts, inp, segments: SegmentTable):

@@ -56,6 +56,12 @@ typedef enum fmoe_activation {
   FMOE_ACT_RELU = 2
 } fmoe_activation;
 
+/* The gates with a load-balance loss. */
+typedef enum fmoe_balance_gate {
+  FMOE_GATE_GSHARD = 0, /* top-2, fmoe/gates/gshard_gate.py:25-62 */
+  FMOE_GATE_SWITCH = 1  /* top-1, fmoe/gates/switch_gate.py:24-60 */
+} fmoe_balance_gate;
+
 /* Largest number of experts the routing kernels keep in LDS. */
 #define FMOE_MAX_EXPERTS 4096
 /* Largest top_k of the fused gate kernels. */
@@ -167,6 +173,17 @@ int fmoe_prune_gate_by_capacity(const int64_t* gate_idx, int64_t* new_gate_idx,
                                 int32_t* ec, int64_t numel, int64_t n_expert,
                                 int64_t n_worker, void* workspace,
                                 int64_t workspace_bytes, void* stream);
+
+/*
+ * The capacity limit as the gates use it (fmoe/gates/utils.py:9-26 at one worker): every
+ * expert keeps its first `capacity` slots.  new_gate[i] = gate[i], or -1 where dropped (entries
+ * outside [0, n_expert) stay as they are); new_count[e] = slots that survive.  One call for
+ * fmoe_expert_count, fmoe_limit_by_capacity and fmoe_prune_gate_by_capacity.
+ */
+int fmoe_limit_gate(const int64_t* gate, int64_t numel, int32_t n_expert, int64_t capacity,
+                    int64_t* new_gate, int64_t* new_count, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+
 
 /* ----------------------------------------------------------------- dispatch */
 
@@ -395,6 +412,24 @@ int fmoe_topk_softmax_fwd(const void* logits, int64_t n_tokens, int32_t n_expert
  */
 int fmoe_naive_gate_fwd(const void* logits, int64_t n_tokens, int32_t n_expert, int32_t top_k,
                         int64_t* idx, void* score, float* zero_loss, int dtype, void* stream);
+
+/*
+ * A gate with a load-balance loss from its logits [T, E] (f32, f16 or bf16, E <= 512): idx and
+ * score [T, 2] (GShard) or [T, 1] (Switch) before any capacity limit, the loss (float[1]) and,
+ * for the backward, d loss / d p[t][e] per expert (coef, float[E]), p the softmax of all
+ * logits.  `capacity` (Switch): the loss counts the slots that survive it.
+ * Replaces torch code of fmoe/gates/gshard_gate.py:25-62 and fmoe/gates/switch_gate.py:24-60;
+ * no counterpart in the reference's extension.
+ */
+int64_t fmoe_balance_gate_workspace_bytes(int32_t n_expert);
+int fmoe_balance_gate_fwd(const void* logits, int64_t n_tokens, int32_t n_expert, int kind,
+                          int64_t capacity, int64_t* idx, void* score, float* loss, float* coef,
+                          void* workspace, int64_t workspace_bytes, int dtype, void* stream);
+/* dlogits of both outputs; dloss (float[1]) or dscore may be NULL. */
+int fmoe_balance_gate_bwd(const void* logits, const float* coef, const float* dloss,
+                          const void* dscore, const void* score, const int64_t* idx,
+                          void* dlogits, int64_t n_tokens, int32_t n_expert, int kind, int dtype,
+                          void* stream);
 
 /*
  * Backward of fmoe_topk_softmax_fwd with respect to the logits:

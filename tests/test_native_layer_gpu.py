@@ -75,3 +75,105 @@ def test_gate_hooks_and_no_tokens():
     out.sum().backward()
     assert out.shape == (0, 64) and empty.grad.shape == (0, 64)
     assert not any(p.grad.any().item() for p in moe.experts.parameters())
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
+@pytest.mark.parametrize("gate,top_k", [("NaiveGate", 2), ("GShardGate", 2), ("SwitchGate", 1)])
+@pytest.mark.parametrize("fused", [True, False])
+def test_gates_activations_and_layouts_match_the_chain(dt, act, gate, top_k, fused):
+    """Every gate, activation and expert layout through the native nodes against the Python
+    chain with torch's own gate arithmetic.  The routing and the survivors of the capacity are
+    the same; values differ by the roundings of the storage type in the gate's loss, whose
+    gradient the chain rounds once per torch operation (a few units in the last place of a
+    sum over the tokens: 4 roundings of eps each on values of the sum's scale)."""
+    import fastmoe_amd
+    from fastmoe_amd import FMoETransformerMLP, fmoe_cuda
+
+    dtype = DTYPES[dt]
+    torch.manual_seed(11)
+    moe = FMoETransformerMLP(8, 64, 96, top_k=top_k, gate=getattr(fastmoe_amd, gate),
+                             activation=act(), fused=fused).to(dtype).cuda()
+    moe.gate.capacity = (0.9, 0.9)          # some slots are dropped
+    moe.gate.random_routing, moe.gate.switch_eps = False, 0.0
+    x = torch.randn(500, 64, device="cuda").to(dtype)
+    dy = torch.randn(500, 64, device="cuda").to(dtype)
+    got = []
+    for watched in (False, True):
+        fmoe_cuda.profile_hook = (lambda *a: None) if watched else None
+        try:
+            for p in moe.parameters():
+                p.grad = None
+            a = x.clone().requires_grad_(True)
+            out = moe(a)
+            loss = moe.gate.get_loss()
+            torch.autograd.backward([out, loss], [dy, None if gate != "NaiveGate" else
+                                                  torch.zeros_like(loss)])
+            with torch.no_grad():
+                idx = moe.gate(x)[0]
+        finally:
+            fmoe_cuda.profile_hook = None
+        got.append([idx, out, loss, a.grad] + [p.grad for p in moe.parameters()])
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert (got[0][0] == -1).any() or gate == "NaiveGate"
+    tol = 4 * torch.finfo(dtype).eps
+    for g, w in zip(got[0][2:], got[1][2:]):
+        assert (g - w).double().norm() <= tol * w.double().norm()
+
+
+@pytest.mark.parametrize("n,e,cap", [(0, 4, 2), (100, 4, 0), (4096, 7, 300), (4097, 512, 8),
+                                     (9000, 513, 5), (70000, 16, 4000)])
+def test_limit_gate_matches_count_limit_prune(n, e, cap):
+    from fastmoe_amd import fmoe_cuda
+    from fastmoe_amd.gates import limit_by_capacity
+
+    g = torch.Generator().manual_seed(n)
+    gate = torch.randint(-1, e, (n, 1), generator=g).cuda()
+    new = limit_by_capacity(gate, e, 1, cap)
+    fmoe_cuda.profile_hook = lambda *a: None
+    try:
+        want = limit_by_capacity(gate, e, 1, cap)
+    finally:
+        fmoe_cuda.profile_hook = None
+    for a, b in zip(new, want):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+@pytest.mark.parametrize("kind,k", [("GATE_GSHARD", 2), ("GATE_SWITCH", 1)])
+@pytest.mark.parametrize("t,e", [(1, 2), (33, 16), (500, 17), (300, 64), (700, 65), (9000, 129),
+                                 (300, 512)])
+def test_balance_gate_against_float64(dt, kind, k, t, e):
+    """Indices, scores, loss and the gradient of both outputs against torch in float64 on the
+    same rounded logits.  Ties go to the lower expert.  Bounds: one rounding of the storage type
+    on the outputs; the loss is a sum of T * E float32 terms (its error stays below
+    1e-5 of it)."""
+    from fastmoe_amd import fmoe_cuda
+
+    m, dtype = fmoe_cuda.native(), DTYPES[dt]
+    g = torch.Generator().manual_seed(t + e)
+    logits = torch.randn(t, e, generator=g).to(dtype).cuda()
+    cap = max(1, int(1.1 * t * k / e))
+    a = logits.clone().requires_grad_(True)
+    idx, score, loss = m.balance_gate(a, getattr(m, kind), cap)
+    ds = torch.randn(t, k, generator=g).to(dtype).cuda()
+    torch.autograd.backward([score, loss], [ds, torch.tensor(3.0, device="cuda")])
+    ref = logits.double().requires_grad_(True)
+    p = torch.softmax(ref, -1)
+    order = torch.argsort(logits.double(), dim=-1, descending=True, stable=True)[:, :k]
+    chosen = torch.gather(ref, 1, order)
+    want = torch.softmax(chosen, -1) if k == 2 else torch.gather(p, 1, order)
+    count = torch.bincount(order[:, 0], minlength=e).double()
+    if k == 2:
+        want_loss = (count / t * p.mean(0)).mean() * e ** 2
+    else:
+        kept = count.clamp(max=cap)
+        want_loss = (kept / kept.sum() * p.sum(0) / kept.sum()).sum() * e
+    torch.autograd.backward([want, want_loss],
+                            [ds.double(), torch.tensor(3.0, device="cuda", dtype=torch.float64)])
+    live = m.limit_gate(order.contiguous(), e, cap)[1]
+    assert torch.equal(idx, live)
+    eps = torch.finfo(dtype).eps
+    assert (score.double() - want).abs().max() <= eps
+    assert abs(loss.item() - want_loss.item()) <= 1e-5 * abs(want_loss.item())
+    assert (a.grad.double() - ref.grad).abs().max() <= 4 * eps * ref.grad.abs().max()
