@@ -62,6 +62,14 @@ void* stream_of(const Tensor& t) {
 
 void* ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
+bool is_capturing(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess)
+    return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // Scratch memory for a call on torch's current stream of `like`'s device.  One buffer per
 // (device, stream) is kept and reused: launches on one stream run in order, and nothing in
 // it outlives a call.  A stream under graph capture gets a fresh tensor instead, which then
@@ -71,12 +79,7 @@ Tensor workspace_of(int64_t bytes, const Tensor& like) {
   if (bytes < 1) bytes = 1;
   auto opts = like.options().dtype(at::kByte);
   void* stream = stream_of(like);
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess ||
-      capturing != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return torch::empty({bytes}, opts);
-  }
+  if (is_capturing(stream)) return torch::empty({bytes}, opts);
   static std::mutex mu;
   // (never destroyed: at process exit the tensors must not be freed after torch's
   // allocator has gone)

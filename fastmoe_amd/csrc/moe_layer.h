@@ -31,30 +31,39 @@ struct RouteLayout {
 };
 
 // Device pointer tables of per-expert parameter lists (w1, b1, w2, b2), rebuilt only when a
-// parameter's storage has moved (optimizers update in place, so normally never).
+// parameter's storage has moved (optimizers update in place, so normally never) or the call
+// comes on another stream than the last one (nothing orders it behind the kernel that wrote
+// the table).  A call under graph capture gets a table of its own: its writing is a node of
+// the graph, so nobody outside may rely on it, and it has to live as long as the graph.
 struct ParamTables {
   std::vector<const void*> key;
   Tensor table;   // int64 [4, E]; rows of absent biases stay zero
+  void* stream = nullptr;
 
-  const Tensor& get(const std::vector<Tensor>& params, int64_t n_expert, bool has_b1, bool has_b2) {
+  Tensor get(const std::vector<Tensor>& params, int64_t n_expert, bool has_b1, bool has_b2) {
     std::vector<const void*> now(4 * n_expert, nullptr);
     const bool present[4] = {true, has_b1, true, has_b2};
     size_t at = 0;
     for (int row = 0; row < 4; ++row)
       if (present[row])
         for (int64_t e = 0; e < n_expert; ++e) now[row * n_expert + e] = params[at++].data_ptr();
-    if (!table.defined() || table.device() != params[0].device() || now != key) {
+    void* on = stream_of(params[0]);
+    const bool capturing = is_capturing(on);
+    if (capturing || !table.defined() || table.device() != params[0].device() || now != key ||
+        on != stream) {
       for (const Tensor& t : params) {
         dev(t, "expert parameter", params[0].scalar_type());
         need(t.device() == params[0].device(), "expert parameters must share their device");
         need((uintptr_t)t.data_ptr() % 16 == 0, "expert parameters must be 16-byte aligned");
       }
       // (a new tensor: kernels of an earlier call may still be reading the old one)
-      table = torch::empty({4, n_expert}, params[0].options().dtype(at::kLong));
-      check(fmoe_pointer_table(now.data(), (int64_t)now.size(), (const void**)table.data_ptr(),
-                               stream_of(params[0])),
+      Tensor fresh = torch::empty({4, n_expert}, params[0].options().dtype(at::kLong));
+      check(fmoe_pointer_table(now.data(), (int64_t)now.size(), (const void**)fresh.data_ptr(), on),
             "pointer_table");
+      if (capturing) return fresh;
+      table = fresh;
       key = std::move(now);
+      stream = on;
     }
     return table;
   }
@@ -493,6 +502,26 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     ctx->set_materialize_grads(false);
     return {kept, score, loss};
   }
+  // The backward as torch operations, for gradients of higher order: the loss reaches
+  // softmax(logits) with one constant per expert, the scores are the softmax of the chosen
+  // logits (GShard) or the chosen values of softmax(logits) (Switch).
+  static Tensor differentiable(int64_t kind, const Tensor& logits, const Tensor& coef,
+                               const Tensor& idx, const Tensor& dscore, const Tensor& dloss) {
+    const Tensor x = logits.to(at::kFloat), p = at::softmax(x, -1);
+    Tensor dp = at::zeros_like(p), dx = at::zeros_like(p);
+    if (dloss.defined()) dp = dp + coef * dloss;
+    if (dscore.defined()) {
+      const Tensor ds = dscore.to(at::kFloat);
+      if (kind == FMOE_GATE_GSHARD) {
+        const Tensor s = at::softmax(x.gather(1, idx), -1);
+        dx = dx.scatter_add(1, idx, s * (ds - (ds * s).sum(-1, true)));
+      } else {
+        dp = dp.scatter_add(1, idx, ds);
+      }
+    }
+    return (dx + p * (dp - (dp * p).sum(-1, true))).to(logits.scalar_type());
+  }
+
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list v = ctx->get_saved_variables();
     const Tensor &logits = v[0], &coef = v[1], &score = v[2], &idx = v[3];
@@ -500,6 +529,9 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     const Tensor dloss = grads[2];
     if (!dscore.defined() && !dloss.defined()) return {Tensor(), Tensor(), Tensor()};
     c10::DeviceGuard guard(logits.device());
+    if (at::GradMode::is_enabled())   // a gradient that will itself be differentiated
+      return {differentiable(ctx->saved_data["kind"].toInt(), logits, coef, idx, dscore, dloss),
+              Tensor(), Tensor()};
     Tensor dlogits = at::empty_like(logits);
     check(fmoe_balance_gate_bwd(logits.data_ptr(), coef.data_ptr<float>(),
                                 dloss.defined() ? dloss.data_ptr<float>() : nullptr,

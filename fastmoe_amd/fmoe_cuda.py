@@ -26,6 +26,7 @@ import os
 import warnings
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _ctypes_ops as ctypes_ops
 
@@ -92,9 +93,16 @@ _compiled = None    # the extension, once bound
 def native():
     """The compiled extension with its whole-layer and gate nodes (expert_layer, gated_layer,
     balance_gate, limit_gate): one autograd node each that enters Python nowhere between its
-    launches.  None where they do not apply: on the ctypes binding, and while `profile_hook`
-    watches the single operators."""
-    return None if profile_hook is not None else _compiled
+    launches.  None where they do not apply: on the ctypes binding, while `profile_hook`
+    watches the single operators, and under anything that has to see the torch operations
+    of a gate one by one (tracing, dispatch modes, vmap, forward-mode differentiation)."""
+    if (profile_hook is not None or forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.compiler.is_compiling()):
+        return None
+    return _compiled
 
 
 def _bind(binding: str) -> None:

@@ -131,6 +131,22 @@ class ParamTables:
         return self._table[name]
 
 
+class NativeTables:
+    r"""The extension's table of a list of expert modules, made at the first call.  A copy or
+    a pickle of the list starts without one."""
+
+    def __init__(self):
+        self._tables = None
+
+    def get(self, native):
+        if self._tables is None:
+            self._tables = native.ParamTables()
+        return self._tables
+
+    def __reduce__(self):
+        return NativeTables, ()
+
+
 def _split_params(params, n_expert, has_bias):
     weights = params[:n_expert]
     biases = params[n_expert:2 * n_expert] if has_bias else None

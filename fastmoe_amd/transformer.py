@@ -8,7 +8,7 @@ from torch.autograd import Function
 from . import fmoe_cuda
 from .functions import SegmentTable
 from .layers import FMoE
-from .linear import (FMoELinear, MOELinear, ParamTables, act_linear, is_exact_gelu,
+from .linear import (FMoELinear, MOELinear, NativeTables, ParamTables, act_linear, is_exact_gelu,
                      linear_act_linear, linear_act_linear_list, native_act)
 
 
@@ -238,6 +238,8 @@ class _Expert(nn.Module):
             elif act is not first:
                 return None
             p1, p2 = l1.__dict__["_parameters"], l2.__dict__["_parameters"]
+            if not {"weight", "bias"} <= p1.keys() & p2.keys():
+                return None   # somebody keeps a plain tensor in a parameter's place
             for kind, p in zip(kinds, (p1["weight"], p1["bias"], p2["weight"], p2["bias"])):
                 kind.append(p)
         act = native_act(first, inp)
@@ -254,10 +256,10 @@ class _Expert(nn.Module):
                 params += kind
         tables = getattr(experts, "_fmoe_native_tables", None)
         if tables is None:
-            tables = fmoe_cuda.native().ParamTables()
+            tables = NativeTables()
             object.__setattr__(experts, "_fmoe_native_tables", tables)
         return (params, len(kinds[0]), kinds[1][0] is not None, kinds[3][0] is not None, act,
-                tables)
+                tables.get(fmoe_cuda.native()))
 
     @staticmethod
     def run_list(experts, inp, segments: SegmentTable):

@@ -1,6 +1,9 @@
 """The layer as one native autograd node against the chain of Python nodes it replaces
 (which still runs while a per-op event hook is set): the same kernels in the same order,
 so the same bits, with and without gradients, for every subset of gradients asked for."""
+import copy
+import io
+
 import pytest
 import torch
 
@@ -177,3 +180,89 @@ def test_balance_gate_against_float64(dt, kind, k, t, e):
     assert (score.double() - want).abs().max() <= eps
     assert abs(loss.item() - want_loss.item()) <= 1e-5 * abs(want_loss.item())
     assert (a.grad.double() - ref.grad).abs().max() <= 4 * eps * ref.grad.abs().max()
+
+
+def _list_layer():
+    from fastmoe_amd import FMoETransformerMLP
+
+    torch.manual_seed(5)
+    return FMoETransformerMLP(4, 64, 96, top_k=2, fused=False).cuda()
+
+
+def test_list_layer_copies_and_pickles_after_a_call():
+    """A layer that has run is still one that can be copied and saved; its copy reads its own
+    parameters."""
+    moe = _list_layer()
+    x = torch.randn(50, 64, device="cuda")
+    want = moe(x).detach()
+    twin = copy.deepcopy(moe)
+    file = io.BytesIO()
+    torch.save(moe, file)
+    file.seek(0)
+    for other in (twin, torch.load(file, weights_only=False)):
+        assert torch.equal(other(x), want)
+        with torch.no_grad():
+            for p in other.experts.parameters():
+                p.zero_()
+        assert not other(x).any() and torch.equal(moe(x), want)
+
+
+def test_list_layer_first_called_under_capture_or_on_another_stream():
+    """The table of the experts' addresses is written by the stream that reads it: a graph
+    that has not run yet leaves nothing behind for eager calls, nor do calls on one stream
+    for those on another."""
+    moe, x = _list_layer(), torch.randn(50, 64, device="cuda")
+    with torch.no_grad():
+        want = copy.deepcopy(moe)(x)
+        warm = torch.cuda.Stream()
+        warm.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(warm):
+            copy.deepcopy(moe)(x)
+        torch.cuda.current_stream().wait_stream(warm)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = moe(x)
+        assert torch.equal(moe(x), want)          # before the first replay
+        other = torch.cuda.Stream()
+        other.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(other):
+            assert torch.equal(moe(x), want)
+        torch.cuda.synchronize()
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and torch.equal(moe(x), want)
+
+
+@pytest.mark.parametrize("gate,top_k", [("GShardGate", 2), ("SwitchGate", 1)])
+def test_balance_loss_differentiates_twice_and_forwards(gate, top_k):
+    """The gradient of a balance loss has a gradient of its own, and the Switch gate takes
+    forward-mode tangents, as the torch operations that the gates consist of do.  Against the
+    gate run operation by operation in float32: sums of 200 x 8 terms, 1e-5 of their size."""
+    import fastmoe_amd
+    from fastmoe_amd import fmoe_cuda
+    from torch.autograd import forward_ad
+
+    torch.manual_seed(9)
+    layer = getattr(fastmoe_amd, gate)(32, 8, 1, topk=top_k).cuda()
+    layer.random_routing, layer.switch_eps = False, 0.0
+    x = torch.randn(200, 32, device="cuda")
+    got = []
+    for watched in (False, True):
+        fmoe_cuda.profile_hook = (lambda *a: None) if watched else None
+        try:
+            a = x.clone().requires_grad_(True)
+            _, score = layer(a)
+            loss = layer.get_loss() + (score[:, 0] ** 2).sum() * (gate == "SwitchGate")
+            (da,) = torch.autograd.grad(loss, a, create_graph=True)
+            (dda,) = torch.autograd.grad((da ** 2).sum(), a)
+        finally:
+            fmoe_cuda.profile_hook = None
+        got.append((da.detach(), dda))
+    for g, w in zip(*got):
+        assert w.any() and (g - w).norm() <= 1e-5 * w.norm()
+    if gate == "SwitchGate":
+        with forward_ad.dual_level():
+            layer(forward_ad.make_dual(x, torch.ones_like(x)))
+            assert forward_ad.unpack_dual(layer.get_loss()).tangent is not None
