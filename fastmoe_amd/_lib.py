@@ -81,6 +81,13 @@ SIGNATURES = {
                                       c_void_p, c_int64, c_int32, c_int, c_int, c_void_p]),
     "fmoe_naive_gate_fwd": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
                                     c_void_p, c_int, c_void_p]),
+    "fmoe_gate_slot_grad": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),
+    "fmoe_scatter_reduce_gate": (c_int, [c_void_p] * 6 + [c_int64, c_int64, c_int64, c_int32, c_int,
+                                                          c_void_p]),
+    "fmoe_gate_linear_grad_workspace_bytes": (c_int64, [c_void_p, c_int64, c_int64, c_int64, c_int32,
+                                                        c_int]),
+    "fmoe_gate_linear_grad": (c_int, [c_void_p] * 6 + [c_int64, c_int64, c_int64, c_int32, c_void_p,
+                                                       c_int64, c_int, c_void_p]),
     "fmoe_topk_softmax_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                       c_int32, c_int, c_void_p]),
     "fmoe_scatter_tokens": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64,

@@ -20,7 +20,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libfmoe_hip.so")
 
 # the two heavy translation units first, so that they compile side by side
 SOURCES = ["gemm_mfma_bf16.hip", "gemm_mfma_f16.hip", "api.hip", "route.hip", "dispatch.hip",
-           "gate.hip", "act.hip", "gemm_simt.hip", "gemm_mfma.hip", "gemm_plain.hip",
+           "gate.hip", "gate_grad.hip", "act.hip", "gemm_simt.hip", "gemm_mfma.hip", "gemm_plain.hip",
            "gemm_mfma_wide.hip"]
 HEADERS = ["common.h", "gemm.h", "gemm_tiles.h", "act_math.h",
            "dma_desc.h", "gemm_mfma_impl.h",

@@ -133,11 +133,23 @@ __device__ __forceinline__ double lane_value(double v, int j) {
 // that a wave holds 2 to 4 packs per lane of each row: measured on rows of
 // 8 KiB, one wave per token reaches 0.60-0.66 of the HBM peak, four waves 0.75+;
 // short rows (2 KiB) do best with one wave and 2 packs per lane.
-template <typename T, int VEC, int SPLIT, int UNROLL>
-__global__ __launch_bounds__(kDispThreads) void combine_fwd_kernel(
+//
+// GATE: the gradient of a layer's input also has the gate's share,
+// sum_j dl[t,j] * wg[idx[t,j]] (the gradient of the logits is zero for all other experts), whose
+// rows come from L2.  As a dense product and an addition it was two launches and two more
+// passes over y: 14 + 9 us behind 12 us of reduction at 8192 x 1024 bf16, 52 + 56 behind 68 at
+// 16384 x 4096; here the reduction takes them along.
+template <typename T> struct GateShare {
+  const int64_t* idx;
+  const typename Elem<T>::acc_t* dl;
+  const T* wg;
+  int n_expert;
+};
+template <typename T, int VEC, int SPLIT, int UNROLL, bool GATE>
+__device__ __forceinline__ void combine_rows(
     const T* __restrict__ buf, const int32_t* __restrict__ inv,
     const T* __restrict__ score, T* __restrict__ y, int64_t n_tokens, int top_k,
-    int64_t d) {
+    int64_t d, const GateShare<T>& gate) {
   using acc_t = typename Elem<T>::acc_t;
   struct alignas(sizeof(T) * VEC) Pk { T v[VEC]; };
   constexpr int kTokPerBlock = kDispWaves / SPLIT;
@@ -155,10 +167,16 @@ __global__ __launch_bounds__(kDispThreads) void combine_fwd_kernel(
     if (t >= n_tokens) continue;
     // lane j keeps the row and weight of slot j
     int32_t my_r = -1;
-    acc_t my_s = 0;
+    acc_t my_s = 0, my_g = 0;
+    int32_t my_e = -1;
     if (lane < top_k) {
       my_r = inv[t * top_k + lane];
       my_s = score ? Elem<T>::to_acc(score[t * top_k + lane]) : (acc_t)1;
+      if (GATE) {
+        my_g = gate.dl[t * top_k + lane];
+        const int64_t at = gate.idx[t * top_k + lane];
+        my_e = at >= 0 && at < gate.n_expert ? (int32_t)at : -1;
+      }
     }
     // UNROLL packs per lane per step: all their loads are issued before the
     // first is used
@@ -186,6 +204,24 @@ __global__ __launch_bounds__(kDispThreads) void combine_fwd_kernel(
 #pragma unroll
           for (int v = 0; v < VEC; ++v) acc[u][v] += s * Elem<T>::to_acc(p[u].v[v]);
       }
+      if (GATE) {
+        for (int j = 0; j < top_k; ++j) {
+          const int32_t ge = lane_value(my_e, j);
+          const acc_t gs = lane_value(my_g, j);
+          if (ge < 0) continue;
+          const T* src = gate.wg + (int64_t)ge * d;
+          Pk p[UNROLL];
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) {
+            const int64_t c = c0 + (int64_t)u * kWave;
+            if (c < c_end) p[u] = *reinterpret_cast<const Pk*>(src + c * VEC);
+          }
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[u][v] += gs * Elem<T>::to_acc(p[u].v[v]);
+        }
+      }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const int64_t c = c0 + (int64_t)u * kWave;
@@ -198,6 +234,21 @@ __global__ __launch_bounds__(kDispThreads) void combine_fwd_kernel(
       }
     }
   }
+}
+
+template <typename T, int VEC, int SPLIT, int UNROLL>
+__global__ __launch_bounds__(kDispThreads) void combine_fwd_kernel(
+    const T* __restrict__ buf, const int32_t* __restrict__ inv,
+    const T* __restrict__ score, T* __restrict__ y, int64_t n_tokens, int top_k,
+    int64_t d) {
+  combine_rows<T, VEC, SPLIT, UNROLL, false>(buf, inv, score, y, n_tokens, top_k, d, {});
+}
+
+template <typename T, int VEC, int SPLIT, int UNROLL>
+__global__ __launch_bounds__(kDispThreads) void reduce_gate_kernel(
+    const T* __restrict__ buf, const int32_t* __restrict__ inv, GateShare<T> gate,
+    T* __restrict__ y, int64_t n_tokens, int top_k, int64_t d) {
+  combine_rows<T, VEC, SPLIT, UNROLL, true>(buf, inv, nullptr, y, n_tokens, top_k, d, gate);
 }
 
 // dbuf[inv[i]] = score[i] * dy[i/k];  dscore[i] = <dy[i/k], buf[inv[i]]>
@@ -385,6 +436,18 @@ static int launch_combine_fwd(const void* buf, const int32_t* inv,
   FMOE_COMBINE_DISPATCH(combine_fwd_kernel, (const T*)buf, inv, (const T*)score, (T*)y, n_tokens,
                         top_k, d);
   FMOE_LAUNCH_CHECK("combine_fwd");
+  return FMOE_OK;
+}
+
+template <typename T>
+static int launch_reduce_gate(const void* dbuf, const int32_t* inv, const int64_t* idx,
+                              const void* dl, const void* wg, int n_expert, void* dx,
+                              int64_t n_tokens, int top_k, int64_t d, hipStream_t s) {
+  constexpr int kVec = 16 / sizeof(T);
+  const bool vec = d % kVec == 0 && aligned(dbuf, 16) && aligned(dx, 16) && aligned(wg, 16);
+  const GateShare<T> gate{idx, (const typename Elem<T>::acc_t*)dl, (const T*)wg, n_expert};
+  FMOE_COMBINE_DISPATCH(reduce_gate_kernel, (const T*)dbuf, inv, gate, (T*)dx, n_tokens, top_k, d);
+  FMOE_LAUNCH_CHECK("scatter_reduce_gate");
   return FMOE_OK;
 }
 
@@ -607,6 +670,25 @@ extern "C" int fmoe_scatter_reduce(const void* dbuf, const int32_t* inv, void* d
     case FMOE_F64: return launch_combine_fwd<double>(dbuf, inv, nullptr, dx, n_tokens, (int)top_k, d, s);
     case FMOE_F16: return launch_combine_fwd<__half>(dbuf, inv, nullptr, dx, n_tokens, (int)top_k, d, s);
     default: return launch_combine_fwd<__hip_bfloat16>(dbuf, inv, nullptr, dx, n_tokens, (int)top_k, d, s);
+  }
+}
+
+extern "C" int fmoe_scatter_reduce_gate(const void* dbuf, const int32_t* inv, const int64_t* idx,
+                                        const void* dslot, const void* wg, void* dx,
+                                        int64_t n_tokens, int64_t top_k, int64_t d,
+                                        int32_t n_expert, int dtype, void* stream) {
+  int rc = check_combine("scatter_reduce_gate", n_tokens, top_k, d, dtype);
+  if (rc) return rc;
+  FMOE_REQUIRE(n_expert >= 1, FMOE_ERR_INVALID, "scatter_reduce_gate: no experts");
+  if (n_tokens == 0 || d == 0) return FMOE_OK;
+  FMOE_REQUIRE(inv && idx && dslot && wg && dx, FMOE_ERR_INVALID,
+               "scatter_reduce_gate: null pointer");
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case FMOE_F32: return launch_reduce_gate<float>(dbuf, inv, idx, dslot, wg, n_expert, dx, n_tokens, (int)top_k, d, s);
+    case FMOE_F64: return launch_reduce_gate<double>(dbuf, inv, idx, dslot, wg, n_expert, dx, n_tokens, (int)top_k, d, s);
+    case FMOE_F16: return launch_reduce_gate<__half>(dbuf, inv, idx, dslot, wg, n_expert, dx, n_tokens, (int)top_k, d, s);
+    default: return launch_reduce_gate<__hip_bfloat16>(dbuf, inv, idx, dslot, wg, n_expert, dx, n_tokens, (int)top_k, d, s);
   }
 }
 

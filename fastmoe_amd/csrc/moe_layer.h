@@ -195,8 +195,12 @@ LayerPass experts_forward(const LayerConfig& c, const LayerSizes& s, const Exper
   return p;
 }
 
+// A gate that ran inside the node: its operands in the backward.
+struct GateGrad {
+  Tensor x, wg, idx;
+};
 struct LayerGrads {
-  Tensor dx, dscore, dw1, db1, dw2, db2;
+  Tensor dx, dslot, dscore, dw1, db1, dw2, db2;
 };
 struct LayerNeeds {
   bool dx, w1, b1, w2, b2;
@@ -205,7 +209,8 @@ struct LayerNeeds {
 void* out_ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const ExpertParams& w,
-                            const LayerPass& p, const Tensor& dy, const LayerNeeds& want) {
+                            const LayerPass& p, const Tensor& dy, const LayerNeeds& want,
+                            const GateGrad* gate) {
   const auto opts = dy.options();
   void* stream = stream_of(dy);
   const RouteLayout at_(s.n, s.e);
@@ -218,6 +223,13 @@ LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const Exp
   check(fmoe_gather_combine_bwd(dy.data_ptr(), p.out.data_ptr(), inv, p.score.data_ptr(),
                                 d_out.data_ptr(), g.dscore.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
         "gather_combine_bwd");
+  if (gate) {
+    g.dslot = at::empty({s.t, s.k},
+                        opts.dtype(dy.scalar_type() == at::kDouble ? at::kDouble : at::kFloat));
+    check(fmoe_gate_slot_grad(g.dscore.data_ptr(), p.score.data_ptr(), g.dslot.data_ptr(), s.t, s.k,
+                              s.dtype, stream),
+          "gate_slot_grad");
+  }
   const bool first = want.dx || want.w1 || want.b1;   // whether the first layer has a backward
   Tensor dpre;
   if (first) dpre = at::empty({s.n, s.h}, opts);
@@ -240,8 +252,14 @@ LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const Exp
         "expert_linear_bwd");
   if (want.dx) {
     g.dx = at::empty({s.t, s.d}, opts);
-    check(fmoe_scatter_reduce(dbuf.data_ptr(), inv, g.dx.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
-          "scatter_reduce");
+    if (gate)
+      check(fmoe_scatter_reduce_gate(dbuf.data_ptr(), inv, gate->idx.data_ptr<int64_t>(),
+                                     g.dslot.data_ptr(), gate->wg.data_ptr(), g.dx.data_ptr(), s.t,
+                                     s.k, s.d, (int32_t)s.e, s.dtype, stream),
+            "scatter_reduce_gate");
+    else
+      check(fmoe_scatter_reduce(dbuf.data_ptr(), inv, g.dx.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
+            "scatter_reduce");
   }
   return g;
 }
@@ -261,8 +279,9 @@ void gate_topk(const LayerSizes& s, const Tensor& logits, Tensor& idx, Tensor& s
 
 // Forward of the layer.  vars: x, then (wg, bg if any) of a gate to be run here, or (idx,
 // score) of a gate that has been run; then the expert parameters.  The gate's linear map
-// stays the library call it is in torch.nn.Linear, in both directions, so the logits (and
-// with them the routing) and every gradient have the bits of the gate module.
+// stays the library call it is in torch.nn.Linear, so the logits (and with them the routing)
+// have the bits of the gate module; its gradients come from the top-k slots alone
+// (gate_grad.hip).
 LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, LayerSizes* sizes,
                         Tensor* x_out, Tensor* idx_out) {
   at::AutoDispatchBelowADInplaceOrView below;
@@ -352,20 +371,28 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     want.b1 = any(c.has_b1, per);
     want.w2 = any(true, per);
     want.b2 = any(c.has_b2, per);
-    LayerGrads g = experts_backward(c, s, w, p, dy, want);
+    const bool gate_grads = c.gated && (dx || nwg || nbg);
+    GateGrad gate;
+    if (gate_grads) gate = {v[6], v[7].contiguous(), v[8]};
+    LayerGrads g = experts_backward(c, s, w, p, dy, want, gate_grads ? &gate : nullptr);
     variable_list out;
     if (c.gated) {
-      const Tensor &x = v[6], &wg = v[7], &idx = v[8];
       Tensor dwg, dbg;
-      if (dx || nwg || nbg) {
-        Tensor dlogits = at::empty({s.t, s.e}, dy.options());
-        check(fmoe_topk_softmax_bwd(g.dscore.data_ptr(), p.score.data_ptr(), idx.data_ptr<int64_t>(),
-                                    dlogits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k, s.dtype,
-                                    stream_of(dy)),
-              "topk_softmax_bwd");
-        if (nwg) dwg = at::mm(dlogits.t(), x);
-        if (nbg) dbg = dlogits.sum(0);
-        if (dx) g.dx.add_(at::mm(dlogits, wg));
+      if (nwg || nbg) {
+        const Tensor& x = gate.x;
+        if (nwg) dwg = at::empty({s.e, s.d}, dy.options());
+        if (nbg) dbg = at::empty({s.e}, dy.options());
+        const RouteLayout at_(s.n, s.e);
+        const char* meta = (const char*)p.route.data_ptr();
+        const int64_t bytes = fmoe_gate_linear_grad_workspace_bytes(x.data_ptr(), s.t, s.k, s.d,
+                                                                    (int32_t)s.e, s.dtype);
+        check(bytes < 0 ? (int)bytes : 0, "gate_linear_grad");
+        Tensor ws = at::empty({bytes}, dy.options().dtype(at::kByte));
+        check(fmoe_gate_linear_grad(x.data_ptr(), (const int64_t*)meta,
+                                    (const int32_t*)(meta + at_.seg), g.dslot.data_ptr(),
+                                    out_ptr(dwg), out_ptr(dbg), s.t, s.k, s.d, (int32_t)s.e,
+                                    ws.data_ptr(), bytes, s.dtype, stream_of(dy)),
+              "gate_linear_grad");
       }
       out = {g.dx, dwg};
       if (c.has_bg) out.push_back(dbg);

@@ -443,6 +443,29 @@ int fmoe_topk_softmax_bwd(const void* dscore, const void* score, const int64_t* 
                           int32_t top_k, int dtype, void* stream);
 
 /*
+ * The gradient of the plain gate (Linear -> top-k -> softmax) without its dense logits:
+ *   dslot[t][j] = score_j * (dscore_j - sum_i dscore_i * score_i)
+ * in the accumulation type (f32; f64 for doubles) is the gradient of logit idx[t][j], all
+ * others are zero;
+ *   fmoe_scatter_reduce_gate:  dx[t] = sum_j dbuf[inv[t][j]] + sum_j dslot[t][j] * wg[idx[t][j]]
+ *   fmoe_gate_linear_grad:     dwg[e] = sum over the rows r of expert e (seg_off, pos of
+ *     fmoe_route) of dslot[pos[r]] * x[pos[r] / top_k], dbg[e] = sum of dslot[pos[r]]
+ * wg, dwg [n_expert, d], dbg [n_expert]; either of dwg, dbg may be null.  The workspace depends
+ * on the alignment of x.
+ */
+int fmoe_gate_slot_grad(const void* dscore, const void* score, void* dslot, int64_t n_tokens,
+                        int64_t top_k, int dtype, void* stream);
+int fmoe_scatter_reduce_gate(const void* dbuf, const int32_t* inv, const int64_t* idx,
+                             const void* dslot, const void* wg, void* dx, int64_t n_tokens,
+                             int64_t top_k, int64_t d, int32_t n_expert, int dtype, void* stream);
+int64_t fmoe_gate_linear_grad_workspace_bytes(const void* x, int64_t n_tokens, int64_t top_k,
+                                              int64_t d, int32_t n_expert, int dtype);
+int fmoe_gate_linear_grad(const void* x, const int64_t* pos, const int32_t* seg_off,
+                          const void* dslot, void* dwg, void* dbg, int64_t n_tokens, int64_t top_k,
+                          int64_t d, int32_t n_expert, void* workspace, int64_t workspace_bytes,
+                          int dtype, void* stream);
+
+/*
  * y[i] = gelu(x[i]) = 0.5 x (1 + erf(x / sqrt 2)) over n elements, and
  * dx[i] = dy[i] * gelu'(x[i]): the activation between the two expert layers,
  * fmoe/transformer.py:28-30 with the default torch.nn.GELU() of

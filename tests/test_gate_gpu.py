@@ -154,3 +154,55 @@ def test_naive_gate_uses_the_kernel_and_errors():
         fmoe_cuda.topk_softmax_fwd(torch.zeros(4, 3, device="cuda"), 4)      # k > experts
     with pytest.raises(RuntimeError):
         fmoe_cuda.topk_softmax_fwd(torch.zeros(4, 40, device="cuda"), 17)    # k > supported
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32", "f64"])
+@pytest.mark.parametrize("t,e,k,d", [(1, 1, 1, 1), (33, 4, 2, 7), (500, 5, 2, 264), (700, 130, 8, 520),
+                                     (5000, 3, 2, 1032), (4096, 16, 1, 4100)])
+def test_gate_gradients_from_slots(dt, t, e, k, d):
+    """The plain gate's gradients from its top-k slots (one slot in eight dropped, expert 0
+    popular) against the dense products in float64.  A sum of n products in the accumulation
+    type is off by at most (n + 8) units of the sum of their magnitudes (8: the gradient of the
+    slot itself), the result by one rounding of the storage type."""
+    from fastmoe_amd import _lib, fmoe_cuda
+
+    lib, dtype = _lib.load(), DTYPES[dt]
+    acc = torch.float64 if dt == "f64" else torch.float32
+    g = torch.Generator().manual_seed(t + d)
+    idx = torch.argsort(torch.rand(t, e, generator=g) - torch.eye(1, e) * 0.4, 1)[:, :k]
+    idx[torch.rand(t, k, generator=g) < 0.125] = -1
+    rnd = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64).to(dtype)
+    x, wg, dbuf, dscore = rnd(t, d), rnd(e, d), rnd(t * k, d), rnd(t, k)
+    score = torch.softmax(rnd(t, k).double(), 1).to(dtype)
+    c = {n: v.cuda().contiguous() for n, v in dict(idx=idx, x=x, wg=wg, dbuf=dbuf, dscore=dscore,
+                                                   score=score).items()}
+    pos, _, seg, inv = fmoe_cuda.route(c["idx"], e)
+    code = {"f32": 0, "f64": 1, "f16": 2, "bf16": 3}[dt]
+    stream = torch.cuda.current_stream().cuda_stream
+    dl = torch.empty(t, k, device="cuda", dtype=acc)
+    dx, dwg = torch.empty_like(c["x"]), torch.empty_like(c["wg"])
+    dbg = torch.empty(e, device="cuda", dtype=dtype)
+    n = lib.fmoe_gate_linear_grad_workspace_bytes(c["x"].data_ptr(), t, k, d, e, code)
+    ws = torch.empty(n, device="cuda", dtype=torch.uint8)
+    p = lambda a: a.data_ptr()
+    assert lib.fmoe_gate_slot_grad(p(c["dscore"]), p(c["score"]), p(dl), t, k, code, stream) == 0
+    assert lib.fmoe_scatter_reduce_gate(p(c["dbuf"]), p(inv), p(c["idx"]), p(dl), p(c["wg"]), p(dx),
+                                        t, k, d, e, code, stream) == 0
+    assert lib.fmoe_gate_linear_grad(p(c["x"]), p(pos), p(seg), p(dl), p(dwg), p(dbg), t, k, d, e,
+                                     p(ws), n, code, stream) == 0
+    s, ds = score.double(), dscore.double()
+    want_dl = s * (ds - (ds * s).sum(1, keepdim=True))
+    mag_dl = s * (ds.abs() + (ds * s).abs().sum(1, keepdim=True))
+    rows = inv.cpu().view(t, k).long()
+    live = (idx >= 0)[..., None].double()
+    moved = dbuf.double()[rows.clamp(min=0)] * live
+    dense = torch.zeros(t, e, dtype=torch.float64).scatter_add_(1, idx.clamp(min=0), want_dl * live[..., 0])
+    mags = torch.zeros(t, e, dtype=torch.float64).scatter_add_(1, idx.clamp(min=0), mag_dl * live[..., 0])
+    unit, eps = torch.finfo(acc).eps, torch.finfo(dtype).eps
+    for got, want, mag, terms in (
+            (dx, moved.sum(1) + dense @ wg.double(), moved.abs().sum(1) + mags @ wg.double().abs(), 2 * k),
+            (dwg, dense.t() @ x.double(), mags.t() @ x.double().abs(), t),
+            (dbg, dense.sum(0), mags.sum(0), t)):
+        err = (got.double().cpu() - want).abs()
+        # (f16 below its smallest normal number: half a step of 2^-24)
+        assert (err <= eps * want.abs() + unit * (terms + 8 + k) * mag + (2 ** -25 if dt == "f16" else 0)).all()

@@ -1,6 +1,7 @@
 """The layer as one native autograd node against the chain of Python nodes it replaces
 (which still runs while a per-op event hook is set): the same kernels in the same order,
-so the same bits, with and without gradients, for every subset of gradients asked for."""
+so the same bits, with and without gradients, for every subset of gradients asked for; only
+the gate's own gradients are summed by kernels of their own."""
 import copy
 import io
 
@@ -60,9 +61,19 @@ def test_native_node_matches_the_chain(dt, top_k, bias, frozen):
     x = torch.randn(130, 64, device="cuda").to(DTYPES[dt])
     dy = torch.randn(130, 64, device="cuda").to(DTYPES[dt])
     got, want = (_run(moe, x, dy, frozen, w) for w in (False, True))
-    for g, w in zip(got, want):
+    names = ["y", "x"] + [n for n, _ in moe.named_parameters()]
+    for name, g, w in zip(names, got, want):
         assert (g is None) == (w is None)
-        assert g is None or torch.equal(g, w)
+        if g is None or not (name == "x" or name.startswith("gate.")):
+            assert g is None or torch.equal(g, w)
+        else:
+            # the chain rounds the logits' gradient, the gate's share of dx and the experts'
+            # share of dx to the storage type (half an eps each) before it adds them up, this
+            # node the result alone: 2 eps of the gradient's size; f32 sums in another order
+            # differ by less than the 130 terms times 2^-24, i.e. 65 eps
+            eps = torch.finfo(g.dtype).eps
+            bound = (2 if dt == "bf16" else 65) * eps
+            assert (g - w).double().norm() <= bound * w.double().norm(), name
 
 
 def test_gate_hooks_and_no_tokens():
