@@ -138,7 +138,9 @@ __device__ __forceinline__ double lane_value(double v, int j) {
 // sum_j dl[t,j] * wg[idx[t,j]] (the gradient of the logits is zero for all other experts), whose
 // rows come from L2.  As a dense product and an addition it was two launches and two more
 // passes over y: 14 + 9 us behind 12 us of reduction at 8192 x 1024 bf16, 52 + 56 behind 68 at
-// 16384 x 4096; here the reduction takes them along.
+// 16384 x 4096; here the reduction takes them along.  Both shares are rounded to the storage
+// type before they are added, as when the gate is an autograd node of its own: the same bits
+// either way.  Without `inv` only the gate's share is written.
 template <typename T> struct GateShare {
   const int64_t* idx;
   const typename Elem<T>::acc_t* dl;
@@ -170,7 +172,7 @@ __device__ __forceinline__ void combine_rows(
     acc_t my_s = 0, my_g = 0;
     int32_t my_e = -1;
     if (lane < top_k) {
-      my_r = inv[t * top_k + lane];
+      my_r = GATE && !inv ? -1 : inv[t * top_k + lane];
       my_s = score ? Elem<T>::to_acc(score[t * top_k + lane]) : (acc_t)1;
       if (GATE) {
         my_g = gate.dl[t * top_k + lane];
@@ -205,6 +207,14 @@ __device__ __forceinline__ void combine_rows(
           for (int v = 0; v < VEC; ++v) acc[u][v] += s * Elem<T>::to_acc(p[u].v[v]);
       }
       if (GATE) {
+        acc_t rows[UNROLL][VEC];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) {
+            rows[u][v] = Elem<T>::to_acc(Elem<T>::from_acc(acc[u][v]));
+            acc[u][v] = 0;
+          }
         for (int j = 0; j < top_k; ++j) {
           const int32_t ge = lane_value(my_e, j);
           const acc_t gs = lane_value(my_g, j);
@@ -221,6 +231,11 @@ __device__ __forceinline__ void combine_rows(
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[u][v] += gs * Elem<T>::to_acc(p[u].v[v]);
         }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+          for (int v = 0; v < VEC; ++v)
+            acc[u][v] = rows[u][v] + Elem<T>::to_acc(Elem<T>::from_acc(acc[u][v]));
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
@@ -444,6 +459,7 @@ static int launch_reduce_gate(const void* dbuf, const int32_t* inv, const int64_
                               const void* dl, const void* wg, int n_expert, void* dx,
                               int64_t n_tokens, int top_k, int64_t d, hipStream_t s) {
   constexpr int kVec = 16 / sizeof(T);
+  // (a null dbuf goes with a null inv)
   const bool vec = d % kVec == 0 && aligned(dbuf, 16) && aligned(dx, 16) && aligned(wg, 16);
   const GateShare<T> gate{idx, (const typename Elem<T>::acc_t*)dl, (const T*)wg, n_expert};
   FMOE_COMBINE_DISPATCH(reduce_gate_kernel, (const T*)dbuf, inv, gate, (T*)dx, n_tokens, top_k, d);
@@ -681,7 +697,7 @@ extern "C" int fmoe_scatter_reduce_gate(const void* dbuf, const int32_t* inv, co
   if (rc) return rc;
   FMOE_REQUIRE(n_expert >= 1, FMOE_ERR_INVALID, "scatter_reduce_gate: no experts");
   if (n_tokens == 0 || d == 0) return FMOE_OK;
-  FMOE_REQUIRE(inv && idx && dslot && wg && dx, FMOE_ERR_INVALID,
+  FMOE_REQUIRE(idx && dslot && wg && dx && (dbuf || !inv), FMOE_ERR_INVALID,
                "scatter_reduce_gate: null pointer");
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {

@@ -594,6 +594,8 @@ PYBIND11_MODULE(fmoe_cuda, m) {
   m.def("gated_layer", &gated_layer, py::arg("x"), py::arg("gate_weight"), py::arg("gate_bias"),
         py::arg("params"), py::arg("n_expert"), py::arg("has_b1"), py::arg("has_b2"),
         py::arg("act"), py::arg("top_k"), py::arg("tables") = py::none());
+  m.def("plain_gate", &plain_gate, py::arg("x"), py::arg("gate_weight"), py::arg("gate_bias"),
+        py::arg("top_k"));
   m.def("limit_gate", &limit_gate, py::arg("gate"), py::arg("n_expert"), py::arg("capacity"));
   m.def("balance_gate", &balance_gate, py::arg("logits"), py::arg("kind"), py::arg("capacity"));
   m.attr("GATE_GSHARD") = (int)FMOE_GATE_GSHARD;

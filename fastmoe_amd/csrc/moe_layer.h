@@ -151,6 +151,19 @@ struct LayerPass {
   Tensor y, buf, pre, act, out, score, route;
 };
 
+// The routing results of `idx` in one allocation (RouteLayout).
+Tensor route_slots(const LayerSizes& s, const Tensor& idx) {
+  const RouteLayout at_(s.n, s.e);
+  Tensor route = at::empty({at_.bytes}, idx.options().dtype(at::kByte));
+  char* meta = (char*)route.data_ptr();
+  Tensor ws = workspace(s.n, s.e, idx);
+  check(fmoe_route(idx.data_ptr<int64_t>(), s.n, (int32_t)s.e, nullptr, (int32_t*)(meta + at_.seg),
+                   (int64_t*)meta, (int32_t*)(meta + at_.inv), ws.data_ptr(), ws.numel(),
+                   stream_of(idx)),
+        "route");
+  return route;
+}
+
 LayerPass experts_forward(const LayerConfig& c, const LayerSizes& s, const ExpertParams& w,
                           const Tensor& x, const Tensor& idx, const Tensor& score, bool train) {
   const auto opts = x.options();
@@ -158,15 +171,11 @@ LayerPass experts_forward(const LayerConfig& c, const LayerSizes& s, const Exper
   const RouteLayout at_(s.n, s.e);
   LayerPass p;
   p.score = score;
-  p.route = at::empty({at_.bytes}, opts.dtype(at::kByte));
-  char* meta = (char*)p.route.data_ptr();
-  int64_t* pos = (int64_t*)meta;
-  int32_t* inv = (int32_t*)(meta + at_.inv);
-  int32_t* seg = (int32_t*)(meta + at_.seg);
-  Tensor ws = workspace(s.n, s.e, x);
-  check(fmoe_route(idx.data_ptr<int64_t>(), s.n, (int32_t)s.e, nullptr, seg, pos, inv, ws.data_ptr(),
-                   ws.numel(), stream),
-        "route");
+  p.route = route_slots(s, idx);
+  const char* meta = (const char*)p.route.data_ptr();
+  const int64_t* pos = (const int64_t*)meta;
+  const int32_t* inv = (const int32_t*)(meta + at_.inv);
+  const int32_t* seg = (const int32_t*)(meta + at_.seg);
   p.buf = at::empty({s.n, s.d}, opts);
   if (s.k >= 4)   // token order: a row is read once for its k copies
     check(fmoe_scatter_tokens(x.data_ptr(), inv, p.buf.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
@@ -208,6 +217,38 @@ struct LayerNeeds {
 
 void* out_ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
+// dlogits at the top-k slots, in the accumulation type
+Tensor gate_slot_grads(const LayerSizes& s, const Tensor& dscore, const Tensor& score) {
+  Tensor dslot = at::empty({s.t, s.k}, score.options().dtype(
+      score.scalar_type() == at::kDouble ? at::kDouble : at::kFloat));
+  check(fmoe_gate_slot_grad(dscore.data_ptr(), score.data_ptr(), dslot.data_ptr(), s.t, s.k, s.dtype,
+                            stream_of(score)),
+        "gate_slot_grad");
+  return dslot;
+}
+
+// Gradients of the gate's weight and bias from the routing results.
+std::tuple<Tensor, Tensor> gate_linear_grads(const LayerSizes& s, const Tensor& x,
+                                             const Tensor& route, const Tensor& dslot, bool weight,
+                                             bool bias) {
+  Tensor dwg, dbg;
+  if (weight) dwg = at::empty({s.e, s.d}, x.options());
+  if (bias) dbg = at::empty({s.e}, x.options());
+  const RouteLayout at_(s.n, s.e);
+  const char* meta = (const char*)route.data_ptr();
+  const int64_t bytes = fmoe_gate_linear_grad_workspace_bytes(x.data_ptr(), s.t, s.k, s.d,
+                                                              (int32_t)s.e, s.dtype);
+  check(bytes < 0 ? (int)bytes : 0, "gate_linear_grad");
+  // (of this call alone: two launches, between which another thread may use the stream)
+  Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+  check(fmoe_gate_linear_grad(x.data_ptr(), (const int64_t*)meta, (const int32_t*)(meta + at_.seg),
+                              dslot.data_ptr(), weight ? dwg.data_ptr() : nullptr,
+                              bias ? dbg.data_ptr() : nullptr, s.t, s.k, s.d, (int32_t)s.e,
+                              ws.data_ptr(), bytes, s.dtype, stream_of(x)),
+        "gate_linear_grad");
+  return {dwg, dbg};
+}
+
 LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const ExpertParams& w,
                             const LayerPass& p, const Tensor& dy, const LayerNeeds& want,
                             const GateGrad* gate) {
@@ -223,13 +264,7 @@ LayerGrads experts_backward(const LayerConfig& c, const LayerSizes& s, const Exp
   check(fmoe_gather_combine_bwd(dy.data_ptr(), p.out.data_ptr(), inv, p.score.data_ptr(),
                                 d_out.data_ptr(), g.dscore.data_ptr(), s.t, s.k, s.d, s.dtype, stream),
         "gather_combine_bwd");
-  if (gate) {
-    g.dslot = at::empty({s.t, s.k},
-                        opts.dtype(dy.scalar_type() == at::kDouble ? at::kDouble : at::kFloat));
-    check(fmoe_gate_slot_grad(g.dscore.data_ptr(), p.score.data_ptr(), g.dslot.data_ptr(), s.t, s.k,
-                              s.dtype, stream),
-          "gate_slot_grad");
-  }
+  if (gate) g.dslot = gate_slot_grads(s, g.dscore, p.score);
   const bool first = want.dx || want.w1 || want.b1;   // whether the first layer has a backward
   Tensor dpre;
   if (first) dpre = at::empty({s.n, s.h}, opts);
@@ -378,22 +413,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     variable_list out;
     if (c.gated) {
       Tensor dwg, dbg;
-      if (nwg || nbg) {
-        const Tensor& x = gate.x;
-        if (nwg) dwg = at::empty({s.e, s.d}, dy.options());
-        if (nbg) dbg = at::empty({s.e}, dy.options());
-        const RouteLayout at_(s.n, s.e);
-        const char* meta = (const char*)p.route.data_ptr();
-        const int64_t bytes = fmoe_gate_linear_grad_workspace_bytes(x.data_ptr(), s.t, s.k, s.d,
-                                                                    (int32_t)s.e, s.dtype);
-        check(bytes < 0 ? (int)bytes : 0, "gate_linear_grad");
-        Tensor ws = at::empty({bytes}, dy.options().dtype(at::kByte));
-        check(fmoe_gate_linear_grad(x.data_ptr(), (const int64_t*)meta,
-                                    (const int32_t*)(meta + at_.seg), g.dslot.data_ptr(),
-                                    out_ptr(dwg), out_ptr(dbg), s.t, s.k, s.d, (int32_t)s.e,
-                                    ws.data_ptr(), bytes, s.dtype, stream_of(dy)),
-              "gate_linear_grad");
-      }
+      if (nwg || nbg)
+        std::tie(dwg, dbg) = gate_linear_grads(s, gate.x, p.route, g.dslot, nwg, nbg);
       out = {g.dx, dwg};
       if (c.has_bg) out.push_back(dbg);
     } else {
@@ -502,6 +523,65 @@ std::tuple<Tensor, Tensor> limit_gate(const Tensor& gate_in, int64_t n_expert, i
                         stream_of(gate)),
         "limit_gate");
   return {count, out};
+}
+
+// The plain gate as a node of its own (a layer that cannot fold it in: masks, experts of the
+// user's), with the kernels and so the bits of the folded one: (idx, score)
+struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& wg,
+                               const OptTensor& bg, int64_t top_k) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor x = x_in.contiguous();
+    const LayerSizes s{x.size(0), x.size(1), 0, wg.size(0), top_k, x.size(0) * top_k, dt(x, "x")};
+    const bool has_bg = bg.has_value() && bg->defined();
+    const Tensor logits = at::linear(x, wg, has_bg ? bg : OptTensor());
+    Tensor idx = at::empty({s.t, s.k}, logits.options().dtype(at::kLong));
+    Tensor score = at::empty({s.t, s.k}, logits.options());
+    check(fmoe_topk_softmax_fwd(logits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k,
+                                idx.data_ptr<int64_t>(), score.data_ptr(), s.dtype, stream_of(x)),
+          "topk_softmax_fwd");
+    ctx->save_for_backward({x_in, wg, idx, score, has_bg ? *bg : Tensor()});
+    ctx->mark_non_differentiable({idx});
+    ctx->set_materialize_grads(false);
+    return {idx, score};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const Tensor &wg = v[1], &idx = v[2], &score = v[3], &bg = v[4];
+    const bool dx = ctx->needs_input_grad(0), nwg = ctx->needs_input_grad(1),
+               nbg = bg.defined() && ctx->needs_input_grad(2);
+    if (!grads[1].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
+    c10::DeviceGuard guard(wg.device());
+    if (at::GradMode::is_enabled()) {   // gradients that will themselves be differentiated
+      const Tensor chosen = at::linear(v[0], wg, bg.defined() ? OptTensor(bg) : OptTensor()).gather(1, idx);
+      const Tensor p = at::softmax(chosen, -1);
+      const Tensor dchosen = p * (grads[1] - (grads[1] * p).sum(-1, true));
+      const Tensor dlogits = at::zeros({v[0].size(0), wg.size(0)}, wg.options()).scatter_add(1, idx, dchosen);
+      return {dx ? at::mm(dlogits, wg) : Tensor(), nwg ? at::mm(dlogits.t(), v[0]) : Tensor(),
+              nbg ? dlogits.sum(0) : Tensor(), Tensor()};
+    }
+    const Tensor x = v[0].contiguous(), w = wg.contiguous();
+    const LayerSizes s{x.size(0), x.size(1), 0, w.size(0), idx.size(1), idx.numel(), dt(x, "x")};
+    const Tensor dslot = gate_slot_grads(s, grads[1].contiguous(), score);
+    Tensor gx, dwg, dbg;
+    if (dx) {
+      gx = at::empty({s.t, s.d}, x.options());
+      check(fmoe_scatter_reduce_gate(nullptr, nullptr, idx.data_ptr<int64_t>(), dslot.data_ptr(),
+                                     w.data_ptr(), gx.data_ptr(), s.t, s.k, s.d, (int32_t)s.e,
+                                     s.dtype, stream_of(x)),
+            "scatter_reduce_gate");
+    }
+    if (nwg || nbg) std::tie(dwg, dbg) = gate_linear_grads(s, x, route_slots(s, idx), dslot, nwg, nbg);
+    return {gx, dwg, dbg, Tensor()};
+  }
+};
+
+std::tuple<Tensor, Tensor> plain_gate(const Tensor& x, const Tensor& wg, const OptTensor& bg,
+                                      int64_t top_k) {
+  need(x.is_cuda() && x.dim() == 2 && wg.dim() == 2, "x must be a 2-d CUDA tensor");
+  c10::DeviceGuard guard(x.device());
+  variable_list r = PlainGateNode::apply(x, wg, bg, top_k);
+  return {r[0], r[1]};
 }
 
 // A gate with a balance loss behind its linear map: logits -> (idx limited to the capacity,

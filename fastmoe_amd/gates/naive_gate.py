@@ -43,6 +43,11 @@ class NaiveGate(BaseGate):
         return None
 
     def forward(self, inp, return_all_scores=False):
+        native = fmoe_cuda.native() if not return_all_scores else None
+        if native is not None and inp.dim() == 2 and inp.is_cuda and self.is_plain(inp):
+            top_idx, score = native.plain_gate(inp, self.gate.weight, self.gate.bias, self.top_k)
+            self.set_loss(torch.zeros(1, device=inp.device, requires_grad=True))
+            return top_idx, score
         logits = self.gate(inp)
         top_idx, score = topk_softmax(logits, self.top_k)
         # idx keeps the leading dimensions of the input, score is [tokens, k]

@@ -447,7 +447,8 @@ int fmoe_topk_softmax_bwd(const void* dscore, const void* score, const int64_t* 
  *   dslot[t][j] = score_j * (dscore_j - sum_i dscore_i * score_i)
  * in the accumulation type (f32; f64 for doubles) is the gradient of logit idx[t][j], all
  * others are zero;
- *   fmoe_scatter_reduce_gate:  dx[t] = sum_j dbuf[inv[t][j]] + sum_j dslot[t][j] * wg[idx[t][j]]
+ *   fmoe_scatter_reduce_gate:  dx[t] = sum_j dbuf[inv[t][j]] + sum_j dslot[t][j] * wg[idx[t][j]],
+ *     either sum rounded to the storage type before the addition; without inv the second alone
  *   fmoe_gate_linear_grad:     dwg[e] = sum over the rows r of expert e (seg_off, pos of
  *     fmoe_route) of dslot[pos[r]] * x[pos[r] / top_k], dbg[e] = sum of dslot[pos[r]]
  * wg, dwg [n_expert, d], dbg [n_expert]; either of dwg, dbg may be null.  The workspace depends

@@ -196,13 +196,19 @@ def test_gate_gradients_from_slots(dt, t, e, k, d):
     rows = inv.cpu().view(t, k).long()
     live = (idx >= 0)[..., None].double()
     moved = dbuf.double()[rows.clamp(min=0)] * live
+    alone = torch.empty_like(dx)      # the gate's share without rows of the experts
+    assert lib.fmoe_scatter_reduce_gate(None, None, p(c["idx"]), p(dl), p(c["wg"]), p(alone), t, k,
+                                        d, e, code, stream) == 0
     dense = torch.zeros(t, e, dtype=torch.float64).scatter_add_(1, idx.clamp(min=0), want_dl * live[..., 0])
     mags = torch.zeros(t, e, dtype=torch.float64).scatter_add_(1, idx.clamp(min=0), mag_dl * live[..., 0])
     unit, eps = torch.finfo(acc).eps, torch.finfo(dtype).eps
     for got, want, mag, terms in (
             (dx, moved.sum(1) + dense @ wg.double(), moved.abs().sum(1) + mags @ wg.double().abs(), 2 * k),
+            (alone, dense @ wg.double(), mags @ wg.double().abs(), k),
             (dwg, dense.t() @ x.double(), mags.t() @ x.double().abs(), t),
             (dbg, dense.sum(0), mags.sum(0), t)):
         err = (got.double().cpu() - want).abs()
         # (f16 below its smallest normal number: half a step of 2^-24)
+        if got is dx:   # either share is rounded before the addition
+            err = err - eps * (moved.sum(1).abs() + (dense @ wg.double()).abs())
         assert (err <= eps * want.abs() + unit * (terms + 8 + k) * mag + (2 ** -25 if dt == "f16" else 0)).all()
