@@ -166,10 +166,11 @@ static int run_bwd(Family family, const GemmArgs& gd, const GemmArgs& gw, int dt
 
 // Up to this many values the small 16-bit tiles look the activation up in its table in
 // memory while they store; a bigger product leaves it to the activation kernel, which
-// keeps the table in LDS.
+// keeps the table in LDS.  ReLU needs no table and always runs in the tiles (4096 tokens,
+// 768 -> 3072: a kernel of 10 us less; 6002 rows f16: 13 us forward, 18 backward).
 constexpr int64_t kTableInMemoryMax = 4 << 20;
 
-// The tables of a 16-bit activation.
+// The tables of a 16-bit activation (the 256-row kernels look ReLU up as well).
 static int act_tables(int act, int dtype, hipStream_t s, GemmArgs* g, bool fwd) {
   if (dtype != FMOE_BF16 && dtype != FMOE_F16) return FMOE_OK;
   if (act == FMOE_ACT_RELU)
@@ -277,7 +278,8 @@ static int linear_fwd(const char* who, const void* x, const void* w, const void*
   if (family == kBig)
     fused = fused && dtype == FMOE_BF16 && (g_tile != 0 || n_rows >= 768 * n_expert);
   else if (family == kPlain)
-    fused = fused && (dtype == FMOE_F32 || g_tile != 0 || n_rows * out_feat <= kTableInMemoryMax);
+    fused = fused && (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
+                      n_rows * out_feat <= kTableInMemoryMax);
   else
     fused = false;
   // A pre-activation whose sign is decided in its last bit switches a whole gradient on or
@@ -397,7 +399,8 @@ static int linear_bwd(const void* dy, const void* x, const void* w, const void* 
   else if (family == kPlain)
     // (f16 GELU: the activation kernel rounds its product once, not through f32 first)
     act_fused = act_fused && (dtype != FMOE_F16 || act == FMOE_ACT_RELU) &&
-                (dtype == FMOE_F32 || g_tile != 0 || n_rows * in_feat <= kTableInMemoryMax);
+                (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
+                 n_rows * in_feat <= kTableInMemoryMax);
   else
     act_fused = false;
   if (act_fused) {

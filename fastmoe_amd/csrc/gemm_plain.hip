@@ -250,11 +250,18 @@ __device__ __forceinline__ float act_fwd(const GemmArgs& g, float v) {
 __device__ __forceinline__ float act_bwd(const GemmArgs& g, float d, float pre) {
   return g.act == FMOE_ACT_RELU ? (pre <= 0.f ? 0.f : d) : d * gelu_grad_direct(pre);
 }
+// (16-bit ReLU: whether a negative value is a NaN only its bits above infinity's tell)
+template <typename T> constexpr uint16_t kInf16 = std::is_same<T, __half>::value ? 0x7c00 : 0x7f80;
+template <typename T>
 __device__ __forceinline__ uint16_t act_fwd16(const GemmArgs& g, uint16_t v) {
+  if (g.act == FMOE_ACT_RELU) return (v & 0x8000u) && (v & 0x7fffu) <= kInf16<T> ? 0 : v;
   return load_global<uint16_t>(g.act_fwd_table + v);
 }
 template <typename T>
 __device__ __forceinline__ uint16_t act_bwd16(const GemmArgs& g, uint16_t d, uint16_t pre) {
+  // (zero or negative, and no NaN)
+  if (g.act == FMOE_ACT_RELU)
+    return pre == 0 || ((pre & 0x8000u) && (pre & 0x7fffu) <= kInf16<T>) ? 0 : d;
   const float n = load_global<float>(g.act_table + (pre & 0x7fffu));
   return __builtin_bit_cast(uint16_t, Elem<T>::from_acc(
       Elem<T>::to_acc(__builtin_bit_cast(T, d)) * ((pre & 0x8000u) ? n : 1.f - n)));
@@ -520,7 +527,7 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
       if (!kFwd || g.c) *reinterpret_cast<Unit*>(C + at) = v.u;
       if (kFwd && g.act_out) {
 #pragma unroll
-        for (int q = 0; q < kUnit; ++q) v.h[q] = act_fwd16(g, v.h[q]);
+        for (int q = 0; q < kUnit; ++q) v.h[q] = act_fwd16<T>(g, v.h[q]);
         *reinterpret_cast<Unit*>((uint16_t*)g.act_out + (int64_t)row0 * ldc + at) = v.u;
       }
     }

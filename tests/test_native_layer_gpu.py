@@ -277,3 +277,31 @@ def test_balance_loss_differentiates_twice_and_forwards(gate, top_k):
         with forward_ad.dual_level():
             layer(forward_ad.make_dual(x, torch.ones_like(x)))
             assert forward_ad.unpack_dual(layer.get_loss()).tangent is not None
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_relu_in_the_tiles_of_a_large_product(dt):
+    """More than 4 Mi values behind the first layer: ReLU forward and backward inside the
+    products' tiles against torch's.  The same sums, a ReLU is exact: the same bits forward; the
+    chain's gradients pass through the same roundings (bounds as above)."""
+    from fastmoe_amd import fmoe_cuda
+
+    dtype = DTYPES[dt]
+    moe = _layer(dtype, 2, d=64, h=1032, activation=torch.nn.ReLU())
+    x = torch.randn(2100, 64, device="cuda").to(dtype)
+    dy = torch.randn(2100, 64, device="cuda").to(dtype)
+    got = []
+    for watched in (False, True):
+        fmoe_cuda.profile_hook = (lambda *a: None) if watched else None
+        try:
+            for p in moe.parameters():
+                p.grad = None
+            a = x.clone().requires_grad_(True)
+            out = moe(a)
+            out.backward(dy)
+        finally:
+            fmoe_cuda.profile_hook = None
+        got.append([out, a.grad] + [p.grad for p in moe.parameters()])
+    assert torch.equal(got[0][0], got[1][0])
+    for g, w in zip(got[0][1:], got[1][1:]):
+        assert (g - w).double().norm() <= 4 * torch.finfo(dtype).eps * w.double().norm()
