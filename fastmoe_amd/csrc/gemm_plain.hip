@@ -696,7 +696,14 @@ int bwd_shape(const GemmArgs& gd, const GemmArgs& gw, const Shape (&shapes)[2], 
 //             4, 1000, 256 -> 512                    16  9.6  7.1  (8.2)
 //             8, 8000, 512 -> 2048                   56   49   69  (71)
 //            32, 16000, 1024 -> 2048                167  196  275
-enum Kind { k256, k128, k64, kMixed };
+//          (128 x 256 tiles, dX + dW, against the best of the others)
+//            64, 18790, 1152 -> 4032           627  581  648   543
+//            32, 8307, 2304 -> 1536            221  210  237   186
+//           128, 16376, 2048 -> 1408           469  513  511   446
+//             8, 16620, 1664 -> 3328           355  377  474   370
+//             4, 24620, 1600 -> 6400           960 1030 1404  1050
+// Over 38 such launches the choice takes 1.3 % longer than the best of the four.
+enum Kind { k256, k128, k64, kMixed, kTall };
 
 struct Spread {   // rows of an expert: three equally spaced points and their weights
   double rows[3];
@@ -736,6 +743,10 @@ Work row_product(Kind kind, const GemmArgs& g, double N, double K, bool narrow_q
     }
     return w;
   }
+  if (kind == kTall) {
+    const double tiles = g.n_expert * sp.mean([&](double r) { return ceil(r / 128); }) * ceil(N / 256);
+    return Work{tiles * (slices * 1.1 + 2.0), slices * 1.4, tiles};
+  }
   const double side = kind == k128 ? 128 : 64;
   const double tiles = g.n_expert * sp.mean([&](double r) { return ceil(r / side); }) * ceil(N / side);
   return kind == k128 ? Work{tiles * (slices * 0.65 + 0.8), slices * 0.8, tiles}
@@ -768,22 +779,25 @@ double bwd_us(Kind kind, const GemmArgs& gd, const GemmArgs& gw) {
   if (gd.c) w = row_product(kind == kMixed ? k64 : kind, gd, gd.in_feat, gd.out_feat, false);
   if (gw.c) {
     const double side = kind == k256 ? 256 : kind == k64 ? 64 : 128;
-    const double n = E * ceil(gw.out_feat / side) * ceil(gw.in_feat / side);
+    const double n = E * ceil(gw.out_feat / side) * ceil(gw.in_feat / (kind == kTall ? 256 : side));
     const double tile = kind == k256 ? 8.7 + ceil(r / 32) * 0.7
                         : kind == k128 ? 2.2 + ceil(r / 64) * 0.42
+                        : kind == kTall ? 2.0 + ceil(r / 64) * 0.75
                         : kind == kMixed ? 1.45 + ceil(r / 32) * 0.23 : 0.9 + ceil(r / 64) * 0.15;
     w.total += n * tile;
     w.longest = std::max(w.longest, tile * (kind == k256 ? 1 : 2));
     w.tiles += n;
   }
-  const double side = kind == k256 ? 256 : kind == k128 ? 128 : 64;
+  const double side = kind == k256 ? 256 : kind == k128 || kind == kTall ? 128 : 64;
   const double tiles = kind == k256 ? launch_us(w, 0.5) : 4 + launch_us(w, 0.3);
   return std::max(tiles, memory_us(gw, (gd.c ? 1 : 0) + (gw.c ? 1 : 0), 1.5, side));
 }
 
-int bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
-  const double a = bwd_us(k128, gd, gw), b = bwd_us(kMixed, gd, gw), c = bwd_us(k64, gd, gw);
-  return a <= b && a <= c ? k128 : b <= c ? kMixed : k64;
+Kind bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
+  Kind best = k128;
+  for (Kind kind : {kMixed, k64, kTall})
+    if (bwd_us(kind, gd, gw) < bwd_us(best, gd, gw)) best = kind;
+  return best;
 }
 
 template <typename T, int DMA>
@@ -810,11 +824,19 @@ int bwd_typed(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
                                                  : launch_bwd<T, Small, Small, DMA>(gd, gw, s);
   } else if constexpr (DMA == 16) {
     const int forced = gd.tile ? gd.tile : gw.tile;
-    const int kind = forced ? (forced == 3 ? kMixed : k128) : bwd_choice(gd, gw);
+    // (forced, by tests: the shapes for 128 rows are told apart by the parity of the experts)
+    const Kind kind = !forced ? bwd_choice(gd, gw)
+                      : forced == 3 ? kMixed : gw.n_expert % 2 ? kTall : k128;
     using Big = Tile<128, 128, 2, 128>;
     if (kind == k128) return launch_bwd<T, Big, Big, DMA>(gd, gw, s);
     // short dW sums: half as deep slices, so that four workgroups fit a CU and their output
     // stores (which bound such products) overlap
+    // Experts of some hundred rows: dW tiles that are half output.  Twice the columns of the
+    // 128 x 128 tile in three stages of half slices load a quarter less per product, and the
+    // two workgroups of a CU store and multiply at the same time, which the one of the
+    // 256-row kernels cannot.
+    using Tall = Tile<128, 256, 3, 64>;
+    if (kind == kTall) return launch_bwd<T, Tall, Tall, DMA>(gd, gw, s);
     if (kind == kMixed)
       return launch_bwd<T, Tile<64, 64, 2, 128>, Tile<128, 128, 2, 64>, DMA>(gd, gw, s);
     return launch_bwd<T, Tile<64, 64, 3, 128>, Tile<64, 64, 3, 128>, DMA>(gd, gw, s);
@@ -856,7 +878,7 @@ bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype)
   if (dtype == FMOE_F32 || !gemm_plain_supported(gd, dtype) || !gemm_plain_supported(gw, dtype))
     return dtype == FMOE_F32;
   if (gd.tile) return gd.tile == 2 || gd.tile == 3;
-  return bwd_us((Kind)bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw);
+  return bwd_us(bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw);
 }
 
 int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s) {

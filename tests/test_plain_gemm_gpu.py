@@ -58,3 +58,12 @@ def test_f32_activation_inside_the_tiles(in_f, out_f):
         for got, ref in zip(fmoe_cuda.grouped_linear_bwd(dy, x, seg, w, **kw), want):
             assert (got is None) == (ref is None)
             assert got is None or max_rel_err(got, ref) <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("counts,in_f,out_f", [([1], 8, 8), ([128, 129, 0, 31, 32], 256, 128),
+                                               ([127, 0, 300], 264, 136), ([33, 5, 97], 520, 248)])
+def test_wide_column_tiles(dt, counts, in_f, out_f):
+    """The backward's 128 x 256 tiles (forced for 128-row tiles and an odd number of experts):
+    edges of tiles, of K slices of 32 and of the three stages."""
+    _run(counts, in_f, out_f, DTYPES[dt], True, 3, extra_rows=3)
