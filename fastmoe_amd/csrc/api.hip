@@ -119,22 +119,23 @@ static int check_linear(const char* who, int64_t n_rows, int64_t in_feat,
 // Which family of kernels runs a product (fmoe_set_gemm_path may force one).
 enum Family { kScalar, kWide, kPlain, kBig };
 
-static Family fwd_family(const GemmArgs& g, int dtype) {
+// `lead`: microseconds by which the 256-row kernels are behind to begin with.
+static Family fwd_family(const GemmArgs& g, int dtype, double lead) {
   if (g_gemm_path != 0) return kScalar;
   const bool plain = gemm_plain_supported(g, dtype);
   if (gemm_mfma_supported(GEMM_FWD, g, dtype))
-    return plain && gemm_plain_fwd_preferred(g, dtype) ? kPlain : kBig;
+    return plain && gemm_plain_fwd_preferred(g, dtype, lead) ? kPlain : kBig;
   if (plain) return kPlain;
   return gemm_mfma_wide_supported(GEMM_FWD, g, dtype) ? kWide : kScalar;
 }
 
 // dX (gd) and dW (gw), either of which may be absent (c null).
-static Family bwd_family(const GemmArgs& gd, const GemmArgs& gw, int dtype) {
+static Family bwd_family(const GemmArgs& gd, const GemmArgs& gw, int dtype, double lead) {
   if (g_gemm_path != 0) return kScalar;
   const bool plain = gemm_plain_supported(gd, dtype) && gemm_plain_supported(gw, dtype);
   if ((!gd.c || gemm_mfma_supported(GEMM_DGRAD, gd, dtype)) &&
       (!gw.c || gemm_mfma_supported(GEMM_WGRAD, gw, dtype)))
-    return plain && gemm_plain_bwd_preferred(gd, gw, dtype) ? kPlain : kBig;
+    return plain && gemm_plain_bwd_preferred(gd, gw, dtype, lead) ? kPlain : kBig;
   if (plain) return kPlain;
   return gemm_mfma_wide_supported(GEMM_DGRAD, gd, dtype) &&
                  gemm_mfma_wide_supported(GEMM_WGRAD, gw, dtype) ? kWide : kScalar;
@@ -169,6 +170,33 @@ static int run_bwd(Family family, const GemmArgs& gd, const GemmArgs& gw, int dt
 // keeps the table in LDS.  ReLU needs no table and always runs in the tiles (4096 tokens,
 // 768 -> 3072: a kernel of 10 us less; 6002 rows f16: 13 us forward, 18 backward).
 constexpr int64_t kTableInMemoryMax = 4 << 20;
+
+// Which kernels take an activation into their tiles.
+// 256-row tiles forward: worth it from about 768 rows per expert on (measured: 12 % of GEMM +
+// activation kernel at 1024 rows per expert, 5 % at 4096, level at 512, where half of the
+// tiles are remainder tiles that pay the table and the second store for few rows).  Small
+// tiles: f32 always (the activation costs what evaluating it costs either way, and the
+// pass over memory is saved).  A forced tile shape (tests, tuning) fuses at any size.
+static bool fwd_act_fused(Family family, int act, int dtype, int64_t n_rows, int64_t out_feat,
+                          int64_t n_expert) {
+  if (!g_fuse_fwd_act) return false;
+  if (family == kBig) return dtype == FMOE_BF16 && (g_tile != 0 || n_rows >= 768 * n_expert);
+  return family == kPlain && (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
+                              n_rows * out_feat <= kTableInMemoryMax);
+}
+static bool bwd_act_fused(Family family, int act, int dtype, int64_t n_rows, int64_t in_feat) {
+  if (family == kBig) return dtype == FMOE_BF16;
+  // (f16 GELU: the activation kernel rounds its product once, not through f32 first)
+  return family == kPlain && (dtype != FMOE_F16 || act == FMOE_ACT_RELU) &&
+         (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
+          n_rows * in_feat <= kTableInMemoryMax);
+}
+// A 16-bit activation as a kernel of its own: a launch and its passes over memory (measured
+// 5.6 us for 64 x 4096 values, 87 for 134 million of which half are live, 60 for 92 million
+// with the live rows in the last-level cache).
+static double act_kernel_us(int64_t values, int passes) {
+  return 5 + 2.0 * passes * (double)values / 5e6;
+}
 
 // The tables of a 16-bit activation (the 256-row kernels look ReLU up as well).
 static int act_tables(int act, int dtype, hipStream_t s, GemmArgs* g, bool fwd) {
@@ -267,21 +295,18 @@ static int linear_fwd(const char* who, const void* x, const void* w, const void*
   GemmArgs g{x, w, y ? y : y_act, bias, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   g.w_table = w_table;
   g.bias_table = bias_table;
-  Family family = fwd_family(g, dtype);
+  // the tiles that leave the activation to its kernel pay for that in the choice: 32 tokens
+  // through 16 experts, 1024 -> 4096, are level without it (25 us) and 31 to 25 us with it
+  double lead = 0;
+  if (act) {
+    const double us = act_kernel_us(n_rows * out_feat, 2);
+    lead = (fwd_act_fused(kBig, act, dtype, n_rows, out_feat, n_expert) ? 0 : us) -
+           (fwd_act_fused(kPlain, act, dtype, n_rows, out_feat, n_expert) ? 0 : us);
+  }
+  Family family = fwd_family(g, dtype, lead);
   if (!act) return run_fwd(family, g, dtype, s);
-  // 256-row tiles: worth it from about 768 rows per expert on (measured: 12 % of GEMM +
-  // activation kernel at 1024 rows per expert, 5 % at 4096, level at 512, where half of the
-  // tiles are remainder tiles that pay the table and the second store for few rows).  Small
-  // tiles: f32 always (the activation costs what evaluating it costs either way, and the
-  // pass over memory is saved).  A forced tile shape (tests, tuning) fuses at any size.
-  bool fused = g_fuse_fwd_act && (uintptr_t)y_act % 16 == 0;
-  if (family == kBig)
-    fused = fused && dtype == FMOE_BF16 && (g_tile != 0 || n_rows >= 768 * n_expert);
-  else if (family == kPlain)
-    fused = fused && (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
-                      n_rows * out_feat <= kTableInMemoryMax);
-  else
-    fused = false;
+  bool fused = (uintptr_t)y_act % 16 == 0 &&
+               fwd_act_fused(family, act, dtype, n_rows, out_feat, n_expert);
   // A pre-activation whose sign is decided in its last bit switches a whole gradient on or
   // off behind a ReLU: feature sizes off the 8-element grid keep the sums in ascending order.
   if (act == FMOE_ACT_RELU && dtype != FMOE_F32 && family == kPlain &&
@@ -386,23 +411,21 @@ static int linear_bwd(const void* dy, const void* x, const void* w, const void* 
   GemmArgs gw{dy, x, dw, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   GemmArgs gd{dy, w, dx, nullptr, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   gd.w_table = w_table;
-  const Family family = bwd_family(gd, gw, dtype);
+  double lead = 0;
+  if (act_pre && dx) {
+    const double us = act_kernel_us(n_rows * in_feat, 3);
+    lead = (bwd_act_fused(kBig, act, dtype, n_rows, in_feat) ? 0 : us) -
+           (bwd_act_fused(kPlain, act, dtype, n_rows, in_feat) ? 0 : us);
+  }
+  const Family family = bwd_family(gd, gw, dtype, lead);
   // The matrix-core kernels for 16-bit types and f32 sum the columns of dY inside their dW
   // tiles; f64 and the scalar kernel leave the bias gradient to the reduction kernel below.
   if (dw && dbias && (family == kBig || family == kPlain)) {
     gw.bias = dbias;
     dbias = nullptr;
   }
-  bool act_fused = act_pre && dx && (uintptr_t)act_pre % 16 == 0;
-  if (family == kBig)
-    act_fused = act_fused && dtype == FMOE_BF16;
-  else if (family == kPlain)
-    // (f16 GELU: the activation kernel rounds its product once, not through f32 first)
-    act_fused = act_fused && (dtype != FMOE_F16 || act == FMOE_ACT_RELU) &&
-                (dtype == FMOE_F32 || act == FMOE_ACT_RELU || g_tile != 0 ||
-                 n_rows * in_feat <= kTableInMemoryMax);
-  else
-    act_fused = false;
+  const bool act_fused = act_pre && dx && (uintptr_t)act_pre % 16 == 0 &&
+                         bwd_act_fused(family, act, dtype, n_rows, in_feat);
   if (act_fused) {
     gd.act = act;
     gd.act_pre = act_pre;

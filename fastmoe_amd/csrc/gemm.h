@@ -125,9 +125,9 @@ int launch_gemm_mfma_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipS
 // through act_fwd_table / act_table.
 bool gemm_plain_supported(const GemmArgs& g, int dtype);
 // Whether these kernels are expected to beat the 256-row ones (16-bit types that both take;
-// always for f32, which only these take).
-bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype);
-bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype);
+// always for f32, which only these take); `lead`: microseconds the 256-row ones are behind.
+bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype, double lead);
+bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype, double lead);
 int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s);
 // dX (gd) and dW (gw) in one launch; a null gd.c or gw.c leaves that product out.
 int launch_gemm_plain_bwd(const GemmArgs& gd, const GemmArgs& gw, int dtype, hipStream_t s);

@@ -868,17 +868,17 @@ bool gemm_plain_supported(const GemmArgs& g, int dtype) {
   return copy_width(g, dtype) != 0;
 }
 
-bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype) {
+bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype, double lead) {
   if (dtype == FMOE_F32 || !gemm_plain_supported(g, dtype)) return dtype == FMOE_F32;
   if (g.tile) return g.tile == 2 || g.tile == 3;   // forced (tests)
-  return std::min(fwd_us(k128, g), fwd_us(k64, g)) < fwd_us(k256, g);
+  return std::min(fwd_us(k128, g), fwd_us(k64, g)) < fwd_us(k256, g) + lead;
 }
 
-bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype) {
+bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype, double lead) {
   if (dtype == FMOE_F32 || !gemm_plain_supported(gd, dtype) || !gemm_plain_supported(gw, dtype))
     return dtype == FMOE_F32;
   if (gd.tile) return gd.tile == 2 || gd.tile == 3;
-  return bwd_us(bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw);
+  return bwd_us(bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw) + lead;
 }
 
 int launch_gemm_plain_fwd(const GemmArgs& g, int dtype, hipStream_t s) {
