@@ -72,7 +72,9 @@ bool is_capturing(void* stream) {
 
 // Scratch memory for a call on torch's current stream of `like`'s device.  One buffer per
 // (device, stream) is kept and reused: launches on one stream run in order, and nothing in
-// it outlives a call.  A stream under graph capture gets a fresh tensor instead, which then
+// it outlives a call.  Only for callers that hold the interpreter lock from here to their last
+// launch that uses the buffer: the stream's order alone does not keep another thread's launches
+// out from between them.  A stream under graph capture gets a fresh tensor instead, which then
 // belongs to the graph's own memory pool.
 Tensor workspace_of(int64_t bytes, const Tensor& like) {
   need(bytes >= 0, "workspace: bad sizes");

@@ -151,12 +151,12 @@ struct LayerPass {
   Tensor y, buf, pre, act, out, score, route;
 };
 
-// The routing results of `idx` in one allocation (RouteLayout).
-Tensor route_slots(const LayerSizes& s, const Tensor& idx) {
+// The routing results of `idx` in one allocation (RouteLayout).  `ws`: scratch of
+// fmoe_route_workspace_bytes(), written by one launch and read by the next two.
+Tensor route_slots(const LayerSizes& s, const Tensor& idx, const Tensor& ws) {
   const RouteLayout at_(s.n, s.e);
   Tensor route = at::empty({at_.bytes}, idx.options().dtype(at::kByte));
   char* meta = (char*)route.data_ptr();
-  Tensor ws = workspace(s.n, s.e, idx);
   check(fmoe_route(idx.data_ptr<int64_t>(), s.n, (int32_t)s.e, nullptr, (int32_t*)(meta + at_.seg),
                    (int64_t*)meta, (int32_t*)(meta + at_.inv), ws.data_ptr(), ws.numel(),
                    stream_of(idx)),
@@ -171,7 +171,7 @@ LayerPass experts_forward(const LayerConfig& c, const LayerSizes& s, const Exper
   const RouteLayout at_(s.n, s.e);
   LayerPass p;
   p.score = score;
-  p.route = route_slots(s, idx);
+  p.route = route_slots(s, idx, workspace(s.n, s.e, idx));
   const char* meta = (const char*)p.route.data_ptr();
   const int64_t* pos = (const int64_t*)meta;
   const int32_t* inv = (const int32_t*)(meta + at_.inv);
@@ -571,7 +571,14 @@ struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
                                      s.dtype, stream_of(x)),
             "scatter_reduce_gate");
     }
-    if (nwg || nbg) std::tie(dwg, dbg) = gate_linear_grads(s, x, route_slots(s, idx), dslot, nwg, nbg);
+    if (nwg || nbg) {
+      // (scratch of this call alone: a backward runs without the interpreter lock, so another
+      // thread may use the stream's shared buffer between the launches)
+      const int64_t bytes = fmoe_route_workspace_bytes(s.n, (int32_t)s.e);
+      need(bytes >= 0, "workspace: bad sizes");
+      const Tensor ws = at::empty({std::max<int64_t>(bytes, 1)}, idx.options().dtype(at::kByte));
+      std::tie(dwg, dbg) = gate_linear_grads(s, x, route_slots(s, idx, ws), dslot, nwg, nbg);
+    }
     return {gx, dwg, dbg, Tensor()};
   }
 };

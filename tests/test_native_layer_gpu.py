@@ -4,6 +4,7 @@ so the same bits, with and without gradients, for every subset of gradients aske
 the gate's own gradients are summed by kernels of their own."""
 import copy
 import io
+import threading
 
 import pytest
 import torch
@@ -191,6 +192,63 @@ def test_balance_gate_against_float64(dt, kind, k, t, e):
     assert (score.double() - want).abs().max() <= eps
     assert abs(loss.item() - want_loss.item()) <= 1e-5 * abs(want_loss.item())
     assert (a.grad.double() - ref.grad).abs().max() <= 4 * eps * ref.grad.abs().max()
+
+
+def _gate(d, e, k, dtype=torch.float32):
+    from fastmoe_amd import NaiveGate
+
+    torch.manual_seed(2)
+    return NaiveGate(d, e, 1, k).to(dtype).cuda()
+
+
+def test_gate_backward_leaves_the_shared_routing_scratch_alone():
+    """The backward of the gate module runs without the interpreter lock, so what it routes
+    with has to be its own: no scratch of its size stays behind for the stream (512 experts and
+    a million slots: a megabyte; the first, small call sets up the stream's other buffers)."""
+    gate, stream = _gate(8, 512, 8), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for tokens in (64, 1 << 17):
+            torch.cuda.synchronize()
+            before = torch.cuda.memory_allocated()
+            x = torch.randn(tokens, 8, device="cuda", requires_grad=True)
+            score = gate(x)[1]
+            grads = torch.autograd.grad(score, [gate.gate.weight, gate.gate.bias],
+                                        torch.ones_like(score))
+            torch.cuda.synchronize()
+            assert all(g.shape[0] == 512 for g in grads)
+            del x, score, grads
+    assert torch.cuda.memory_allocated() - before < 1 << 16
+
+
+def test_two_threads_on_one_stream():
+    """One thread differentiates a gate while another routes on the same stream, both with
+    slots enough for three launches each: everybody gets what they get alone, bit for bit."""
+    gate, moe = _gate(64, 16, 2), _layer(torch.float32, 2)
+    x, y = torch.randn(6000, 64, device="cuda"), torch.randn(9000, 64, device="cuda")
+
+    def differentiate():
+        a = x.clone().requires_grad_(True)
+        score = gate(a)[1]
+        return torch.autograd.grad((score * score).sum(), [a, gate.gate.weight, gate.gate.bias])
+
+    def forward():
+        with torch.no_grad():
+            return (moe(y),)
+
+    want, failed = {f: f() for f in (differentiate, forward)}, []
+
+    def loop(f):
+        for _ in range(40):
+            if not all(torch.equal(g, w) for g, w in zip(f(), want[f])):
+                failed.append(f.__name__)
+
+    threads = [threading.Thread(target=loop, args=(f,)) for f in want]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
 
 
 def _list_layer():
