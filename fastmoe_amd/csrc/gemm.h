@@ -14,9 +14,14 @@ enum GemmMode { GEMM_FWD = 0, GEMM_DGRAD = 1, GEMM_WGRAD = 2,
                 // matrix-core family (callers pass GEMM_FWD and set act_out)
                 GEMM_FWD_ACT = 3,
                 // DGRAD with GemmArgs::act_pre, likewise (callers pass GEMM_DGRAD)
-                GEMM_DGRAD_ACT = 4 };
-constexpr bool is_fwd(int mode) { return mode == GEMM_FWD || mode == GEMM_FWD_ACT; }
-constexpr bool is_dgrad(int mode) { return mode == GEMM_DGRAD || mode == GEMM_DGRAD_ACT; }
+                GEMM_DGRAD_ACT = 4,
+                // the two with a ReLU (GemmArgs::act), which needs no table
+                GEMM_FWD_RELU = 5,
+                GEMM_DGRAD_RELU = 6 };
+constexpr bool fuses_fwd(int mode) { return mode == GEMM_FWD_ACT || mode == GEMM_FWD_RELU; }
+constexpr bool fuses_dgrad(int mode) { return mode == GEMM_DGRAD_ACT || mode == GEMM_DGRAD_RELU; }
+constexpr bool is_fwd(int mode) { return mode == GEMM_FWD || fuses_fwd(mode); }
+constexpr bool is_dgrad(int mode) { return mode == GEMM_DGRAD || fuses_dgrad(mode); }
 
 struct GemmArgs {
   const void* a;        // FWD: x      DGRAD: dy     WGRAD: dy
@@ -31,14 +36,14 @@ struct GemmArgs {
   int out_feat;
   int n_expert;
   int tile;             // 0 = choose the tile shape automatically, 1..4 = force one
-  // DGRAD on the bf16 matrix-core and f32 kernels only: if not null, dx = (dy W) * gelu'(act_pre)
-  // with act_pre [n_rows, in_feat] the pre-activations behind the layer's input,
-  // and act_table (bf16) the device table of gelu'(-|x|) (gelu_bwd_table()).
+  // DGRAD, where the kernel takes it: if not null, dx = (dy W) * act'(act_pre) with act_pre
+  // [n_rows, in_feat] the pre-activations behind the layer's input (ReLU: or the activations),
+  // and act_table (16-bit GELU) the device table of gelu'(-|x|) (gelu_bwd_table()).
   const void* act_pre = nullptr;
   const float* act_table = nullptr;
-  // FWD on the bf16 matrix-core and f32 kernels only: if not null, act_out
-  // [n_rows, out_feat] receives gelu(y) next to y; bf16 through act_fwd_table, the device
-  // table of gelu(x) by 16-bit pattern of x (gelu_fwd_table()).
+  // FWD, where the kernel takes it: if not null, act_out [n_rows, out_feat] receives act(y)
+  // next to y; 16-bit GELU through act_fwd_table, the device table of gelu(x) by 16-bit
+  // pattern of x (gelu_fwd_table()).
   // With act_out the forward product's c may be null: only the activation is wanted.
   int act = FMOE_ACT_GELU;      // fmoe_activation behind act_pre / act_out
   void* act_out = nullptr;

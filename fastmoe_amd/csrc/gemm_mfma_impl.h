@@ -44,6 +44,7 @@
 #include <utility>
 
 #include "dma_desc.h"
+#include "act_math.h"
 #include "gemm_tiles.h"
 
 namespace fmoe {
@@ -707,8 +708,8 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
   // is all in or all out) gets an offset no descriptor reaches.
   const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(C + (int64_t)m0 * ldc + n0), (short)0,
-      // (FWD_ACT without a place for the pre-activations: an empty descriptor drops the stores)
-      MODE == GEMM_FWD_ACT && g.c == nullptr ? 0 : ((m_valid - 1) * ldc + n_valid) * 2,
+      // (without a place for the pre-activations: an empty descriptor drops the stores)
+      fuses_fwd(MODE) && g.c == nullptr ? 0 : ((m_valid - 1) * ldc + n_valid) * 2,
       kRsrcFlags);
   const int c_off = n0 + pk * 8 < N ? (r0 * ldc + pk * 8) * 2 : (int)kOutOfRange;
   // FWD with the activation fused in (g.act_out): the tile is written twice, as it
@@ -716,8 +717,8 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
   // gelu(x) for 16-bit x, whose slice for 2^-28 <= |x| < 16 (both signs, 8192
   // results) sits in LDS behind the staged tile; a pack with an argument outside
   // that range (zeros, denormals, |x| >= 16, infinities, NaNs) is looked up in the
-  // full table in memory.
-  constexpr bool fuse_fwd = MODE == GEMM_FWD_ACT;
+  // full table in memory.  A ReLU is two compares per value and needs no table.
+  constexpr bool fuse_fwd = fuses_fwd(MODE), kTable = MODE == GEMM_FWD_ACT;
   // (behind this instantiation's own staged tile: a small tile shape then needs little
   // LDS and two of its workgroups fit a CU)
   constexpr int kTabOffset = BM * kLdc * 2;
@@ -730,7 +731,7 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
 #pragma unroll
   for (int i = 0; i < kTabPerThread; ++i) tab_regs[i] = i32x4_t{0, 0, 0, 0};
   __amdgpu_buffer_rsrc_t a_rsrc = c_rsrc;
-  if constexpr (fuse_fwd) {
+  if constexpr (kTable) {
     // 16-byte piece L of the slice: 8 results from pattern 0x3180 + 8 L on, the
     // second half of the pieces from 0xB180 on (the negative arguments)
     constexpr int kHalfPieces = kActTabBytes / 16 / 2;
@@ -741,13 +742,20 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
                                             : 0x8000 + kActTabFirst + 8 * (piece - kHalfPieces);
       tab_regs[i] = *reinterpret_cast<const i32x4_t*>(g.act_fwd_table + first);
     }
+  }
+  if constexpr (fuse_fwd) {
     a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)((T*)g.act_out + (int64_t)row0 * ldc + (int64_t)m0 * ldc + n0), (short)0,
         ((m_valid - 1) * ldc + n_valid) * 2, kRsrcFlags);
   }
-  // gelu of the 8 values of a pack
+  // the activation of the 8 values of a pack
   auto act_of = [&](i32x4_t pre) -> i32x4_t {
     i32x4_t out;
+    if constexpr (MODE == GEMM_FWD_RELU) {
+#pragma unroll
+      for (int wd = 0; wd < 4; ++wd) out[wd] = (int)relu_fwd_pair<T>((uint32_t)pre[wd]);
+      return out;
+    }
     uint32_t seen = 0;
 #pragma unroll
     for (int wd = 0; wd < 4; ++wd) {
@@ -784,7 +792,7 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
       constexpr int b = decltype(b_tag)::value;
       stage_block(std::integral_constant<int, b % (TM / 2)>{}, std::integral_constant<int, b / (TM / 2)>{});
     });
-    if constexpr (fuse_fwd) {
+    if constexpr (kTable) {
 #pragma unroll
       for (int i = 0; i < kTabPerThread; ++i)
         reinterpret_cast<i32x4_t*>(fwd_tab_w)[tid + i * NT] = tab_regs[i];
@@ -833,7 +841,7 @@ __device__ __forceinline__ void gemm_tile16(const GemmArgs& g, uint16_t* smem, T
       constexpr int b = decltype(b_tag)::value;
       stage_block(std::integral_constant<int, b % TM>{}, std::integral_constant<int, b / TM>{});
     });
-    if constexpr (fuse_fwd) {
+    if constexpr (kTable) {
 #pragma unroll
       for (int i = 0; i < kTabPerThread; ++i)
         reinterpret_cast<i32x4_t*>(fwd_tab_w)[tid + i * NT] = tab_regs[i];
@@ -1174,8 +1182,9 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
   constexpr int kLdc = BN + 8;   // elements per staged row
   T* stage_c = reinterpret_cast<T*>(smem);
   // DGRAD with the activation's backward fused in: the slice of the gelu' table
-  // goes into LDS behind the staged tile (its loads fly during the staging)
-  constexpr bool fuse_act = MODE == GEMM_DGRAD_ACT;
+  // goes into LDS behind the staged tile (its loads fly during the staging); a ReLU
+  // needs none
+  constexpr bool fuse_act = fuses_dgrad(MODE), kTable = MODE == GEMM_DGRAD_ACT;
   constexpr int kTabOffset = BM * kLdc * 2;   // behind this instantiation's own staged tile
   static_assert(kTabOffset % 16 == 0 && kTabOffset <= kActTabLdsOffset, "place of the table");
   float* act_tab_w = reinterpret_cast<float*>(smem + kTabOffset / 2);
@@ -1187,7 +1196,7 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
   i32x4_t tab_regs[kTabPerThread];
 #pragma unroll
   for (int i = 0; i < kTabPerThread; ++i) tab_regs[i] = i32x4_t{0, 0, 0, 0};
-  if constexpr (fuse_act) {
+  if constexpr (kTable) {
     const i32x4_t* src = reinterpret_cast<const i32x4_t*>(g.act_table + kActTabFirst);
 #pragma unroll
     for (int i = 0; i < kTabPerThread; ++i) tab_regs[i] = src[tid + i * NT];
@@ -1251,7 +1260,7 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
   constexpr int kBlocksLo = kHalfRows * TN * 4, kBlocksHi = (TM - kHalfRows) * TN * 4;
   stage_blocks(std::integral_constant<int, 0>{}, std::integral_constant<int, kHalfRows>{},
                std::integral_constant<int, 0>{}, std::integral_constant<int, kBlocksLo>{});
-  if constexpr (fuse_act) {
+  if constexpr (kTable) {
 #pragma unroll
     for (int i = 0; i < kTabPerThread; ++i)
       reinterpret_cast<i32x4_t*>(act_tab_w)[tid + i * NT] = tab_regs[i];
@@ -1302,6 +1311,7 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
     // as a separate activation kernel would read it) times the table value of
     // the matching pre-activation pack, fetched through a descriptor with the
     // tile's own bounds (a pack outside reads as zeros and its store is dropped).
+    // ReLU: dH where the unit is active.
     if (n0 + pk * 8 < N) {
       const __amdgpu_buffer_rsrc_t p_rsrc = __builtin_amdgcn_make_buffer_rsrc(
           (void*)((const T*)g.act_pre + ((int64_t)row0 + m0) * ldc + n0), (short)0,
@@ -1326,20 +1336,28 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
 #pragma unroll
         for (int u = 0; u < kChunk; ++u)
           hv[u] = *reinterpret_cast<const i32x4_t*>(sp + (c * kChunk + u) * kRowsPerStep * kLdc);
-        uint32_t seen = 0;
-#pragma unroll
-        for (int u = 0; u < kChunk; ++u)
-#pragma unroll
-          for (int wd = 0; wd < 4; ++wd)
-            ov[u][wd] = (int)gelu_bwd_pair_fast<T>((uint32_t)hv[u][wd], (uint32_t)pv[c & 1][u][wd],
-                                                   act_tab, seen);
-        if (__builtin_amdgcn_ballot_w64(seen >= (uint32_t)kActTabCount) != 0) {
+        if constexpr (kTable) {
+          uint32_t seen = 0;
 #pragma unroll
           for (int u = 0; u < kChunk; ++u)
 #pragma unroll
             for (int wd = 0; wd < 4; ++wd)
-              ov[u][wd] = (int)gelu_bwd_pair_any<T>((uint32_t)hv[u][wd],
-                                                    (uint32_t)pv[c & 1][u][wd], g.act_table);
+              ov[u][wd] = (int)gelu_bwd_pair_fast<T>((uint32_t)hv[u][wd], (uint32_t)pv[c & 1][u][wd],
+                                                     act_tab, seen);
+          if (__builtin_amdgcn_ballot_w64(seen >= (uint32_t)kActTabCount) != 0) {
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+              for (int wd = 0; wd < 4; ++wd)
+                ov[u][wd] = (int)gelu_bwd_pair_any<T>((uint32_t)hv[u][wd],
+                                                      (uint32_t)pv[c & 1][u][wd], g.act_table);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+            for (int wd = 0; wd < 4; ++wd)
+              ov[u][wd] = (int)relu_bwd_pair<T>((uint32_t)hv[u][wd], (uint32_t)pv[c & 1][u][wd]);
         }
 #pragma unroll
         for (int u = 0; u < kChunk; ++u)
@@ -1370,7 +1388,7 @@ __device__ __forceinline__ void gemm_tile32(const GemmArgs& g, uint16_t* smem, T
 // FWD 1.29-1.31 vs 1.24-1.26 PFLOP/s with 16x16x32, DGRAD 1.21 vs 1.35 and
 // WGRAD 1.24 vs 1.27 the other way round.
 #ifndef FMOE_MFMA16_MODES
-#define FMOE_MFMA16_MODES ((1 << GEMM_FWD) | (1 << GEMM_FWD_ACT))
+#define FMOE_MFMA16_MODES ((1 << GEMM_FWD) | (1 << GEMM_FWD_ACT) | (1 << GEMM_FWD_RELU))
 #endif
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NS, int MODE>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint16_t* smem, TileRows where,
@@ -1535,13 +1553,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs g,
 // The tail of one product overlaps the head of the next instead of leaving CUs
 // idle between two launches.  gd / gw are the arguments the two products
 // would get on their own.
-template <typename T, int BM, int BN, int BK, int WM, int WN, int NS, bool ACT>
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NS, int DMODE>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_bwd_kernel(GemmArgs gd, GemmArgs gw,
                                                                int tiles_n_d, int tiles_n_w,
                                                                int tiles_m_w, int small_first) {
   constexpr int NW = WM * WN;
-  // dX with gelu' of the pre-activations applied in its tiles (gd.act_pre), or plain
-  constexpr int DMODE = ACT ? GEMM_DGRAD_ACT : GEMM_DGRAD;
+  // (DMODE: dX with the activation's derivative applied in its tiles (gd.act_pre), or plain)
   constexpr bool kSmall = has_small_tiles<BM, BN, DMODE>();
   static_assert(!kSmall || NW == 4, "remainder tiles put 4 waves side by side");
   extern __shared__ __attribute__((aligned(1024))) uint16_t smem[];
@@ -1649,14 +1666,18 @@ static int launch_t(int mode, const GemmArgs& g, hipStream_t s) {
   switch (mode) {
     case GEMM_FWD:
       if constexpr (std::is_same<T, __hip_bfloat16>::value) {
-        if (g.act_out) return launch_mode<T, GEMM_FWD_ACT>(g, s);
+        if (g.act_out)
+          return g.act == FMOE_ACT_RELU ? launch_mode<T, GEMM_FWD_RELU>(g, s)
+                                        : launch_mode<T, GEMM_FWD_ACT>(g, s);
       }
       FMOE_REQUIRE(g.act_out == nullptr, FMOE_ERR_UNSUPPORTED,
                    "grouped GEMM: the fused activation is a bf16 kernel");
       return launch_mode<T, GEMM_FWD>(g, s);
     case GEMM_DGRAD:
       if constexpr (std::is_same<T, __hip_bfloat16>::value) {
-        if (g.act_pre) return launch_mode<T, GEMM_DGRAD_ACT>(g, s);
+        if (g.act_pre)
+          return g.act == FMOE_ACT_RELU ? launch_mode<T, GEMM_DGRAD_RELU>(g, s)
+                                        : launch_mode<T, GEMM_DGRAD_ACT>(g, s);
       }
       FMOE_REQUIRE(g.act_pre == nullptr, FMOE_ERR_UNSUPPORTED,
                    "grouped GEMM: the fused activation is a bf16 kernel");
@@ -1666,7 +1687,7 @@ static int launch_t(int mode, const GemmArgs& g, hipStream_t s) {
 }
 
 // dX and dW of one linear in one launch of 256x256 tiles, K slices of BK in NS stages.
-template <typename T, int BK, int NS, bool ACT = false>
+template <typename T, int BK, int NS, int DMODE = GEMM_DGRAD>
 static int launch_bwd_fused(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
   constexpr int BM = 256, BN = 256, WM = 2, WN = 2, NT = WM * WN * 64;
   constexpr size_t pipe_bytes = (size_t)NS * (BM + BN) * BK * 2;
@@ -1677,13 +1698,15 @@ static int launch_bwd_fused(const GemmArgs& gd, const GemmArgs& gw, hipStream_t 
   static_assert(lds_bytes + 1024 <= 160 * 1024, "LDS budget of a gfx950 CU");
   if (gd.act_pre) {
     if constexpr (std::is_same<T, __hip_bfloat16>::value) {
-      if (!ACT) return launch_bwd_fused<T, BK, NS, true>(gd, gw, s);
+      if (DMODE == GEMM_DGRAD)
+        return gd.act == FMOE_ACT_RELU ? launch_bwd_fused<T, BK, NS, GEMM_DGRAD_RELU>(gd, gw, s)
+                                       : launch_bwd_fused<T, BK, NS, GEMM_DGRAD_ACT>(gd, gw, s);
     } else {
       FMOE_REQUIRE(false, FMOE_ERR_UNSUPPORTED,
                    "grouped GEMM: the fused activation is a bf16 kernel");
     }
   }
-  auto kern = gemm_bwd_kernel<T, BM, BN, BK, WM, WN, NS, ACT>;
+  auto kern = gemm_bwd_kernel<T, BM, BN, BK, WM, WN, NS, DMODE>;
   FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds_bytes);
   const int tiles_n_d = ceil_div(gd.in_feat, BN);
   const int tiles_n_w = ceil_div(gw.in_feat, BN), tiles_m_w = ceil_div(gw.out_feat, BM);

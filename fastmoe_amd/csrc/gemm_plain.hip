@@ -250,16 +250,6 @@ __device__ __forceinline__ float act_fwd(const GemmArgs& g, float v) {
 __device__ __forceinline__ float act_bwd(const GemmArgs& g, float d, float pre) {
   return g.act == FMOE_ACT_RELU ? (pre <= 0.f ? 0.f : d) : d * gelu_grad_direct(pre);
 }
-// ReLU of 16-bit patterns: whether a negative value is a NaN only its bits above infinity's tell.
-template <typename T> constexpr uint16_t kInf16 = std::is_same<T, __half>::value ? 0x7c00 : 0x7f80;
-template <typename T>
-__device__ __forceinline__ uint16_t relu_fwd16(uint16_t v) {
-  return (v & 0x8000u) && (v & 0x7fffu) <= kInf16<T> ? 0 : v;
-}
-template <typename T>
-__device__ __forceinline__ uint16_t relu_bwd16(uint16_t d, uint16_t pre) {
-  return pre == 0 || ((pre & 0x8000u) && (pre & 0x7fffu) <= kInf16<T>) ? 0 : d;
-}
 __device__ __forceinline__ uint16_t act_fwd16(const GemmArgs& g, uint16_t v) {
   return load_global<uint16_t>(g.act_fwd_table + v);
 }

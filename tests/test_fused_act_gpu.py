@@ -1,6 +1,7 @@
 """The backward of `linear(gelu(pre))` with gelu' applied inside the grouped
 GEMM's epilogue (fmoe_grouped_linear_bwd_act) against the two separate steps it
-replaces: the same bits out, on every kernel path, for every 16-bit argument."""
+replaces: the same bits out, on every kernel path, for every 16-bit argument; ReLU in the
+tiles of both directions likewise."""
 import numpy as np
 import pytest
 import torch
@@ -202,3 +203,67 @@ def test_other_activations_keep_their_own_backward():
     y0 = h @ ref.h4toh.weight[0].t() + ref.h4toh.bias[0]
     y0.sum().backward()
     assert (x.grad[:20] - xr.grad[:20]).abs().max().item() <= 1e-4
+
+
+def _expert_linear(lib, dtype, counts, in_f, out_f, path):
+    """Calls of the two-layer expert's products on one set of operands: forward(act, keep_y) ->
+    (y, y_act) and backward(dy, act, act_pre) -> (dx, dw, db), every kernel family forced."""
+    code = {torch.float32: 0, torch.float64: 1, torch.float16: 2, torch.bfloat16: 3}[dtype]
+    n, e = sum(counts), len(counts)
+    x, w, b = (randn(s, dtype, i, 0.3).cuda()
+               for i, s in enumerate([(n, in_f), (e, out_f, in_f), (e, out_f)]))
+    seg = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def forced(fn, *args):
+        assert lib.fmoe_set_gemm_path(path) == 0
+        try:
+            assert fn(*args, n, in_f, out_f, e, code, stream) == 0, lib.fmoe_last_error()
+            torch.cuda.synchronize()
+        finally:
+            lib.fmoe_set_gemm_path(0)
+
+    def ptr(t):
+        return None if t is None else t.data_ptr()
+
+    def forward(act, keep_y=True):
+        y = torch.empty(n, out_f, dtype=dtype, device="cuda") if keep_y else None
+        a = torch.empty(n, out_f, dtype=dtype, device="cuda") if act else None
+        forced(lib.fmoe_expert_linear_fwd, ptr(x), ptr(w), None, ptr(b), None, ptr(seg), ptr(y),
+               ptr(a), act)
+        return y, a
+
+    def backward(dy, act, act_pre):
+        dx, dw, db = torch.empty_like(x), torch.empty_like(w), torch.empty_like(b)
+        forced(lib.fmoe_expert_linear_bwd, ptr(dy), ptr(x), ptr(w), None, ptr(seg), ptr(act_pre),
+               act, ptr(dx), ptr(dw), ptr(db))
+        return dx, dw, db
+
+    return x, forward, backward
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("path", [2, 3, 4, 5])
+@pytest.mark.parametrize("counts,in_f,out_f", [([300, 0, 257, 64, 1, 200, 513], 136, 264),
+                                               ([130, 255, 70], 264, 72), ([513], 264, 1032)])
+def test_relu_inside_every_tile(dt, path, counts, in_f, out_f):
+    """ReLU in the output tiles of either direction, infinities and NaNs included: the product
+    without one, then max(y, 0) and `unit active ? dx : 0`, bit for bit."""
+    from fastmoe_amd import _lib
+
+    x, forward, backward = _expert_linear(_lib.load(), DTYPES[dt], counts, in_f, out_f, path)
+    x[3, 1], x[7, 2] = float("inf"), float("nan")
+    y, _ = forward(0)
+    want = torch.where(y <= 0, torch.zeros_like(y), y)
+    for keep in (True, False):
+        kept, a = forward(2, keep)
+        assert _same_bits(a, want) and (not keep or _same_bits(kept, y))
+    assert want[7].isnan().all() and (want == 0).any()
+    dy = randn((sum(counts), out_f), DTYPES[dt], 7).cuda()
+    dy[5], dy[11, 0], dy[12, 1] = float("inf"), float("-inf"), float("nan")
+    pre = randn((sum(counts), in_f), DTYPES[dt], 8).cuda().relu()
+    pre[0, 0] = float("nan")
+    plain, got = backward(dy, 0, None), backward(dy, 2, pre)
+    assert plain[0][5].isinf().any() or plain[0][5].isnan().any()
+    assert _same_bits(got[0], torch.where(pre <= 0, torch.zeros_like(pre), plain[0]))
+    assert _same_bits(got[1], plain[1]) and _same_bits(got[2], plain[2])
