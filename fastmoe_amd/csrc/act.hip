@@ -25,10 +25,6 @@ constexpr int kTabBwd = 32768;           // entries: every pattern without its s
 // One copy per GPU; [0] = bf16, [1] = f16.
 __device__ uint16_t g_gelu_fwd_tab[2][kTabFwd];
 __device__ float g_gelu_bwd_tab[2][kTabBwd];
-// The same for ReLU; the backward one (for both types) by pattern of the activation, which is
-// never negative: 1 for zero, 0 for everything else, NaNs included.
-__device__ uint16_t g_relu_fwd_tab[2][kTabFwd];
-__device__ float g_relu_bwd_tab[kTabBwd];
 
 __device__ __forceinline__ double bits_to_double(int which, uint16_t b) {
   if (which == 0) return (double)__uint_as_float((uint32_t)b << 16);
@@ -48,10 +44,6 @@ __global__ void gelu_table_kernel() {
     g_gelu_fwd_tab[which][i] = float_to_bits(which, (float)gelu_f64(x));
     if (i < kTabBwd) g_gelu_bwd_tab[which][i] = (float)gelu_grad_f64(-x);
   }
-  // negative numbers to zero, negative NaNs as they are
-  g_relu_fwd_tab[0][i] = i >= 0x8000 && i <= 0xff80 ? 0 : (uint16_t)i;
-  g_relu_fwd_tab[1][i] = i >= 0x8000 && i <= 0xfc00 ? 0 : (uint16_t)i;
-  if (i < kTabBwd) g_relu_bwd_tab[i] = i == 0 ? 1.f : 0.f;
 }
 
 // Elements that need work: all n, or the first *n_rows_dev rows of row_len when
@@ -279,23 +271,6 @@ int gelu_fwd_table(int dtype, hipStream_t s, const uint16_t** table) {
   uint16_t* base = nullptr;
   FMOE_HIP_CHECK(hipGetSymbolAddress((void**)&base, HIP_SYMBOL(g_gelu_fwd_tab)));
   *table = base + (dtype == FMOE_BF16 ? 0 : kTabFwd);
-  return FMOE_OK;
-}
-
-int relu_fwd_table(int dtype, hipStream_t s, const uint16_t** table) {
-  int cus = 0;
-  const int rc = ensure_tables(s, &cus);
-  if (rc) return rc;
-  uint16_t* base = nullptr;
-  FMOE_HIP_CHECK(hipGetSymbolAddress((void**)&base, HIP_SYMBOL(g_relu_fwd_tab)));
-  *table = base + (dtype == FMOE_BF16 ? 0 : kTabFwd);
-  return FMOE_OK;
-}
-int relu_bwd_table(hipStream_t s, const float** table) {
-  int cus = 0;
-  const int rc = ensure_tables(s, &cus);
-  if (rc) return rc;
-  FMOE_HIP_CHECK(hipGetSymbolAddress((void**)table, HIP_SYMBOL(g_relu_bwd_tab)));
   return FMOE_OK;
 }
 

@@ -198,11 +198,9 @@ static double act_kernel_us(int64_t values, int passes) {
   return 5 + 2.0 * passes * (double)values / 5e6;
 }
 
-// The tables of a 16-bit activation (the 256-row kernels look ReLU up as well).
+// The tables of a 16-bit GELU (a ReLU needs none, so that its first call may be captured).
 static int act_tables(int act, int dtype, hipStream_t s, GemmArgs* g, bool fwd) {
-  if (dtype != FMOE_BF16 && dtype != FMOE_F16) return FMOE_OK;
-  if (act == FMOE_ACT_RELU)
-    return fwd ? relu_fwd_table(dtype, s, &g->act_fwd_table) : relu_bwd_table(s, &g->act_table);
+  if (act != FMOE_ACT_GELU || (dtype != FMOE_BF16 && dtype != FMOE_F16)) return FMOE_OK;
   return fwd ? gelu_fwd_table(dtype, s, &g->act_fwd_table) : gelu_bwd_table(dtype, s, &g->act_table);
 }
 

@@ -95,11 +95,6 @@ constexpr int kActTabLdsOffset = 256 * (256 + 8) * 2;   // bytes from the start 
 int gelu_bwd_table(int dtype, hipStream_t s, const float** table);
 // Device table of gelu(x) by the 16-bit pattern of x (65536 results of the dtype).
 int gelu_fwd_table(int dtype, hipStream_t s, const uint16_t** table);
-// The same two for ReLU: a forward table of max(x, 0) by pattern, and (for either dtype)
-// 1 - relu'(a) by pattern of the ACTIVATION a = relu(x) (never negative), so that the
-// kernels' rule "a positive argument takes 1 - the entry" holds for both activations.
-int relu_fwd_table(int dtype, hipStream_t s, const uint16_t** table);
-int relu_bwd_table(hipStream_t s, const float** table);
 // y = max(x, 0) and dx = x > 0 ? dy : 0 (NaN passes), over the first *n_rows_dev rows
 int relu_fwd(const void* x, void* y, int64_t n, const int32_t* n_rows_dev, int64_t row_len,
              int dtype, hipStream_t s);

@@ -1,8 +1,13 @@
 """HIP-graph capture and replay of the whole layer (forward + backward).  Kept
 in a file of its own that pytest collects last."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
+from conftest import ROOT
 from test_layer_gpu import _make
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +100,52 @@ def test_make_graphed_callables_replays_the_layer():
             assert torch.equal(a, b)
         _ = run(twin, xs[(i + 1) % 4], dys[(i + 1) % 4])
         torch.cuda.synchronize()
+
+
+FIRST_RELU = """
+import sys, torch
+sys.path.insert(0, {tests!r}); sys.path.insert(0, {root!r})
+from helpers import DTYPES, randn
+from fastmoe_amd import _lib
+lib, dtype, code = _lib.load(), DTYPES[{dt!r}], {{"f16": 2, "bf16": 3}}[{dt!r}]
+counts, n_in, n_out = [300, 0, 257, 70], 64, 96
+n, e = sum(counts), len(counts)
+x, w, dy = (randn(s, dtype, i, 0.3).cuda() for i, s in enumerate([(n, n_in), (e, n_out, n_in), (n, n_in)]))
+seg = torch.tensor([0] + counts).cumsum(0).int().cuda()
+a, dpre = (torch.empty(n, n_out, dtype=dtype, device="cuda") for _ in range(2))
+w2, dw2 = randn((e, n_in, n_out), dtype, 4, 0.3).cuda(), torch.empty(e, n_in, n_out, dtype=dtype, device="cuda")
+assert lib.fmoe_set_gemm_path({path}) == 0
+def call():
+    s = torch.cuda.current_stream().cuda_stream
+    for rc in (lib.fmoe_expert_linear_fwd(x.data_ptr(), w.data_ptr(), None, None, None, seg.data_ptr(), None,
+                                          a.data_ptr(), 2, n, n_in, n_out, e, code, s),
+               lib.fmoe_expert_linear_bwd(dy.data_ptr(), a.data_ptr(), w2.data_ptr(), None, seg.data_ptr(),
+                                          a.data_ptr(), 2, dpre.data_ptr(), dw2.data_ptr(), None, n, n_out,
+                                          n_in, e, code, s)):
+        assert rc == 0, lib.fmoe_last_error()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    call()
+got = []
+for _ in range(3):
+    a.zero_(), dpre.zero_(), dw2.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    got.append([t.clone() for t in (a, dpre, dw2)])
+call()
+torch.cuda.synchronize()
+for r in got:
+    assert all(torch.equal(p, q) for p, q in zip(r, (a, dpre, dw2)))
+assert a.any() and dpre.any() and (a == 0).any()
+print("captured")
+"""
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("path", [0, 2])
+def test_the_first_relu_of_a_process_can_be_captured(dt, path):
+    """A ReLU needs no table, so nothing has to be set up outside the graph: in a process of its
+    own, on the small tiles and on the 256-row ones."""
+    code = FIRST_RELU.format(root=ROOT, tests=os.path.join(ROOT, "tests"), dt=dt, path=path)
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0 and "captured" in res.stdout, (res.stdout + res.stderr)[-2000:]
