@@ -241,7 +241,8 @@ def apply_activation(activation, x, n_rows_dev=None):
     library's kernel, anything else as the module itself.  `n_rows_dev` (device
     int32[1], optional): the rows of x behind that count are dead (slots a
     capacity limit dropped) and the kernel skips them."""
-    if (type(activation) is torch.nn.GELU and getattr(activation, "approximate", "none") == "none"
+    if (type(activation) is torch.nn.GELU and "forward" not in activation.__dict__
+            and getattr(activation, "approximate", "none") == "none"
             and x.is_cuda and x.dtype in (torch.float32, torch.float64, torch.float16,
                                           torch.bfloat16)):
         return Gelu.apply(x, n_rows_dev)

@@ -20,10 +20,11 @@ class NaiveGate(BaseGate):
 
     def is_plain(self, x) -> bool:
         r"""Whether running this module on the 2-d tensor `x` is exactly Linear -> top-k ->
-        softmax in one dtype, with nobody watching: a layer may then fold the gate into its
-        own autograd node."""
+        softmax in one dtype, with nobody watching and no `forward` set on an instance: a
+        layer may then fold the gate into its own autograd node."""
         lin = self.gate
         return (type(self).forward is NaiveGate.forward and type(lin) is nn.Linear
+                and "forward" not in self.__dict__ and "forward" not in lin.__dict__
                 and lin.weight.dtype == x.dtype and lin.weight.is_cuda
                 and self.top_k <= fmoe_cuda.MAX_GATE_TOP_K
                 and torch.get_default_dtype() == torch.float32

@@ -286,7 +286,7 @@ def linear_act_linear_list(activation, inp, fwd_expert_count, weights1, biases1,
 
 def is_exact_gelu(activation, x: torch.Tensor) -> bool:
     r"""Whether `activation(x)` is the erf GELU the library has kernels for."""
-    return (type(activation) is torch.nn.GELU
+    return (type(activation) is torch.nn.GELU and "forward" not in activation.__dict__
             and getattr(activation, "approximate", "none") == "none" and x.is_cuda
             and x.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16))
 
@@ -295,8 +295,9 @@ def native_act(activation, x: torch.Tensor) -> int:
     r"""The library's code of `activation` (FMOE_ACT_*), 0 if it has no kernels for it."""
     if is_exact_gelu(activation, x):
         return 1
-    return 2 if type(activation) is torch.nn.ReLU or activation is torch.relu \
-        or activation is torch.nn.functional.relu else 0
+    if type(activation) is torch.nn.ReLU:
+        return 0 if "forward" in activation.__dict__ else 2
+    return 2 if activation is torch.relu or activation is torch.nn.functional.relu else 0
 
 
 def act_linear(activation, pre, fwd_expert_count, weight, bias):

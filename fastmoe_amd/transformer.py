@@ -12,20 +12,26 @@ from .linear import (FMoELinear, MOELinear, NativeTables, ParamTables, act_linea
                      linear_act_linear, linear_act_linear_list, native_act)
 
 
-def _watched(*modules) -> bool:
-    r"""Whether anybody has hooks on one of `modules` that only a call of the module
-    itself (forward hooks) or its own autograd nodes (backward hooks) would run."""
-    return any(m is not None and isinstance(m, nn.Module) and
-               (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or
-                getattr(m, "_backward_pre_hooks", None))
-               for m in modules)
-
-
 def _hooked(module) -> bool:
-    r"""_watched() of one module, through its dictionary."""
+    r"""Whether `module` has hooks that only a call of the module itself (forward hooks) or
+    its own autograd nodes (backward hooks) would run, or a `forward` of its own, set on
+    the instance as wrapping tools do."""
     d = module.__dict__
     return bool(d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                or d.get("_backward_pre_hooks"))
+                or d.get("_backward_pre_hooks") or "forward" in d)
+
+
+def _watched(*modules) -> bool:
+    r"""_hooked() of any of `modules` that is a module."""
+    return any(isinstance(m, nn.Module) and _hooked(m) for m in modules)
+
+
+def _plain(cls, *modules) -> bool:
+    r"""Whether calling any of `modules` runs `cls.forward` and nothing else, so that its
+    arithmetic may be done without calling it: a subclass with a `forward` of its own, a
+    wrapper and a watched module have to be called."""
+    return all(getattr(type(m), "forward", None) is cls.forward and not _hooked(m)
+               for m in modules)
 
 
 class FusedExpertLayer(Function):
@@ -122,11 +128,11 @@ class _Expert(nn.Module):
         self.activation = activation
 
     def forward(self, inp, fwd_expert_count):
-        if _watched(self.htoh4, self.h4toh, self.activation):
-            # somebody watches the linear modules or the activation: call them as
-            # modules, the way the reference does (fmoe/transformer.py:25-33)
+        if not _plain(FMoELinear, self.htoh4, self.h4toh) or _watched(self.activation):
+            # somebody watches or has replaced the linear modules or the activation: call
+            # them as modules, the way the reference does (fmoe/transformer.py:25-33)
             x = self.htoh4(inp, fwd_expert_count)
-            if _watched(self.h4toh, self.activation):
+            if not _plain(FMoELinear, self.h4toh) or _watched(self.activation):
                 return self.h4toh(self.activation(x), fwd_expert_count)
             return act_linear(self.activation, x, fwd_expert_count, self.h4toh.weight,
                               self.h4toh.bias)
@@ -139,14 +145,16 @@ class _Expert(nn.Module):
         r"""Whether the whole layer (dispatch included) can run as one autograd node:
         one 2-d GPU tensor in the parameters' dtype, an activation the library has kernels
         for (ReLU in the extension only) between the two layers, and nobody watching the
-        modules inside."""
+        modules inside or giving them another `forward`."""
+        if not (_plain(_Expert, self) and _plain(FMoELinear, self.htoh4, self.h4toh)
+                and not _watched(self.activation)):
+            return False
         w1, w2 = self.htoh4.weight, self.h4toh.weight
         return (torch.is_tensor(inp) and inp.dim() == 2 and inp.is_cuda
                 and inp.dtype == w1.dtype == w2.dtype and 1 <= top_k <= 64
                 and (is_exact_gelu(self.activation, inp)
                      or (native_act(self.activation, inp) != 0
-                         and fmoe_cuda.native() is not None))
-                and not _watched(self, self.htoh4, self.h4toh, self.activation))
+                         and fmoe_cuda.native() is not None)))
 
     def _native_args(self, inp):
         r"""The experts' share of a call of the extension's layer nodes."""
@@ -195,24 +203,24 @@ class _Expert(nn.Module):
     def can_run_list(experts) -> bool:
         r"""Whether `experts` (the reference's layout: one `_Expert(1, ...)` per
         expert) can run as ONE grouped call per layer on per-expert weight pointers:
-        single-expert modules of one shape, dtype and device, and nobody watching them
-        (hooks on a list module run only when that module is called, which the
+        single-expert modules of one shape, dtype and device, and nobody watching them or
+        giving them another `forward` (which runs only when that module is called, as the
         reference-shaped route does)."""
         first = experts[0] if len(experts) else None
-        if not isinstance(first, _Expert):
+        if not isinstance(first, _Expert) or not _plain(FMoELinear, first.htoh4, first.h4toh):
             return False
         w1, w2 = first.htoh4.weight, first.h4toh.weight
         for e in experts:
-            if not (isinstance(e, _Expert) and e.activation is first.activation
-                    and e.htoh4.num_expert == 1 and e.h4toh.num_expert == 1
+            if not (isinstance(e, _Expert) and _plain(_Expert, e)
+                    and _plain(FMoELinear, e.htoh4, e.h4toh)
+                    and e.activation is first.activation and e.htoh4.num_expert == 1 and e.h4toh.num_expert == 1
                     and e.htoh4.weight.shape == w1.shape and e.h4toh.weight.shape == w2.shape
                     and (e.htoh4.bias is None) == (first.htoh4.bias is None)
                     and (e.h4toh.bias is None) == (first.h4toh.bias is None)
                     and e.htoh4.weight.dtype == w1.dtype and e.h4toh.weight.dtype == w1.dtype
                     and e.htoh4.weight.device == w1.device
                     and e.h4toh.weight.device == w1.device
-                    and e.htoh4.weight.is_cuda
-                    and not _watched(e, e.htoh4, e.h4toh)):
+                    and e.htoh4.weight.is_cuda):
                 return False
         return not _watched(first.activation)
 

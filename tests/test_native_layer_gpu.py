@@ -194,6 +194,52 @@ def test_balance_gate_against_float64(dt, kind, k, t, e):
     assert (a.grad.double() - ref.grad).abs().max() <= 4 * eps * ref.grad.abs().max()
 
 
+def _replace_forward(module, seen):
+    """`module` wrapped in place: its calls are counted and their first result doubled."""
+    inner = module.forward
+
+    def forward(*args):
+        seen.append(module)
+        out = inner(*args)
+        return (out[0], out[1] * 2) if isinstance(out, tuple) else out * 2
+
+    module.forward = forward
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
+@pytest.mark.parametrize("where", ["gate", "gate.gate", "experts", "htoh4", "h4toh", "activation"])
+@pytest.mark.parametrize("how", ["instance", "class"])
+def test_modules_with_another_forward_are_called(fused, act, where, how):
+    """A `forward` set on an instance or by a subclass is what runs, wherever in the layer: twice
+    the logits, hidden values or scores there change the output, and the module is counted."""
+    from fastmoe_amd import FMoETransformerMLP
+
+    torch.manual_seed(4)
+    moe = FMoETransformerMLP(4, 32, 48, top_k=2, activation=act(), fused=fused).cuda()
+    x = torch.randn(60, 32, device="cuda", requires_grad=True)
+    want, seen = moe(x), []
+    if where.startswith("gate"):
+        modules = [moe.get_submodule(where)]
+    else:
+        experts = [moe.experts] if fused else list(moe.experts)
+        modules = experts if where == "experts" else [getattr(e, where) for e in experts]
+    for m in set(modules):
+        if how == "instance":
+            _replace_forward(m, seen)
+        else:
+            def forward(self, *args, _parent=type(m)):
+                seen.append(self)
+                out = _parent.forward(self, *args)
+                return (out[0], out[1] * 2) if isinstance(out, tuple) else out * 2
+
+            m.__class__ = type("Other", (type(m),), {"forward": forward})
+    got = moe(x)
+    got.sum().backward()
+    assert set(seen) == set(modules) and not torch.allclose(got, want, rtol=1e-2)
+    assert x.grad is not None and x.grad.any()
+
+
 def _gate(d, e, k, dtype=torch.float32):
     from fastmoe_amd import NaiveGate
 
