@@ -265,7 +265,10 @@ class _Expert(nn.Module):
         tables = getattr(experts, "_fmoe_native_tables", None)
         if tables is None:
             tables = NativeTables()
-            object.__setattr__(experts, "_fmoe_native_tables", tables)
+            try:
+                object.__setattr__(experts, "_fmoe_native_tables", tables)
+            except AttributeError:   # a plain list: no place to keep them
+                pass
         return (params, len(kinds[0]), kinds[1][0] is not None, kinds[3][0] is not None, act,
                 tables.get(fmoe_cuda.native()))
 

@@ -322,6 +322,27 @@ def test_list_layer_copies_and_pickles_after_a_call():
         assert not other(x).any() and torch.equal(moe(x), want)
 
 
+@pytest.mark.parametrize("container", [list, tuple])
+@pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
+def test_experts_in_a_plain_container(container, act):
+    """Experts kept in a Python list or tuple instead of a ModuleList: the same layer."""
+    from fastmoe_amd import FMoETransformerMLP
+
+    torch.manual_seed(5)
+    moe = FMoETransformerMLP(4, 64, 96, top_k=2, fused=False, activation=act()).cuda()
+    x, got = torch.randn(50, 64, device="cuda"), []
+    experts = moe.experts
+    for holder in (experts, container(experts)):
+        del moe.experts
+        moe.experts = holder
+        for p in experts.parameters():
+            p.grad = None
+        out = moe(x)
+        out.sum().backward()
+        got.append([out.detach()] + [p.grad for p in experts.parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 def test_list_layer_first_called_under_capture_or_on_another_stream():
     """The table of the experts' addresses is written by the stream that reads it: a graph
     that has not run yet leaves nothing behind for eager calls, nor do calls on one stream
