@@ -629,19 +629,23 @@ extern "C" int fmoe_limit_gate(const int64_t* gate, int64_t numel, int32_t n_exp
     FMOE_LAUNCH_CHECK("limit_gate_single");
     return FMOE_OK;
   }
-  hipLaunchKernelGGL(route_hist_kernel, dim3(ws.n_blocks), dim3(kRouteThreads),
-                     n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert, ws.block_hist,
-                     (int32_t*)nullptr);
-  FMOE_LAUNCH_CHECK("route_hist");
+  if (ws.n_blocks > 0) {   // (no slots: the scan alone writes the zero counts)
+    hipLaunchKernelGGL(route_hist_kernel, dim3(ws.n_blocks), dim3(kRouteThreads),
+                       n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert, ws.block_hist,
+                       (int32_t*)nullptr);
+    FMOE_LAUNCH_CHECK("route_hist");
+  }
   hipLaunchKernelGGL(route_scan_kernel<MODE_LIMIT>, dim3(1), dim3(kScanThreads),
                      (2 * n_expert + 1) * sizeof(int32_t), s, ws.block_hist, ws.n_blocks,
                      (int)n_expert, new_count, (int32_t*)nullptr, (int32_t*)nullptr,
                      (int32_t*)nullptr, limit);
   FMOE_LAUNCH_CHECK("route_scan");
-  hipLaunchKernelGGL(route_place_kernel<MODE_LIMIT>, dim3(ws.n_blocks), dim3(kRouteThreads),
-                     kRouteWaves * n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert,
-                     ws.block_hist, (const int32_t*)nullptr, (int64_t*)nullptr, (int32_t*)nullptr,
-                     new_gate, (const int32_t*)nullptr, limit);
-  FMOE_LAUNCH_CHECK("route_place");
+  if (ws.n_blocks > 0) {
+    hipLaunchKernelGGL(route_place_kernel<MODE_LIMIT>, dim3(ws.n_blocks), dim3(kRouteThreads),
+                       kRouteWaves * n_expert * sizeof(int32_t), s, gate, numel, (int)n_expert,
+                       ws.block_hist, (const int32_t*)nullptr, (int64_t*)nullptr,
+                       (int32_t*)nullptr, new_gate, (const int32_t*)nullptr, limit);
+    FMOE_LAUNCH_CHECK("route_place");
+  }
   return FMOE_OK;
 }

@@ -136,7 +136,7 @@ def test_gates_activations_and_layouts_match_the_chain(dt, act, gate, top_k, fus
         assert (g - w).double().norm() <= tol * w.double().norm()
 
 
-@pytest.mark.parametrize("n,e,cap", [(0, 4, 2), (100, 4, 0), (4096, 7, 300), (4097, 512, 8),
+@pytest.mark.parametrize("n,e,cap", [(0, 4, 2), (0, 513, 2), (100, 4, 0), (4096, 7, 300), (4097, 512, 8),
                                      (9000, 513, 5), (70000, 16, 4000)])
 def test_limit_gate_matches_count_limit_prune(n, e, cap):
     from fastmoe_amd import fmoe_cuda
