@@ -154,7 +154,11 @@ class _Expert(nn.Module):
                 and inp.dtype == w1.dtype == w2.dtype and 1 <= top_k <= 64
                 and (is_exact_gelu(self.activation, inp)
                      or (native_act(self.activation, inp) != 0
-                         and fmoe_cuda.native() is not None)))
+                         and fmoe_cuda.native() is not None
+                         # (parameters kept in another layout are copied on the way, which
+                         # only the chain of single operators does)
+                         and all(p is None or p.is_contiguous() for p in
+                                 (w1, self.htoh4.bias, w2, self.h4toh.bias)))))
 
     def _native_args(self, inp):
         r"""The experts' share of a call of the extension's layer nodes."""

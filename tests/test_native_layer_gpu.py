@@ -322,6 +322,26 @@ def test_list_layer_copies_and_pickles_after_a_call():
         assert not other(x).any() and torch.equal(moe(x), want)
 
 
+@pytest.mark.parametrize("name", ["htoh4.weight", "htoh4.bias", "h4toh.weight", "h4toh.bias"])
+def test_relu_experts_with_parameters_in_another_layout(name):
+    """A parameter whose memory is not in [E, out, in] order: the same values and gradients, up
+    to the order in which 70 tokens are summed (fewer than 65 units)."""
+    moe = _layer(torch.float32, 2, activation=torch.nn.ReLU())
+    x, got = torch.randn(70, 64, device="cuda"), []
+    p = moe.experts.get_parameter(name)
+    for other in (False, True):
+        if other:
+            p.data = p.data.transpose(0, -1).contiguous().transpose(0, -1)
+            assert not p.is_contiguous()
+        for q in moe.parameters():
+            q.grad = None
+        out = moe(x)
+        out.sum().backward()
+        got.append([out.detach()] + [q.grad for q in moe.parameters()])
+    for a, b in zip(*got):
+        assert (a - b).norm() <= 65 * torch.finfo(a.dtype).eps * a.norm()
+
+
 @pytest.mark.parametrize("container", [list, tuple])
 @pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
 def test_experts_in_a_plain_container(container, act):
