@@ -154,11 +154,16 @@ class _Expert(nn.Module):
                 and inp.dtype == w1.dtype == w2.dtype and 1 <= top_k <= 64
                 and (is_exact_gelu(self.activation, inp)
                      or (native_act(self.activation, inp) != 0
-                         and fmoe_cuda.native() is not None
+                         and fmoe_cuda.native() is not None and self._keeps_width()
                          # (parameters kept in another layout are copied on the way, which
                          # only the chain of single operators does)
                          and all(p is None or p.is_contiguous() for p in
                                  (w1, self.htoh4.bias, w2, self.h4toh.bias)))))
+
+    def _keeps_width(self) -> bool:
+        r"""Whether the experts' output is as wide as their input, as the extension's layer
+        nodes take it."""
+        return self.h4toh.weight.shape[1] == self.htoh4.weight.shape[2]
 
     def _native_args(self, inp):
         r"""The experts' share of a call of the extension's layer nodes."""
@@ -170,9 +175,9 @@ class _Expert(nn.Module):
     def run_layer(self, inp, gate_idx, score):
         r"""`sum_j score[t, j] * expert_{gate_idx[t, j]}(inp[t])` over the live slots,
         as one autograd node: the extension's own, or FusedExpertLayer where a Python node
-        is wanted (ctypes binding, per-op profiling)."""
+        is wanted (ctypes binding, per-op profiling) or the output has another width."""
         native = fmoe_cuda.native()
-        if native is not None:
+        if native is not None and self._keeps_width():
             return native.expert_layer(inp, gate_idx, score, *self._native_args(inp))
         return FusedExpertLayer.apply(inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
                                       self.h4toh.weight, self.h4toh.bias)
@@ -182,7 +187,7 @@ class _Expert(nn.Module):
         native autograd node, the gate's zero loss included; None where the gate has to run
         as the module it is.  Only called after can_run_layer()."""
         native = fmoe_cuda.native()
-        if native is None or not gate.is_plain(inp):
+        if native is None or not gate.is_plain(inp) or not self._keeps_width():
             return None
         lin = gate.gate
         out, loss = native.gated_layer(inp, lin.weight, lin.bias, *self._native_args(inp),
@@ -266,6 +271,8 @@ class _Expert(nn.Module):
                     return None
             if present:
                 params += kind
+        if kinds[2][0].shape[1] != kinds[0][0].shape[2]:
+            return None   # an output of another width than the input
         tables = getattr(experts, "_fmoe_native_tables", None)
         if tables is None:
             tables = NativeTables()

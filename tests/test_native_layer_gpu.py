@@ -342,6 +342,41 @@ def test_relu_experts_with_parameters_in_another_layout(name):
         assert (a - b).norm() <= 65 * torch.finfo(a.dtype).eps * a.norm()
 
 
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
+def test_experts_whose_output_has_another_width(fused, act):
+    """An FMoE layer of experts 32 -> 48 -> 40 against the sum over the experts in float64."""
+    from fastmoe_amd import FMoE
+    from fastmoe_amd.linear import FMoELinear
+    from fastmoe_amd.transformer import _Expert
+
+    def expert(n):
+        e = _Expert(n, 32, 48, activation)
+        e.h4toh = FMoELinear(n, 48, 40)
+        return e
+
+    torch.manual_seed(6)
+    activation = act()
+    moe = FMoE(4, 32, top_k=2, expert=None if fused else lambda d: expert(1))
+    if fused:
+        moe.experts = expert(4)
+    moe.cuda()
+    x = torch.randn(60, 32, device="cuda", requires_grad=True)
+    out = moe(x)
+    out.sum().backward()
+    idx, score = moe.gate(x)
+    want = torch.zeros(60, 40, dtype=torch.float64, device="cuda")
+    for e in range(4):
+        m = moe.experts[e]
+        w = [t.double()[0] for t in (m.htoh4.weight, m.htoh4.bias, m.h4toh.weight, m.h4toh.bias)]
+        y = torch.nn.functional.linear(activation(torch.nn.functional.linear(
+            x.double(), w[0], w[1])), w[2], w[3])
+        want = want + y * (score.double() * (idx == e)).sum(1, keepdim=True)
+    # (sums of 32 and 48 products in float32)
+    assert out.shape == (60, 40) and (out - want).norm() <= 1e-6 * want.norm()
+    assert x.grad.any() and all(p.grad is not None for p in moe.parameters())
+
+
 @pytest.mark.parametrize("container", [list, tuple])
 @pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
 def test_experts_in_a_plain_container(container, act):
