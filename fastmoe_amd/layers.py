@@ -153,7 +153,8 @@ class FMoE(nn.Module):
         args = get(self.experts, inp)
         if args is None:
             return None
-        if self.gate_hook is None and isinstance(self.gate, NaiveGate) and self.gate.is_plain(inp):
+        if self.gate_hook is None and isinstance(self.gate, NaiveGate) and self.gate.is_plain(inp) \
+                and self.gate.gate.weight.shape[0] == len(self.experts):
             lin = self.gate.gate
             out, loss = native.gated_layer(inp, lin.weight, lin.bias, *args[:5],
                                            self.gate.top_k, args[5])

@@ -186,10 +186,10 @@ class _Expert(nn.Module):
         r"""The layer with the plain top-k gate `gate` (NaiveGate) in front of it as one
         native autograd node, the gate's zero loss included; None where the gate has to run
         as the module it is.  Only called after can_run_layer()."""
-        native = fmoe_cuda.native()
-        if native is None or not gate.is_plain(inp) or not self._keeps_width():
-            return None
-        lin = gate.gate
+        native, lin = fmoe_cuda.native(), gate.gate
+        if (native is None or not gate.is_plain(inp) or not self._keeps_width()
+                or lin.weight.shape[0] != self.htoh4.num_expert):
+            return None   # (a choice that is none of the experts drops the slot)
         out, loss = native.gated_layer(inp, lin.weight, lin.bias, *self._native_args(inp),
                                        gate.top_k)
         gate.set_loss(loss)

@@ -377,6 +377,34 @@ def test_experts_whose_output_has_another_width(fused, act):
     assert x.grad.any() and all(p.grad is not None for p in moe.parameters())
 
 
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("outputs", [5, 9])
+def test_gate_with_more_or_fewer_outputs_than_experts(fused, outputs):
+    """A gate may choose among more numbers than there are experts (a choice of none: the slot is
+    dropped) or never choose some of them."""
+    from fastmoe_amd import FMoETransformerMLP, fmoe_cuda
+
+    torch.manual_seed(6)
+    moe = FMoETransformerMLP(6, 64, 96, top_k=2, fused=fused).cuda()
+    moe.gate.gate = torch.nn.Linear(64, outputs).cuda()
+    x, got = torch.randn(130, 64, device="cuda"), []
+    for watched in (False, True):
+        fmoe_cuda.profile_hook = (lambda *a: None) if watched else None
+        try:
+            for p in moe.parameters():
+                p.grad = None
+            a = x.clone().requires_grad_(True)
+            out = moe(a)
+            out.sum().backward()
+        finally:
+            fmoe_cuda.profile_hook = None
+        got.append([out, a.grad] + [p.grad for p in moe.parameters()])
+    assert torch.equal(got[0][0], got[1][0]) and moe.gate(x)[0].max() == outputs - 1
+    # (the gate's gradients are sums of 130 terms in another order: 65 units)
+    for g, w in zip(got[0][1:], got[1][1:]):
+        assert (g - w).norm() <= 65 * torch.finfo(g.dtype).eps * w.norm()
+
+
 @pytest.mark.parametrize("container", [list, tuple])
 @pytest.mark.parametrize("act", [torch.nn.GELU, torch.nn.ReLU])
 def test_experts_in_a_plain_container(container, act):
