@@ -603,6 +603,7 @@ def scatter_reduce(dbuf: torch.Tensor, inv: torch.Tensor, n_tokens: int,
 
 
 MAX_GATE_TOP_K = 16   # FMOE_MAX_GATE_TOP_K of the C ABI
+MAX_EXPERTS = 4096    # FMOE_MAX_EXPERTS
 
 
 def topk_softmax_fwd(logits: torch.Tensor, top_k: int) -> Tuple[torch.Tensor, torch.Tensor]:

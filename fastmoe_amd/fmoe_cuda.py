@@ -39,6 +39,7 @@ profile_hook = None
 profile_only = None
 
 MAX_GATE_TOP_K = ctypes_ops.MAX_GATE_TOP_K   # FMOE_MAX_GATE_TOP_K of the C ABI
+MAX_EXPERTS = ctypes_ops.MAX_EXPERTS         # FMOE_MAX_EXPERTS: what routing takes
 init = ctypes_ops.init                       # one-time GPU set-up (fmoe_init), either binding
 
 OPERATORS = ("expert_count", "assign_pos", "linear_forward", "linear_backward",

@@ -27,6 +27,7 @@ class NaiveGate(BaseGate):
                 and "forward" not in self.__dict__ and "forward" not in lin.__dict__
                 and lin.weight.dtype == x.dtype and lin.weight.is_cuda
                 and self.top_k <= fmoe_cuda.MAX_GATE_TOP_K
+                and lin.weight.shape[0] <= fmoe_cuda.MAX_EXPERTS   # (its gradients are routed)
                 and torch.get_default_dtype() == torch.float32
                 and not torch.is_autocast_enabled()
                 and not _has_any_global_hook()

@@ -212,3 +212,21 @@ def test_gate_gradients_from_slots(dt, t, e, k, d):
         if got is dx:   # either share is rounded before the addition
             err = err - eps * (moved.sum(1).abs() + (dense @ wg.double()).abs())
         assert (err <= eps * want.abs() + unit * (terms + 8 + k) * mag + (2 ** -25 if dt == "f16" else 0)).all()
+
+
+def test_gate_over_more_experts_than_can_be_routed():
+    """Choosing needs no routing, so a gate module may have more outputs than a layer may have
+    experts, and differentiate.  Against torch's own operations: sums of 50 terms in float32."""
+    from fastmoe_amd import NaiveGate
+
+    torch.manual_seed(8)
+    gate = NaiveGate(16, 5000, 1, 2).cuda()
+    x = torch.randn(50, 16, device="cuda", requires_grad=True)
+    params = [x, gate.gate.weight, gate.gate.bias]
+    idx, score = gate(x)
+    got = torch.autograd.grad((score * score).sum(), params)
+    val, want_idx = torch.topk(gate.gate(x), 2)
+    want = torch.autograd.grad((torch.softmax(val, -1) ** 2).sum(), params)
+    assert torch.equal(idx, want_idx)
+    for g, w in zip(got, want):
+        assert (g - w).norm() <= 1e-5 * w.norm()
