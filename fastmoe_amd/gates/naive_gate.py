@@ -39,7 +39,8 @@ class NaiveGate(BaseGate):
     def native_balance(self, logits):
         r"""The extension where its balance-gate node takes these logits, else None."""
         if (logits.is_cuda and logits.dim() == 2 and logits.shape[0] > 0
-                and 2 <= logits.shape[1] <= 512 and self.world_size == 1
+                and 2 <= logits.shape[1] <= 512 and logits.shape[1] == self.tot_expert
+                and self.world_size == 1
                 and logits.dtype in (torch.float32, torch.float16, torch.bfloat16)):
             return fmoe_cuda.native()
         return None

@@ -230,3 +230,16 @@ def test_gate_over_more_experts_than_can_be_routed():
     assert torch.equal(idx, want_idx)
     for g, w in zip(got, want):
         assert (g - w).norm() <= 1e-5 * w.norm()
+
+
+@pytest.mark.parametrize("gate", ["GShardGate", "SwitchGate"])
+def test_balance_gates_refuse_another_number_of_outputs(gate):
+    """Their loss has one term per expert: a linear map with more outputs is an error, not a
+    loss over something else."""
+    import fastmoe_amd
+
+    layer = getattr(fastmoe_amd, gate)(16, 4, 1).cuda()
+    layer(torch.randn(50, 16, device="cuda"))
+    layer.gate = torch.nn.Linear(16, 6).cuda()
+    with pytest.raises(RuntimeError, match="size"):
+        layer(torch.randn(50, 16, device="cuda"))
