@@ -525,6 +525,23 @@ std::tuple<Tensor, Tensor> limit_gate(const Tensor& gate_in, int64_t n_expert, i
   return {count, out};
 }
 
+// The gradients of the plain gate's linear map (x, weight, bias) from dscore as torch operations,
+// for gradients that will themselves be differentiated.  The softmax over the chosen logits is
+// taken at the scores of the forward pass, whatever has become of the bias since.
+variable_list differentiable_gate_grads(const Tensor& x, const Tensor& wg, const Tensor& bg,
+                                        const Tensor& idx, const Tensor& score,
+                                        const Tensor& dscore, bool dx, bool nwg, bool nbg) {
+  const auto acc = score.scalar_type() == at::kDouble ? at::kDouble : at::kFloat;
+  const Tensor chosen =
+      at::linear(x, wg, bg.defined() ? OptTensor(bg) : OptTensor()).gather(1, idx).to(acc);
+  const Tensor shift = score.detach().to(acc).log() - chosen.detach();
+  const Tensor p = at::softmax(chosen + shift, -1), ds = dscore.to(acc);
+  const Tensor dchosen = (p * (ds - (ds * p).sum(-1, true))).to(wg.scalar_type());
+  const Tensor dlogits = at::zeros({x.size(0), wg.size(0)}, wg.options()).scatter_add(1, idx, dchosen);
+  return {dx ? at::mm(dlogits, wg) : Tensor(), nwg ? at::mm(dlogits.t(), x) : Tensor(),
+          nbg ? dlogits.sum(0) : Tensor()};
+}
+
 // The plain gate as a node of its own (a layer that cannot fold it in: masks, experts of the
 // user's), with the kernels and so the bits of the folded one: (idx, score)
 struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
@@ -540,25 +557,25 @@ struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
     check(fmoe_topk_softmax_fwd(logits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k,
                                 idx.data_ptr<int64_t>(), score.data_ptr(), s.dtype, stream_of(x)),
           "topk_softmax_fwd");
-    ctx->save_for_backward({x_in, wg, idx, score, has_bg ? *bg : Tensor()});
+    ctx->save_for_backward({x_in, wg, idx, score});
+    // (not a saved variable: its value is not needed, and may be updated before the backward)
+    ctx->saved_data["bias"] = has_bg ? *bg : Tensor();
     ctx->mark_non_differentiable({idx});
     ctx->set_materialize_grads(false);
     return {idx, score};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list v = ctx->get_saved_variables();
-    const Tensor &wg = v[1], &idx = v[2], &score = v[3], &bg = v[4];
+    const Tensor &wg = v[1], &idx = v[2], &score = v[3], bg = ctx->saved_data["bias"].toTensor();
     const bool dx = ctx->needs_input_grad(0), nwg = ctx->needs_input_grad(1),
                nbg = bg.defined() && ctx->needs_input_grad(2);
     if (!grads[1].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
     c10::DeviceGuard guard(wg.device());
     if (at::GradMode::is_enabled()) {   // gradients that will themselves be differentiated
-      const Tensor chosen = at::linear(v[0], wg, bg.defined() ? OptTensor(bg) : OptTensor()).gather(1, idx);
-      const Tensor p = at::softmax(chosen, -1);
-      const Tensor dchosen = p * (grads[1] - (grads[1] * p).sum(-1, true));
-      const Tensor dlogits = at::zeros({v[0].size(0), wg.size(0)}, wg.options()).scatter_add(1, idx, dchosen);
-      return {dx ? at::mm(dlogits, wg) : Tensor(), nwg ? at::mm(dlogits.t(), v[0]) : Tensor(),
-              nbg ? dlogits.sum(0) : Tensor(), Tensor()};
+      variable_list out =
+          differentiable_gate_grads(v[0], wg, bg, idx, score, grads[1], dx, nwg, nbg);
+      out.push_back(Tensor());
+      return out;
     }
     const Tensor x = v[0].contiguous(), w = wg.contiguous();
     const LayerSizes s{x.size(0), x.size(1), 0, w.size(0), idx.size(1), idx.numel(), dt(x, "x")};

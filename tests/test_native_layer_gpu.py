@@ -297,6 +297,24 @@ def test_two_threads_on_one_stream():
     assert not failed
 
 
+@pytest.mark.parametrize("alone", [True, False])
+def test_gate_bias_may_change_before_the_backward(alone):
+    """No gradient depends on the value of the gate's bias, so updating it in place (as balancing
+    without a loss does) between the forward and the backward pass is allowed."""
+    gate, moe = _gate(64, 6, 2), _layer(torch.float32, 2)
+    if not alone:
+        gate = moe.gate
+    x, got = torch.randn(70, 64, device="cuda"), []
+    for change in (False, True):
+        a = x.clone().requires_grad_(True)
+        out = gate(a)[1] if alone else moe(a)
+        if change:
+            with torch.no_grad():
+                gate.gate.bias.add_(0.5 * torch.randn_like(gate.gate.bias))
+        got.append(torch.autograd.grad((out * out).sum(), [a, gate.gate.weight, gate.gate.bias]))
+    assert all(torch.equal(p, q) for p, q in zip(*got))
+
+
 def _list_layer():
     from fastmoe_amd import FMoETransformerMLP
 
