@@ -317,8 +317,7 @@ void gate_topk(const LayerSizes& s, const Tensor& logits, Tensor& idx, Tensor& s
 // stays the library call it is in torch.nn.Linear, so the logits (and with them the routing)
 // have the bits of the gate module; its gradients come from the top-k slots alone
 // (gate_grad.hip).
-LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, LayerSizes* sizes,
-                        Tensor* x_out, Tensor* idx_out) {
+LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, Tensor* idx_out) {
   at::AutoDispatchBelowADInplaceOrView below;
   const Tensor x = vars[0].contiguous();
   c10::DeviceGuard guard(x.device());
@@ -333,22 +332,59 @@ LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, L
     score = vars[2].reshape({s.t, s.k}).contiguous().to(x.scalar_type());
   }
   LayerPass p = experts_forward(c, s, expert_params(c, params), x, idx, score, train);
-  if (sizes) *sizes = s;
-  if (x_out) *x_out = x;
   if (idx_out) *idx_out = idx;
   return p;
 }
 
+// What a node saves of the plain gate's linear map: as in torch.nn.Linear the input only for the
+// parameters' gradients and the weight only for the input's, so that what no gradient needs may
+// be written in place before the backward.  (The parameters themselves are kept as well, without
+// the check of saved variables: for gradients of higher order.)
+void save_gate(AutogradContext* ctx, variable_list& saved, const Tensor& x, const Tensor& wg,
+               const Tensor& bg) {
+  saved.push_back(wg.requires_grad() || (bg.defined() && bg.requires_grad()) ? x : Tensor());
+  saved.push_back(x.requires_grad() ? wg : Tensor());
+  ctx->saved_data["gate"] = std::vector<Tensor>{wg, bg};
+}
+struct GateOperands {
+  Tensor x, wg, bg;   // x: undefined where no parameter wants a gradient
+};
+GateOperands saved_gate(AutogradContext* ctx, const Tensor& x, const Tensor& wg) {
+  const std::vector<Tensor> kept = ctx->saved_data["gate"].toTensorVector();
+  return {x, wg.defined() ? wg : kept[0], kept[1]};
+}
+
+// The gradients of the plain gate's linear map (x, weight, bias) from dscore as torch operations,
+// for gradients that will themselves be differentiated.  The softmax over the chosen logits is
+// taken at the scores of the forward pass, whatever has become of the bias since; it is a
+// constant where the gate is.
+variable_list differentiable_gate_grads(const GateOperands& gate, const Tensor& idx,
+                                        const Tensor& score, const Tensor& dscore, bool dx,
+                                        bool nwg, bool nbg) {
+  const auto acc = score.scalar_type() == at::kDouble ? at::kDouble : at::kFloat;
+  Tensor p = score.detach().to(acc);
+  if (gate.x.defined()) {
+    const Tensor chosen =
+        at::linear(gate.x, gate.wg, gate.bg.defined() ? OptTensor(gate.bg) : OptTensor())
+            .gather(1, idx).to(acc);
+    p = at::softmax(chosen + (p.log() - chosen.detach()), -1);
+  }
+  const Tensor ds = dscore.to(acc);
+  const Tensor dchosen = (p * (ds - (ds * p).sum(-1, true))).to(gate.wg.scalar_type());
+  const Tensor dlogits =
+      at::zeros({idx.size(0), gate.wg.size(0)}, gate.wg.options()).scatter_add(1, idx, dchosen);
+  return {dx ? at::mm(dlogits, gate.wg) : Tensor(), nwg ? at::mm(dlogits.t(), gate.x) : Tensor(),
+          nbg ? dlogits.sum(0) : Tensor()};
+}
+
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static Tensor forward(AutogradContext* ctx, at::TensorList vars, const LayerConfig& c) {
-    Tensor x, idx;
-    LayerSizes s;
-    LayerPass p = layer_forward(c, vars, true, &s, &x, &idx);
+    Tensor idx;
+    LayerPass p = layer_forward(c, vars, true, &idx);
     variable_list saved{p.buf, p.pre, p.act, p.out, p.score, p.route};
     if (c.gated) {
-      saved.push_back(x);
-      saved.push_back(vars[1]);
       saved.push_back(idx);
+      save_gate(ctx, saved, vars[0], vars[1], c.has_bg ? vars[2] : Tensor());
     } else {
       ctx->saved_data["shape"] = vars[2].sizes();
       ctx->saved_data["dtype"] = (int64_t)vars[2].scalar_type();
@@ -408,13 +444,16 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     want.b2 = any(c.has_b2, per);
     const bool gate_grads = c.gated && (dx || nwg || nbg);
     GateGrad gate;
-    if (gate_grads) gate = {v[6], v[7].contiguous(), v[8]};
+    if (gate_grads) {
+      const GateOperands op = saved_gate(ctx, v[7], v[8]);
+      gate = {op.x, op.wg.contiguous(), v[6]};
+    }
     LayerGrads g = experts_backward(c, s, w, p, dy, want, gate_grads ? &gate : nullptr);
     variable_list out;
     if (c.gated) {
       Tensor dwg, dbg;
       if (nwg || nbg)
-        std::tie(dwg, dbg) = gate_linear_grads(s, gate.x, p.route, g.dslot, nwg, nbg);
+        std::tie(dwg, dbg) = gate_linear_grads(s, gate.x.contiguous(), p.route, g.dslot, nwg, nbg);
       out = {g.dx, dwg};
       if (c.has_bg) out.push_back(dbg);
     } else {
@@ -450,7 +489,7 @@ bool wants_grad(at::TensorList ts) {
 
 Tensor run_layer(const LayerConfig& c, at::TensorList vars) {
   if (wants_grad(vars)) return LayerNode::apply(vars, c);
-  return layer_forward(c, vars, false, nullptr, nullptr, nullptr).y;
+  return layer_forward(c, vars, false, nullptr).y;
 }
 
 // The expert parameters' share of a call: `params` holds w1, b1, w2, b2 in that order, the
@@ -525,23 +564,6 @@ std::tuple<Tensor, Tensor> limit_gate(const Tensor& gate_in, int64_t n_expert, i
   return {count, out};
 }
 
-// The gradients of the plain gate's linear map (x, weight, bias) from dscore as torch operations,
-// for gradients that will themselves be differentiated.  The softmax over the chosen logits is
-// taken at the scores of the forward pass, whatever has become of the bias since.
-variable_list differentiable_gate_grads(const Tensor& x, const Tensor& wg, const Tensor& bg,
-                                        const Tensor& idx, const Tensor& score,
-                                        const Tensor& dscore, bool dx, bool nwg, bool nbg) {
-  const auto acc = score.scalar_type() == at::kDouble ? at::kDouble : at::kFloat;
-  const Tensor chosen =
-      at::linear(x, wg, bg.defined() ? OptTensor(bg) : OptTensor()).gather(1, idx).to(acc);
-  const Tensor shift = score.detach().to(acc).log() - chosen.detach();
-  const Tensor p = at::softmax(chosen + shift, -1), ds = dscore.to(acc);
-  const Tensor dchosen = (p * (ds - (ds * p).sum(-1, true))).to(wg.scalar_type());
-  const Tensor dlogits = at::zeros({x.size(0), wg.size(0)}, wg.options()).scatter_add(1, idx, dchosen);
-  return {dx ? at::mm(dlogits, wg) : Tensor(), nwg ? at::mm(dlogits.t(), x) : Tensor(),
-          nbg ? dlogits.sum(0) : Tensor()};
-}
-
 // The plain gate as a node of its own (a layer that cannot fold it in: masks, experts of the
 // user's), with the kernels and so the bits of the folded one: (idx, score)
 struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
@@ -557,35 +579,36 @@ struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
     check(fmoe_topk_softmax_fwd(logits.data_ptr(), s.t, (int32_t)s.e, (int32_t)s.k,
                                 idx.data_ptr<int64_t>(), score.data_ptr(), s.dtype, stream_of(x)),
           "topk_softmax_fwd");
-    ctx->save_for_backward({x_in, wg, idx, score});
-    // (not a saved variable: its value is not needed, and may be updated before the backward)
-    ctx->saved_data["bias"] = has_bg ? *bg : Tensor();
+    variable_list saved{idx, score};
+    save_gate(ctx, saved, x_in, wg, has_bg ? *bg : Tensor());
+    ctx->save_for_backward(std::move(saved));
     ctx->mark_non_differentiable({idx});
     ctx->set_materialize_grads(false);
     return {idx, score};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list v = ctx->get_saved_variables();
-    const Tensor &wg = v[1], &idx = v[2], &score = v[3], bg = ctx->saved_data["bias"].toTensor();
+    const Tensor &idx = v[0], &score = v[1];
+    const GateOperands gate = saved_gate(ctx, v[2], v[3]);
     const bool dx = ctx->needs_input_grad(0), nwg = ctx->needs_input_grad(1),
-               nbg = bg.defined() && ctx->needs_input_grad(2);
+               nbg = gate.bg.defined() && ctx->needs_input_grad(2);
     if (!grads[1].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
-    c10::DeviceGuard guard(wg.device());
+    c10::DeviceGuard guard(score.device());
     if (at::GradMode::is_enabled()) {   // gradients that will themselves be differentiated
-      variable_list out =
-          differentiable_gate_grads(v[0], wg, bg, idx, score, grads[1], dx, nwg, nbg);
+      variable_list out = differentiable_gate_grads(gate, idx, score, grads[1], dx, nwg, nbg);
       out.push_back(Tensor());
       return out;
     }
-    const Tensor x = v[0].contiguous(), w = wg.contiguous();
-    const LayerSizes s{x.size(0), x.size(1), 0, w.size(0), idx.size(1), idx.numel(), dt(x, "x")};
+    const int64_t d = gate.wg.size(1);
+    const LayerSizes s{idx.size(0), d, 0, gate.wg.size(0), idx.size(1), idx.numel(), dt(score, "score")};
     const Tensor dslot = gate_slot_grads(s, grads[1].contiguous(), score);
     Tensor gx, dwg, dbg;
     if (dx) {
-      gx = at::empty({s.t, s.d}, x.options());
+      const Tensor w = gate.wg.contiguous();
+      gx = at::empty({s.t, s.d}, score.options());
       check(fmoe_scatter_reduce_gate(nullptr, nullptr, idx.data_ptr<int64_t>(), dslot.data_ptr(),
                                      w.data_ptr(), gx.data_ptr(), s.t, s.k, s.d, (int32_t)s.e,
-                                     s.dtype, stream_of(x)),
+                                     s.dtype, stream_of(score)),
             "scatter_reduce_gate");
     }
     if (nwg || nbg) {
@@ -594,7 +617,8 @@ struct PlainGateNode : public torch::autograd::Function<PlainGateNode> {
       const int64_t bytes = fmoe_route_workspace_bytes(s.n, (int32_t)s.e);
       need(bytes >= 0, "workspace: bad sizes");
       const Tensor ws = at::empty({std::max<int64_t>(bytes, 1)}, idx.options().dtype(at::kByte));
-      std::tie(dwg, dbg) = gate_linear_grads(s, x, route_slots(s, idx, ws), dslot, nwg, nbg);
+      std::tie(dwg, dbg) =
+          gate_linear_grads(s, gate.x.contiguous(), route_slots(s, idx, ws), dslot, nwg, nbg);
     }
     return {gx, dwg, dbg, Tensor()};
   }

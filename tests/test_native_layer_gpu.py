@@ -315,6 +315,34 @@ def test_gate_bias_may_change_before_the_backward(alone):
     assert all(torch.equal(p, q) for p, q in zip(*got))
 
 
+@pytest.mark.parametrize("alone", [True, False])
+@pytest.mark.parametrize("what", ["weight", "x"])
+def test_what_no_gradient_needs_may_change_before_the_backward(alone, what):
+    """As in torch.nn.Linear: the gate's weight where x wants no gradient, x where the gate is
+    frozen.  Where they are needed, the change is an error."""
+    gate, moe = _gate(64, 6, 2), _layer(torch.float32, 2)
+    if not alone:
+        gate = moe.gate
+    x, got = torch.randn(70, 64, device="cuda"), []
+    gate.requires_grad_(what == "weight")
+    for change in (False, True):
+        a = (x.clone().requires_grad_(True) * 1) if what == "x" else x.clone()
+        out = gate(a)[1] if alone else moe(a)
+        wanted = a if what == "x" else gate.gate.weight
+        if change:
+            with torch.no_grad():
+                (a if what == "x" else gate.gate.weight).add_(1.0)
+        got.append(torch.autograd.grad((out * out).sum(), wanted)[0])
+    assert torch.equal(*got)
+    gate.requires_grad_(True)
+    a = x.clone().requires_grad_(True) * 1
+    out = gate(a)[1] if alone else moe(a)
+    with torch.no_grad():
+        (a if what == "x" else gate.gate.weight).add_(1.0)
+    with pytest.raises(RuntimeError, match="inplace"):
+        (out * out).sum().backward()
+
+
 def _list_layer():
     from fastmoe_amd import FMoETransformerMLP
 
