@@ -399,6 +399,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     return p.y;
   }
 
+  // Under create_graph the gate's share is made of torch operations, as where the gate is a
+  // module; the experts' kernels have no derivative, so their share is a constant then.
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     LayerConfig c = LayerConfig::from(ctx->saved_data["c"].toIntVector());
     const variable_list v = ctx->get_saved_variables();
@@ -406,7 +408,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     size_t at = 6 + (c.gated ? 3 : 0);
     if (c.list) c.table = v[at++];
     const at::TensorList weights = at::TensorList(v).slice(at);
-    at::AutoDispatchBelowADInplaceOrView below;
+    const bool twice = at::GradMode::is_enabled();
+    std::optional<at::AutoDispatchBelowADInplaceOrView> below(std::in_place);
     const Tensor dy = grads[0].contiguous();
     c10::DeviceGuard guard(dy.device());
     const LayerPass p{Tensor(), v[0], v[1], v[2], v[3], v[4], v[5]};
@@ -442,7 +445,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     want.b1 = any(c.has_b1, per);
     want.w2 = any(true, per);
     want.b2 = any(c.has_b2, per);
-    const bool gate_grads = c.gated && (dx || nwg || nbg);
+    const bool gate_grads = c.gated && !twice && (dx || nwg || nbg);
     GateGrad gate;
     if (gate_grads) {
       const GateOperands op = saved_gate(ctx, v[7], v[8]);
@@ -452,8 +455,16 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     variable_list out;
     if (c.gated) {
       Tensor dwg, dbg;
-      if (nwg || nbg)
+      if (gate_grads && (nwg || nbg))
         std::tie(dwg, dbg) = gate_linear_grads(s, gate.x.contiguous(), p.route, g.dslot, nwg, nbg);
+      if (twice) {
+        below.reset();
+        const variable_list own = differentiable_gate_grads(saved_gate(ctx, v[7], v[8]), v[6],
+                                                            p.score, g.dscore, dx, nwg, nbg);
+        if (dx) g.dx = g.dx + own[0];
+        dwg = own[1];
+        dbg = own[2];
+      }
       out = {g.dx, dwg};
       if (c.has_bg) out.push_back(dbg);
     } else {

@@ -533,6 +533,48 @@ def test_balance_loss_differentiates_twice_and_forwards(gate, top_k):
             assert forward_ad.unpack_dual(layer.get_loss()).tangent is not None
 
 
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("alone", [True, False])
+def test_plain_gate_differentiates_twice(alone, bias):
+    """The gradient of the plain gate has a gradient of its own, as a module and folded into the
+    layer (where the gradient of the scores and the experts' share count as constants).  Against
+    torch in float64: sums of up to 300 float32 terms, off by at most 300 units of 2^-24 each
+    time, a handful in a row: 1e-4 of the norm."""
+    from fastmoe_amd import FMoETransformerMLP
+
+    torch.manual_seed(12)
+    moe = FMoETransformerMLP(6, 64, 96, top_k=2, gate_bias=bias).cuda()
+    lin = moe.gate.gate
+    x = torch.randn(300, 64, device="cuda", requires_grad=True)
+    c = torch.randn(300, 2 if alone else 64, device="cuda")
+    idx, score = moe.gate(x)
+    params = [p for p in (lin.weight, lin.bias) if p is not None]
+    ref = [t.detach().double().requires_grad_(True) for t in (x, *params)]
+    want = torch.softmax(torch.nn.functional.linear(*ref).gather(1, idx), -1)
+    if alone:
+        dscore, share = c.double(), 0.0
+        out = score
+    else:
+        out = moe(x)
+        rows = [moe.experts[e].h4toh(moe.experts.activation(moe.experts[e].htoh4(x, torch.tensor([300]))),
+                                     torch.tensor([300])) for e in range(6)]
+        y = torch.stack(rows, 1).gather(1, idx[..., None].expand(-1, -1, 64))     # [T, k, d]
+        dscore = (y.detach().double() * c.double()[:, None]).sum(-1)
+        share = torch.autograd.grad((y * score.detach()[..., None]).sum(1), x, c)[0].double()
+    once = torch.autograd.grad(out, [x, *params], c, create_graph=True)
+    g = torch.autograd.grad(want, ref, dscore, create_graph=True)
+    g = [g[0] + share, *g[1:]]
+    for a, b in zip(once, g):
+        assert (a - b).norm() <= 1e-4 * b.norm()
+    twice = torch.autograd.grad(sum((t ** 2).sum() for t in once), [x, *params])
+    want2 = torch.autograd.grad(sum((t ** 2).sum() for t in g), ref)
+    for a, b in zip(twice, want2):
+        assert b.any() and (a - b).norm() <= 1e-4 * b.norm()
+    plain = torch.autograd.grad(moe(x) if not alone else moe.gate(x)[1], [x, *params], c)
+    for a, b in zip(once, plain):
+        assert (a - b).norm() <= 1e-6 * b.norm()
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_relu_in_the_tiles_of_a_large_product(dt):
     """More than 4 Mi values behind the first layer: ReLU forward and backward inside the
