@@ -98,19 +98,22 @@ __global__ __launch_bounds__(kThreads) void gate_wgrad_kernel(
       b += g;
       const int n = std::min(kWave, (end - base + kWaves - 1) / kWaves);
       for (int q = 0; q < n; q += kRowsInFlight) {
+        // (other lanes' values are read by the whole wave: a lane beyond the last column holds
+        // rows and gradients too, which a branch that leaves it out need not keep)
         Pk p[kRowsInFlight];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u)
-          if (q + u < n && in)
-            p[u] = *reinterpret_cast<const Pk*>(
-                x + (int64_t)__builtin_amdgcn_readlane(tok, q + u) * d + col);
+        for (int u = 0; u < kRowsInFlight; ++u) {
+          const int row = __builtin_amdgcn_readlane(tok, q + u);
+          if (q + u < n && in) p[u] = *reinterpret_cast<const Pk*>(x + (int64_t)row * d + col);
+        }
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u)
+        for (int u = 0; u < kRowsInFlight; ++u) {
+          const acc_t gu = bcast(g, q + u);
           if (q + u < n && in) {
-            const acc_t gu = bcast(g, q + u);
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[v] += gu * Elem<T>::to_acc(p[u].v[v]);
           }
+        }
       }
     }
 #pragma unroll
