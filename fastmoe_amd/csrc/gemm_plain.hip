@@ -820,7 +820,7 @@ int fwd_typed(const GemmArgs& g, hipStream_t s) {
     return fwd_shape(g, kShapesF32, 4) == 0 ? launch_fwd<T, Tile<64, 128, 2, 128>, DMA>(g, s)
                                             : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
   } else if constexpr (DMA == 16) {
-    const bool big = g.tile ? g.tile != 3 : fwd_us(k128, g) <= fwd_us(k64, g);
+    const bool big = g.tile ? g.tile != 3 && g.tile != 5 : fwd_us(k128, g) <= fwd_us(k64, g);
     return big ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
                : launch_fwd<T, Tile<64, 64, 4, 128>, DMA>(g, s);
   } else {
@@ -838,9 +838,8 @@ int bwd_typed(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
                                                  : launch_bwd<T, Small, Small, DMA>(gd, gw, s);
   } else if constexpr (DMA == 16) {
     const int forced = gd.tile ? gd.tile : gw.tile;
-    // (forced, by tests: the shapes for 128 rows are told apart by the parity of the experts)
     const Kind kind = !forced ? bwd_choice(gd, gw)
-                      : forced == 3 ? kMixed : gw.n_expert % 2 ? kTall : k128;
+                      : forced == 3 ? kMixed : forced == 5 ? k64 : forced == 6 ? kTall : k128;
     using Big = Tile<128, 128, 2, 128>;
     if (kind == k128) return launch_bwd<T, Big, Big, DMA>(gd, gw, s);
     // short dW sums: half as deep slices, so that four workgroups fit a CU and their output
@@ -873,6 +872,10 @@ int copy_width(const GemmArgs& g, int dtype) {
   return rows % 4 == 0 && bases % 4 == 0 ? 4 : 0;
 }
 
+// Forced configurations (tests) that are this file's: 128 x 128 tiles; 64 x 64 with 128 x 128
+// ones for dW; 64 x 64 for all; 128 x 128 forward with 128 x 256 backward
+bool forced_plain(int tile) { return tile == 2 || tile == 3 || tile == 5 || tile == 6; }
+
 }  // namespace
 
 bool gemm_plain_supported(const GemmArgs& g, int dtype) {
@@ -884,14 +887,14 @@ bool gemm_plain_supported(const GemmArgs& g, int dtype) {
 
 bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype, double lead) {
   if (dtype == FMOE_F32 || !gemm_plain_supported(g, dtype)) return dtype == FMOE_F32;
-  if (g.tile) return g.tile == 2 || g.tile == 3;   // forced (tests)
+  if (g.tile) return forced_plain(g.tile);
   return std::min(fwd_us(k128, g), fwd_us(k64, g)) < fwd_us(k256, g) + lead;
 }
 
 bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype, double lead) {
   if (dtype == FMOE_F32 || !gemm_plain_supported(gd, dtype) || !gemm_plain_supported(gw, dtype))
     return dtype == FMOE_F32;
-  if (gd.tile) return gd.tile == 2 || gd.tile == 3;
+  if (gd.tile) return forced_plain(gd.tile);
   return bwd_us(bwd_choice(gd, gw), gd, gw) < bwd_us(k256, gd, gw) + lead;
 }
 

@@ -489,11 +489,14 @@ int fmoe_gelu_bwd(const void* dy, const void* x, void* dx, int64_t n,
  * Selects the grouped-GEMM kernel family for the CALLING THREAD's later calls:
  * 0 = automatic (MFMA where the shape allows, tile shape from the library's cost
  * model), 1 = force the scalar kernel, 2..5 = MFMA with bf16/f16 tile
- * configuration 1..4 forced (256x256, 128x256, 128x128, 256x256 with K slices of
- * 64; f32/f64 have one tile shape), 6 = automatic, with the forward activation of
- * fmoe_grouped_linear_fwd_act always as a kernel of its own.  A testing aid with
- * no counterpart in the reference; the setting is thread-local (every thread
- * starts at 0), so concurrent callers do not disturb each other.
+ * configuration 1..4 forced (256x256; 128x128; 64x64, dW 128x128; 256x256 with K
+ * slices of 64; f32 and even feature sizes off the 8-element grid: 1 and 3 their
+ * larger shape, 2 and 4 their smaller one; f64 has one), 6 = automatic, with the
+ * forward activation of fmoe_grouped_linear_fwd_act always as a kernel of its own,
+ * 8 and 9 = configurations 5 (64x64 throughout) and 6 (128x128, backward 128x256).
+ * 7 is refused, as is everything else.  A testing aid with no counterpart in the
+ * reference; the setting is thread-local (every thread starts at 0), so
+ * concurrent callers do not disturb each other.
  */
 int fmoe_set_gemm_path(int path);
 

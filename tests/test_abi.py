@@ -45,6 +45,7 @@ def test_argument_errors_are_reported_not_fatal():
     rc = lib.fmoe_gather_combine_fwd(None, None, None, None, 4, 65, 8, 3, None)
     assert rc == -2
     assert lib.fmoe_set_gemm_path(7) == -1 and lib.fmoe_set_gemm_path(6) == 0
+    assert lib.fmoe_set_gemm_path(10) == -1 and lib.fmoe_set_gemm_path(9) == 0
     assert lib.fmoe_set_gemm_path(0) == 0
 
 

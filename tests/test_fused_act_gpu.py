@@ -243,7 +243,7 @@ def _expert_linear(lib, dtype, counts, in_f, out_f, path):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
-@pytest.mark.parametrize("path", [2, 3, 4, 5])
+@pytest.mark.parametrize("path", [2, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("counts,in_f,out_f", [([300, 0, 257, 64, 1, 200, 513], 136, 264),
                                                ([130, 255, 70], 264, 72), ([513], 264, 1032)])
 def test_relu_inside_every_tile(dt, path, counts, in_f, out_f):

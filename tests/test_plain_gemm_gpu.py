@@ -1,7 +1,7 @@
-"""The plain-pipeline matrix-core GEMMs (f32 of any shape; bf16 / f16 whose feature sizes
-are even but no multiples of 8): every tile shape forced at sizes on and around the edges
-of its tiles and K slices, against float64; the f32 activation inside the tiles against
-the activation kernel, bit for bit."""
+"""The plain-pipeline matrix-core GEMMs (f32 of any shape; bf16 / f16 of even feature
+sizes): every tile shape forced at sizes on and around the edges of its tiles and K
+slices, against float64; the f32 activation inside the tiles against the activation
+kernel, bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -64,6 +64,16 @@ def test_f32_activation_inside_the_tiles(in_f, out_f):
 @pytest.mark.parametrize("counts,in_f,out_f", [([1], 8, 8), ([128, 129, 0, 31, 32], 256, 128),
                                                ([127, 0, 300], 264, 136), ([33, 5, 97], 520, 248)])
 def test_wide_column_tiles(dt, counts, in_f, out_f):
-    """The backward's 128 x 256 tiles (forced for 128-row tiles and an odd number of experts):
-    edges of tiles, of K slices of 32 and of the three stages."""
-    _run(counts, in_f, out_f, DTYPES[dt], True, 3, extra_rows=3)
+    """The backward's 128 x 256 tiles: edges of tiles, of K slices of 32 and of the three
+    stages."""
+    _run(counts, in_f, out_f, DTYPES[dt], True, 9, extra_rows=3)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("path", [3, 4, 8, 9])
+@pytest.mark.parametrize("counts,in_f,out_f", [([1, 1], 8, 8), ([64, 65, 0, 127], 64, 72),
+                                               ([129, 63, 128, 1], 136, 256), ([200], 200, 56)])
+def test_sixteen_bit_rows_of_sixteen_bytes(dt, path, counts, in_f, out_f):
+    """All four kinds of small tiles at the edges of each, with one and with several experts, an
+    odd number of them among others."""
+    _run(counts, in_f, out_f, DTYPES[dt], True, path, extra_rows=3)
