@@ -602,8 +602,6 @@ PYBIND11_MODULE(fmoe_cuda, m) {
   m.def("balance_gate", &balance_gate, py::arg("logits"), py::arg("kind"), py::arg("capacity"));
   m.attr("GATE_GSHARD") = (int)FMOE_GATE_GSHARD;
   m.attr("GATE_SWITCH") = (int)FMOE_GATE_SWITCH;
-  m.attr("ACT_GELU") = (int)FMOE_ACT_GELU;
-  m.attr("ACT_RELU") = (int)FMOE_ACT_RELU;
   m.def("set_gemm_path", &set_gemm_path);
   m.def("_seg_off_from_counts",
         [](Tensor expert_count, py::object device) {

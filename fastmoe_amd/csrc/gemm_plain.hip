@@ -253,11 +253,12 @@ __device__ __forceinline__ float act_bwd(const GemmArgs& g, float d, float pre) 
 __device__ __forceinline__ uint16_t act_fwd16(const GemmArgs& g, uint16_t v) {
   return load_global<uint16_t>(g.act_fwd_table + v);
 }
-template <typename T>
-__device__ __forceinline__ uint16_t act_bwd16(const GemmArgs& g, uint16_t d, uint16_t pre) {
+// (bf16; the derivative behind an f16 product is the activation kernel's)
+__device__ __forceinline__ uint16_t gelu_bwd16(const GemmArgs& g, uint16_t d, uint16_t pre) {
+  using B = __hip_bfloat16;
   const float n = load_global<float>(g.act_table + (pre & 0x7fffu));
-  return __builtin_bit_cast(uint16_t, Elem<T>::from_acc(
-      Elem<T>::to_acc(__builtin_bit_cast(T, d)) * ((pre & 0x8000u) ? n : 1.f - n)));
+  return __builtin_bit_cast(uint16_t, Elem<B>::from_acc(
+      Elem<B>::to_acc(__builtin_bit_cast(B, d)) * ((pre & 0x8000u) ? n : 1.f - n)));
 }
 
 template <typename T, typename S, int MODE, int DMA>
@@ -526,9 +527,9 @@ __device__ __forceinline__ void plain_tile(const GemmArgs& g, char* smem, TileRo
         if (relu) {
 #pragma unroll
           for (int q = 0; q < kUnit; ++q) v.h[q] = relu_bwd16<T>(v.h[q], p.h[q]);
-        } else {
+        } else if constexpr (std::is_same<T, __hip_bfloat16>::value) {
 #pragma unroll
-          for (int q = 0; q < kUnit; ++q) v.h[q] = act_bwd16<T>(g, v.h[q], p.h[q]);
+          for (int q = 0; q < kUnit; ++q) v.h[q] = gelu_bwd16(g, v.h[q], p.h[q]);
         }
       }
       if (!kFwd || g.c) *reinterpret_cast<Unit*>(C + at) = v.u;
