@@ -1,7 +1,7 @@
 """The K loops of the matrix-core GEMM as the compiler emits them: no wait of the
 compiler's own on the memory counter, no accumulator moves, no scratch access (see
 tests/check_mfma_loops.py for why each of them is expensive here).  Needs
-hipcc but no GPU; about a minute and a half."""
+hipcc but no GPU; about three minutes."""
 import os
 import subprocess
 import sys
