@@ -42,6 +42,7 @@ class GShardGate(NaiveGate):
             self.set_loss(loss)
         else:
             topk_idx, topk_val = topk_softmax(logits, self.top_k)
+            topk_idx = topk_idx.view(*logits.shape[:-1], self.top_k)
             top1 = topk_idx.view(-1, self.top_k)[:, 0]
             frac = _histogram(top1, self.tot_expert).to(torch.float) / logits.shape[0]
             prob = F.softmax(logits, dim=1).mean(dim=0)

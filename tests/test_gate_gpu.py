@@ -232,6 +232,22 @@ def test_gate_over_more_experts_than_can_be_routed():
         assert (g - w).norm() <= 1e-5 * w.norm()
 
 
+def test_gshard_indices_keep_the_leading_dimensions():
+    """On a [S, B, d] input the choices come as [S, B, 2], the scores as [S * B, 2], as those of
+    the plain gate."""
+    from fastmoe_amd import GShardGate, NaiveGate
+
+    torch.manual_seed(3)
+    gate = GShardGate(16, 4, 1, capacity=(8.0, 8.0), random_routing=False).cuda()
+    plain = NaiveGate(16, 4, 1, 2).cuda()
+    plain.load_state_dict(gate.state_dict())
+    x = torch.randn(10, 6, 16, device="cuda")
+    idx, score = gate(x)
+    want_idx, want = plain(x)
+    assert idx.shape == (10, 6, 2) and torch.equal(score, want)
+    assert ((idx == want_idx) | (idx == -1)).all() and (idx >= 0).any()
+
+
 @pytest.mark.parametrize("gate", ["GShardGate", "SwitchGate"])
 def test_balance_gates_refuse_another_number_of_outputs(gate):
     """Their loss has one term per expert: a linear map with more outputs is an error, not a
