@@ -30,8 +30,10 @@ def _plain(cls, *modules) -> bool:
     r"""Whether calling any of `modules` runs `cls.forward` and nothing else, so that its
     arithmetic may be done without calling it: a subclass with a `forward` of its own, a
     wrapper and a watched module have to be called."""
-    return all(getattr(type(m), "forward", None) is cls.forward and not _hooked(m)
-               for m in modules)
+    for m in modules:
+        if getattr(type(m), "forward", None) is not cls.forward or _hooked(m):
+            return False
+    return True
 
 
 class FusedExpertLayer(Function):
@@ -146,30 +148,35 @@ class _Expert(nn.Module):
         one 2-d GPU tensor in the parameters' dtype, an activation the library has kernels
         for (ReLU in the extension only) between the two layers, and nobody watching the
         modules inside or giving them another `forward`."""
-        if not (_plain(_Expert, self) and _plain(FMoELinear, self.htoh4, self.h4toh)
-                and not _watched(self.activation)):
+        # (a small layer's time is the host's, so the modules are looked up once each and
+        # past nn.Module.__getattr__: 3 us instead of 7)
+        modules = self.__dict__["_modules"]
+        l1, l2 = modules.get("htoh4"), modules.get("h4toh")
+        act = modules["activation"] if "activation" in modules else self.activation
+        if not _plain(_Expert, self) or not _plain(FMoELinear, l1, l2) or (
+                isinstance(act, nn.Module) and _hooked(act)):
             return False
-        w1, w2 = self.htoh4.weight, self.h4toh.weight
+        w1, w2 = l1.weight, l2.weight
         return (torch.is_tensor(inp) and inp.dim() == 2 and inp.is_cuda
                 and inp.dtype == w1.dtype == w2.dtype and 1 <= top_k <= 64
-                and (is_exact_gelu(self.activation, inp)
-                     or (native_act(self.activation, inp) != 0
-                         and fmoe_cuda.native() is not None and self._keeps_width()
+                and (is_exact_gelu(act, inp)
+                     or (native_act(act, inp) != 0
+                         and fmoe_cuda.native() is not None
+                         and self._native_args(inp) is not None
                          # (parameters kept in another layout are copied on the way, which
                          # only the chain of single operators does)
-                         and all(p is None or p.is_contiguous() for p in
-                                 (w1, self.htoh4.bias, w2, self.h4toh.bias)))))
-
-    def _keeps_width(self) -> bool:
-        r"""Whether the experts' output is as wide as their input, as the extension's layer
-        nodes take it."""
-        return self.h4toh.weight.shape[1] == self.htoh4.weight.shape[2]
+                         and all(p is None or p.is_contiguous()
+                                 for p in (w1, l1.bias, w2, l2.bias)))))
 
     def _native_args(self, inp):
-        r"""The experts' share of a call of the extension's layer nodes."""
+        r"""The experts' share of a call of the extension's layer nodes, which take experts
+        whose output is as wide as their input; None for others."""
         l1, l2 = self.htoh4, self.h4toh
-        params = [p for p in (l1.weight, l1.bias, l2.weight, l2.bias) if p is not None]
-        return (params, l1.num_expert, l1.bias is not None, l2.bias is not None,
+        w1, b1, w2, b2 = l1.weight, l1.bias, l2.weight, l2.bias
+        if w2.shape[1] != w1.shape[2]:
+            return None
+        params = [p for p in (w1, b1, w2, b2) if p is not None]
+        return (params, l1.num_expert, b1 is not None, b2 is not None,
                 native_act(self.activation, inp))
 
     def run_layer(self, inp, gate_idx, score):
@@ -177,8 +184,9 @@ class _Expert(nn.Module):
         as one autograd node: the extension's own, or FusedExpertLayer where a Python node
         is wanted (ctypes binding, per-op profiling) or the output has another width."""
         native = fmoe_cuda.native()
-        if native is not None and self._keeps_width():
-            return native.expert_layer(inp, gate_idx, score, *self._native_args(inp))
+        args = self._native_args(inp) if native is not None else None
+        if args is not None:
+            return native.expert_layer(inp, gate_idx, score, *args)
         return FusedExpertLayer.apply(inp, gate_idx, score, self.htoh4.weight, self.htoh4.bias,
                                       self.h4toh.weight, self.h4toh.bias)
 
@@ -186,12 +194,15 @@ class _Expert(nn.Module):
         r"""The layer with the plain top-k gate `gate` (NaiveGate) in front of it as one
         native autograd node, the gate's zero loss included; None where the gate has to run
         as the module it is.  Only called after can_run_layer()."""
-        native, lin = fmoe_cuda.native(), gate.gate
-        if (native is None or not gate.is_plain(inp) or not self._keeps_width()
-                or lin.weight.shape[0] != self.htoh4.num_expert):
+        native = fmoe_cuda.native()
+        args = self._native_args(inp) if native is not None and gate.is_plain(inp) else None
+        if args is None:
+            return None
+        lin = gate.gate
+        weight = lin.weight
+        if weight.shape[0] != args[1]:
             return None   # (a choice that is none of the experts drops the slot)
-        out, loss = native.gated_layer(inp, lin.weight, lin.bias, *self._native_args(inp),
-                                       gate.top_k)
+        out, loss = native.gated_layer(inp, weight, lin.bias, *args, gate.top_k)
         gate.set_loss(loss)
         return out
 
