@@ -17,6 +17,7 @@
 #include <torch/extension.h>
 
 #include <ATen/core/grad_mode.h>
+#include <c10/core/InferenceMode.h>
 
 namespace {
 
@@ -56,7 +57,9 @@ struct ParamTables {
         need(t.device() == params[0].device(), "expert parameters must share their device");
         need((uintptr_t)t.data_ptr() % 16 == 0, "expert parameters must be 16-byte aligned");
       }
-      // (a new tensor: kernels of an earlier call may still be reading the old one)
+      // (a new tensor: kernels of an earlier call may still be reading the old one; an ordinary
+      // one also under inference mode, as a later training call saves it for its backward)
+      c10::InferenceMode ordinary(false);
       Tensor fresh = torch::empty({4, n_expert}, params[0].options().dtype(at::kLong));
       check(fmoe_pointer_table(now.data(), (int64_t)now.size(), (const void**)fresh.data_ptr(), on),
             "pointer_table");

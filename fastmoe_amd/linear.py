@@ -126,7 +126,8 @@ class ParamTables:
             return None
         key = tuple(t.data_ptr() for t in tensors)
         if self._key.get(name) != key:
-            self._table[name] = fmoe_cuda.pointer_table([t.detach() for t in tensors])
+            with torch.inference_mode(False):   # (a later training call saves the table)
+                self._table[name] = fmoe_cuda.pointer_table([t.detach() for t in tensors])
             self._key[name] = key
         return self._table[name]
 

@@ -472,6 +472,24 @@ def test_experts_in_a_plain_container(container, act):
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
+@pytest.mark.parametrize("watched", [True, False])
+def test_list_layer_trains_after_inference_mode(watched):
+    """The table of the experts' addresses made by a call under inference mode serves a training
+    call as well, through the native node and through the chain."""
+    from fastmoe_amd import fmoe_cuda
+
+    moe, x = _list_layer(), torch.randn(50, 64, device="cuda")
+    fmoe_cuda.profile_hook = (lambda *a: None) if watched else None
+    try:
+        with torch.inference_mode():
+            want = moe(x)
+        out = moe(x)
+        out.sum().backward()
+    finally:
+        fmoe_cuda.profile_hook = None
+    assert torch.equal(out, want) and all(p.grad.any() for p in moe.experts.parameters())
+
+
 def test_list_layer_first_called_under_capture_or_on_another_stream():
     """The table of the experts' addresses is written by the stream that reads it: a graph
     that has not run yet leaves nothing behind for eager calls, nor do calls on one stream
