@@ -671,8 +671,8 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     ctx->set_materialize_grads(false);
     return {kept, score, loss};
   }
-  // The backward as torch operations, for gradients of higher order: the loss reaches
-  // softmax(logits) with one constant per expert, the scores are the softmax of the chosen
+  // The backward as torch operations, for gradients of higher order and for batches of
+  // gradients (torch's vmap over a backward): the loss reaches softmax(logits) with one constant per expert, the scores are the softmax of the chosen
   // logits (GShard) or the chosen values of softmax(logits) (Switch).
   static Tensor differentiable(int64_t kind, const Tensor& logits, const Tensor& coef,
                                const Tensor& idx, const Tensor& dscore, const Tensor& dloss) {
@@ -698,7 +698,10 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     const Tensor dloss = grads[2];
     if (!dscore.defined() && !dloss.defined()) return {Tensor(), Tensor(), Tensor()};
     c10::DeviceGuard guard(logits.device());
-    if (at::GradMode::is_enabled())   // a gradient that will itself be differentiated
+    // (a batch of gradients has no memory of its own)
+    const bool batched = (dscore.defined() && !dscore.has_storage()) ||
+                         (dloss.defined() && !dloss.has_storage());
+    if (at::GradMode::is_enabled() || batched)
       return {differentiable(ctx->saved_data["kind"].toInt(), logits, coef, idx, dscore, dloss),
               Tensor(), Tensor()};
     Tensor dlogits = at::empty_like(logits);

@@ -259,3 +259,24 @@ def test_balance_gates_refuse_another_number_of_outputs(gate):
     layer.gate = torch.nn.Linear(16, 6).cuda()
     with pytest.raises(RuntimeError, match="size"):
         layer(torch.randn(50, 16, device="cuda"))
+
+
+@pytest.mark.parametrize("which", ["score", "loss"])
+def test_batches_of_gradients_through_the_balance_gates(which):
+    """Several gradients at once (is_grads_batched) are those taken one by one, up to the 20 or
+    so roundings of each way to them."""
+    from fastmoe_amd import GShardGate, SwitchGate
+
+    torch.manual_seed(5)
+    gates = [SwitchGate(16, 4, 1).cuda()]
+    if which == "loss":   # (GShard's scores have no batched gradient)
+        gates.append(GShardGate(16, 4, 1, random_routing=False).cuda())
+    for gate in gates:
+        x = torch.randn(50, 16, device="cuda", requires_grad=True)
+        score = gate(x)[1]
+        out = score if which == "score" else gate.get_loss()
+        dy = torch.randn((3,) + out.shape, device="cuda")
+        got = torch.autograd.grad(out, x, dy, is_grads_batched=True, retain_graph=True)[0]
+        for g, d in zip(got, dy):
+            want = torch.autograd.grad(out, x, d, retain_graph=True)[0]
+            assert want.any() and (g - want).norm() <= 20 * torch.finfo(g.dtype).eps * want.norm()
