@@ -6,6 +6,7 @@ import math
 import torch
 import torch.nn as nn
 from torch.autograd import Function
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import fmoe_cuda
 from .functions import SegmentTable, apply_activation
@@ -293,9 +294,12 @@ def is_exact_gelu(activation, x: torch.Tensor) -> bool:
 
 
 def native_act(activation, x: torch.Tensor) -> int:
-    r"""The library's code of `activation` (FMOE_ACT_*), 0 if it has no kernels for it."""
+    r"""The library's code of `activation` (FMOE_ACT_*), 0 if it has no kernels for it, or if it
+    is ReLU and there are hooks on all modules, which see such experts called as modules."""
     if is_exact_gelu(activation, x):
         return 1
+    if _has_any_global_hook():
+        return 0
     if type(activation) is torch.nn.ReLU:
         return 0 if "forward" in activation.__dict__ else 2
     return 2 if activation is torch.relu or activation is torch.nn.functional.relu else 0

@@ -240,6 +240,27 @@ def test_modules_with_another_forward_are_called(fused, act, where, how):
     assert x.grad is not None and x.grad.any()
 
 
+@pytest.mark.parametrize("fused", [True, False])
+def test_hooks_on_all_modules_see_relu_experts(fused):
+    """A hook on every module (as profilers and loggers set) sees the gate's linear map, the
+    activation and, where it holds all experts, the expert module called; the output stays."""
+    from fastmoe_amd import FMoETransformerMLP
+
+    torch.manual_seed(4)
+    moe = FMoETransformerMLP(4, 32, 48, top_k=2, activation=torch.nn.ReLU(), fused=fused).cuda()
+    x, seen = torch.randn(60, 32, device="cuda"), []
+    want = moe(x)
+    hook = torch.nn.modules.module.register_module_forward_hook(lambda m, *_: seen.append(m))
+    try:
+        got = moe(x)
+    finally:
+        hook.remove()
+    called = [moe, moe.gate, moe.gate.gate] + ([moe.experts, moe.experts.activation] if fused
+                                               else [moe.experts[0].activation])
+    assert all(any(m is s for s in seen) for m in called)
+    assert (got - want).norm() <= 65 * torch.finfo(x.dtype).eps * want.norm()
+
+
 def _gate(d, e, k, dtype=torch.float32):
     from fastmoe_amd import NaiveGate
 
