@@ -162,9 +162,9 @@ class _Expert(nn.Module):
                 and (is_exact_gelu(act, inp)
                      or (native_act(act, inp) != 0
                          and fmoe_cuda.native() is not None
-                         and self._native_args(inp) is not None
-                         # (parameters kept in another layout are copied on the way, which
-                         # only the chain of single operators does)
+                         # (an output of another width, and parameters kept in another layout,
+                         # which are copied on the way, are for the chain of single operators)
+                         and w2.shape[1] == w1.shape[2]
                          and all(p is None or p.is_contiguous()
                                  for p in (w1, l1.bias, w2, l2.bias)))))
 
