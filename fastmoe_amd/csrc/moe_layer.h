@@ -321,18 +321,21 @@ void gate_topk(const LayerSizes& s, const Tensor& logits, Tensor& idx, Tensor& s
 // have the bits of the gate module; its gradients come from the top-k slots alone
 // (gate_grad.hip).
 LayerPass layer_forward(const LayerConfig& c, at::TensorList vars, bool train, Tensor* idx_out) {
+  // (a view of the caller's scores is taken where views keep the version of their base: the
+  // backward needs the values, so a change in place before it is an error)
+  Tensor score = c.gated ? Tensor() : vars[2].reshape({vars[0].size(0), c.top_k});
   at::AutoDispatchBelowADInplaceOrView below;
   const Tensor x = vars[0].contiguous();
   c10::DeviceGuard guard(x.device());
   const at::TensorList params = vars.slice(c.gated ? 2 + c.has_bg : 3);
   const LayerSizes s = layer_sizes(c, x, params);
-  Tensor idx, score;
+  Tensor idx;
   if (c.gated) {
     gate_topk(s, at::linear(x, vars[1], c.has_bg ? OptTensor(vars[2]) : OptTensor()), idx, score,
               c.zero_loss);
   } else {
     idx = vars[1];
-    score = vars[2].reshape({s.t, s.k}).contiguous().to(x.scalar_type());
+    score = score.contiguous().to(x.scalar_type());
   }
   LayerPass p = experts_forward(c, s, expert_params(c, params), x, idx, score, train);
   if (idx_out) *idx_out = idx;

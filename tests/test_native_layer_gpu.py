@@ -68,10 +68,10 @@ def test_native_node_matches_the_chain(dt, top_k, bias, frozen):
         if g is None or not (name == "x" or name.startswith("gate.")):
             assert g is None or torch.equal(g, w)
         else:
-            # the chain rounds the logits' gradient, the gate's share of dx and the experts'
-            # share of dx to the storage type (half an eps each) before it adds them up, this
-            # node the result alone: 2 eps of the gradient's size; f32 sums in another order
-            # differ by less than the 130 terms times 2^-24, i.e. 65 eps
+            # the chain rounds the logits' gradient to the storage type, which this node keeps
+            # in the accumulation type; both round the gate's share of dx, the experts' share
+            # and their sum (half an eps each): 2 eps of the gradient's size; f32 sums in
+            # another order differ by less than the 130 terms times 2^-24, i.e. 65 eps
             eps = torch.finfo(g.dtype).eps
             bound = (2 if dt == "bf16" else 65) * eps
             assert (g - w).double().norm() <= bound * w.double().norm(), name
@@ -369,6 +369,24 @@ def _list_layer():
 
     torch.manual_seed(5)
     return FMoETransformerMLP(4, 64, 96, top_k=2, fused=False).cuda()
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("shape", [(70, 2), (140,)])
+def test_scores_may_not_change_before_the_backward(fused, shape):
+    """The gradients need the scores that the forward used, so changing a user's gate's scores in
+    place between the two is an error, whatever shape they come in."""
+    from fastmoe_amd import FMoETransformerMLP
+
+    moe = FMoETransformerMLP(6, 64, 96, top_k=2, fused=fused).cuda()
+    idx = torch.randint(0, 6, (70, 2), device="cuda")
+    score = torch.rand(shape, device="cuda", requires_grad=True) * 1
+    moe.gate.forward = lambda x: (idx, score)
+    out = moe(torch.randn(70, 64, device="cuda"))
+    with torch.no_grad():
+        score.mul_(2)
+    with pytest.raises(RuntimeError, match="inplace"):
+        out.sum().backward()
 
 
 def test_list_layer_copies_and_pickles_after_a_call():
