@@ -571,6 +571,7 @@ std::tuple<Tensor, Tensor> gated_layer(const Tensor& inp, const Tensor& wg, cons
 std::tuple<Tensor, Tensor> limit_gate(const Tensor& gate_in, int64_t n_expert, int64_t capacity) {
   const Tensor gate = gate_in.contiguous();
   dev(gate, "gate", at::kLong);
+  need(capacity == (int32_t)capacity, "capacity exceeds the range of int32");
   c10::DeviceGuard guard(gate.device());
   Tensor count = at::empty({n_expert}, gate.options()), out = at::empty_like(gate);
   Tensor ws = workspace(gate.numel(), n_expert, gate);
@@ -675,8 +676,9 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     return {kept, score, loss};
   }
   // The backward as torch operations, for gradients of higher order and for batches of
-  // gradients (torch's vmap over a backward): the loss reaches softmax(logits) with one constant per expert, the scores are the softmax of the chosen
-  // logits (GShard) or the chosen values of softmax(logits) (Switch).
+  // gradients (torch's vmap over a backward): the loss reaches softmax(logits) with one
+  // constant per expert, the scores are the softmax of the chosen logits (GShard) or the
+  // chosen values of softmax(logits) (Switch).
   static Tensor differentiable(int64_t kind, const Tensor& logits, const Tensor& coef,
                                const Tensor& idx, const Tensor& dscore, const Tensor& dloss) {
     const Tensor x = logits.to(at::kFloat), p = at::softmax(x, -1);

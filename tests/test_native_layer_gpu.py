@@ -154,6 +154,21 @@ def test_limit_gate_matches_count_limit_prune(n, e, cap):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("cap", [2 ** 31, -2 ** 31 - 1])
+def test_capacity_is_a_number_of_32_bits(cap):
+    """Any other is refused: by the helper and, where it comes from the rate, by the gates."""
+    from fastmoe_amd import GShardGate, SwitchGate
+    from fastmoe_amd.gates import limit_by_capacity
+
+    with pytest.raises(RuntimeError):
+        limit_by_capacity(torch.zeros(8, 1, dtype=torch.int64, device="cuda"), 4, 1, cap)
+    x = torch.randn(8, 16, device="cuda")
+    for gate in (GShardGate(16, 4, 1), SwitchGate(16, 4, 1)):
+        gate.capacity = (cap, cap)
+        with pytest.raises(RuntimeError):
+            gate.cuda()(x)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
 @pytest.mark.parametrize("kind,k", [("GATE_GSHARD", 2), ("GATE_SWITCH", 1)])
 @pytest.mark.parametrize("t,e", [(1, 2), (33, 16), (500, 17), (300, 64), (700, 65), (9000, 129),
