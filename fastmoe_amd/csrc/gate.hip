@@ -710,8 +710,8 @@ extern "C" int fmoe_balance_gate_bwd(const void* logits, const float* coef, cons
                                      int dtype, void* stream) {
   int rc = check_balance("balance_gate_bwd", n_tokens, n_expert, kind, dtype);
   if (rc) return rc;
-  FMOE_REQUIRE(logits && coef && score && idx && dlogits, FMOE_ERR_INVALID,
-               "balance_gate_bwd: null pointer");
+  FMOE_REQUIRE(logits && coef && (score || kind == GATE_SWITCH) && idx && dlogits,
+               FMOE_ERR_INVALID, "balance_gate_bwd: null pointer");
   hipStream_t s = (hipStream_t)stream;
   FMOE_BALANCE_DISPATCH(launch_balance_bwd, logits, coef, dloss, dscore, score, idx, dlogits,
                         n_tokens, n_expert, s);

@@ -669,7 +669,8 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
                                 dt(logits, "logits"), stream_of(logits)),
           "balance_gate_fwd");
     Tensor kept = std::get<1>(limit_gate(idx, e, capacity));
-    ctx->save_for_backward({logits, coef, score, idx});
+    // (Switch's gradient does not need the score, which its caller may then write in place)
+    ctx->save_for_backward({logits, coef, kind == FMOE_GATE_GSHARD ? score : Tensor(), idx});
     ctx->saved_data["kind"] = kind;
     ctx->mark_non_differentiable({kept});
     ctx->set_materialize_grads(false);
@@ -712,7 +713,7 @@ struct BalanceGateNode : public torch::autograd::Function<BalanceGateNode> {
     Tensor dlogits = at::empty_like(logits);
     check(fmoe_balance_gate_bwd(logits.data_ptr(), coef.data_ptr<float>(),
                                 dloss.defined() ? dloss.data_ptr<float>() : nullptr,
-                                dscore.defined() ? dscore.data_ptr() : nullptr, score.data_ptr(),
+                                dscore.defined() ? dscore.data_ptr() : nullptr, out_ptr(score),
                                 idx.data_ptr<int64_t>(), dlogits.data_ptr(), logits.size(0),
                                 (int32_t)logits.size(1), (int)ctx->saved_data["kind"].toInt(),
                                 dt(logits, "logits"), stream_of(logits)),

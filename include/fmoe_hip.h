@@ -425,7 +425,7 @@ int64_t fmoe_balance_gate_workspace_bytes(int32_t n_expert);
 int fmoe_balance_gate_fwd(const void* logits, int64_t n_tokens, int32_t n_expert, int kind,
                           int64_t capacity, int64_t* idx, void* score, float* loss, float* coef,
                           void* workspace, int64_t workspace_bytes, int dtype, void* stream);
-/* dlogits of both outputs; dloss (float[1]) or dscore may be NULL. */
+/* dlogits of both outputs; dloss (float[1]) or dscore may be NULL, Switch's score as well. */
 int fmoe_balance_gate_bwd(const void* logits, const float* coef, const float* dloss,
                           const void* dscore, const void* score, const int64_t* idx,
                           void* dlogits, int64_t n_tokens, int32_t n_expert, int kind, int dtype,

@@ -422,6 +422,26 @@ def test_list_layer_copies_and_pickles_after_a_call():
         assert not other(x).any() and torch.equal(moe(x), want)
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_switch_score_may_change_before_the_backward(dt):
+    """Its gradient depends on the logits alone, so a caller may scale the score in place: the
+    gradients are those of a scaled copy."""
+    from fastmoe_amd import SwitchGate
+
+    torch.manual_seed(5)
+    gate = SwitchGate(16, 4, 1).to(DTYPES[dt]).cuda().eval()
+    x = torch.randn(40, 16, device="cuda", dtype=DTYPES[dt])
+
+    def grads(in_place):
+        _, score = gate(x)
+        score = score.mul_(2) if in_place else score * 2
+        return torch.autograd.grad(score.float().square().sum() + gate.get_loss(),
+                                   list(gate.parameters()))
+
+    for a, b in zip(grads(True), grads(False)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("name", ["htoh4.weight", "htoh4.bias", "h4toh.weight", "h4toh.bias"])
 def test_relu_experts_with_parameters_in_another_layout(name):
     """A parameter whose memory is not in [E, out, in] order: the same values and gradients, up
