@@ -5,9 +5,9 @@
 // that torch makes of it leave most of the chip idle (few experts: 16384 tokens, 4096
 // features, 8 experts ran on 64 workgroups) and cost four launches with the bias: 80 + 12 + 5
 // us there, 86 + 15 + 5 for 8192 tokens, 2048 features, 128 experts, top-8.  Together with the
-// gate's share of dx (dispatch.hip) a step went from 18997 to 18353 us and from 3543 to 3356 us
-// (boxes differ by 2 %: 1.2 and 2.2 % within one run), 1000 tokens of 300 features from 252 to
-// 210 us, 512 of 128 from 248 to 213 us.
+// gate's share of dx (dispatch.hip) a step of these two takes 1.2 and 2.2 % less (both sides in
+// turn, within one run), one of 1000 tokens of 300 features 210 us instead of 252, of 512 of 128
+// 213 instead of 248.
 #include <algorithm>
 
 #include "common.h"

@@ -1,15 +1,18 @@
 // Grouped GEMM on the matrix cores for what the 256-row bf16/f16 kernels
-// (gemm_mfma_impl.h) do not take: f32 of any shape, and bf16/f16 whose feature sizes
-// are even but no multiples of 8 (rows then start on 4-byte boundaries).
+// (gemm_mfma_impl.h) do not take, f32 of any shape and bf16/f16 whose feature sizes are
+// even but no multiples of 8 (rows then start on 4-byte boundaries), and for bf16/f16 on
+// 16-byte rows where the estimate at the end finds smaller tiles faster (few rows per
+// expert, few tiles).
 //
 // One pipeline for all of them.  A workgroup of 4 waves (2 x 2) computes a BM x BN tile;
-// a K slice is 128 BYTES of every operand row (32 values of f32, 64 of bf16/f16), two LDS
-// stages of it alternate, copied by `buffer_load ... lds` (16 or 4 bytes per lane,
-// no staging registers), with one wait and one barrier per slice.  There is no
-// interleaving plan as in the 256-row kernels: f32 MFMAs are 16 times slower, so one
-// slice of a 64 x 128 tile is 2048 cycles of them per SIMD, and three or four workgroups per
-// CU cover each other's barriers; with 4-byte copies (dword-aligned rows) the CU's address
-// unit bounds the kernel (a quarter of a KiB per 20 cycles).
+// a K slice is 128 BYTES of every operand row (32 values of f32, 64 of bf16/f16), or 64
+// where that lets more workgroups share a CU; two to four LDS stages of it take turns,
+// copied by `buffer_load ... lds` (16 or 4 bytes per lane, no staging registers), with one
+// wait and one barrier per slice.  There is no interleaving plan as in the 256-row kernels:
+// f32 MFMAs are 16 times slower, so one slice of a 64 x 128 tile is 2048 cycles of them per
+// SIMD, and two to four workgroups per CU cover each other's barriers; with 4-byte copies
+// (dword-aligned rows) the CU's address unit bounds the kernel (a quarter of a KiB per 20
+// cycles).
 //
 // Both operand layouts are kept in LDS as they come:
 //   K-contiguous rows  [row][128 bytes], 16-byte packs XORed by row bits;
@@ -717,7 +720,8 @@ int bwd_shape(const GemmArgs& gd, const GemmArgs& gw, const Shape (&shapes)[2], 
 //           128, 16376, 2048 -> 1408           469  513  511   446
 //             8, 16620, 1664 -> 3328           355  377  474   370
 //             4, 24620, 1600 -> 6400           960 1030 1404  1050
-// Over 38 such launches the choice takes 1.3 % longer than the best of the four.
+// The constants come from 38 such launches.  How much longer than the best of the five kinds
+// the chosen one takes has not been measured since the 128 x 256 tiles came.
 enum Kind { k256, k128, k64, kMixed, kTall };
 
 struct Spread {   // rows of an expert: three equally spaced points and their weights
@@ -843,14 +847,14 @@ int bwd_typed(const GemmArgs& gd, const GemmArgs& gw, hipStream_t s) {
                       : forced == 3 ? kMixed : forced == 5 ? k64 : forced == 6 ? kTall : k128;
     using Big = Tile<128, 128, 2, 128>;
     if (kind == k128) return launch_bwd<T, Big, Big, DMA>(gd, gw, s);
-    // short dW sums: half as deep slices, so that four workgroups fit a CU and their output
-    // stores (which bound such products) overlap
     // Experts of some hundred rows: dW tiles that are half output.  Twice the columns of the
     // 128 x 128 tile in three stages of half slices load a quarter less per product, and the
     // two workgroups of a CU store and multiply at the same time, which the one of the
     // 256-row kernels cannot.
     using Tall = Tile<128, 256, 3, 64>;
     if (kind == kTall) return launch_bwd<T, Tall, Tall, DMA>(gd, gw, s);
+    // short dW sums: half as deep slices, so that four workgroups fit a CU and their output
+    // stores (which bound such products) overlap
     if (kind == kMixed)
       return launch_bwd<T, Tile<64, 64, 2, 128>, Tile<128, 128, 2, 64>, DMA>(gd, gw, s);
     return launch_bwd<T, Tile<64, 64, 3, 128>, Tile<64, 64, 3, 128>, DMA>(gd, gw, s);
