@@ -819,13 +819,46 @@ Kind bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
   return best;
 }
 
+// Forward product of few rows per expert (decode steps, many experts): the weights' way from
+// HBM bounds it, and a tile higher than the experts spends copies, LDS reads and matrix
+// instructions on rows that are not there.  32 x 64 tiles in three stages, four workgroups to
+// a CU, while experts hold 32 rows (what random routing spreads around the average included);
+// 64 x 128 in three stages in place of 128 x 128 while they hold 64.  Measured, us (256-row
+// kernels, 128 x 128, 64 x 64 and these):
+//    16 experts,   64 rows, 1024 -> 4096     25   24   25     22.4
+//     8,  128, 4096 -> 14336                183  170  167    162
+//     8,  128, 14336 -> 4096                167  218  159    160
+//    64,  512, 2048 -> 4096                 252  254  247    227
+//   128,  256, 1408 -> 2048                 141  129  122    117
+//   128, 2048, 1024 -> 2048                 115  108  115    100
+//    64, 2560, 1024 -> 2048                  53   49   52     47.6
+//    64, 2560, 2048 -> 1024                  47   44   47     43.6
+//    32, 1920, 2688 -> 768                   39   33   29     27.5
+// (Weights that stay in the last-level cache between launches, as in that table, hide one
+// thing: with at most one 32 x 64 tile for each of the 256 CUs, three stages are too few bytes
+// under way to HBM.  Six there: an inference pass of 32 tokens, 1024 -> 4096, 16 experts, top-2
+// takes 67.4 us with the other tiles, 68.6 with three stages and 65.4 with six; with 320 to 512
+// tiles three are 1 % of a pass ahead.)
+// At 100 rows per expert the 64 x 128 tiles are behind (32, 3200, 2048 -> 4096: 145 against 152).
+enum Low { kLow32, kLow64, kNotLow };
+Low low_rows(const GemmArgs& g) {
+  const double most = Spread(g).rows[2];
+  return most <= 32 ? kLow32 : most <= 64 ? kLow64 : kNotLow;
+}
+
 template <typename T, int DMA>
 int fwd_typed(const GemmArgs& g, hipStream_t s) {
   if constexpr (std::is_same<T, float>::value) {
     return fwd_shape(g, kShapesF32, 4) == 0 ? launch_fwd<T, Tile<64, 128, 2, 128>, DMA>(g, s)
                                             : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
   } else if constexpr (DMA == 16) {
+    const Low low = g.tile ? kNotLow : low_rows(g);
+    if (low == kLow32)
+      return (int64_t)g.n_expert * ceil_div(g.out_feat, 64) <= 256
+                 ? launch_fwd<T, Tile<32, 64, 6, 128>, DMA>(g, s)
+                 : launch_fwd<T, Tile<32, 64, 3, 128>, DMA>(g, s);
     const bool big = g.tile ? g.tile != 3 && g.tile != 5 : fwd_us(k128, g) <= fwd_us(k64, g);
+    if (big && low == kLow64) return launch_fwd<T, Tile<64, 128, 3, 128>, DMA>(g, s);
     return big ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
                : launch_fwd<T, Tile<64, 64, 4, 128>, DMA>(g, s);
   } else {
@@ -893,7 +926,14 @@ bool gemm_plain_supported(const GemmArgs& g, int dtype) {
 bool gemm_plain_fwd_preferred(const GemmArgs& g, int dtype, double lead) {
   if (dtype == FMOE_F32 || !gemm_plain_supported(g, dtype)) return dtype == FMOE_F32;
   if (g.tile) return forced_plain(g.tile);
-  return std::min(fwd_us(k128, g), fwd_us(k64, g)) < fwd_us(k256, g) + lead;
+  const double plain = std::min(fwd_us(k128, g), fwd_us(k64, g)), wide = fwd_us(k256, g) + lead;
+  // few rows: where the estimates meet at the time HBM needs, the lower tiles come closer to it
+  // (copies of 4 bytes have none)
+  if (copy_width(g, dtype) == 16) {
+    const Low low = low_rows(g);
+    if (low != kNotLow) return low == kLow32 || plain <= wide;
+  }
+  return plain < wide;
 }
 
 bool gemm_plain_bwd_preferred(const GemmArgs& gd, const GemmArgs& gw, int dtype, double lead) {

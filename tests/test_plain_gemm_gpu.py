@@ -77,3 +77,16 @@ def test_sixteen_bit_rows_of_sixteen_bytes(dt, path, counts, in_f, out_f):
     """All four kinds of small tiles at the edges of each, with one and with several experts, an
     odd number of them among others."""
     _run(counts, in_f, out_f, DTYPES[dt], True, path, extra_rows=3)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("counts,in_f,out_f", [([1], 8, 8), ([32, 33, 0, 31, 1], 136, 72),
+                                               ([0, 0, 150, 0, 0, 0, 2, 1], 264, 128),
+                                               ([65, 63, 0, 64, 1, 33], 136, 264),
+                                               ([0, 0, 300, 3, 0, 0], 520, 136),
+                                               ([3, 0, 40, 1, 9], 200, 3328)])
+def test_tiles_of_few_rows_per_expert(dt, counts, in_f, out_f):
+    """The forward's 32- and 64-row tiles, which the average number of rows chooses: edges of
+    tiles, of K slices of 64 and of the stages (six with up to 256 tiles, three beyond), and
+    experts far above the average."""
+    _run(counts, in_f, out_f, DTYPES[dt], True, 0, extra_rows=3)
