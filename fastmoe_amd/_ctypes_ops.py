@@ -687,7 +687,7 @@ def init(device=None) -> None:
 
 def set_gemm_path(path: int) -> None:
     """0 = matrix-core kernel where the shape allows (tile shape chosen by the
-    library), 1 = scalar kernel only, 2..5 and 8, 9 = matrix-core kernel with bf16/f16
-    tile configuration 1..4 and 5, 6 forced, 6 = automatic with the forward activation as
-    a kernel of its own (for tests; the setting belongs to the calling thread)."""
+    library), 1 = scalar kernel only, 2..5, 8, 9 and 11, 12 = matrix-core kernel with
+    bf16/f16 tile configuration 1..4, 5, 6 and 7, 8 forced, 6 = automatic with the forward
+    activation as a kernel of its own (for tests; the setting belongs to the calling thread)."""
     _lib.check(_L.fmoe_set_gemm_path(path), "set_gemm_path")

@@ -232,14 +232,15 @@ extern "C" int fmoe_init(void* stream) {
 }
 
 extern "C" int fmoe_set_gemm_path(int path) {
-  FMOE_REQUIRE(path >= 0 && path <= 9 && path != 7, FMOE_ERR_INVALID,
-               "gemm path must be 0..6, 8 or 9");
+  FMOE_REQUIRE(path >= 0 && path <= 12 && path != 7 && path != 10, FMOE_ERR_INVALID,
+               "gemm path must be 0..6, 8, 9, 11 or 12");
   // 2..5: tile configuration 1..4 forced (16-bit types: 256 rows; 128; 64 with 128-row dW; 256
   // with K slices of 64 in two stages; f32 and odd feature sizes: their larger, smaller shape);
   // 6: automatic, but the forward activation runs as a kernel of its own behind the GEMM;
   // 8, 9: configurations 5 and 6 (16-bit types: 64 rows throughout; 128 x 256 backward)
+  // 11, 12: configurations 7 and 8 (16-bit types: forward tiles of few rows, 32 x 64, 64 x 128)
   g_gemm_path = path == 1 ? 1 : 0;
-  g_tile = path >= 2 && path <= 5 ? path - 1 : path >= 8 ? path - 3 : 0;
+  g_tile = path >= 2 && path <= 5 ? path - 1 : path >= 11 ? path - 4 : path >= 8 ? path - 3 : 0;
   g_fuse_fwd_act = path != 6;
   return FMOE_OK;
 }

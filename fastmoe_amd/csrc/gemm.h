@@ -35,7 +35,7 @@ struct GemmArgs {
   int in_feat;
   int out_feat;
   int n_expert;
-  int tile;             // 0 = choose the tile shape automatically, 1..6 = force one
+  int tile;             // 0 = choose the tile shape automatically, 1..8 = force one
   // DGRAD, where the kernel takes it: if not null, dx = (dy W) * act'(act_pre) with act_pre
   // [n_rows, in_feat] the pre-activations behind the layer's input (ReLU: or the activations),
   // and act_table (16-bit GELU) the device table of gelu'(-|x|) (gelu_bwd_table()).

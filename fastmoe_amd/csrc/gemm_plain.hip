@@ -852,7 +852,7 @@ int fwd_typed(const GemmArgs& g, hipStream_t s) {
     return fwd_shape(g, kShapesF32, 4) == 0 ? launch_fwd<T, Tile<64, 128, 2, 128>, DMA>(g, s)
                                             : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
   } else if constexpr (DMA == 16) {
-    const Low low = g.tile ? kNotLow : low_rows(g);
+    const Low low = g.tile == 7 ? kLow32 : g.tile == 8 ? kLow64 : g.tile ? kNotLow : low_rows(g);
     if (low == kLow32)
       return (int64_t)g.n_expert * ceil_div(g.out_feat, 64) <= 256
                  ? launch_fwd<T, Tile<32, 64, 6, 128>, DMA>(g, s)
@@ -911,8 +911,9 @@ int copy_width(const GemmArgs& g, int dtype) {
 }
 
 // Forced configurations (tests) that are this file's: 128 x 128 tiles; 64 x 64 with 128 x 128
-// ones for dW; 64 x 64 for all; 128 x 128 forward with 128 x 256 backward
-bool forced_plain(int tile) { return tile == 2 || tile == 3 || tile == 5 || tile == 6; }
+// ones for dW; 64 x 64 for all; 128 x 128 forward with 128 x 256 backward; the forward tiles of
+// few rows, 32 x 64 and 64 x 128, with 128 x 128 backward
+bool forced_plain(int tile) { return tile == 2 || tile == 3 || tile >= 5; }
 
 }  // namespace
 

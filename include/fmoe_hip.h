@@ -493,8 +493,9 @@ int fmoe_gelu_bwd(const void* dy, const void* x, void* dx, int64_t n,
  * slices of 64; f32 and even feature sizes off the 8-element grid: 1 and 3 their
  * larger shape, 2 and 4 their smaller one; f64 has one), 6 = automatic, with the
  * forward activation of fmoe_grouped_linear_fwd_act always as a kernel of its own,
- * 8 and 9 = configurations 5 (64x64 throughout) and 6 (128x128, backward 128x256).
- * 7 is refused, as is everything else.  A testing aid with no counterpart in the
+ * 8 and 9 = configurations 5 (64x64 throughout) and 6 (128x128, backward 128x256),
+ * 11 and 12 = configurations 7 and 8 (forward tiles of few rows, 32x64 and 64x128;
+ * backward 128x128).  7 and 10 are refused, as is everything else.  A testing aid with no counterpart in the
  * reference; the setting is thread-local (every thread starts at 0), so
  * concurrent callers do not disturb each other.
  */

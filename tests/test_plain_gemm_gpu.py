@@ -84,9 +84,55 @@ def test_sixteen_bit_rows_of_sixteen_bytes(dt, path, counts, in_f, out_f):
                                                ([0, 0, 150, 0, 0, 0, 2, 1], 264, 128),
                                                ([65, 63, 0, 64, 1, 33], 136, 264),
                                                ([0, 0, 300, 3, 0, 0], 520, 136),
-                                               ([3, 0, 40, 1, 9], 200, 3328)])
+                                               ([3, 0, 40, 1, 9], 200, 3328),
+                                               ([40, 64, 0, 33, 65, 38] * 85, 64, 136)])
 def test_tiles_of_few_rows_per_expert(dt, counts, in_f, out_f):
-    """The forward's 32- and 64-row tiles, which the average number of rows chooses: edges of
-    tiles, of K slices of 64 and of the stages (six with up to 256 tiles, three beyond), and
-    experts far above the average."""
+    """The forward as the average number of rows chooses it, experts far above the average among
+    them: 32 x 64 tiles, 64 x 64 ones for few tiles (the fourth and fifth), 64 x 128 ones for many
+    (the last); each kind at its edges is below."""
     _run(counts, in_f, out_f, DTYPES[dt], True, 0, extra_rows=3)
+
+
+def _bits(t):
+    return t.view(torch.int16)
+
+
+# rows at the edges of 32, 64 and 128, columns at those of 64 and 128, and K slices of 64 from one
+# to more than twice round a ring of six stages, with and without a tail
+LOW_TILES = [([1], 8, 8), ([32, 33, 0, 31, 1], 384, 72), ([64, 65, 0, 63, 2], 392, 128),
+             ([128, 129, 0, 127, 30], 776, 136), ([0, 0, 300, 3, 96, 97], 1032, 264),
+             ([3, 0, 40, 1, 9], 448, 3328)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("path", [11, 12])
+@pytest.mark.parametrize("counts,in_f,out_f", LOW_TILES)
+def test_every_tile_of_few_rows(dt, path, counts, in_f, out_f):
+    """Forward tiles of few rows against float64 and, bit for bit, against the 128 x 128 ones:
+    with and without a bias, weights behind pointer tables, both activations, and a ReLU whose
+    argument is not kept."""
+    from fastmoe_amd import _lib, fmoe_cuda
+    from test_fused_act_gpu import _expert_linear
+
+    dtype = DTYPES[dt]
+    for with_bias in (True, False):
+        _run(counts, in_f, out_f, dtype, with_bias, path, extra_rows=3)
+    n, e = sum(counts), len(counts)
+    seg = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    x, w, b = (randn(s, dtype, i, 0.3).cuda()
+               for i, s in enumerate([(n + 3, in_f), (e, out_f, in_f), (e, out_f)]))
+    got = {}
+    for p in (path, 3):
+        fmoe_cuda.set_gemm_path(p)
+        try:
+            y, a = fmoe_cuda.grouped_linear_fwd(x, seg, w, b, with_gelu=True)
+            apart = [[t[i:i + 1].clone() for i in range(e)] for t in (w, b)]
+            z = fmoe_cuda.grouped_linear_fwd_ptrs(x, seg, *map(fmoe_cuda.pointer_table, apart),
+                                                  out_f)
+            relu = _expert_linear(_lib.load(), dtype, counts, in_f, out_f, p)[1]
+            got[p] = [y[:n], a[:n], fmoe_cuda.grouped_linear_fwd(x, seg, w, None)[:n],
+                      relu(2, True)[1], relu(2, False)[1]]
+            assert torch.equal(_bits(z[:n]), _bits(y[:n]))
+        finally:
+            fmoe_cuda.set_gemm_path(0)
+    assert all(torch.equal(_bits(g), _bits(h)) for g, h in zip(got[path], got[3]))
