@@ -19,8 +19,11 @@ EPILOGUE, never to the loop itself):
 
 The script compiles the files to assembly for gfx950 (of gemm_mfma_impl.h the bf16
 kernels only unless --all-dtypes: about 3 instead of 5 minutes), finds every loop with
-at least 8 MFMAs and fewer than 700 lines, and reports the three counts; exit status 1
-if any is not zero.  A `flat_load` anywhere in a kernel of the files is reported as well.
+at least 4 MFMAs (a slice of the smallest tile, 32 x 64) and fewer than 700 lines, and
+reports the three counts; exit status 1 if any is not zero.  A kernel whose MFMAs lie outside
+all of these loops was not checked and is reported too: any at all in gemm_plain.hip, where
+every one belongs to a K loop, and a kernel without a loop in gemm_mfma_impl.h.  So is a
+`flat_load` anywhere in a kernel of the files.
 """
 from __future__ import annotations
 
@@ -68,10 +71,11 @@ def compile_to_assembly(out_path: str, all_dtypes: bool) -> None:
 
 def scan(asm_text: str):
     """([(kernel, [(mfmas, lines, compiler_vmcnt_waits, accvgpr_moves, scratch_ops)])],
-    {kernel: flat loads anywhere in its body})"""
+    {kernel: flat loads anywhere in its body}, {kernel: MFMAs that no loop accounts for})"""
     lines = asm_text.split("\n")
     out = []
     flat = {}
+    unseen = {}
     for start in (i for i, l in enumerate(lines) if re.match(r"^_ZN4fmoe\S+:", l)):
         name = lines[start].split(":")[0]
         end = next((i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end")),
@@ -88,13 +92,14 @@ def scan(asm_text: str):
             if m:
                 labels[m.group(1)] = i
         loops = []
+        outside = {i for i, x in enumerate(body) if "v_mfma" in x}
         for i, l in enumerate(body):
             m = re.search(r"s_c?branch\w*\s+(\.LBB\d+_\d+)", l)
             if not (m and m.group(1) in labels and labels[m.group(1)] < i):
                 continue
             block = body[labels[m.group(1)]:i + 1]
             mfmas = sum(1 for x in block if "v_mfma" in x)
-            if mfmas < 8 or len(block) >= 700:
+            if mfmas < 4 or len(block) >= 700:
                 continue
             in_asm = False
             waits = moves = scratch = 0
@@ -108,9 +113,12 @@ def scan(asm_text: str):
                 moves += "v_accvgpr" in x
                 scratch += "scratch_" in x
             loops.append((mfmas, len(block), waits, moves, scratch))
+            outside -= set(range(labels[m.group(1)], i))
         if loops:
             out.append((name, loops))
-    return out, flat
+        if outside and ("plain_" in name or not loops):
+            unseen[name] = len(outside)
+    return out, flat, unseen
 
 
 def main() -> int:
@@ -131,7 +139,7 @@ def main() -> int:
         finally:
             if not args.keep and os.path.exists(path):
                 os.remove(path)
-    found, flat = scan(text)
+    found, flat, unseen = scan(text)
     bad = 0
     # The activation epilogues index an LDS table with an offset that may lie outside
     # the table (the result is then recomputed): harmless as an LDS read, a wild global
@@ -139,6 +147,9 @@ def main() -> int:
     for name, n in flat.items():
         print("%s: %d flat_load instructions (LDS / global pointers must keep their "
               "address spaces)" % (name[:80], n))
+        bad += n
+    for name, n in unseen.items():
+        print("%s: %d MFMAs outside the loops that were checked" % (name[:100], n))
         bad += n
     for name, loops in found:
         short = re.sub(r"_ZN4fmoe\d+", "", name).replace("14__hip_bfloat16", "bf16")
