@@ -1522,7 +1522,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs g,
         g, smem, {e, m_tile * BM, row0, g.seg_off[e + 1] - row0}, n_tile);
     return;
   }
-  RowTiles<BM, kSmall, NW> rows;
+  RowTiles<BM, kSmall ? kRemainder : kOneHeight, NW> rows;
   rows.scan(g.seg_off, g.n_expert, s_wave_sum);
   constexpr int kF = kSmall ? narrow_factor<BM, BN, MODE>() : 1;
   const int wide_s = rows.rows_s * tiles_n;
@@ -1564,7 +1564,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_bwd_kernel(GemmArgs gd, Gem
   extern __shared__ __attribute__((aligned(1024))) uint16_t smem[];
   __shared__ int s_owner[4], s_wave_sum[2 * NW];
 
-  RowTiles<BM, kSmall, NW> rows;
+  RowTiles<BM, kSmall ? kRemainder : kOneHeight, NW> rows;
   rows.scan(gd.seg_off, gd.n_expert, s_wave_sum);
   constexpr int kF = kSmall ? narrow_factor<BM, BN, DMODE>() : 1;
   const bool narrow = kF > 1 && rows.rows_s * tiles_n_d <= kNarrowMax &&

@@ -6,7 +6,7 @@
 //
 // One pipeline for all of them.  A workgroup of 4 waves (2 x 2) computes a BM x BN tile;
 // a K slice is 128 BYTES of every operand row (32 values of f32, 64 of bf16/f16), or 64
-// where that lets more workgroups share a CU; two to four LDS stages of it take turns,
+// where that lets more workgroups share a CU; two to six LDS stages of it take turns,
 // copied by `buffer_load ... lds` (16 or 4 bytes per lane, no staging registers), with one
 // wait and one barrier per slice.  There is no interleaving plan as in the 256-row kernels:
 // f32 MFMAs are 16 times slower, so one slice of a 64 x 128 tile is 2048 cycles of them per
@@ -32,6 +32,7 @@
 //
 // Tile shape: the cost model and the measurements at the end.
 #include <algorithm>
+#include <climits>
 
 #include "act_math.h"
 #include "dma_desc.h"
@@ -557,7 +558,7 @@ __global__ __launch_bounds__(kThreads, (workgroups_per_cu(S::kLds))) void plain_
     GemmArgs g, int tiles_n) {
   extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
   __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
-  RowTiles<S::BM, false, kWaves> rows;
+  RowTiles<S::BM, kOneHeight, kWaves> rows;
   rows.scan(g.seg_off, g.n_expert, s_wave_sum);
   const int live = rows.rows_f * tiles_n;
   if (live == 0) return;
@@ -569,6 +570,42 @@ __global__ __launch_bounds__(kThreads, (workgroups_per_cu(S::kLds))) void plain_
   plain_tile<T, S, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * S::BN);
 }
 
+// Forward product of few rows per expert on average, cut by the rows that each expert really
+// has: tiles Low, but tiles High for experts of more than kFewRows rows where these fill the
+// chip.  Low tiles of a long expert copy its weights into LDS again and again; while there are
+// fewer High tiles than CUs, though, the wait for memory counts and not the copies, and Low
+// tiles spread it wider.  Measured: see low_rows().
+constexpr int kFewRows = 64, kCus = 256;
+template <typename T, typename Low, typename High, int DMA>
+__global__ __launch_bounds__(kThreads, (workgroups_per_cu(std::max(Low::kLds, High::kLds)))) void
+plain_fwd_few_kernel(GemmArgs g, int tiles_n_low, int tiles_n_high) {
+  extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
+  __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
+  RowTiles<High::BM, kTwoHeights, kWaves, Low::BM> rows;
+  rows.low_most = kFewRows;
+  rows.scan(g.seg_off, g.n_expert, s_wave_sum);
+  if (rows.rows_f > 0 && rows.rows_f * tiles_n_high < kCus) {
+    rows.low_most = INT_MAX;
+    __syncthreads();   // the sums of the first scan have been read
+    rows.scan(g.seg_off, g.n_expert, s_wave_sum);
+  }
+  const int live_high = rows.rows_f * tiles_n_high;
+  const int live = live_high + rows.rows_s * tiles_n_low;
+  if (live == 0) return;
+  const int t = tile_number(blockIdx.x, live);
+  if (t >= live) return;
+  int v, n_tile;
+  if (t < live_high) {
+    tile_order(t, rows.rows_f, tiles_n_high, v, n_tile);
+    const TileRows where = rows.find(g.seg_off, v, false, s_owner);
+    plain_tile<T, High, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * High::BN);
+  } else {
+    tile_order(t - live_high, rows.rows_s, tiles_n_low, v, n_tile);
+    const TileRows where = rows.find(g.seg_off, v, true, s_owner);
+    plain_tile<T, Low, GEMM_FWD, DMA>(g, plain_smem, where, n_tile * Low::BN);
+  }
+}
+
 // dX (tiles D) and dW with the bias gradient (tiles W) in one launch, dX tiles first;
 // either may be absent (no tiles).
 template <typename T, typename D, typename W, int DMA>
@@ -576,7 +613,7 @@ __global__ __launch_bounds__(kThreads, (workgroups_per_cu(std::max(D::kLds, W::k
 plain_bwd_kernel(GemmArgs gd, GemmArgs gw, int tiles_n_d, int tiles_n_w, int tiles_m_w) {
   extern __shared__ __attribute__((aligned(1024))) char plain_smem[];
   __shared__ int s_owner[4], s_wave_sum[2 * kWaves];
-  RowTiles<D::BM, false, kWaves> rows;
+  RowTiles<D::BM, kOneHeight, kWaves> rows;
   rows.scan(gd.seg_off, gd.n_expert, s_wave_sum);
   const int live_d = rows.rows_f * tiles_n_d;
   const int per_expert_w = tiles_n_w * tiles_m_w;
@@ -616,6 +653,23 @@ int launch_fwd(const GemmArgs& g, hipStream_t s) {
   const int rc = round_up_blocks(tiles_n * (g.n_rows / S::BM + (int64_t)g.n_expert), &blocks);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), S::kLds, s, g, tiles_n);
+  FMOE_LAUNCH_CHECK("gemm_plain");
+  return FMOE_OK;
+}
+
+template <typename T, typename Low, typename High, int DMA>
+int launch_fwd_few(const GemmArgs& g, hipStream_t s) {
+  static_assert(Low::BM <= High::BM && Low::BN <= High::BN, "Low must be the smaller tile");
+  constexpr size_t lds = std::max(Low::kLds, High::kLds);
+  auto kern = plain_fwd_few_kernel<T, Low, High, DMA>;
+  FMOE_SET_DYNAMIC_LDS_ONCE(kern, lds);
+  const int tiles_n_low = ceil_div(g.out_feat, Low::BN);
+  const int tiles_n_high = ceil_div(g.out_feat, High::BN);
+  unsigned blocks = 0;
+  // (an expert in High tiles has no more of them than it would have of Low ones)
+  const int rc = round_up_blocks(tiles_n_low * (g.n_rows / Low::BM + (int64_t)g.n_expert), &blocks);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds, s, g, tiles_n_low, tiles_n_high);
   FMOE_LAUNCH_CHECK("gemm_plain");
   return FMOE_OK;
 }
@@ -823,8 +877,8 @@ Kind bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
 // HBM bounds it, and a tile higher than the experts spends copies, LDS reads and matrix
 // instructions on rows that are not there.  32 x 64 tiles in three stages, four workgroups to
 // a CU, while experts hold 32 rows (what random routing spreads around the average included);
-// 64 x 128 in three stages in place of 128 x 128 while they hold 64.  Measured, us (256-row
-// kernels, 128 x 128, 64 x 64 and these):
+// 64 x 128 in three stages in place of 128 x 128 while they hold 64.  Measured, us, routing
+// near uniform (256-row kernels, 128 x 128, 64 x 64 and these):
 //    16 experts,   64 rows, 1024 -> 4096     25   24   25     22.4
 //     8,  128, 4096 -> 14336                183  170  167    162
 //     8,  128, 14336 -> 4096                167  218  159    160
@@ -833,13 +887,28 @@ Kind bwd_choice(const GemmArgs& gd, const GemmArgs& gw) {
 //   128, 2048, 1024 -> 2048                 115  108  115    100
 //    64, 2560, 1024 -> 2048                  53   49   52     47.6
 //    64, 2560, 2048 -> 1024                  47   44   47     43.6
-//    32, 1920, 2688 -> 768                   39   33   29     27.5
-// (Weights that stay in the last-level cache between launches, as in that table, hide one
-// thing: with at most one 32 x 64 tile for each of the 256 CUs, three stages are too few bytes
-// under way to HBM.  Six there: an inference pass of 32 tokens, 1024 -> 4096, 16 experts, top-2
-// takes 67.4 us with the other tiles, 68.6 with three stages and 65.4 with six; with 320 to 512
-// tiles three are 1 % of a pass ahead.)
 // At 100 rows per expert the 64 x 128 tiles are behind (32, 3200, 2048 -> 4096: 145 against 152).
+//
+// With at most one 32 x 64 tile for each of the 256 CUs, three stages are too few bytes under way
+// to HBM: six there.  (Weights from HBM each time, us, three stages and six: 16 experts, 64 rows,
+// 4096 -> 1024 33.0 and 31.1; 8, 100, 2048 -> 1408 16.4 and 13.8; 32, 200, 3072 -> 512 23.6 and
+// 21.1; with more tiles 24, 200, 2048 -> 768 21.4 and 25.0; 16, 256, 4096 -> 2048 62.6 and 77.6.)
+//
+// The host knows the average only.  Experts far above it are cut on the device
+// (plain_fwd_few_kernel), into 64 x 64 and 128 x 128 tiles.  Skewed loads, weights from HBM each
+// time, us: the choice before there were tiles for few rows, those tiles for all experts, as
+// it is.  (Popularity p_e ~ e^-1.2; all rows on two experts; on one.)
+//    64 experts, 1024 rows, 4096 -> 14336    1302 1353 1289    130 261 193    93 240 170
+//   128, 3400, 2048 -> 1408                   164  166  168     45  51  43    44  50  42
+//    64,  512, 2048 -> 4096                   225  165  175     45  31  22    43  23  19
+//   128, 2048, 1024 -> 2048                   111  108  111     27  30  26    27  25  20
+//     8,  128, 4096 -> 14336                  205  166  166     53  64  53    27  39  34
+//     8,  128, 14336 -> 4096                  187  203  202     68  72  72    67  60  60
+//    32, 1280, 4096 -> 4096                   284  239  228     80  75  63    77  72  62
+//   128, 6000, 1408 -> 2048                   187  178  174     37  54  46    37  52  45
+// Left behind: experts of 33 to 64 rows in two 32-row tiles where K is long (the sixth), and
+// wide products with all rows on one or two of many experts, which the 256-row kernels run
+// faster still; these take a seventh to a third of what the call takes under a uniform load.
 enum Low { kLow32, kLow64, kNotLow };
 Low low_rows(const GemmArgs& g) {
   const double most = Spread(g).rows[2];
@@ -853,14 +922,14 @@ int fwd_typed(const GemmArgs& g, hipStream_t s) {
                                             : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);
   } else if constexpr (DMA == 16) {
     const Low low = g.tile == 7 ? kLow32 : g.tile == 8 ? kLow64 : g.tile ? kNotLow : low_rows(g);
+    using Big = Tile<128, 128, 2, 128>;
     if (low == kLow32)
-      return (int64_t)g.n_expert * ceil_div(g.out_feat, 64) <= 256
+      return (int64_t)g.n_expert * ceil_div(g.out_feat, 64) <= kCus
                  ? launch_fwd<T, Tile<32, 64, 6, 128>, DMA>(g, s)
-                 : launch_fwd<T, Tile<32, 64, 3, 128>, DMA>(g, s);
+                 : launch_fwd_few<T, Tile<32, 64, 3, 128>, Tile<64, 64, 2, 128>, DMA>(g, s);
     const bool big = g.tile ? g.tile != 3 && g.tile != 5 : fwd_us(k128, g) <= fwd_us(k64, g);
-    if (big && low == kLow64) return launch_fwd<T, Tile<64, 128, 3, 128>, DMA>(g, s);
-    return big ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
-               : launch_fwd<T, Tile<64, 64, 4, 128>, DMA>(g, s);
+    if (low == kLow64 && big) return launch_fwd_few<T, Tile<64, 128, 3, 128>, Big, DMA>(g, s);
+    return big ? launch_fwd<T, Big, DMA>(g, s) : launch_fwd<T, Tile<64, 64, 4, 128>, DMA>(g, s);
   } else {
     return fwd_shape(g, kShapes16, 2) == 0 ? launch_fwd<T, Tile<128, 128, 2, 128>, DMA>(g, s)
                                            : launch_fwd<T, Tile<64, 64, 2, 128>, DMA>(g, s);

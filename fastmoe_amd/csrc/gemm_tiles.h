@@ -53,16 +53,26 @@ constexpr int kSmallRows = 64;
 constexpr int kSmallBK = 32;
 constexpr int kSmallStages = 6;
 
-// How expert rows are cut into tiles: `full` tiles of BM rows from row 0 on
+// How expert rows are cut into tiles.
+// kOneHeight: tiles of BM rows.
+// kRemainder: `full` tiles of BM rows from row 0 on
 // and, for a remainder of at most BM / 2 rows, one remainder tile (`small` is
 // 0 or 1) of 64 rows, or of 128 rows when the remainder is longer than 64;
 // a remainder above BM / 2 rows takes one more BM tile.  Remainder tiles cost
 // about 0.45 (64 rows) and 0.6 (128 rows) of a 256-row tile.
-template <int BM, bool SMALL>
-__device__ __forceinline__ void cut_rows(int cnt, int& full, int& small) {
-  if (!SMALL) {
-    full = (cnt + BM - 1) / BM;
-    small = 0;
+// kTwoHeights: an expert of up to `low_most` rows in `small` tiles of LOW rows, a longer one
+// in tiles of BM rows.
+enum Cut { kOneHeight, kRemainder, kTwoHeights };
+template <int BM, Cut CUT, int LOW>
+__device__ __forceinline__ void cut_rows(int cnt, int low_most, int& full, int& small) {
+  full = (cnt + BM - 1) / BM;
+  small = 0;
+  if (CUT == kOneHeight) return;
+  if (CUT == kTwoHeights) {
+    if (cnt <= low_most) {
+      full = 0;
+      small = (cnt + LOW - 1) / LOW;
+    }
     return;
   }
   full = cnt / BM;
@@ -103,7 +113,7 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
 }
 
 // Row tiles of a ragged product.  The BM-row tiles of all experts are numbered
-// first, one expert after the other, the remainder tiles behind them.
+// first, one expert after the other, the remainder (or lower) tiles behind them.
 //
 // Up to 64 experts: lane x of EVERY wave cuts the rows of expert x and a wave
 // scan turns the counts into first-tile numbers, so no LDS and no barrier are
@@ -111,14 +121,15 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
 // thread cuts the rows of a contiguous run of experts, the scan runs over the
 // whole block through LDS, and the thread whose run contains a given row tile
 // walks the run to find its owner.
-template <int BM, bool SMALL, int NW>
+template <int BM, Cut CUT, int NW, int LOW = BM>
 struct RowTiles {
   bool by_lane;            // the up-to-64-experts scheme
   int x_lo, x_hi;          // this thread's run of experts
-  int mine_f, mine_s;      // BM-row / remainder tiles in the run
+  int mine_f, mine_s;      // BM-row / small tiles in the run
   int first_f, first_s;    // number of the run's first tile of either kind
   int rows_f, rows_s;      // totals over all experts
   int my_row0, my_cnt;     // by_lane: the expert of this lane
+  int low_most = BM;       // kTwoHeights: rows of the longest expert in small tiles
 
   // May contain a __syncthreads(); s_wave_sum has 2 * NW entries.
   __device__ __forceinline__ void scan(const int32_t* seg_off, int n_expert, int* s_wave_sum) {
@@ -132,7 +143,7 @@ struct RowTiles {
       if (lane < n_expert) {
         my_row0 = seg_off[lane];
         my_cnt = seg_off[lane + 1] - my_row0;
-        cut_rows<BM, SMALL>(my_cnt, mine_f, mine_s);
+        cut_rows<BM, CUT, LOW>(my_cnt, low_most, mine_f, mine_s);
       }
     } else {
       const int per_thread = (n_expert + NW * 64 - 1) / (NW * 64);
@@ -140,14 +151,14 @@ struct RowTiles {
       x_hi = min(x_lo + per_thread, n_expert);
       for (int x = x_lo; x < x_hi; ++x) {
         int f, sm;
-        cut_rows<BM, SMALL>(seg_off[x + 1] - seg_off[x], f, sm);
+        cut_rows<BM, CUT, LOW>(seg_off[x + 1] - seg_off[x], low_most, f, sm);
         mine_f += f;
         mine_s += sm;
       }
     }
     // inclusive scans inside the wave
     const int incl_f = wave_inclusive_sum(mine_f);
-    const int incl_s = SMALL ? wave_inclusive_sum(mine_s) : 0;
+    const int incl_s = CUT != kOneHeight ? wave_inclusive_sum(mine_s) : 0;
     first_f = incl_f - mine_f;
     first_s = incl_s - mine_s;
     if (by_lane) {
@@ -173,7 +184,13 @@ struct RowTiles {
     }
   }
 
-  // Owner of row tile v (of the remainder kind if `small`), v below the total
+  // First row of an expert's tile `i` of its kind, behind `full` BM-row ones.
+  static __device__ __forceinline__ int first_row(int i, int full, bool small) {
+    if (CUT == kTwoHeights) return i * (small ? LOW : BM);
+    return (small ? full : i) * BM;
+  }
+
+  // Owner of row tile v (of the small kind if `small`), v below the total
   // of its kind.  s_out has 4 entries; may contain a __syncthreads().
   __device__ __forceinline__ TileRows find(const int32_t* seg_off, int v, bool small,
                                            int* s_out) const {
@@ -185,7 +202,7 @@ struct RowTiles {
       const int at = __builtin_amdgcn_readlane(first, owner);
       const int f = __builtin_amdgcn_readlane(mine_f, owner);
       t.e = owner;
-      t.m0 = small ? f * BM : (v - at) * BM;
+      t.m0 = first_row(v - at, f, small);
       t.row0 = __builtin_amdgcn_readlane(my_row0, owner);
       t.cnt = __builtin_amdgcn_readlane(my_cnt, owner);
       return t;
@@ -195,11 +212,11 @@ struct RowTiles {
       for (int x = x_lo; x < x_hi; ++x) {
         const int r0 = seg_off[x], c = seg_off[x + 1] - r0;
         int f, sm;
-        cut_rows<BM, SMALL>(c, f, sm);
+        cut_rows<BM, CUT, LOW>(c, low_most, f, sm);
         const int tx = small ? sm : f;
         if (v < at + tx) {
           s_out[0] = x;
-          s_out[1] = small ? f * BM : (v - at) * BM;
+          s_out[1] = first_row(v - at, f, small);
           s_out[2] = r0;
           s_out[3] = c;
           break;

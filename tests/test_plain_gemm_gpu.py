@@ -101,7 +101,10 @@ def _bits(t):
 # to more than twice round a ring of six stages, with and without a tail
 LOW_TILES = [([1], 8, 8), ([32, 33, 0, 31, 1], 384, 72), ([64, 65, 0, 63, 2], 392, 128),
              ([128, 129, 0, 127, 30], 776, 136), ([0, 0, 300, 3, 96, 97], 1032, 264),
-             ([3, 0, 40, 1, 9], 448, 3328)]
+             ([3, 0, 40, 1, 9], 448, 3328),
+             # long experts: few tiles of them, and enough to be cut higher; also above 64 experts
+             ([70, 1, 20, 33, 0], 136, 3464), ([70, 1, 200, 33, 0], 136, 11016),
+             ([0, 1, 33, 130, 96] * 14, 72, 200), ([0, 1, 33, 130, 96] * 14, 72, 808)]
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
@@ -136,3 +139,31 @@ def test_every_tile_of_few_rows(dt, path, counts, in_f, out_f):
         finally:
             fmoe_cuda.set_gemm_path(0)
     assert all(torch.equal(_bits(g), _bits(h)) for g, h in zip(got[path], got[3]))
+
+
+def test_all_rows_on_one_of_many_experts():
+    """The choice of tiles sees the average number of rows, 16 here; an expert that holds all of
+    them is cut into higher tiles.  Tiles of 128 rows, which know no average, are the measure
+    (129 us where tiles of 32 rows took 250; 1.3 times that is the expectation)."""
+    from fastmoe_amd import fmoe_cuda
+
+    e, n, in_f, out_f = 64, 1024, 4096, 14336
+    w = randn((1, 112, 8), torch.bfloat16, 1, 0.02).cuda().repeat(1, out_f // 112, in_f // 8)
+    x = randn((n, in_f), torch.bfloat16, 2).cuda()
+    seg = torch.tensor([0] * 21 + [n] * (e + 1 - 21), dtype=torch.int32).cuda()
+    table = fmoe_cuda.pointer_table([w] * e)
+    best = {0: float("inf"), 3: float("inf")}
+    for _ in range(6):
+        for path in best:
+            fmoe_cuda.set_gemm_path(path)
+            try:
+                start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                start.record()
+                for _ in range(10):
+                    fmoe_cuda.grouped_linear_fwd_ptrs(x, seg, table, None, out_f)
+                end.record()
+                end.synchronize()
+            finally:
+                fmoe_cuda.set_gemm_path(0)
+            best[path] = min(best[path], start.elapsed_time(end))
+    assert best[0] <= 1.6 * best[3], best
