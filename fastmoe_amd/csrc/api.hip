@@ -296,8 +296,9 @@ static int linear_fwd(const char* who, const void* x, const void* w, const void*
   GemmArgs g{x, w, y ? y : y_act, bias, seg_off, n_rows, (int)in_feat, (int)out_feat, (int)n_expert, g_tile};
   g.w_table = w_table;
   g.bias_table = bias_table;
-  // the tiles that leave the activation to its kernel pay for that in the choice: 32 tokens
-  // through 16 experts, 1024 -> 4096, are level without it (25 us) and 31 to 25 us with it
+  // the tiles that leave the activation to its kernel pay for that in the choice: 800 rows
+  // through 8 experts, 2048 -> 1024, are level in the estimate without it (and 64 x 64 tiles take
+  // 15.3 us, 256-row ones 19.6) and 16.5 to 25.1 us with a GELU
   double lead = 0;
   if (act) {
     const double us = act_kernel_us(n_rows * out_feat, 2);
